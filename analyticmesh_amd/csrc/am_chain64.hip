@@ -24,6 +24,7 @@
 #include "am_device.h"
 #include "am_kernels.h"
 #include "am_walk.h"
+#include "am_near.h"
 
 namespace am {
 
@@ -555,7 +556,7 @@ __device__ __forceinline__ void chain_tile_half(const NetDev& net, const ChainIO
 }
 
 __global__ __launch_bounds__(AM_CHAIN_THREADS) void k_chain_tile_fp64(NetDev net, ChainIO io) {
-  if (io.zero && blockIdx.x == 0 && threadIdx.x == 0) *io.zero = 0;
+  if (io.zero && blockIdx.x == 0 && threadIdx.x < 2) io.zero[threadIdx.x] = 0;
   const int r0 = blockIdx.x * AM_CT;
   const int cnt = launch_count(io);
   if (r0 >= cnt) return;
@@ -564,7 +565,7 @@ __global__ __launch_bounds__(AM_CHAIN_THREADS) void k_chain_tile_fp64(NetDev net
 }
 
 __global__ __launch_bounds__(AM_HALF_THREADS) void k_chain_tile_mfma(NetDev net, ChainIO io) {
-  if (io.zero && blockIdx.x == 0 && threadIdx.x == 0) *io.zero = 0;
+  if (io.zero && blockIdx.x == 0 && threadIdx.x < 2) io.zero[threadIdx.x] = 0;
   const int r0 = blockIdx.x * AM_HT;
   const int cnt = launch_count(io);
   if (r0 >= cnt) return;
@@ -693,30 +694,83 @@ __device__ __forceinline__ void walk_ray64_body(const NetDev& net, const RegionI
 }
 
 // NW waves per region (the records do not depend on NW: every reduction breaks
-// ties by constraint index and each serial step runs on one wave).
-// With `left` (the counter zeroed before the launch), a region the walk
-// leaves undecided puts its chunk-local slot on the candidate scan's list and
-// counts itself and its reasons in left.run (as k_collect_slots would).
+// ties by constraint index and each serial step runs on one wave).  A region
+// the walk leaves undecided goes on the candidate scan's list (its counter
+// zeroed before) and counts itself and its reasons in left.run (as
+// k_collect_slots would).
 template <int NW>
 __global__ __launch_bounds__(64 * NW, 24 / NW) void k_walk_ray64(NetDev net, RegionIO io, int rid0, WalkParams wp,
                                                         const double* planes, const double* eqb, int Cs_hbm,
-                                                        int only_undecided, SlotList left) {
-  if ((int)blockIdx.x >= launch_count(io)) return;
-  const int rid = io.ids ? io.ids[blockIdx.x] : rid0 + blockIdx.x;
-  // a region an earlier walk decided keeps its records (its flag is 0 and stays 0)
-  if (only_undecided && !(io.flags[rid - io.first] & AM_UNDECIDED)) return;
-  walk_ray64_body<NW>(net, io, rid, blockIdx.x, wp, planes, eqb, Cs_hbm);
-  // thread 0 wrote the region's flag (finish_region)
-  if (left.cnt && threadIdx.x == 0) {
-    const unsigned f = io.flags[rid - io.first];
-    if (f & AM_UNDECIDED) {
-      left.slots[atomicAdd(left.cnt, 1)] = (int)blockIdx.x;
-      atomicAdd(left.run, 1);
-      for (int w = 0; w < AM_WHY_COUNT; ++w)
-        if (f & AM_WHY_BIT(w)) atomicAdd(left.run + 1 + w, 1);
+                                                        NearList list, SlotList left) {
+  const int total = min(*list.cnt, io.count);
+  for (int i = blockIdx.x; i < total; i += gridDim.x) {
+    const int b = list.slots[i];
+    const int rid = io.ids ? io.ids[b] : rid0 + b;
+    walk_ray64_body<NW>(net, io, rid, b, wp, planes, eqb, Cs_hbm);
+    // thread 0 wrote the region's flag (finish_region)
+    if (threadIdx.x == 0) {
+      const unsigned f = io.flags[rid - io.first];
+      if (f & AM_UNDECIDED) {
+        left.slots[atomicAdd(left.cnt, 1)] = b;
+        atomicAdd(left.run, 1);
+        for (int w = 0; w < AM_WHY_COUNT; ++w)
+          if (f & AM_WHY_BIT(w)) atomicAdd(left.run + 1 + w, 1);
+      }
     }
+    __syncthreads();   // this region's LDS is free for the next
   }
 }
+
+// One region's planes as the tiled chain stores them (plane64), for the near walk.
+struct TilePlanes {
+  const double* src;
+  int Cs, n1;
+  const double* W0;
+  const double* b0;
+  const uint32_t* mask;
+  int C;
+  // the constraints in two parts: hidden layer 1's, rebuilt from its weights, and the others
+  __device__ __forceinline__ int parts() const { return 2; }
+  __device__ __forceinline__ int first(int l) const { return l ? n1 : 0; }
+  __device__ __forceinline__ int size(int l) const { return l ? C - n1 : n1; }
+  __device__ __forceinline__ double err(int) const { return 0.0; }
+  __device__ __forceinline__ void load(int l, int j, double* p) const {
+    if (l == 0) {
+      const uint32_t sm = mbit(mask, j) ? 0x80000000u : 0u;
+      const double v[4] = {W0[j * 3 + 0], W0[j * 3 + 1], W0[j * 3 + 2], b0[j]};
+      for (int q = 0; q < 4; ++q) p[q] = flip_sign(v[q], sm);
+    } else {
+      for (int q = 0; q < 4; ++q) p[q] = src[(size_t)q * Cs + n1 + j];
+    }
+  }
+  __device__ __forceinline__ void get(int g, double* p) const { load(g < n1 ? 0 : 1, g < n1 ? g : g - n1, p); }
+};
+
+template <bool SCAN>
+__global__ __launch_bounds__(64) void k_near64(NetDev net, RegionIO io, int rid0, WalkParams wp, const double* planes,
+                                               const double* eqb, int Cs_hbm, int only_undecided, NearList left) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int b = blockIdx.x;
+  if (b >= launch_count(io)) return;
+  const int rid = io.ids ? io.ids[b] : rid0 + b;
+  // a region an earlier walk decided keeps its records (its flag is 0 and stays 0)
+  if (only_undecided && !(io.flags[rid - io.first] & AM_UNDECIDED)) return;
+  const NearLds<double> S = carve_near<double>(smem_raw, net.C, net.Wd, net.vm, false);
+  const int start = io.reg_start[rid];
+  for (int w = threadIdx.x; w < net.Wd; w += 64) S.mask[w] = io.reg_mask[(size_t)rid * net.Wd + w];
+  double p[3], eq[4];
+  for (int q = 0; q < 3; ++q) p[q] = io.reg_point[(size_t)rid * 3 + q];
+  for (int q = 0; q < 4; ++q) eq[q] = eqb[(size_t)b * 4 + q];
+  __syncthreads();
+  const TilePlanes P{planes + (size_t)b * 4 * Cs_hbm, Cs_hbm, net.nodes[1], net.W0, net.b[0], S.mask, net.C};
+  const bool done = near_or_full_walk<double, SCAN>(net, io, wp, rid, rid - io.first, P, S, eq, p, start);
+  // (thread 0 wrote the flag in finish_region: the orientation may be undecided)
+  if (threadIdx.x == 0 && (!done || (!SCAN && (io.flags[rid - io.first] & AM_UNDECIDED)))) near_left(left, b);
+}
+template __global__ void k_near64<true>(NetDev, RegionIO, int, WalkParams, const double*, const double*, int, int,
+                                        NearList);
+template __global__ void k_near64<false>(NetDev, RegionIO, int, WalkParams, const double*, const double*, int, int,
+                                         NearList);
 
 template <int NW>
 __global__ __launch_bounds__(64 * NW, 24 / NW) void k_walk_ray64_multi(const NetDev* nets, RegionIO io, int Wd, int rid0,
@@ -727,11 +781,11 @@ __global__ __launch_bounds__(64 * NW, 24 / NW) void k_walk_ray64_multi(const Net
   walk_ray64_body<NW>(nets[region_net(io, Wd, rid)], io, rid, blockIdx.x, wp, planes, eqb, Cs_hbm);
 }
 
-template __global__ void k_walk_ray64<2>(NetDev, RegionIO, int, WalkParams, const double*, const double*, int, int,
+template __global__ void k_walk_ray64<2>(NetDev, RegionIO, int, WalkParams, const double*, const double*, int, NearList,
                                          SlotList);
-template __global__ void k_walk_ray64<4>(NetDev, RegionIO, int, WalkParams, const double*, const double*, int, int,
+template __global__ void k_walk_ray64<4>(NetDev, RegionIO, int, WalkParams, const double*, const double*, int, NearList,
                                          SlotList);
-template __global__ void k_walk_ray64<8>(NetDev, RegionIO, int, WalkParams, const double*, const double*, int, int,
+template __global__ void k_walk_ray64<8>(NetDev, RegionIO, int, WalkParams, const double*, const double*, int, NearList,
                                          SlotList);
 template __global__ void k_walk_ray64_multi<2>(const NetDev*, RegionIO, int, int, WalkParams, const double*,
                                                const double*, int);

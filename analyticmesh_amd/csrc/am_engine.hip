@@ -28,6 +28,7 @@
 #include "am_adjoint.h"
 #include "am_newton.h"
 #include "am_combine.h"
+#include "am_near.h"
 #include "am_scan.h"
 
 using namespace am;
@@ -536,23 +537,25 @@ ChainIO chain_io(const am_ctx* c, const int* ids, int first, int n, int Ch) {
   return cio;
 }
 
-// The FP64 ray walk with the context's waves per region.
-void launch_ray64(am_ctx* c, int n, size_t lds, const RegionIO& io, int rid0, int Ch, int only_undecided,
-                  const WalkParams& kRay64, const SlotList& left = SlotList{}) {
+// The FP64 ray walk over all constraints of the listed regions, with the
+// context's waves per region (a grid that strides over the list).
+void launch_ray64(am_ctx* c, int n, size_t lds, const RegionIO& io, int rid0, int Ch, const WalkParams& kRay64,
+                  const NearList& list, const SlotList& left) {
   const double* P = c->tplanes.p;
   const double* E = c->teq.p;
+  n = std::min(n, c->scan_blocks);
   switch (c->ray_waves) {
     case 2:
       hipLaunchKernelGGL(k_walk_ray64<2>, dim3(n), dim3(128), lds, c->stream, c->net, io, rid0, kRay64, P, E, Ch,
-                         only_undecided, left);
+                         list, left);
       break;
     case 8:
       hipLaunchKernelGGL(k_walk_ray64<8>, dim3(n), dim3(512), lds, c->stream, c->net, io, rid0, kRay64, P, E, Ch,
-                         only_undecided, left);
+                         list, left);
       break;
     default:
       hipLaunchKernelGGL(k_walk_ray64<4>, dim3(n), dim3(256), lds, c->stream, c->net, io, rid0, kRay64, P, E, Ch,
-                         only_undecided, left);
+                         list, left);
   }
 }
 
@@ -572,8 +575,8 @@ size_t fp64_prepare(am_ctx* c, int count) {
   const size_t cap = std::min<size_t>(chunk, (size_t)count);
   ensure(c->tplanes, cap * 4 * Ch, false, c->stream);
   ensure(c->teq, cap * 4, false, c->stream);
-  ensure(c->tslots, cap, false, c->stream);
-  ensure(c->tcnt, 1, false, c->stream);
+  ensure(c->tslots, 2 * cap, false, c->stream);   // the near walk's leavings, then the ray walk's
+  ensure(c->tcnt, 2, false, c->stream);
   return chunk;
 }
 
@@ -603,15 +606,18 @@ void run_fp64_regions(am_ctx* c, int lvl_first, int first, int count, const int*
   // FP32 form's Newton modes leave none)
   const WalkParams& rw = c->fast.wp;
   const bool vert64 = rw.lam_v < 0.f || (rw.lam_v > 0.f && !rw.vsel);
-  // the FP64 ray walk lists what it leaves undecided for the candidate scan
-  // itself (the chain zeroes the list's counter)
-  const bool fused = mode == 1;
+  // the near walk lists the regions it leaves to the walk over all constraints,
+  // the ray walk those it leaves to the candidate scan (the chain zeroes both
+  // counters)
+  const size_t nlds = near_lds_bytes(c->C, c->Wd, c->vm, 8, false);
+  const NearList near{c->tcnt.p, c->tslots.p};
+  const size_t lcap = std::min<size_t>(chunk, (size_t)count);
   for (int off = 0; off < count; off += (int)chunk) {
     const int n = std::min<int>((int)chunk, count - off);
     ChainIO cio = chain_io(c, ids ? ids + off : nullptr, first + off, n, Ch);
     cio.dcount = dcount;
     cio.dbase = off;
-    if (fused) cio.zero = c->tcnt.p;
+    cio.zero = c->tcnt.p;
     RegionIO io;
     io.reg_mask = c->reg_mask.p;
     io.reg_start = c->reg_start.p;
@@ -656,16 +662,23 @@ void run_fp64_regions(am_ctx* c, int lvl_first, int first, int count, const int*
     }
     if (after_walk && undecided == 0) continue;
     if (mode == 0 && !after_walk) {
-      hipLaunchKernelGGL(k_walk_fp64, dim3(n), dim3(64), wlds, c->stream, c->net, io, first + off, (const int*)nullptr,
-                         (const int*)nullptr, (const double*)c->tplanes.p, (const double*)c->teq.p, Ch);
+      hipLaunchKernelGGL(k_near64<true>, dim3(n), dim3(64), nlds, c->stream, c->net, io, first + off, kRay64,
+                         (const double*)c->tplanes.p, (const double*)c->teq.p, Ch, 0, near);
+      hipLaunchKernelGGL(k_walk_fp64, dim3(std::min(n, c->scan_blocks)), dim3(64), wlds, c->stream, c->net, io,
+                         first + off, (const int*)near.cnt, (const int*)near.slots, (const double*)c->tplanes.p,
+                         (const double*)c->teq.p, Ch);
       HIPCHK(hipGetLastError());
       tm.span(m1, tm.mark(c->stream), T_SCAN64);
       t.scanned_host += n;
       continue;
     }
     if (mode == 1) {
-      launch_ray64(c, n, rlds, io, first + off, Ch, after_walk ? 1 : 0, mf ? kRay64Mf : kRay64,
-                   SlotList{c->tcnt.p, c->tslots.p, c->runacc.p});
+      hipLaunchKernelGGL(k_near64<false>, dim3(n), dim3(64), nlds, c->stream, c->net, io, first + off,
+                         mf ? kRay64Mf : kRay64, (const double*)c->tplanes.p, (const double*)c->teq.p, Ch,
+                         after_walk ? 1 : 0, near);
+      HIPCHK(hipGetLastError());
+      launch_ray64(c, n, rlds, io, first + off, Ch, mf ? kRay64Mf : kRay64, near,
+                   SlotList{c->tcnt.p + 1, c->tslots.p + lcap, c->runacc.p});
       HIPCHK(hipGetLastError());
       const size_t m2 = tm.mark(c->stream);
       tm.span(m1v, m2, T_RAY64);
@@ -679,7 +692,8 @@ void run_fp64_regions(am_ctx* c, int lvl_first, int first, int count, const int*
     io.flags = nullptr;
     const size_t m3 = tm.mark(c->stream);
     hipLaunchKernelGGL(k_walk_fp64, dim3(std::min(n, c->scan_blocks)), dim3(64), wlds, c->stream, c->net, io, first + off,
-                       (const int*)c->tcnt.p, (const int*)c->tslots.p, (const double*)c->tplanes.p,
+                       (const int*)(mode == 1 ? c->tcnt.p + 1 : c->tcnt.p),
+                       (const int*)(mode == 1 ? c->tslots.p + lcap : c->tslots.p), (const double*)c->tplanes.p,
                        (const double*)c->teq.p, Ch);
     HIPCHK(hipGetLastError());
     tm.span(m3, tm.mark(c->stream), T_SCAN64);

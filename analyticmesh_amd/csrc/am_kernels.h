@@ -86,7 +86,7 @@ struct ChainIO {
   int noutp[AM_MAX_LINEAR];         // n_out rounded up to AM_CR
   const int* dcount = nullptr;      // as in RegionIO: regions past *dcount - dbase are not valid
   int dbase = 0;
-  int* zero = nullptr;              // set to 0 by the launch (a counter that later launches of the chunk fill)
+  int* zero = nullptr;              // two counters set to 0 by the launch (later launches of the chunk fill them)
 };
 
 // A list of chunk-local slots filled by atomics (cnt zeroed before), with
@@ -96,6 +96,12 @@ struct SlotList {
   int* cnt = nullptr;
   int* slots = nullptr;
   int* run = nullptr;
+};
+
+// Launch slots of the regions a near walk leaves, in no particular order.
+struct NearList {
+  int* cnt = nullptr;
+  int* slots = nullptr;
 };
 
 // The regions and plane buffers of one tiled-chain launch.
@@ -123,12 +129,18 @@ __global__ void k_chain_tile_fp64_multi(const NetDev* nets, const ChainIO* cios,
 __global__ void k_walk_fp64(NetDev net, RegionIO io, int rid0, const int* count, const int* slots,
                             const double* planes, const double* eq, int Cs_hbm);
 struct WalkParams;
-// only_undecided: blocks whose region is not flagged AM_UNDECIDED in io.flags exit.
-// NW waves per region: 2, 4 or 8.  With left.cnt, the regions the walk leaves
-// undecided are listed as k_collect_slots lists them.
+// The near walk (am_near.h) on the planes of the chain: SCAN decides as
+// k_walk_fp64, else as k_walk_ray64.  Regions it leaves are listed (launch
+// slots, *left.cnt zeroed before) for those kernels.
+template <bool SCAN>
+__global__ void k_near64(NetDev net, RegionIO io, int rid0, WalkParams wp, const double* planes, const double* eq,
+                         int Cs_hbm, int only_undecided, NearList left);
+// The checked ray walk over all constraints of the regions the near walk left
+// (list; blocks stride over it).  NW waves per region: 2, 4 or 8.  The regions
+// it leaves undecided are listed in `left` as k_collect_slots lists them.
 template <int NW>
 __global__ void k_walk_ray64(NetDev net, RegionIO io, int rid0, WalkParams wp, const double* planes,
-                             const double* eq, int Cs_hbm, int only_undecided, SlotList left);
+                             const double* eq, int Cs_hbm, NearList list, SlotList left);
 // Batch-of-networks forms (region rid0 + b; its network is mask word Wd - 1;
 // the scan's LDS layout follows each network's C, the launch is sized for the
 // widest network).
