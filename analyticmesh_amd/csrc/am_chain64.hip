@@ -747,7 +747,7 @@ struct TilePlanes {
 };
 
 template <bool SCAN>
-__global__ __launch_bounds__(64) void k_near64(NetDev net, RegionIO io, int rid0, WalkParams wp, const double* planes,
+__global__ __launch_bounds__(64, 5) void k_near64(NetDev net, RegionIO io, int rid0, WalkParams wp, const double* planes,
                                                const double* eqb, int Cs_hbm, int only_undecided, NearList left) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int b = blockIdx.x;
@@ -763,7 +763,7 @@ __global__ __launch_bounds__(64) void k_near64(NetDev net, RegionIO io, int rid0
   for (int q = 0; q < 4; ++q) eq[q] = eqb[(size_t)b * 4 + q];
   __syncthreads();
   const TilePlanes P{planes + (size_t)b * 4 * Cs_hbm, Cs_hbm, net.nodes[1], net.W0, net.b[0], S.mask, net.C};
-  const bool done = near_or_full_walk<double, SCAN>(net, io, wp, rid, rid - io.first, P, S, eq, p, start);
+  const bool done = near_or_full_walk<double, SCAN>(net, io, wp, rid, rid - io.first, P, S, eq, p, start) == NEAR_DONE;
   // (thread 0 wrote the flag in finish_region: the orientation may be undecided)
   if (threadIdx.x == 0 && (!done || (!SCAN && (io.flags[rid - io.first] & AM_UNDECIDED)))) near_left(left, b);
 }

@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "am_fast.h"
+#include "am_near.h"
 #include "am_scan.h"
 
 namespace am {
@@ -498,6 +499,43 @@ __global__ __launch_bounds__(64 * NW, 24 / NW) void k_walk_ray_f32(NetDev net, R
   walk_ray<float, NW>(net, io, wp, rid, rid - io.first, P, smask, eq, p, rec, start_in, with_sigma ? eb[4] : 0.f);
 }
 
+// One region's FP32 planes and error estimates as the face kernel stores them.
+struct FacePlanes {
+  const float* src;
+  int Cs, C;
+  __device__ __forceinline__ int parts() const { return 1; }
+  __device__ __forceinline__ int first(int) const { return 0; }
+  __device__ __forceinline__ int size(int) const { return C; }
+  __device__ __forceinline__ float err(int g) const { return src[4 * (size_t)Cs + g]; }
+  __device__ __forceinline__ void load(int, int j, float* p) const {
+    for (int q = 0; q < 4; ++q) p[q] = src[(size_t)q * Cs + j];
+  }
+  __device__ __forceinline__ void get(int g, float* p) const { load(0, g, p); }
+};
+
+// The near walk on the FP32 planes (per-plane error estimates): decides as
+// k_walk_ray_f32, one wave per region.  Every region has a start plane (seeds
+// take k_walk_ray_f32).
+__global__ __launch_bounds__(64, 5) void k_near_f32(NetDev net, RegionIO io, WalkParams wp, const float* planes,
+                                                 const float* eqbuf, int Cs_hbm, int chunk_first) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  const int b = blockIdx.x;
+  if (b >= io.count) return;
+  const int rid = chunk_first + b;
+  const NearLds<float> S = carve_near<float>(smem_raw, net.C, net.Wd, net.vm, true);
+  const int start = io.reg_start[rid];
+  for (int w = threadIdx.x; w < net.Wd; w += 64) S.mask[w] = io.reg_mask[(size_t)rid * net.Wd + w];
+  const float* eb = eqbuf + (size_t)b * AM_EQS;
+  const float eq[4] = {eb[0], eb[1], eb[2], eb[3]};
+  const float p[3] = {(float)io.reg_point[(size_t)rid * 3 + 0], (float)io.reg_point[(size_t)rid * 3 + 1],
+                      (float)io.reg_point[(size_t)rid * 3 + 2]};
+  __syncthreads();
+  const FacePlanes P{planes + (size_t)b * AM_PCOMP * Cs_hbm, Cs_hbm, net.C};
+  const int w = near_or_full_walk<float, false>(net, io, wp, rid, rid - io.first, P, S, eq, p, start, eb[4]);
+  if (w != NEAR_DONE && threadIdx.x == 0)
+    io.flags[rid - io.first] = AM_UNDECIDED | (w > 0 ? (unsigned)w : AM_WHY_BIT(AM_WHY_SEED));
+}
+
 // The level's regions the walk left to FP64 in one launch: their ids (first +
 // level index, in region order, through a one-pass scan of 2048-region
 // tiles) and count, and the counters: undecided regions added to acc[0],
@@ -806,6 +844,7 @@ void fast_level(FastNet& f, FastBuffers& b, const NetDev& net, const FastLevel& 
   const size_t wlds = walk_scan_lds(net);
   const size_t rlds = walk_ray_lds(net);
   const size_t glds = gemm_lds(d, prec);
+  const size_t nlds = near_lds_bytes(net.C, net.Wd, net.vm, 4, true);
 
   for (int c0 = 0; c0 < lvl.count; c0 += CH) {
     const int n = std::min(CH, lvl.count - c0);
@@ -843,7 +882,10 @@ void fast_level(FastNet& f, FastBuffers& b, const NetDev& net, const FastLevel& 
     io.Csort = Csort;
     io.flags = flags;
     io.ids = nullptr;
-    if (f.walk_mode == 0 && f.ray_waves == 2)
+    // a level past the seeds, planes with estimates: the near walk
+    if (f.walk_mode == 0 && prec == 0 && lvl.first > 0)
+      hipLaunchKernelGGL(k_near_f32, dim3(n), dim3(64), nlds, st, net, io, f.wp, planes, eqb, d.Cs, lvl.first + c0);
+    else if (f.walk_mode == 0 && f.ray_waves == 2)
       hipLaunchKernelGGL(k_walk_ray_f32<2>, dim3(n), dim3(128), rlds, st, net, io, f.wp, planes, eqb, d.Cs,
                          lvl.first + c0);
     else if (f.walk_mode == 0 && f.ray_waves == 8)

@@ -17,8 +17,8 @@
 // What bounds it: VALU issue and the planes' read (32 bytes per constraint).
 // The walks over all constraints read every plane once per vertex, from LDS
 // that leaves 4 to 6 regions per CU.  4x256 network, 1,022,340 regions, one
-// MI355X: candidate scan 75.3 -> 9.4 ms, FP64 ray walk 21.4 -> 9.2 ms; the
-// trained 4x60 network (248,231 regions) 11.6 -> 3.8 ms.
+// MI355X: candidate scan 75.3 -> 9.2 ms, FP64 ray walk 21.4 -> 9.9 ms, FP32 ray
+// walk 17.5 -> 10.8 ms; the trained 4x60 network (248,231 regions) 11.6 -> 3.8 ms.
 #pragma once
 #include "am_device.h"
 #include "am_kernels.h"
@@ -204,9 +204,13 @@ __device__ __forceinline__ bool near_covers(const T* v, const T* p, T r, T E, T 
 // FULL: every constraint takes part (each pass reads all planes again), for a
 // region whose polygon the near constraints do not cover: about one in a hundred
 // on the geometric networks, a third on the trained chair (long thin faces).
-// Returns whether the region was settled and its record written.
+// Returns NEAR_DONE (settled, record written), NEAR_RETRY (the constraints at
+// hand do not suffice), or the reason bits (AM_WHY_BIT) for which the checked ray
+// walk would leave the region undecided.
+#define NEAR_DONE 0
+#define NEAR_RETRY (-1)
 template <typename T, bool SCAN, bool FULL, typename Src>
-__device__ __forceinline__ bool near_walk(const NetDev& net, const RegionIO& io, const WalkParams& wp, int rid,
+__device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, const WalkParams& wp, int rid,
                                           int slot_region, const Src& P, const NearLds<T>& S, const T* eq, const T* p,
                                           int start, T eqe = T(0)) {
   constexpr bool per_plane = sizeof(T) == 4;
@@ -228,7 +232,7 @@ __device__ __forceinline__ bool near_walk(const NetDev& net, const RegionIO& io,
   };
   if (!FULL) {
     const int n = near_constraints<T, SCAN>(P, C, p, S.key, S.cand, r, qmax);
-    if (n < 3) return false;
+    if (n < 3) return NEAR_RETRY;
     have = lane < n;
     g = have ? (int)S.cand[lane] : -1;
     if (have) {
@@ -238,7 +242,7 @@ __device__ __forceinline__ bool near_walk(const NetDev& net, const RegionIO& io,
     }
     for (int q = 0; q < 4; ++q) S.pl[lane * 4 + q] = a[q];
     const unsigned long long sb = __ballot(g == start && have);
-    if (!sb) return false;
+    if (!sb) return NEAR_RETRY;
     sl = __builtin_ctzll(sb);
   } else {
     for (int w = lane; w < (C + 31) >> 5; w += 64) S.used[w] = 0u;
@@ -264,7 +268,7 @@ __device__ __forceinline__ bool near_walk(const NetDev& net, const RegionIO& io,
     } else {
       for (int l = 0; l < P.parts(); ++l) {
         const int n = P.size(l), g0 = P.first(l);
-#pragma unroll 2
+#pragma unroll 1
         for (int j = lane; j < n; j += 64) {
           T x[4];
           P.load(l, j, x);
@@ -292,7 +296,7 @@ __device__ __forceinline__ bool near_walk(const NetDev& net, const RegionIO& io,
     });
     rl = hi.take();
     ql = lo.take();
-    if (rl < 0 || ql < 0) return false;
+    if (rl < 0 || ql < 0) return FULL ? (int)AM_WHY_BIT(AM_WHY_START) : NEAR_RETRY;
     if (SCAN) {
       T kh, kl;
       if (FULL) {
@@ -321,7 +325,7 @@ __device__ __forceinline__ bool near_walk(const NetDev& net, const RegionIO& io,
   while (true) {
     // next edge plane rl: its vertex with the plane walked along and f = iso
     if (FULL) __syncthreads();        // S.used
-    if (is_used(rl) && !(rl == sl && ntab >= 3)) return false;
+    const bool in_tab = is_used(rl) && !(rl == sl && ntab >= 3);
     T pr[4], pc[4], v[3];
     plane(rl, pr);
     plane(cl, pc);
@@ -331,31 +335,23 @@ __device__ __forceinline__ bool near_walk(const NetDev& net, const RegionIO& io,
     T dn[3] = {pr[1] * eq[2] - pr[2] * eq[1], pr[2] * eq[0] - pr[0] * eq[2], pr[0] * eq[1] - pr[1] * eq[0]};
     if (pc[0] * dn[0] + pc[1] * dn[1] + pc[2] * dn[2] > T(0)) { dn[0] = -dn[0]; dn[1] = -dn[1]; dn[2] = -dn[2]; }
     Nearest<T> next;
-    if (ntab >= 2) {                  // the turn
-      T n1[4], n2[4];
+    T n1[4], n2[4];                   // the last two planes of the polygon, for the turn
+    if (ntab >= 2) {
       plane(tab2, n1);
       plane(tab1, n2);
-      if (SCAN) {
-        if (!pivot_valid(eq, n1, n2, pr)) return false;
-      } else {
-        const T A12 = AM_DOT3(n1, n2), A23 = AM_DOT3(n2, pr), A13 = AM_DOT3(n1, pr), A22 = AM_DOT3(n2, n2);
-        const T C1 = AM_DOT3(n1, eq), C2 = AM_DOT3(n2, eq), C3 = AM_DOT3(pr, eq), B = AM_DOT3(eq, eq);
-        const T val = (A12 * A23 - A22 * A13) * B - (A12 * C2 * C3 + A23 * C1 * C2 - A13 * C2 * C2 - A22 * C1 * C3);
-        const T mag = (absT(A12 * A23) + absT(A22 * A13)) * B +
-                      (absT(A12 * C2 * C3) + absT(A23 * C1 * C2) + absT(A13 * C2 * C2) + absT(A22 * C1 * C3));
-        if (!(val > T(wp.eps_turn) * mag)) return false;
-      }
     }
     if (SCAN) {
       solve3(pr, pc, eq, v);
       for (int q = 0; q < 3; ++q) vd[q] = (double)v[q];
-      if (nv > 0 && same_vertex(lastv, vd)) return false;
+      if (in_tab || !near_covers<T>(v, p, r, T(0), T(0)) || (nv > 0 && same_vertex(lastv, vd)) ||
+          (ntab >= 2 && !pivot_valid(eq, n1, n2, pr)))
+        return NEAR_RETRY;
       T pq[4], kw;
       plane(ql, pq);
       if (FULL) kw = order_key(pr);
       else kw = lane_value(key, rl);
       const int gw = index_of(rl);
-      bool fail = !near_covers<T>(v, p, r, T(0), T(0));
+      bool fail = false;
       each([&](const T* x, int h, int gi, T) {
         if (h == cl || h == rl) return;
         const T sv = plane_eval(x[0], x[1], x[2], x[3], v);
@@ -371,7 +367,7 @@ __device__ __forceinline__ bool near_walk(const NetDev& net, const RegionIO& io,
                            (h != ql && violates(pq[0], pq[1], pq[2], pq[3], vt)));
         }
       });
-      if (__any(fail)) return false;
+      if (__any(fail)) return NEAR_RETRY;
     } else {
       if constexpr (sizeof(T) == 4) {
         const double a4[4] = {pr[0], pr[1], pr[2], pr[3]};
@@ -386,7 +382,6 @@ __device__ __forceinline__ bool near_walk(const NetDev& net, const RegionIO& io,
       const T lam = per_plane ? T(wp.lam) : T(0);
       vb = vertex_bound_unit<T>(pr, pc, eq, lam * err_of(rl), lam * err_of(cl), lam * eqe, T(wp.eps), T(wp.h_max), lam,
                                 T(wp.lam_v));
-      if (!vb.ok) return false;
       scale_bound<T>(vb, T(1) + absT(v[0]) + absT(v[1]) + absT(v[2]));
       T E = vb.E, F = T(0);
       if constexpr (sizeof(T) == 4) {
@@ -397,19 +392,32 @@ __device__ __forceinline__ bool near_walk(const NetDev& net, const RegionIO& io,
         E = T(2) * vb.e0;
         F = T(2) * (vb.w1 * l1 + vb.w2 * l2 + vb.w3 * l3 + vb.eg * qmax);
       }
-      bool fail = !FULL && !near_covers<T>(v, p, r, E, F);
-      if (nv > 0) {
-        const double l1 = fabs(vd[0] - lastv[0]) + fabs(vd[1] - lastv[1]) + fabs(vd[2] - lastv[2]);
-        fail = fail || !(l1 > 4.0 * Tol<double>::SAME_EPS);
+      // (a system that is not trusted decides nothing: only its place counts)
+      if (!FULL && !near_covers<T>(v, p, r, vb.ok ? E : T(0), vb.ok ? F : T(0))) return NEAR_RETRY;
+      if (in_tab) return (int)AM_WHY_BIT(AM_WHY_TAB);
+      if (ntab >= 2) {   // the turn (walk_ray's test)
+        const T A12 = AM_DOT3(n1, n2), A23 = AM_DOT3(n2, pr), A13 = AM_DOT3(n1, pr), A22 = AM_DOT3(n2, n2);
+        const T C1 = AM_DOT3(n1, eq), C2 = AM_DOT3(n2, eq), C3 = AM_DOT3(pr, eq), B = AM_DOT3(eq, eq);
+        const T val = (A12 * A23 - A22 * A13) * B - (A12 * C2 * C3 + A23 * C1 * C2 - A13 * C2 * C2 - A22 * C1 * C3);
+        const T mag = (absT(A12 * A23) + absT(A22 * A13)) * B +
+                      (absT(A12 * C2 * C3) + absT(A23 * C1 * C2) + absT(A13 * C2 * C2) + absT(A22 * C1 * C3));
+        if (!(val > T(wp.eps_turn) * mag)) return (int)AM_WHY_BIT(AM_WHY_TURN);
       }
+      int bits = 0;
       each([&](const T* x, int h, int, T e) {
         if (h == cl || h == rl) return;
         const T sv = plane_eval(x[0], x[1], x[2], x[3], v);
-        fail = fail || checked_verdict_at<T>(sv, x[0], x[1], x[2], x[3], e, vb) != 0;
+        bits |= checked_verdict_at<T>(sv, x[0], x[1], x[2], x[3], e, vb);
         const T al = fmaT(x[0], dn[0], fmaT(x[1], dn[1], x[2] * dn[2]));
         next.add(-sv, al, al > T(0), h);
       });
-      if (__any(fail)) return false;
+      if (__any(bits & 1)) return (int)AM_WHY_BIT(AM_WHY_VIOL);
+      if (__any(bits & 2)) return (int)AM_WHY_BIT(AM_WHY_UNSURE);
+      if (!vb.ok) return (int)AM_WHY_BIT(AM_WHY_HMAX);
+      if (nv > 0) {
+        const double l1 = fabs(vd[0] - lastv[0]) + fabs(vd[1] - lastv[1]) + fabs(vd[2] - lastv[2]);
+        if (!(l1 > 4.0 * Tol<double>::SAME_EPS)) return (int)AM_WHY_BIT(AM_WHY_SAME);
+      }
     }
     // record the vertex
     const int gr = index_of(rl), gc = index_of(cl);
@@ -436,9 +444,9 @@ __device__ __forceinline__ bool near_walk(const NetDev& net, const RegionIO& io,
     tab2 = tab1;
     tab1 = rl;
     if (ntab >= 4 && rl == sl) break;       // closed
-    if (ntab >= vm + 1) return false;       // truncated
+    if (ntab >= vm + 1) return SCAN ? NEAR_RETRY : (int)AM_WHY_BIT(AM_WHY_TRUNC);
     const int nx = next.take();
-    if (nx < 0) return false;
+    if (nx < 0) return FULL ? (int)AM_WHY_BIT(AM_WHY_NEXT) : NEAR_RETRY;
     ql = cl;
     cl = rl;
     rl = nx;
@@ -451,16 +459,19 @@ __device__ __forceinline__ bool near_walk(const NetDev& net, const RegionIO& io,
     finish_region<T, true, double>(net, io, wp, rid, slot_region, S.mask, eq, S.rec.tab, S.rec.verts, S.rec.vpair,
                                    ntab, nv, start, start, AM_ST_OK, false, 0u, vinacc,
                                    per_plane ? S.rec.jinv : nullptr);
-  return true;
+  return NEAR_DONE;
 }
 
-// The walk of one region on its near constraints, else on all of them.
+// The walk of one region on its near constraints, else on all of them.  FP64
+// forms retry on all constraints whatever the reason; the FP32 form leaves a
+// fifth of its regions undecided, for reasons all constraints would confirm.
 template <typename T, bool SCAN, typename Src>
-__device__ __forceinline__ bool near_or_full_walk(const NetDev& net, const RegionIO& io, const WalkParams& wp, int rid,
-                                                  int slot_region, const Src& P, const NearLds<T>& S, const T* eq,
-                                                  const T* p, int start, T eqe = T(0)) {
-  if (start < 0 || start >= net.C) return false;
-  if (near_walk<T, SCAN, false>(net, io, wp, rid, slot_region, P, S, eq, p, start, eqe)) return true;
+__device__ __forceinline__ int near_or_full_walk(const NetDev& net, const RegionIO& io, const WalkParams& wp, int rid,
+                                                 int slot_region, const Src& P, const NearLds<T>& S, const T* eq,
+                                                 const T* p, int start, T eqe = T(0)) {
+  if (start < 0 || start >= net.C) return NEAR_RETRY;
+  const int w = near_walk<T, SCAN, false>(net, io, wp, rid, slot_region, P, S, eq, p, start, eqe);
+  if (w == NEAR_DONE || (sizeof(T) == 4 && w != NEAR_RETRY)) return w;
   __syncthreads();
   return near_walk<T, SCAN, true>(net, io, wp, rid, slot_region, P, S, eq, p, start, eqe);
 }
