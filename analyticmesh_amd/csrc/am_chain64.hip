@@ -24,7 +24,6 @@
 #include "am_device.h"
 #include "am_kernels.h"
 #include "am_walk.h"
-#include "am_near.h"
 
 namespace am {
 
@@ -365,212 +364,12 @@ __device__ __forceinline__ void chain_tile_body(const NetDev& net, const ChainIO
   }
 }
 
-// The matrix-core chain on half tiles: 8 regions (32 columns) per workgroup of
-// 8 waves, each wave two 16-row blocks (rows 32 w .. 32 w + 31) by two 16-column
-// blocks, so one A fragment feeds two products and one B fragment two.  Its
-// LDS (about 75 KB) lets two workgroups share a CU: one runs its products while
-// the other parks, stores and compacts a layer.  Planes as chain_tile_body.
-__device__ __forceinline__ void chain_tile_half(const NetDev& net, const ChainIO& io, const ChainLevel& lv, int r0,
-                                                int nreg) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  double* Xs = reinterpret_cast<double*>(smem_raw);                                   // [AM_CXR][AM_HXS]
-  uint16_t* klist = reinterpret_cast<uint16_t*>(Xs + (size_t)AM_CXR * AM_HXS + 1);     // [D][AM_KLS]
-  uint32_t* mk = reinterpret_cast<uint32_t*>(klist + (size_t)net.D * AM_KLS);          // [AM_HT][Wd]
-  __shared__ int s_nk[AM_MAX_LINEAR];
-  for (int idx = tid; idx < AM_HT * net.Wd; idx += AM_HALF_THREADS) {
-    const int t = idx / net.Wd, w = idx - t * net.Wd;
-    uint32_t v = 0u;
-    if (t < nreg) {
-      const int rid = lv.ids ? lv.ids[r0 + t] : lv.first + r0 + t;
-      v = io.reg_mask[(size_t)rid * net.Wd + w];
-    }
-    mk[idx] = v;
-  }
-  __syncthreads();
-  // active-input lists as in chain_tile_body (waves take layers in turn)
-  for (int li = wave + 1; li <= net.D; li += AM_HALF_THREADS / 64) {
-    const int nin = net.nodes[li], in0 = li == 1 ? 0 : net.off[li - 1];
-    uint16_t* kl = klist + (size_t)(li - 1) * AM_KLS;
-    int base = 0;
-    for (int kb = 0; kb < nin; kb += 64) {
-      const int k = kb + lane;
-      bool act = false;
-      if (k < nin)
-        for (int t = 0; t < AM_HT; ++t) act = act || mbit(mk + t * net.Wd, in0 + k);
-      const unsigned long long bal = __ballot(act);
-      if (act) kl[base + __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0u))] = (uint16_t)k;
-      base += __popcll(bal);
-    }
-    const int nkp = (base + AM_CPF - 1) / AM_CPF * AM_CPF;
-    for (int i = base + lane; i < nkp + AM_CPF; i += 64) kl[i] = (uint16_t)AM_CHAIN_MAXW;
-    if (lane == 0) s_nk[li] = nkp;
-  }
-  __syncthreads();
-  const size_t Cs = (size_t)io.Cs;
-  const int n1 = net.nodes[1];
-  // layer-1 input rows: a thread takes list position i and half h of the tile's
-  // regions, reads its row of (W0 | b0) once and writes 4 regions x 4 values
-  {
-    static_assert(AM_HALF_THREADS == 512 && AM_CHAIN_MAXW <= 256, "two halves of 256 positions");
-    const int h = tid >> 8;
-    for (int i = tid & 255; i < s_nk[1]; i += 256) {
-      const int k = klist[i];
-      double w[4] = {0.0, 0.0, 0.0, 0.0};
-      if (k < n1) {
-        w[0] = net.W0[k * 3 + 0];
-        w[1] = net.W0[k * 3 + 1];
-        w[2] = net.W0[k * 3 + 2];
-        w[3] = net.b[0][k];
-      }
-#pragma unroll
-      for (int tt = 0; tt < AM_HT / 2; ++tt) {
-        const int t = h * (AM_HT / 2) + tt;
-        const bool on = k < n1 && mbit(mk + t * net.Wd, k);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) Xs[i * AM_HXS + 4 * t + q] = on ? w[q] : 0.0;
-      }
-    }
-  }
-  for (int idx = tid; idx < AM_HN * net.E; idx += AM_HALF_THREADS) {
-    const int col = idx / net.E, e = idx - col * net.E, t = col >> 2, q = col & 3;
-    if (t < nreg) lv.planes[((size_t)(r0 + t) * 4 + q) * Cs + net.L + e] = q < 3 ? net.ew[e * 3 + q] : net.eb[e];
-  }
-  __syncthreads();
-  const int l16 = lane & 15, l4 = lane >> 4;
-  for (int li = 1; li <= net.D; ++li) {
-    const int nout = net.nodes[li + 1], noutp = io.noutp[li];
-    const int row0 = wave * 32;
-    // row blocks of this wave with rows (W^T holds noutp >= nout columns, zero past nout)
-    const int nrb = row0 >= nout ? 0 : (row0 + 16 >= noutp ? 1 : 2);
-    am_f64x4 acc[2][2];
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-      for (int cb = 0; cb < 2; ++cb) acc[rb][cb] = am_f64x4{0.0, 0.0, 0.0, 0.0};
-    if (nrb > 0) {
-      const uint16_t* kl = klist + (size_t)(li - 1) * AM_KLS;
-      const int nkp = s_nk[li];
-      const double* wcol = io.Wp[li] + row0 + l16;
-      const int rb1 = nrb > 1 ? 16 : 0;   // the second block's column offset (re-reads the first when absent)
-      constexpr int PF = AM_CPF / 4;
-      double a0[PF], a1[PF];
-#pragma unroll
-      for (int u = 0; u < PF; ++u) {
-        const double* w = wcol + (size_t)kl[4 * u + l4] * noutp;
-        a0[u] = w[0];
-        a1[u] = w[rb1];
-      }
-      for (int i0 = 0; i0 < nkp; i0 += AM_CPF) {
-#pragma unroll
-        for (int u = 0; u < PF; ++u) {
-          const int ii = i0 + 4 * u;
-          const double b0 = Xs[(size_t)(ii + l4) * AM_HXS + l16];
-          const double b1 = Xs[(size_t)(ii + l4) * AM_HXS + 16 + l16];
-          const double x0 = a0[u], x1 = a1[u];
-          const double* w = wcol + (size_t)kl[ii + AM_CPF + l4] * noutp;
-          a0[u] = w[0];
-          a1[u] = w[rb1];
-          acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(x0, b0, acc[0][0], 0, 0, 0);
-          acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(x0, b1, acc[0][1], 0, 0, 0);
-          if (nrb > 1) {
-            acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(x1, b0, acc[1][0], 0, 0, 0);
-            acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(x1, b1, acc[1][1], 0, 0, 0);
-          }
-        }
-      }
-    }
-    // the park's biases (column c of each region: lanes with l16 % 4 == 3),
-    // loaded while the other waves finish their products
-    const bool cbias = (l16 & 3) == 3;
-    double bias[2][4];
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int row = row0 + 16 * rb + l4 + 4 * v;
-        bias[rb][v] = cbias && rb < nrb && row < nout ? io.bp[li][row] : 0.0;
-      }
-    __syncthreads();                  // every wave is done reading this layer's input
-    {
-#pragma unroll
-      for (int rb = 0; rb < 2; ++rb) {
-        if (rb >= nrb) continue;
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int row = row0 + 16 * rb + l4 + 4 * v;
-          if (row < nout) {
-            const double b = bias[rb][v];
-            Xs[row * AM_HXS + l16] = acc[rb][0][v] + b;
-            Xs[row * AM_HXS + 16 + l16] = acc[rb][1][v] + b;
-          }
-        }
-      }
-    }
-    __syncthreads();
-    if (li < net.D) {
-      const int out0 = net.off[li];
-      const int jt = tid & 255, ct = tid >> 8;
-      for (int col = ct; col < AM_HN; col += AM_HALF_THREADS / 256) {
-        const int t = col >> 2, q = col & 3;
-        if (t >= nreg) break;
-        double* dst = lv.planes + ((size_t)(r0 + t) * 4 + q) * Cs + out0;
-        for (int j = jt; j < nout; j += 256) {
-          const double y = Xs[j * AM_HXS + col];
-          dst[j] = mbit(mk + t * net.Wd, out0 + j) ? -y : y;
-        }
-      }
-      const uint16_t* kl2 = klist + (size_t)li * AM_KLS;
-      const int nkp2 = s_nk[li + 1];
-      constexpr int PPT = AM_HALF_THREADS / AM_HN;                  // positions per pass of the block
-      constexpr int XH = AM_CHAIN_MAXW / PPT / 2;                   // passes per half
-      int tq = tid;
-      asm volatile("" : "+v"(tq));
-      const int col = tq & (AM_HN - 1), t = col >> 2, p0 = tq / AM_HN;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        double xv[XH];
-#pragma unroll
-        for (int c = 0; c < XH; ++c) {
-          const int i = (h * XH + c) * PPT + p0;
-          xv[c] = 0.0;
-          if (i < nkp2) {
-            const int k = kl2[i];
-            if (k < nout && mbit(mk + t * net.Wd, out0 + k)) xv[c] = Xs[k * AM_HXS + col];
-          }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int c = 0; c < XH; ++c) {
-          const int i = (h * XH + c) * PPT + p0;
-          if (i < nkp2) Xs[i * AM_HXS + col] = xv[c];
-        }
-      }
-    } else if (tid < AM_HN && (tid >> 2) < nreg) {
-      const double y = Xs[tid];
-      lv.eq[(size_t)(r0 + (tid >> 2)) * 4 + (tid & 3)] = (tid & 3) == 3 ? y - net.iso : y;
-    }
-    __syncthreads();
-  }
-}
-
 __global__ __launch_bounds__(AM_CHAIN_THREADS) void k_chain_tile_fp64(NetDev net, ChainIO io) {
-  if (io.zero && blockIdx.x == 0 && threadIdx.x < 2) io.zero[threadIdx.x] = 0;
   const int r0 = blockIdx.x * AM_CT;
   const int cnt = launch_count(io);
   if (r0 >= cnt) return;
   const ChainLevel lv{io.first, cnt, io.ids, io.planes, io.eq};
   chain_tile_body<false>(net, io, lv, r0, min(AM_CT, cnt - r0));
-}
-
-__global__ __launch_bounds__(AM_HALF_THREADS) void k_chain_tile_mfma(NetDev net, ChainIO io) {
-  if (io.zero && blockIdx.x == 0 && threadIdx.x < 2) io.zero[threadIdx.x] = 0;
-  const int r0 = blockIdx.x * AM_HT;
-  const int cnt = launch_count(io);
-  if (r0 >= cnt) return;
-  const ChainLevel lv{io.first, cnt, io.ids, io.planes, io.eq};
-  chain_tile_half(net, io, lv, r0, min(AM_HT, cnt - r0));
 }
 
 // Many networks in one launch: block b takes tiles[b] = (network, r0, regions);
@@ -615,18 +414,6 @@ __device__ __forceinline__ void walk_fp64_body(const NetDev& net, const RegionIO
   const WalkParams wp{0.f, 0.f, 0.f};
   walk_region<double, false>(net, io, wp, rid, rid - io.first, Px, Py, Pz, Pc, keys, order, used, smask, eq, p);
   __syncthreads();   // this region's LDS is free for the next
-}
-
-__global__ __launch_bounds__(64) void k_walk_fp64(NetDev net, RegionIO io, int rid0, const int* count,
-                                                  const int* slots, const double* planes, const double* eqb,
-                                                  int Cs_hbm) {
-  const int total = count ? min(*count, io.count) : io.count;
-  // block-stride over the regions (one iteration per block when the grid covers them)
-  for (int b = blockIdx.x; b < total; b += gridDim.x) {
-    const int sl = slots ? slots[b] : b;     // planes slot of this region
-    const int rid = io.ids ? io.ids[sl] : rid0 + sl;
-    walk_fp64_body(net, io, rid, sl, planes, eqb, Cs_hbm);
-  }
 }
 
 // Network of a region in a batch of networks: the last word of its mask.
@@ -693,85 +480,6 @@ __device__ __forceinline__ void walk_ray64_body(const NetDev& net, const RegionI
   walk_ray<double, NW>(net, io, wp, rid, rid - io.first, P, smask, eq, p, rec, start_in);
 }
 
-// NW waves per region (the records do not depend on NW: every reduction breaks
-// ties by constraint index and each serial step runs on one wave).  A region
-// the walk leaves undecided goes on the candidate scan's list (its counter
-// zeroed before) and counts itself and its reasons in left.run (as
-// k_collect_slots would).
-template <int NW>
-__global__ __launch_bounds__(64 * NW, 24 / NW) void k_walk_ray64(NetDev net, RegionIO io, int rid0, WalkParams wp,
-                                                        const double* planes, const double* eqb, int Cs_hbm,
-                                                        NearList list, SlotList left) {
-  const int total = min(*list.cnt, io.count);
-  for (int i = blockIdx.x; i < total; i += gridDim.x) {
-    const int b = list.slots[i];
-    const int rid = io.ids ? io.ids[b] : rid0 + b;
-    walk_ray64_body<NW>(net, io, rid, b, wp, planes, eqb, Cs_hbm);
-    // thread 0 wrote the region's flag (finish_region)
-    if (threadIdx.x == 0) {
-      const unsigned f = io.flags[rid - io.first];
-      if (f & AM_UNDECIDED) {
-        left.slots[atomicAdd(left.cnt, 1)] = b;
-        atomicAdd(left.run, 1);
-        for (int w = 0; w < AM_WHY_COUNT; ++w)
-          if (f & AM_WHY_BIT(w)) atomicAdd(left.run + 1 + w, 1);
-      }
-    }
-    __syncthreads();   // this region's LDS is free for the next
-  }
-}
-
-// One region's planes as the tiled chain stores them (plane64), for the near walk.
-struct TilePlanes {
-  const double* src;
-  int Cs, n1;
-  const double* W0;
-  const double* b0;
-  const uint32_t* mask;
-  int C;
-  // the constraints in two parts: hidden layer 1's, rebuilt from its weights, and the others
-  __device__ __forceinline__ int parts() const { return 2; }
-  __device__ __forceinline__ int first(int l) const { return l ? n1 : 0; }
-  __device__ __forceinline__ int size(int l) const { return l ? C - n1 : n1; }
-  __device__ __forceinline__ double err(int) const { return 0.0; }
-  __device__ __forceinline__ void load(int l, int j, double* p) const {
-    if (l == 0) {
-      const uint32_t sm = mbit(mask, j) ? 0x80000000u : 0u;
-      const double v[4] = {W0[j * 3 + 0], W0[j * 3 + 1], W0[j * 3 + 2], b0[j]};
-      for (int q = 0; q < 4; ++q) p[q] = flip_sign(v[q], sm);
-    } else {
-      for (int q = 0; q < 4; ++q) p[q] = src[(size_t)q * Cs + n1 + j];
-    }
-  }
-  __device__ __forceinline__ void get(int g, double* p) const { load(g < n1 ? 0 : 1, g < n1 ? g : g - n1, p); }
-};
-
-template <bool SCAN>
-__global__ __launch_bounds__(64, 5) void k_near64(NetDev net, RegionIO io, int rid0, WalkParams wp, const double* planes,
-                                               const double* eqb, int Cs_hbm, int only_undecided, NearList left) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  const int b = blockIdx.x;
-  if (b >= launch_count(io)) return;
-  const int rid = io.ids ? io.ids[b] : rid0 + b;
-  // a region an earlier walk decided keeps its records (its flag is 0 and stays 0)
-  if (only_undecided && !(io.flags[rid - io.first] & AM_UNDECIDED)) return;
-  const NearLds<double> S = carve_near<double>(smem_raw, net.C, net.Wd, net.vm, false);
-  const int start = io.reg_start[rid];
-  for (int w = threadIdx.x; w < net.Wd; w += 64) S.mask[w] = io.reg_mask[(size_t)rid * net.Wd + w];
-  double p[3], eq[4];
-  for (int q = 0; q < 3; ++q) p[q] = io.reg_point[(size_t)rid * 3 + q];
-  for (int q = 0; q < 4; ++q) eq[q] = eqb[(size_t)b * 4 + q];
-  __syncthreads();
-  const TilePlanes P{planes + (size_t)b * 4 * Cs_hbm, Cs_hbm, net.nodes[1], net.W0, net.b[0], S.mask, net.C};
-  const bool done = near_or_full_walk<double, SCAN>(net, io, wp, rid, rid - io.first, P, S, eq, p, start) == NEAR_DONE;
-  // (thread 0 wrote the flag in finish_region: the orientation may be undecided)
-  if (threadIdx.x == 0 && (!done || (!SCAN && (io.flags[rid - io.first] & AM_UNDECIDED)))) near_left(left, b);
-}
-template __global__ void k_near64<true>(NetDev, RegionIO, int, WalkParams, const double*, const double*, int, int,
-                                        NearList);
-template __global__ void k_near64<false>(NetDev, RegionIO, int, WalkParams, const double*, const double*, int, int,
-                                         NearList);
-
 template <int NW>
 __global__ __launch_bounds__(64 * NW, 24 / NW) void k_walk_ray64_multi(const NetDev* nets, RegionIO io, int Wd, int rid0,
                                                               WalkParams wp, const double* planes, const double* eqb,
@@ -781,51 +489,12 @@ __global__ __launch_bounds__(64 * NW, 24 / NW) void k_walk_ray64_multi(const Net
   walk_ray64_body<NW>(nets[region_net(io, Wd, rid)], io, rid, blockIdx.x, wp, planes, eqb, Cs_hbm);
 }
 
-template __global__ void k_walk_ray64<2>(NetDev, RegionIO, int, WalkParams, const double*, const double*, int, NearList,
-                                         SlotList);
-template __global__ void k_walk_ray64<4>(NetDev, RegionIO, int, WalkParams, const double*, const double*, int, NearList,
-                                         SlotList);
-template __global__ void k_walk_ray64<8>(NetDev, RegionIO, int, WalkParams, const double*, const double*, int, NearList,
-                                         SlotList);
 template __global__ void k_walk_ray64_multi<2>(const NetDev*, RegionIO, int, int, WalkParams, const double*,
                                                const double*, int);
 template __global__ void k_walk_ray64_multi<4>(const NetDev*, RegionIO, int, int, WalkParams, const double*,
                                                const double*, int);
 template __global__ void k_walk_ray64_multi<8>(const NetDev*, RegionIO, int, int, WalkParams, const double*,
                                                const double*, int);
-
-// Vertices of a region whose polygon (the tight-constraint pair of every
-// vertex, its order and orientation) a reduced-precision walk certified: each
-// is the intersection of the FP64 planes of its pair with the face plane,
-// solved as the FP64 ray walk solves it (new constraint, constraint walked
-// along, face plane), so the coordinates carry FP64 rounding only.
-__global__ __launch_bounds__(64) void k_vertex_fp64(NetDev net, RegionIO io, int rid0, const double* planes,
-                                                    const double* eqb, int Cs_hbm) {
-  const int b = blockIdx.x;
-  if (b >= launch_count(io)) return;
-  const int rid = io.ids ? io.ids[b] : rid0 + b;
-  if (io.flags && (io.flags[rid - io.first] & AM_UNDECIDED)) return;   // left to the FP64 walk
-  const int vm = net.vm;
-  const int nv = io.reg_info[(size_t)rid * AM_INFO_STRIDE + 2];
-  const double* src = planes + (size_t)b * 4 * Cs_hbm;
-  const uint32_t* mask = io.reg_mask + (size_t)rid * net.Wd;
-  const double eq[4] = {eqb[(size_t)b * 4 + 0], eqb[(size_t)b * 4 + 1], eqb[(size_t)b * 4 + 2],
-                        eqb[(size_t)b * 4 + 3]};
-  for (int i = threadIdx.x; i < nv && i < vm; i += 64) {
-    const int r = io.reg_vpair[((size_t)rid * vm + i) * 2 + 0];
-    const int s = io.reg_vpair[((size_t)rid * vm + i) * 2 + 1];
-    if (r < 0 || r >= net.C || s < 0 || s >= net.C) continue;
-    double pr[4], ps[4];
-    plane64(net, mask, src, Cs_hbm, r, pr);
-    plane64(net, mask, src, Cs_hbm, s, ps);
-    double v[3];
-    solve3_rcp(pr, ps, eq, v);
-    double* out = io.reg_verts + ((size_t)rid * vm + i) * 3;
-    out[0] = v[0];
-    out[1] = v[1];
-    out[2] = v[2];
-  }
-}
 
 // Chunk-local slots of the regions k_walk_ray64 left undecided: region of
 // slot b is ids[b] or rid0 + b; its flag is level-relative.

@@ -29,6 +29,7 @@
 #include "am_newton.h"
 #include "am_combine.h"
 #include "am_near.h"
+#include "am_prefix.h"
 #include "am_scan.h"
 
 using namespace am;
@@ -113,6 +114,31 @@ void ensure_zeroed(DevBuf<unsigned long long>& b, size_t n, hipStream_t st) {
                      b.n * 2, 0u);
   HIPCHK(hipGetLastError());
 }
+
+// Planes of a march's activation prefixes (am_prefix.h): the table, and per
+// depth the blocks of plane storage, kept between runs and reused by the next.
+// The storage is bounded (kPrefixBytes, less when the device is short of memory):
+// a launch that might not fit starts over with an empty table, which costs the
+// sharing with earlier levels and nothing else.
+constexpr size_t kPrefixBytes = (size_t)4 << 30;
+
+struct PrefixStore {
+  DevBuf<unsigned long long> tab;
+  DevBuf<int> tab_id, counts, rslot;       // counts: total, then done
+  DevBuf<char*> blk;
+  DevBuf<int2> fresh;
+  DevBuf<double> layer1, extra;
+  std::vector<DevBuf<char>> arenas;        // the blocks' allocations
+  char* arena = nullptr;                   // the rest of the last one
+  size_t arena_left = 0;
+  std::vector<char*> blocks[AM_MAX_LINEAR + 1];
+  std::vector<DevBuf<double>> tmp;         // transforms of skips, transposed and padded
+  size_t bytes = 0;                        // of the allocations
+  size_t cap = 0;                          // table slots in use
+  long long ub[AM_MAX_LINEAR + 1] = {0};   // upper bounds of the ids given per depth
+  std::vector<char> reset;                 // per chunk of the planned level: start over first
+  PrefixDev dev{};
+};
 
 }  // namespace
 
@@ -199,6 +225,8 @@ struct am_ctx {
   bool tile_ok = false;
   bool chain_mfma = true;     // the certified forms' FP64 chain on the matrix cores ("chain_mfma")
   DevBuf<double> tplanes, teq;
+  // planes shared by activation prefix (am_prefix.h)
+  PrefixStore pfx;
   // am_adjoint's buffers, kept from call to call: dL/dv, dW, db, G and P per layer
   DevBuf<double> adj_gv, adj_dv;
   DevBuf<double> adj_part;   // per-block partial sums of dW / db, added in a fixed order
@@ -209,8 +237,10 @@ struct am_ctx {
   DevBuf<unsigned long long> redo_state;  // tile state of the one-pass scan listing them (zero between uses)
   DevBuf<uint16_t> reg_jinv;              // [R][vm][9] bf16: the reduced walk's inverse vertex systems
   bool jinv_on = false;                   // this run keeps them (reduced form, Newton vertices)
+  int* acc = nullptr;                     // ... its counters
   DevBuf<int> runacc;                     // per run: FP64 ray walk undecided count, then per reason
-  StageTimer timer;
+  StageTimer timer;                       // (batch of networks; the Newton step)
+  StageClock* clock = nullptr;            // a march's stage times, behind its counters in runacc
   std::vector<DevBuf<double>> WTp, bpad;   // W_li^T and b_li with n_out padded to AM_CR (zeros)
 
   double stats[AM_STAT_COUNT] = {0};
@@ -349,6 +379,8 @@ void insert_launch(am_ctx* c, const InsertPlan& p) {
   const size_t tiles = scan_commit_tiles(n);
   io.scan_state = c->scan_state.p;
   io.scan_words = (int)tiles + 1;
+  io.zero = c->tcnt.p;
+  io.clk = c->clock;
   hipLaunchKernelGGL(k_insert, dim3(blocks(n, 256)), dim3(256), 0, st, io);
   HIPCHK(hipGetLastError());
   // the new-region flags' scan in one pass; with the store already large
@@ -360,6 +392,11 @@ void insert_launch(am_ctx* c, const InsertPlan& p) {
   sio.tiles = (int)tiles;
   sio.rank = p.early ? nullptr : c->rank.p;
   sio.total = c->host_total_dev;
+  sio.clk = c->clock;
+  sio.pub = c->pfx.dev.total;
+  sio.npub = c->pfx.dev.total ? c->pfx.dev.nd + 1 : 0;
+  sio.pub_stride = AM_PFX_TS;
+  sio.pub_out = c->host_total_dev + 1;
   hipLaunchKernelGGL(k_scan_commit, dim3((unsigned)tiles), dim3(kScanCommitThreads), 0, st, sio);
   HIPCHK(hipGetLastError());
 }
@@ -367,6 +404,8 @@ void insert_launch(am_ctx* c, const InsertPlan& p) {
 int insert_finish(am_ctx* c, const InsertPlan& p) {
   if (p.n == 0) return 0;
   const int total = wait_total(c);
+  // (every launch of the level has run: its prefixes are counted)
+  for (int d = 1; d <= c->pfx.dev.nd; ++d) c->pfx.ub[d] = reinterpret_cast<volatile int*>(c->host_total)[1 + d];
   if (total == 0) return 0;
   // am_combine indexes (region, vertex slot) items with 32-bit ints: R * vm must stay below 2^31
   long long limit = std::min<long long>((long long)INT_MAX / 2, (long long)INT_MAX / c->vm);
@@ -447,42 +486,9 @@ size_t region_lds_bytes(const am_ctx* c, int& Cs, int& Csort) {
          (size_t)((c->C + 31) / 32) * 4 + (size_t)c->Wd * 4 + 64;
 }
 
-void launch_region_fp64(am_ctx* c, int first, int count, const int* ids = nullptr) {
-  int Cs, Csort;
-  const size_t lds = region_lds_bytes(c, Cs, Csort);
-  RegionIO io;
-  io.reg_mask = c->reg_mask.p;
-  io.reg_start = c->reg_start.p;
-  io.reg_point = c->reg_point.p;
-  io.reg_info = c->reg_info.p;
-  io.reg_tab = c->reg_tab.p;
-  io.reg_verts = c->reg_verts.p;
-  io.reg_vpair = c->reg_vpair.p;
-  io.cand_mask = c->cand_mask.p;
-  io.cand_start = c->cand_start.p;
-  io.cand_point = c->cand_point.p;
-  io.cand_hash = c->cand_hash.p;
-  io.first = first;
-  io.count = count;
-  io.Cs = Cs;
-  io.Csort = Csort;
-  io.flags = nullptr;
-  io.ids = ids;
-  const size_t m0 = c->timer.mark(c->stream);
-  hipLaunchKernelGGL(k_region_fp64, dim3(count), dim3(64), lds, c->stream, c->net, io);
-  HIPCHK(hipGetLastError());
-  c->timer.span(m0, c->timer.mark(c->stream), T_REGION64);
-}
-
 size_t chain_lds_bytes(const am_ctx* c) {
   return ((size_t)AM_CXR * AM_CXS + 1) * sizeof(double) + (size_t)c->D * AM_KLS * sizeof(uint16_t) +
          (size_t)AM_CT * c->Wd * 4 + 16;
-}
-
-// LDS of k_chain_tile_mfma (half tiles: AM_HT regions)
-size_t chain_half_lds_bytes(const am_ctx* c) {
-  return ((size_t)AM_CXR * AM_HXS + 1) * sizeof(double) + (size_t)c->D * AM_KLS * sizeof(uint16_t) +
-         (size_t)AM_HT * c->Wd * 4 + 16;
 }
 
 // Per-run counters of the FP64 stages (kernel times go to the context's timer;
@@ -505,19 +511,6 @@ size_t ray64_lds_bytes(const am_ctx* c) {
          walk_rec_bytes(c->vm, false);
 }
 
-// FP64 planes + walk of `count` regions (region ids first.., or ids[0..count)),
-// through the tiled chain in chunks; candidate slots and flags are numbered
-// from `lvl_first`.  mode 0: the candidate scan on every region (the FP64
-// records of the CPU restatement, bit for bit); mode 1: the checked FP64 ray
-// walk, and the scan on the regions it leaves undecided, reusing their planes
-// (the scan runs a block-stride loop up to the device-side count); mode 2:
-// after a reduced-precision walk that flagged the level in rflags
-// (`undecided` of them, -1 when the count is not known on the host): the
-// regions it decided get FP64 vertices
-// (k_vertex_fp64, their other records stay as written), the others go
-// through mode 1.
-// Nothing here waits for the device.  Falls back to the one-region kernel
-// where the tiled chain does not apply.
 // The tiled chain's arguments for regions first .. first + n - 1 (or ids),
 // planes into the context's tile buffers with component stride Ch.
 ChainIO chain_io(const am_ctx* c, const int* ids, int first, int n, int Ch) {
@@ -539,22 +532,21 @@ ChainIO chain_io(const am_ctx* c, const int* ids, int first, int n, int Ch) {
 
 // The FP64 ray walk over all constraints of the listed regions, with the
 // context's waves per region (a grid that strides over the list).
-void launch_ray64(am_ctx* c, int n, size_t lds, const RegionIO& io, int rid0, int Ch, const WalkParams& kRay64,
+void launch_ray64(am_ctx* c, int n, size_t lds, const RegionIO& io, int rid0, const WalkParams& wp,
                   const NearList& list, const SlotList& left) {
-  const double* P = c->tplanes.p;
   const double* E = c->teq.p;
   n = std::min(n, c->scan_blocks);
   switch (c->ray_waves) {
     case 2:
-      hipLaunchKernelGGL(k_walk_ray64<2>, dim3(n), dim3(128), lds, c->stream, c->net, io, rid0, kRay64, P, E, Ch,
+      hipLaunchKernelGGL(k_walk_ray64<2>, dim3(n), dim3(128), lds, c->stream, c->net, c->pfx.dev, io, rid0, wp, E,
                          list, left);
       break;
     case 8:
-      hipLaunchKernelGGL(k_walk_ray64<8>, dim3(n), dim3(512), lds, c->stream, c->net, io, rid0, kRay64, P, E, Ch,
+      hipLaunchKernelGGL(k_walk_ray64<8>, dim3(n), dim3(512), lds, c->stream, c->net, c->pfx.dev, io, rid0, wp, E,
                          list, left);
       break;
     default:
-      hipLaunchKernelGGL(k_walk_ray64<4>, dim3(n), dim3(256), lds, c->stream, c->net, io, rid0, kRay64, P, E, Ch,
+      hipLaunchKernelGGL(k_walk_ray64<4>, dim3(n), dim3(256), lds, c->stream, c->net, c->pfx.dev, io, rid0, wp, E,
                          list, left);
   }
 }
@@ -565,59 +557,269 @@ void set_ray64_lds(size_t lds) {
   HIPCHK(hipFuncSetAttribute((const void*)k_walk_ray64<8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
 }
 
-// Buffers of run_fp64_regions for a level of `count` regions (planes of one
-// chunk, the undecided-slot list); returns the chunk size.  Idempotent, so it
-// can run before a capture and again, as a no-op, inside it.
-size_t fp64_prepare(am_ctx* c, int count) {
-  const int Ch = (c->C + 63) & ~63;
-  size_t chunk = ((size_t)1 << 30) / ((size_t)32 * Ch);
-  chunk = std::max<size_t>(1024, std::min<size_t>(chunk, 65536)) & ~(size_t)(AM_CT - 1);
+const void* dev_view(am_ctx* c, const void* src, size_t bytes, hipStream_t st);
+
+// Widest input of a layer product and its LDS.
+size_t prefix_layer_lds(const am_ctx* c) {
+  int w = 1;
+  for (int l = 1; l <= c->D; ++l) w = std::max(w, c->nodes[l]);
+  return layer_lds(w);
+}
+
+// Regions per launch of the prefix stages: the new planes of a launch take at
+// most half the storage.
+size_t prefix_chunk(const am_ctx* c) {
+  size_t per = 0;
+  for (int d = 1; d < c->D; ++d) per += (size_t)32 * c->nodes[d + 1];
+  const size_t n = per ? (kPrefixBytes / 2) / per : 65536;
+  return std::max<size_t>(AM_PFX_IDS, std::min<size_t>(n, 65536)) & ~(size_t)(AM_PFX_IDS - 1);
+}
+
+void prefix_clear(am_ctx* c) {
+  PrefixStore& s = c->pfx;
+  hipLaunchKernelGGL(k_prefix_clear, dim3(blocks(s.cap, 256)), dim3(256), 0, c->stream, s.dev, s.cap);
+  HIPCHK(hipGetLastError());
+}
+
+// A table of at least `cap` slots (a power of two), empty when it is new.
+void prefix_table(am_ctx* c, size_t cap) {
+  PrefixStore& s = c->pfx;
+  ensure(s.tab, cap, false, c->stream);
+  ensure(s.tab_id, cap, false, c->stream);
+  s.cap = cap;
+  s.dev.tab = s.tab.p;
+  s.dev.tab_id = s.tab_id.p;
+  s.dev.cap_mask = (uint32_t)(cap - 1);
+}
+
+// Per run: the weights' layouts, an empty table.
+void prefix_setup(am_ctx* c, const void* const* tms, int dtype) {
+  PrefixStore& s = c->pfx;
+  const hipStream_t st = c->stream;
+  PrefixDev& d = s.dev;
+  d.nd = c->D - 1;
+  ensure(s.counts, (size_t)(AM_PFX_TS + 1) * (AM_MAX_LINEAR + 1), false, st);
+  d.total = s.counts.p;
+  d.done = s.counts.p + AM_PFX_TS * (AM_MAX_LINEAR + 1);
+  ensure(s.blk, (size_t)(AM_MAX_LINEAR + 1) * AM_PFX_BLOCKS, false, st);
+  d.blk = s.blk.p;
+  const int n1 = c->nodes[1];
+  ensure(s.layer1, (size_t)4 * n1, false, st);
+  hipLaunchKernelGGL(k_pack_pairs, dim3(blocks(n1, 256)), dim3(256), 0, st, (const double*)c->W0.p,
+                     (const double*)c->b[0].p, n1, reinterpret_cast<double2*>(s.layer1.p));
+  ensure(s.extra, (size_t)4 * std::max(c->E, 1), false, st);
+  if (c->E)
+    hipLaunchKernelGGL(k_pack_pairs, dim3(blocks(c->E, 256)), dim3(256), 0, st, (const double*)c->ew.p,
+                       (const double*)c->eb.p, c->E, reinterpret_cast<double2*>(s.extra.p));
+  HIPCHK(hipGetLastError());
+  d.layer1 = reinterpret_cast<const double2*>(s.layer1.p);
+  d.extra = reinterpret_cast<const double2*>(s.extra.p);
+  for (int li = 1; li <= c->D; ++li) {
+    d.Wp[li] = c->WTp[li].p;
+    d.bp[li] = c->bpad[li].p;
+    d.noutp[li] = (c->nodes[li + 1] + AM_CR - 1) / AM_CR * AM_CR;
+  }
+  s.tmp.resize(c->tm.size());
+  for (size_t t = 0; t < c->tm.size(); ++t) {
+    const int h = c->tm_h[t], w = c->tm_w[t];
+    if (h <= 0 || w <= 0) continue;
+    const int rp = (h + AM_CR - 1) / AM_CR * AM_CR;
+    ensure(s.tmp[t], (size_t)(w + 1) * rp, false, st);
+    launch_transpose_pad(dev_view(c, tms[t], (size_t)h * w * (dtype == AM_DTYPE_F64 ? 8 : 4), st),
+                         dtype == AM_DTYPE_F64, h, w, s.tmp[t].p, rp, w + 1, st);
+    HIPCHK(hipGetLastError());
+    d.tmp[t] = s.tmp[t].p;
+    d.tmpo[t] = rp;
+  }
+  // the surface meets about L^2 cells, a third of them per depth as prefixes
+  size_t cap = (size_t)1 << 15;
+  while (cap < (size_t)2 * c->L * c->L && cap < ((size_t)1 << 21)) cap *= 2;
+  prefix_table(c, std::max(cap, s.cap));
+  prefix_clear(c);
+  std::fill(s.ub, s.ub + AM_MAX_LINEAR + 1, 0);
+}
+
+// Storage for `ids` ids of every depth: more blocks where needed, cut from
+// allocations that at least double the storage (an allocation takes 0.1 to 0.4
+// ms whatever its size).  False when that would pass the bound (or the device's
+// memory) and `must` is not set.
+bool prefix_blocks(am_ctx* c, const long long* ids, bool must) {
+  PrefixStore& s = c->pfx;
+  size_t want = 0;
+  for (int d = 1; d <= s.dev.nd; ++d) {
+    const size_t need = (size_t)((ids[d] + AM_PFX_IDS - 1) >> AM_PFX_SHIFT);
+    if (need > AM_PFX_BLOCKS) {
+      if (must) throw CapErr{"too many activation prefixes in one launch"};
+      return false;
+    }
+    if (need > s.blocks[d].size()) want += (need - s.blocks[d].size()) * prefix_block_bytes(c->nodes[d + 1]);
+  }
+  if (want == 0) return true;
+  if (s.arena_left < want) {
+    size_t bytes = std::max<size_t>(want, std::min<size_t>(s.bytes, kPrefixBytes > s.bytes ? kPrefixBytes - s.bytes : 0));
+    bool fits = s.bytes + want <= kPrefixBytes;
+    if (fits && s.bytes + bytes > ((size_t)512 << 20)) {
+      // many contexts may share the device: leave a quarter of it free
+      size_t fr = 0, all = 0;
+      fits = hipMemGetInfo(&fr, &all) == hipSuccess && fr > all / 4 + bytes;
+    }
+    if (!fits && !must) return false;
+    if (!fits) bytes = want;
+    DevBuf<char> b;
+    const hipError_t er = hipMalloc(&b.p, bytes);
+    if (er != hipSuccess) {
+      (void)hipGetLastError();
+      b.p = nullptr;
+      if (must) throw HipErr{er, "hipMalloc of the activation prefixes' planes"};
+      return false;
+    }
+    b.n = bytes;
+    s.bytes += bytes;
+    s.arena_left = bytes;
+    s.arena = b.p;
+    s.arenas.push_back(std::move(b));
+  }
+  PrefixPtrs ptrs{};
+  auto flush = [&]() {
+    if (!ptrs.n) return;
+    hipLaunchKernelGGL(k_prefix_ptrs, dim3(1), dim3(64), 0, c->stream, s.blk.p, ptrs);
+    HIPCHK(hipGetLastError());
+    ptrs.n = 0;
+  };
+  for (int d = 1; d <= s.dev.nd; ++d) {
+    const size_t need = (size_t)((ids[d] + AM_PFX_IDS - 1) >> AM_PFX_SHIFT), bytes = prefix_block_bytes(c->nodes[d + 1]);
+    while (s.blocks[d].size() < need) {
+      ptrs.at[ptrs.n] = d * AM_PFX_BLOCKS + (int)s.blocks[d].size();
+      ptrs.p[ptrs.n++] = s.arena;
+      s.blocks[d].push_back(s.arena);
+      s.arena += bytes;
+      s.arena_left -= bytes;
+      if (ptrs.n == 24) flush();
+    }
+  }
+  flush();
+  return true;
+}
+
+// Plans the prefix stages of a level of `count` regions in launches of `chunk`:
+// storage, table size, and before which launches the table starts over.  Host
+// work and allocations only happen here, so the launches can be captured.
+void prefix_plan(am_ctx* c, int count, size_t chunk) {
+  PrefixStore& s = c->pfx;
+  const int nd = s.dev.nd;
+  s.reset.clear();
+  ensure(s.rslot, std::min<size_t>(chunk, (size_t)count) * std::max(nd, 1), false, c->stream);
+  s.dev.rslot = s.rslot.p;
+  s.dev.fresh_stride = (int)std::min<size_t>(chunk, (size_t)count);
+  ensure(s.fresh, (size_t)(nd + 1) * s.dev.fresh_stride, false, c->stream);
+  s.dev.fresh = s.fresh.p;
+  size_t most = 0;
+  long long ub0[AM_MAX_LINEAR + 1];
+  std::copy(s.ub, s.ub + AM_MAX_LINEAR + 1, ub0);
+  for (int off = 0; off < count; off += (int)chunk) {
+    const int n = std::min<int>((int)chunk, count - off);
+    long long ids[AM_MAX_LINEAR + 1] = {0};
+    size_t sum = 0;
+    for (int d = 1; d <= nd; ++d) sum += (size_t)(ids[d] = s.ub[d] + n);
+    bool reset = sum > ((size_t)1 << 27) || !prefix_blocks(c, ids, false);
+    if (reset) {
+      sum = 0;
+      for (int d = 1; d <= nd; ++d) sum += (size_t)(ids[d] = n);
+      prefix_blocks(c, ids, true);
+    }
+    s.reset.push_back(reset ? 1 : 0);
+    std::copy(ids, ids + AM_MAX_LINEAR + 1, s.ub);
+    most = std::max(most, sum);
+  }
+  size_t cap = s.cap;
+  while (cap < 2 * most) cap *= 2;
+  if (cap != s.cap) {
+    // the ids so far move to a larger table
+    DevBuf<unsigned long long> old = std::move(s.tab);
+    DevBuf<int> old_id = std::move(s.tab_id);
+    prefix_table(c, cap);
+    hipLaunchKernelGGL(k_fill_u32, dim3(blocks(2 * cap, 256)), dim3(256), 0, c->stream,
+                       reinterpret_cast<uint32_t*>(s.tab.p), 2 * cap, 0xffffffffu);
+    for (int d = 1; d <= nd; ++d)
+      if (ub0[d] > 0)
+        hipLaunchKernelGGL(k_prefix_rehash, dim3(blocks((size_t)ub0[d], 256)), dim3(256), 0, c->stream, c->net, s.dev,
+                           (const uint32_t*)c->reg_mask.p, d, (int)ub0[d]);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(c->stream));   // the old table's last readers
+  }
+}
+
+// The planes of the regions of one launch (chunk k of the plan).
+void prefix_launch(am_ctx* c, size_t k, const int* ids, int first, int n, const int* dcount, int dbase) {
+  PrefixStore& s = c->pfx;
+  if (s.reset[k]) prefix_clear(c);
+  s.dev.clk = c->clock;
+  if (s.dev.nd == 0) return;
+  PrefixRegions rg;
+  rg.reg_mask = c->reg_mask.p;
+  rg.ids = ids;
+  rg.first = first;
+  rg.count = n;
+  rg.dcount = dcount;
+  rg.dbase = dbase;
+  hipLaunchKernelGGL(k_prefix, dim3(blocks(n, AM_PFX_REGIONS), s.dev.nd), dim3(4 * AM_PFX_REGIONS), 0, c->stream, c->net,
+                     s.dev, rg);
+  HIPCHK(hipGetLastError());
+  const size_t lds = prefix_layer_lds(c);
+  for (int d = 1; d <= s.dev.nd; ++d) {
+    const int nout = c->nodes[d + 1];
+    hipLaunchKernelGGL((c->skips[d].empty() ? k_layer<false> : k_layer<true>), dim3(blocks(n, AM_PT), (nout + 127) / 128),
+                       dim3(256), lds, c->stream, c->net, s.dev, rg, d);
+    HIPCHK(hipGetLastError());
+  }
+}
+
+// Buffers of run_fp64_regions for a level of `count` regions and the plan of
+// its prefix stages; to be called once before it (and before a capture).
+void fp64_prepare(am_ctx* c, int count) {
+  const size_t chunk = prefix_chunk(c);
   const size_t cap = std::min<size_t>(chunk, (size_t)count);
-  ensure(c->tplanes, cap * 4 * Ch, false, c->stream);
   ensure(c->teq, cap * 4, false, c->stream);
   ensure(c->tslots, 2 * cap, false, c->stream);   // the near walk's leavings, then the ray walk's
   ensure(c->tcnt, 2, false, c->stream);
-  return chunk;
+  prefix_plan(c, count, chunk);
 }
 
+// FP64 planes + walk of `count` regions (region ids first.., or ids[0..count)),
+// in chunks; candidate slots and flags are numbered from `lvl_first`.  Planes
+// come from the activation prefixes, the walk is the near walk and, for what it
+// leaves, the walk over all constraints.  mode 0: the candidate scan's records
+// (those of the CPU restatement, bit for bit); mode 1: the checked FP64 ray
+// walk's, and the scan's for the regions that leaves undecided; mode 2: after a
+// reduced-precision walk that flagged the level in rflags (`undecided` of them,
+// -1 when the count is not known on the host): the regions it decided get FP64
+// vertices (k_vertex_fp64, their other records stay as written), the others go
+// through mode 1.
+// Nothing here waits for the device.
 void run_fp64_regions(am_ctx* c, int lvl_first, int first, int count, const int* ids, int mode, Fp64Counts& t,
                       long long undecided = -1, const int* dcount = nullptr) {
-  if (!c->tile_ok) {
-    // one region per workgroup: the chain and the candidate scan in one kernel
-    if (ids) {
-      launch_region_fp64(c, lvl_first, count, ids);
-    } else {
-      launch_region_fp64(c, first, count);
-    }
-    t.scanned_host += count;
-    return;
-  }
   const bool after_walk = mode == 2;
   if (after_walk) mode = 1;
-  if (mode == 1 && ray64_lds_bytes(c) > c->max_lds) mode = 0;
+  // nets with skips or layers over 256 wide keep the candidate scan's records in every form
+  if (mode == 1 && (ray64_lds_bytes(c) > c->max_lds || !c->tile_ok)) mode = 0;
   int Cs, Csort;
   const size_t wlds = region_lds_bytes(c, Cs, Csort);
   const size_t rlds = ray64_lds_bytes(c);
-  const int Ch = (c->C + 63) & ~63;
-  const size_t chunk = fp64_prepare(c, count);
-  const size_t clds = chain_lds_bytes(c), hlds = chain_half_lds_bytes(c);
-  StageTimer& tm = c->timer;
+  const size_t chunk = prefix_chunk(c);
   // regions the reduced walk may have decided with a vertex left to FP64 (the
   // FP32 form's Newton modes leave none)
   const WalkParams& rw = c->fast.wp;
   const bool vert64 = rw.lam_v < 0.f || (rw.lam_v > 0.f && !rw.vsel);
+  const WalkParams& kr = c->chain_mfma ? kRay64Mf : kRay64;
   // the near walk lists the regions it leaves to the walk over all constraints,
-  // the ray walk those it leaves to the candidate scan (the chain zeroes both
-  // counters)
+  // the ray walk those it leaves to the candidate scan
   const size_t nlds = near_lds_bytes(c->C, c->Wd, c->vm, 8, false);
+  const size_t qlds = std::max(wlds, nlds);
   const NearList near{c->tcnt.p, c->tslots.p};
   const size_t lcap = std::min<size_t>(chunk, (size_t)count);
-  for (int off = 0; off < count; off += (int)chunk) {
+  size_t k = 0;
+  for (int off = 0; off < count; off += (int)chunk, ++k) {
     const int n = std::min<int>((int)chunk, count - off);
-    ChainIO cio = chain_io(c, ids ? ids + off : nullptr, first + off, n, Ch);
-    cio.dcount = dcount;
-    cio.dbase = off;
-    cio.zero = c->tcnt.p;
     RegionIO io;
     io.reg_mask = c->reg_mask.p;
     io.reg_start = c->reg_start.p;
@@ -638,65 +840,36 @@ void run_fp64_regions(am_ctx* c, int lvl_first, int first, int count, const int*
     io.ids = ids ? ids + off : nullptr;
     io.dcount = dcount;
     io.dbase = off;
-    const size_t m0 = tm.mark(c->stream);
-    // the records of the candidate scan on every region (mode 0) are the
-    // oracle's bit for bit: its planes come from the sequential-fma chain
-    const bool mf = c->chain_mfma && (mode != 0 || after_walk);
-    if (mf)
-      hipLaunchKernelGGL(k_chain_tile_mfma, dim3((n + AM_HT - 1) / AM_HT), dim3(AM_HALF_THREADS), hlds, c->stream,
-                         c->net, cio);
-    else
-      hipLaunchKernelGGL(k_chain_tile_fp64, dim3((n + AM_CT - 1) / AM_CT), dim3(AM_CHAIN_THREADS), clds, c->stream,
-                         c->net, cio);
-    HIPCHK(hipGetLastError());
+    const int rid0 = first + off;
+    io.clk = c->clock;
+    if (k > 0)   // (the level's first launch finds them cleared)
+      hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, c->tcnt.p, (size_t)2, 0);
+    prefix_launch(c, k, io.ids, rid0, n, dcount, off);
     t.chain_launches += 1;
-    const size_t m1 = tm.mark(c->stream);
-    tm.span(m0, m1, T_CHAIN64);
-    size_t m1v = m1;
     if (after_walk && undecided != count && vert64) {
-      hipLaunchKernelGGL(k_vertex_fp64, dim3(n), dim3(64), 0, c->stream, c->net, io, first + off,
-                         (const double*)c->tplanes.p, (const double*)c->teq.p, Ch);
+      hipLaunchKernelGGL(k_vertex_fp64, dim3(n), dim3(64), 0, c->stream, c->net, c->pfx.dev, io, rid0);
       HIPCHK(hipGetLastError());
-      m1v = tm.mark(c->stream);
-      tm.span(m1, m1v, T_VERT64);
     }
-    if (after_walk && undecided == 0) continue;
-    if (mode == 0 && !after_walk) {
-      hipLaunchKernelGGL(k_near64<true>, dim3(n), dim3(64), nlds, c->stream, c->net, io, first + off, kRay64,
-                         (const double*)c->tplanes.p, (const double*)c->teq.p, Ch, 0, near);
-      hipLaunchKernelGGL(k_walk_fp64, dim3(std::min(n, c->scan_blocks)), dim3(64), wlds, c->stream, c->net, io,
-                         first + off, (const int*)near.cnt, (const int*)near.slots, (const double*)c->tplanes.p,
-                         (const double*)c->teq.p, Ch);
+    if (mode == 0) {
+      hipLaunchKernelGGL(k_near64<true>, dim3(n), dim3(64), nlds, c->stream, c->net, c->pfx.dev, io, rid0, kr,
+                         c->teq.p, after_walk ? 1 : 0, near);
+      io.flags = nullptr;
+      hipLaunchKernelGGL(k_walk_fp64, dim3(std::min(n, c->scan_blocks)), dim3(64), qlds, c->stream, c->net,
+                         c->pfx.dev, io, rid0, (const int*)near.cnt, (const int*)near.slots, (const double*)c->teq.p, 1);
       HIPCHK(hipGetLastError());
-      tm.span(m1, tm.mark(c->stream), T_SCAN64);
       t.scanned_host += n;
       continue;
     }
-    if (mode == 1) {
-      hipLaunchKernelGGL(k_near64<false>, dim3(n), dim3(64), nlds, c->stream, c->net, io, first + off,
-                         mf ? kRay64Mf : kRay64, (const double*)c->tplanes.p, (const double*)c->teq.p, Ch,
-                         after_walk ? 1 : 0, near);
-      HIPCHK(hipGetLastError());
-      launch_ray64(c, n, rlds, io, first + off, Ch, mf ? kRay64Mf : kRay64, near,
-                   SlotList{c->tcnt.p + 1, c->tslots.p + lcap, c->runacc.p});
-      HIPCHK(hipGetLastError());
-      const size_t m2 = tm.mark(c->stream);
-      tm.span(m1v, m2, T_RAY64);
-    } else {
-      hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, c->tcnt.p, (size_t)1, 0);
-      hipLaunchKernelGGL(k_collect_slots, dim3((n + 255) / 256), dim3(256), 0, c->stream,
-                         (const unsigned*)c->rflags.p, n, dcount, off, (const int*)(ids ? ids + off : nullptr),
-                         first + off, lvl_first, c->tcnt.p, c->tslots.p, c->runacc.p);
-      HIPCHK(hipGetLastError());
-    }
-    io.flags = nullptr;
-    const size_t m3 = tm.mark(c->stream);
-    hipLaunchKernelGGL(k_walk_fp64, dim3(std::min(n, c->scan_blocks)), dim3(64), wlds, c->stream, c->net, io, first + off,
-                       (const int*)(mode == 1 ? c->tcnt.p + 1 : c->tcnt.p),
-                       (const int*)(mode == 1 ? c->tslots.p + lcap : c->tslots.p), (const double*)c->tplanes.p,
-                       (const double*)c->teq.p, Ch);
+    const SlotList left{c->tcnt.p + 1, c->tslots.p + lcap, c->acc};
+    hipLaunchKernelGGL(k_near64<false>, dim3(n), dim3(64), nlds, c->stream, c->net, c->pfx.dev, io, rid0, kr, c->teq.p,
+                       after_walk ? 1 : 0, near);
     HIPCHK(hipGetLastError());
-    tm.span(m3, tm.mark(c->stream), T_SCAN64);
+    launch_ray64(c, n, rlds, io, rid0, kr, near, left);
+    HIPCHK(hipGetLastError());
+    io.flags = nullptr;
+    hipLaunchKernelGGL(k_walk_fp64, dim3(std::min(n, c->scan_blocks)), dim3(64), wlds, c->stream, c->net, c->pfx.dev,
+                       io, rid0, (const int*)left.cnt, (const int*)left.slots, (const double*)c->teq.p, 0);
+    HIPCHK(hipGetLastError());
   }
 }
 
@@ -999,6 +1172,17 @@ void batch_hist(am_batch* b, long long first, long long count) {
 // ---------------------------------------------------------------------------
 namespace {
 
+// A run's counters, stage clock and walk counters, cleared.
+__global__ void k_run_begin(int* p, int n, StageClock* clk, int* zero) {
+  for (int i = threadIdx.x; i < n; i += 256) p[i] = 0;
+  if (threadIdx.x < 2) zero[threadIdx.x] = 0;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    clk->last = wall_clock64();
+    clk->slot = T_SLOTS;
+  }
+}
+
 // Whether p is ordinary (pageable) host memory: not device, pinned or managed.
 bool pageable_host(const void* p) {
   hipPointerAttribute_t a;
@@ -1269,7 +1453,6 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
     if (lds > c->max_lds)
       throw CapErr{"network too wide for the FP64 region kernel's LDS (" + std::to_string(lds) + " bytes)"};
     if (lds > 65536) {
-      HIPCHK(hipFuncSetAttribute((const void*)k_region_fp64, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
       HIPCHK(hipFuncSetAttribute((const void*)k_walk_fp64, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     }
     c->tile_ok = true;
@@ -1283,12 +1466,9 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
       else if (clds > 65536) {
         HIPCHK(hipFuncSetAttribute((const void*)k_chain_tile_fp64, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)clds));
-        const size_t hlds = chain_half_lds_bytes(c);
-        if (hlds > 65536)
-          HIPCHK(hipFuncSetAttribute((const void*)k_chain_tile_mfma, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)hlds));
       }
     }
+    prefix_setup(c, tms, dtype);
     // The reduced forms need the tiled FP64 chain for their vertices and
     // re-decisions; nets it does not take (skips, layers over 256 wide) run
     // those forms on the FP64 region kernel, with the same topology.
@@ -1339,18 +1519,29 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
     }
     hipLaunchKernelGGL(k_hash_keys, dim3(blocks(n_seeds, 256)), dim3(256), 0, st, (const uint32_t*)c->cand_mask.p,
                        n_seeds, c->Wd, c->cand_hash.p);
+    // run counters on the device: [0, 1 + W) the FP64 ray walk's undecided
+    // regions and reasons, [1 + W, 2 + 2W) the reduced-precision walk's, then
+    // the regions it decided with a vertex left to FP64; then the stage clock
+    constexpr int NACC = 2 * (1 + AM_WHY_COUNT) + 1;
+    struct RunAcc {
+      StageClock clock;
+      int acc[NACC];
+    };
+    ensure(c->runacc, (sizeof(RunAcc) + 3) / 4, false, st);
+    RunAcc* const ra_dev = reinterpret_cast<RunAcc*>(c->runacc.p);
+    int* const acc_dev = ra_dev->acc;
+    c->acc = acc_dev;
+    c->clock = &ra_dev->clock;
+    ensure(c->tcnt, 2, false, st);
+    hipLaunchKernelGGL(k_run_begin, dim3(1), dim3(256), 0, st, c->runacc.p, (int)(sizeof(RunAcc) / 4), c->clock,
+                       c->tcnt.p);
+    HIPCHK(hipGetLastError());
     long long lvl_first = 0;
     long long lvl_count = insert_level(c, (size_t)n_seeds);
     long long levels = 0, cands = 0, launches = 0;
     long long why[AM_WHY_COUNT] = {0};
     Fp64Counts f64;
     c->timer.reset();
-    // run counters on the device: [0, 1 + W) the FP64 ray walk's undecided
-    // regions and reasons, [1 + W, 2 + 2W) the reduced-precision walk's, then
-    // the regions it decided with a vertex left to FP64
-    constexpr int NACC = 2 * (1 + AM_WHY_COUNT) + 1;
-    ensure(c->runacc, NACC, false, st);
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, c->runacc.p, (size_t)NACC, 0);
     while (lvl_count > 0) {
       if (c->max_regions >= 0 && lvl_first >= c->max_regions) break;
       const size_t ncand = (size_t)lvl_count * c->vm;
@@ -1359,7 +1550,7 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
       if (fp64_form && c->graph_levels) {
         // the level's launches (planes, walks, visited-set insert and commit)
         // as one graph; the host work (growth) happens before the capture
-        if (c->tile_ok) fp64_prepare(c, (int)lvl_count);
+        fp64_prepare(c, (int)lvl_count);
         const InsertPlan plan = insert_prepare(c, ncand);
         launch_as_graph(c, (int)levels, [&]() {
           run_fp64_regions(c, (int)lvl_first, (int)lvl_first, (int)lvl_count, nullptr,
@@ -1392,7 +1583,7 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
       if (!fp64_form && c->graph_levels) {
         // as the FP64 forms' graph above: the host work first (buffers, the
         // region store's growth), then every launch of the level in one graph
-        if (c->tile_ok) fp64_prepare(c, (int)lvl_count);
+        fp64_prepare(c, (int)lvl_count);
         fast_level_prepare(c->fast, c->fbuf, n, (int)lvl_count);
         ensure(c->redo_ids, (size_t)lvl_count, false, st);
         ensure(c->redo_cnt, 1, false, st);
@@ -1402,7 +1593,7 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
         const RedoList redo{c->redo_ids.p, c->redo_cnt.p, c->redo_state.p};
         FastTimes ft{};
         launch_as_graph(c, (int)levels, [&]() {
-          fast_level(c->fast, c->fbuf, n, fl, st, c->timer, ft, c->rflags.p, c->runacc.p + 1 + AM_WHY_COUNT, redo,
+          fast_level(c->fast, c->fbuf, n, fl, st, c->clock, ft, c->rflags.p, acc_dev + 1 + AM_WHY_COUNT, redo,
                      true);
           run_fp64_regions(c, (int)lvl_first, (int)lvl_first, (int)lvl_count, c->redo_ids.p, 2, f64, -1,
                            c->redo_cnt.p);
@@ -1417,6 +1608,7 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
         lvl_count = added;
         continue;
       }
+      fp64_prepare(c, (int)lvl_count);
       if (fp64_form) {
         run_fp64_regions(c, (int)lvl_first, (int)lvl_first, (int)lvl_count, nullptr,
                          c->precision == AM_PREC_FP64 ? 0 : 1, f64);
@@ -1428,7 +1620,7 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
         ensure_zeroed(c->redo_state, redo_state_words((int)lvl_count), st);
         const RedoList redo{c->redo_ids.p, c->redo_cnt.p, c->redo_state.p};
         FastTimes ft{};
-        fast_level(c->fast, c->fbuf, n, fl, st, c->timer, ft, c->rflags.p, c->runacc.p + 1 + AM_WHY_COUNT, redo);
+        fast_level(c->fast, c->fbuf, n, fl, st, c->clock, ft, c->rflags.p, acc_dev + 1 + AM_WHY_COUNT, redo);
         // FP64 planes of the regions the walk left to FP64 only (their list,
         // made by fast_level's last launch, and count stay on the device;
         // the launches are sized for the whole
@@ -1441,10 +1633,8 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
                          c->redo_cnt.p);
         launches += ft.launches;
       }
-      const size_t mi = c->timer.mark(st);
       const long long before = c->R;
       const int added = insert_level(c, ncand);   // waits once: the next level's size
-      c->timer.span(mi, c->timer.mark(st), T_INSERT);
       cands += (long long)ncand;
       levels += 1;
       lvl_first = before;
@@ -1460,21 +1650,24 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
       newton_n = newton_refine(c);
       c->timer.span(mn, c->timer.mark(st), T_NEWTON);
     }
-    int acc[NACC] = {0};
-    HIPCHK(hipMemcpyAsync(acc, c->runacc.p, sizeof(acc), hipMemcpyDeviceToHost, st));
+    RunAcc ra{};
+    HIPCHK(hipMemcpyAsync(&ra, ra_dev, sizeof(ra), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    const int* acc = ra.acc;
     const long long redo = fp64_form ? 0 : acc[1 + AM_WHY_COUNT];
     const long long vert64 = fp64_form ? 0 : acc[2 + 2 * AM_WHY_COUNT];
-    HIPCHK(hipStreamSynchronize(st));
     c->timer.resolve();
     const auto t1 = std::chrono::steady_clock::now();
-    const double* T = c->timer.acc;
-    const double fp64_ms = T[T_CHAIN64] + T[T_RAY64] + T[T_SCAN64] + T[T_REGION64] + T[T_VERT64];
+    double T[T_SLOTS];
+    for (int i = 0; i < T_SLOTS; ++i) T[i] = (double)ra.clock.acc[i] * kStageTickMs;
+    T[T_NEWTON] = c->timer.acc[T_NEWTON];
+    const double fp64_ms = T[T_CHAIN64] + T[T_RAY64] + T[T_SCAN64] + T[T_VERT64];
     c->stats[AM_STAT_RUN_MS] = std::chrono::duration<double, std::milli>(t1 - t0).count();
     c->stats[AM_STAT_INSERT_MS] = T[T_INSERT];
     if (fp64_form) {
       c->stats[AM_STAT_REGION_MS] = fp64_ms;
       c->stats[AM_STAT_GEMM_MS] = T[T_CHAIN64];
-      c->stats[AM_STAT_WALK_MS] = T[T_RAY64] + T[T_SCAN64] + T[T_REGION64];
+      c->stats[AM_STAT_WALK_MS] = T[T_RAY64] + T[T_SCAN64];
       c->stats[AM_STAT_REDO_MS] = 0;
       for (int w = 0; w < AM_WHY_COUNT; ++w) why[w] = acc[1 + w];
     } else {
@@ -1490,7 +1683,7 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
     c->stats[AM_STAT_REDO_REGIONS] = (double)redo;
     c->stats[AM_STAT_REGION_LAUNCHES] = (double)launches;
     c->stats[AM_STAT_CHAIN64_MS] = T[T_CHAIN64];
-    c->stats[AM_STAT_WALK64_MS] = T[T_SCAN64] + T[T_REGION64];
+    c->stats[AM_STAT_WALK64_MS] = T[T_SCAN64];
     c->stats[AM_STAT_RAY64_MS] = T[T_RAY64];
     c->stats[AM_STAT_SCAN64_REGIONS] = (double)(f64.scanned_host + acc[0]);
     c->stats[AM_STAT_RAY64_UNDECIDED] = (double)acc[0];

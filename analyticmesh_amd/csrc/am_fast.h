@@ -102,11 +102,11 @@ size_t redo_state_words(int count);
 // undecided or AM_VERT64 into `redo` (in region order) and adds the undecided
 // ones to acc[0], their reasons to acc[1 + w] and the AM_VERT64 ones to
 // acc[1 + AM_WHY_COUNT] on the device; nothing here waits.
-// Kernel times go to `timer` (T_GEMM, T_WALK).
+// Kernel times go to `clk` (T_GEMM, T_WALK).
 // With `prepared`, fast_level_prepare(f, b, net, lvl.count) has run before
 // (then fast_level only enqueues launches: it can be captured into a graph).
 void fast_level(FastNet& f, FastBuffers& b, const NetDev& net, const FastLevel& lvl, hipStream_t st,
-                StageTimer& timer, FastTimes& t, unsigned* flags, int* acc, const RedoList& redo,
+                StageClock* clk, FastTimes& t, unsigned* flags, int* acc, const RedoList& redo,
                 bool prepared = false);
 // Buffers and launch attributes of fast_level for a level of `count` regions.
 void fast_level_prepare(FastNet& f, FastBuffers& b, const NetDev& net, int count);

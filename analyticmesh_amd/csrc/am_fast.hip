@@ -45,6 +45,7 @@ struct GemmIO {
   int count;        // regions in this chunk
   float* planes;    // [count][4][Cs]
   float* eq;        // [count][4]
+  StageClock* clk = nullptr;
 };
 
 __device__ __forceinline__ uint16_t bf16_rn(float x) {
@@ -131,6 +132,7 @@ __device__ void stage_layer1(const FastNetDev& f, const GemmIO& io, const uint32
 
 template <int PREC>
 __global__ __launch_bounds__(256, PREC == 0 ? 4 : 1) void k_gemm(FastNetDev f, GemmIO io) {
+  stage_mark(io.clk, T_GEMM);
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int KS = f.Kpad + 8;   // bf16 column stride (halves)
@@ -428,6 +430,7 @@ __global__ __launch_bounds__(256, PREC == 0 ? 4 : 1) void k_gemm(FastNetDev f, G
 // Checked FP32 walk of one region whose planes the face kernel wrote.
 __global__ __launch_bounds__(64) void k_walk_f32(NetDev net, RegionIO io, WalkParams wp, const float* planes,
                                                  const float* eqbuf, int Cs_hbm, int chunk_first) {
+  stage_mark(io.clk, T_WALK);
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int C = net.C;
   const int Cs = io.Cs, N2 = io.Csort;
@@ -469,6 +472,7 @@ __global__ __launch_bounds__(64) void k_walk_f32(NetDev net, RegionIO io, WalkPa
 template <int NW>
 __global__ __launch_bounds__(64 * NW, 24 / NW) void k_walk_ray_f32(NetDev net, RegionIO io, WalkParams wp, const float* planes,
                                                           const float* eqbuf, int Cs_hbm, int chunk_first) {
+  stage_mark(io.clk, T_WALK);
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int C = net.C;
   const int Cs = io.Cs;
@@ -518,6 +522,7 @@ struct FacePlanes {
 // take k_walk_ray_f32).
 __global__ __launch_bounds__(64, 5) void k_near_f32(NetDev net, RegionIO io, WalkParams wp, const float* planes,
                                                  const float* eqbuf, int Cs_hbm, int chunk_first) {
+  stage_mark(io.clk, T_WALK);
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int b = blockIdx.x;
   if (b >= io.count) return;
@@ -830,7 +835,7 @@ void fast_level_prepare(FastNet& f, FastBuffers& b, const NetDev& net, int count
 }
 
 void fast_level(FastNet& f, FastBuffers& b, const NetDev& net, const FastLevel& lvl, hipStream_t st,
-                StageTimer& timer, FastTimes& t, unsigned* flags, int* acc, const RedoList& redo, bool prepared) {
+                StageClock* clk, FastTimes& t, unsigned* flags, int* acc, const RedoList& redo, bool prepared) {
   const FastNetDev& d = f.dev;
   const int prec = f.precision == 1 ? 1 : 0;
   t.launches = 0;
@@ -854,14 +859,12 @@ void fast_level(FastNet& f, FastBuffers& b, const NetDev& net, const FastLevel& 
     g.count = n;
     g.planes = planes;
     g.eq = eqb;
-    const size_t m0 = timer.mark(st);
+    g.clk = clk;
     if (prec == 0)
       hipLaunchKernelGGL(k_gemm<0>, dim3((n + AM_GT - 1) / AM_GT), dim3(256), glds, st, d, g);
     else
       hipLaunchKernelGGL(k_gemm<1>, dim3((n + AM_GT - 1) / AM_GT), dim3(256), glds, st, d, g);
     FCHK(hipGetLastError());
-    const size_t m1 = timer.mark(st);
-    timer.span(m0, m1, T_GEMM);
 
     RegionIO io;
     io.reg_mask = lvl.reg_mask;
@@ -881,6 +884,7 @@ void fast_level(FastNet& f, FastBuffers& b, const NetDev& net, const FastLevel& 
     io.Cs = CsL;
     io.Csort = Csort;
     io.flags = flags;
+    io.clk = clk;
     io.ids = nullptr;
     // a level past the seeds, planes with estimates: the near walk
     if (f.walk_mode == 0 && prec == 0 && lvl.first > 0)
@@ -898,7 +902,6 @@ void fast_level(FastNet& f, FastBuffers& b, const NetDev& net, const FastLevel& 
       hipLaunchKernelGGL(k_walk_f32, dim3(n), dim3(64), wlds, st, net, io, f.wp, planes, eqb, d.Cs,
                          lvl.first + c0);
     FCHK(hipGetLastError());
-    timer.span(m1, timer.mark(st), T_WALK);
     t.launches += 1;
   }
   const int tiles = (int)redo_state_words(lvl.count) - 2;

@@ -70,6 +70,11 @@ struct ScanCommitIO {
   int n, tiles;
   int* rank;
   int* total;
+  StageClock* clk = nullptr;
+  // further counts handed to the host before the total
+  const int* pub = nullptr;
+  int npub = 0, pub_stride = 1;
+  int* pub_out = nullptr;
 };
 constexpr int kScanCommitThreads = 512;
 constexpr int kScanCommitItems = 8;

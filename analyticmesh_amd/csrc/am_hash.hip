@@ -75,7 +75,9 @@ __global__ __launch_bounds__(256) void k_insert(InsertIO io) {
   __shared__ int s_list[4][64];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int gtid = blockIdx.x * 256 + tid;
+  stage_mark(io.clk, T_INSERT);
   if (gtid < io.scan_words) io.scan_state[gtid] = 0ull;
+  if (io.zero && gtid < 2) io.zero[gtid] = 0;
   const int c = gtid;
   bool live = false;
   if (c < io.n) {
@@ -192,7 +194,12 @@ __global__ __launch_bounds__(kScanCommitThreads) void k_scan_commit(ScanCommitIO
     }
     if (lane == 0) {
       s_excl = excl;
-      if (t == io.tiles - 1 && io.total) *io.total = excl + tot;
+      if (t == io.tiles - 1 && io.total) {
+        for (int i = 0; i < io.npub; ++i) io.pub_out[i] = io.pub[i * io.pub_stride];
+        if (io.clk) stage_mark_now(io.clk, T_SLOTS);
+        if (io.npub) __threadfence_system();
+        *io.total = excl + tot;
+      }
     }
   }
   __syncthreads();

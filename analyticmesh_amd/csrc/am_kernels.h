@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include "am_limits.h"
+#include "am_timer.h"
 
 namespace am {
 
@@ -28,6 +29,7 @@ struct RegionIO {
   const int* ids;             // optional: region ids to process (FP64 re-decision); else first + blockIdx.x
   const int* dcount = nullptr;  // optional: ids past *dcount - dbase are not valid (a launch sized on
   int dbase = 0;                // the host for the worst case; blocks past the device count exit)
+  StageClock* clk = nullptr;    // the march's stage times, if taken
   uint16_t* reg_jinv = nullptr; // optional [R][vm][9] bf16: per vertex the inverse of its 3x3 system
                                 // from the reduced planes (columns for the new, walked and face plane),
                                 // for the FP64 Newton step (a record with it has info[7] = 1)
@@ -52,9 +54,9 @@ struct InsertIO {
   uint32_t cap_mask;
   unsigned long long* scan_state;  // [scan_words] tile states of the level's one-pass scan, cleared here
   int scan_words;
+  int* zero = nullptr;             // two counters of the walks, cleared for the next level
+  StageClock* clk = nullptr;
 };
-
-__global__ void k_region_fp64(NetDev net, RegionIO io);
 
 // Tiled FP64 chain: the planes of a tile of regions in HBM, for the walk kernel.
 #define AM_CT 16                // regions per chain workgroup
@@ -67,12 +69,6 @@ __global__ void k_region_fp64(NetDev net, RegionIO io);
 #define AM_KLS (AM_CHAIN_MAXW + 2 * AM_CPF)   // entries of one layer's active-input list
 #define AM_CXR (AM_CHAIN_MAXW + AM_CPF)       // rows of the chain's layer buffer (list positions + prefetch)
 #define AM_CHAIN_THREADS (64 * AM_CHAIN_MAXW / AM_CR)
-// Half tiles of the matrix-core chain (k_chain_tile_mfma)
-#define AM_HT 8                 // regions per workgroup
-#define AM_HN (4 * AM_HT)       // columns
-#define AM_HXS (AM_HN + 1)      // LDS row stride (doubles)
-#define AM_HALF_THREADS 512     // 8 waves, 32 output rows each
-
 struct ChainIO {
   const uint32_t* reg_mask;   // [R][Wd]
   const int* ids;             // optional region ids; else first + tile-local index
@@ -86,7 +82,6 @@ struct ChainIO {
   int noutp[AM_MAX_LINEAR];         // n_out rounded up to AM_CR
   const int* dcount = nullptr;      // as in RegionIO: regions past *dcount - dbase are not valid
   int dbase = 0;
-  int* zero = nullptr;              // two counters set to 0 by the launch (later launches of the chunk fill them)
 };
 
 // A list of chunk-local slots filled by atomics (cnt zeroed before), with
@@ -113,34 +108,12 @@ struct ChainLevel {
 };
 
 __global__ void k_chain_tile_fp64(NetDev net, ChainIO io);
-// The same planes with the products on the FP64 matrix cores: equal up to the
-// rounding of another summation order (the forms that certify their decisions).
-// Tiles of AM_HT regions, AM_HALF_THREADS threads, LDS chain_half_lds_bytes.
-__global__ void k_chain_tile_mfma(NetDev net, ChainIO io);
 // A batch of networks (each region's network is the last word of its mask):
 // tiles[b] = (network, first slot, regions, -) of one network.
 // MF: the products on the matrix cores (k_chain_tile_mfma).
 template <bool MF>
 __global__ void k_chain_tile_fp64_multi(const NetDev* nets, const ChainIO* cios, ChainLevel lv, const int4* tiles);
-// The walk of k_region_fp64 on planes from k_chain_tile_fp64.  Block b takes
-// planes slot s = slots[b] (or b); its region is io.ids[s] when ids are given,
-// else rid0 + s; candidate slots are numbered from io.first as in k_region_fp64.
-// With `count`, blocks at or past *count exit (a grid sized for the worst case).
-__global__ void k_walk_fp64(NetDev net, RegionIO io, int rid0, const int* count, const int* slots,
-                            const double* planes, const double* eq, int Cs_hbm);
 struct WalkParams;
-// The near walk (am_near.h) on the planes of the chain: SCAN decides as
-// k_walk_fp64, else as k_walk_ray64.  Regions it leaves are listed (launch
-// slots, *left.cnt zeroed before) for those kernels.
-template <bool SCAN>
-__global__ void k_near64(NetDev net, RegionIO io, int rid0, WalkParams wp, const double* planes, const double* eq,
-                         int Cs_hbm, int only_undecided, NearList left);
-// The checked ray walk over all constraints of the regions the near walk left
-// (list; blocks stride over it).  NW waves per region: 2, 4 or 8.  The regions
-// it leaves undecided are listed in `left` as k_collect_slots lists them.
-template <int NW>
-__global__ void k_walk_ray64(NetDev net, RegionIO io, int rid0, WalkParams wp, const double* planes,
-                             const double* eq, int Cs_hbm, NearList list, SlotList left);
 // Batch-of-networks forms (region rid0 + b; its network is mask word Wd - 1;
 // the scan's LDS layout follows each network's C, the launch is sized for the
 // widest network).
@@ -154,12 +127,6 @@ __global__ void k_walk_ray64_multi(const NetDev* nets, RegionIO io, int Wd, int 
 // With dn, entries past *dn - dbase are not valid.
 __global__ void k_collect_slots(const unsigned* flags, int n, const int* dn, int dbase, const int* ids, int rid0,
                                 int lvl_first, int* cnt, int* slots, int* run);
-// FP64 vertices of regions whose topology a reduced-precision walk decided:
-// block b re-solves the face vertices of region io.ids[b] (or rid0 + b) from
-// the FP64 planes of slot b (its two tight constraints and the face plane);
-// with io.flags, regions flagged AM_UNDECIDED are skipped.
-__global__ void k_vertex_fp64(NetDev net, RegionIO io, int rid0, const double* planes, const double* eq,
-                              int Cs_hbm);
 __global__ void k_fill_i32(int* p, size_t n, int v);
 
 // Weight layouts on the device (am_layout.hip): dst[j * ni + i] = src[i * cols + j]

@@ -27,12 +27,15 @@
 namespace am {
 
 #define AM_NEAR_MAX 64        // near constraints: one per lane
+#define AM_NEAR_PL (4 * 66)   // their planes; before, the face plane's inputs [4][66] (a stride of 66: four
+                              // components read together fall into different banks)
 
 // Scratch of the near walk in dynamic LDS, ahead of the walk records.
 template <typename T>
 struct NearLds {
   T* pl;            // [64][4] the near constraints' planes, for broadcast reads
-  float* key;       // [C] squared distance of p inside each constraint (0 where outside, +inf: never a bound)
+  uint16_t* key;    // [C] squared distance of p inside each constraint (0 where outside, +inf: never a
+                    // bound), as the upper half of its FP32 bits, i.e. rounded down
   uint16_t* cand;   // [64] near constraints
   uint32_t* mask;   // [Wd]
   uint32_t* used;   // [C bits] (over key: the walk on all constraints does not need the distances)
@@ -40,7 +43,7 @@ struct NearLds {
 };
 __host__ __device__ inline size_t near_lds_bytes(int C, int Wd, int vm, int tsize, bool jinv) {
   auto a16 = [](size_t x) { return (x + 15) & ~(size_t)15; };
-  return (size_t)AM_NEAR_MAX * 4 * tsize + a16((size_t)C * 4) + AM_NEAR_MAX * 2 + a16((size_t)Wd * 4) +
+  return (size_t)AM_NEAR_PL * tsize + a16((size_t)C * 2) + AM_NEAR_MAX * 2 + a16((size_t)Wd * 4) +
          walk_rec_bytes(vm, jinv);
 }
 template <typename T>
@@ -48,10 +51,10 @@ __device__ inline NearLds<T> carve_near(unsigned char* p, int C, int Wd, int vm,
   auto a16 = [](size_t x) { return (x + 15) & ~(size_t)15; };
   NearLds<T> s;
   s.pl = reinterpret_cast<T*>(p);
-  p += (size_t)AM_NEAR_MAX * 4 * sizeof(T);
-  s.key = reinterpret_cast<float*>(p);
+  p += (size_t)AM_NEAR_PL * sizeof(T);
+  s.key = reinterpret_cast<uint16_t*>(p);
   s.used = reinterpret_cast<uint32_t*>(p);
-  p += a16((size_t)C * 4);
+  p += a16((size_t)C * 2);
   s.cand = reinterpret_cast<uint16_t*>(p);
   p += AM_NEAR_MAX * 2;
   s.mask = reinterpret_cast<uint32_t*>(p);
@@ -110,58 +113,83 @@ struct Nearest {
 // 64 constraints per lane about KT + KT^2 / 128 constraints are then within
 // it), and compacts the constraints within it in index order.
 // qmax: with per-plane estimates, the largest sigma_g / |a_g|.
-template <typename T, bool SCAN, typename Src>
-__device__ __forceinline__ int near_constraints(const Src& P, int C, const T* p, float* key, uint16_t* cand, T& r,
-                                                T& qmax) {
-  const int lane = threadIdx.x;
-  float best = __builtin_inff(), qm = 0.f;
+// One wave's pass over distances, constraint by constraint.
+template <typename T, bool SCAN>
+struct NearScan {
+  uint32_t best = 0x7f80u;              // upper halves of non-negative floats order as the values
+  float qm = 0.f;
   bool bad = false, inf = false;
-  for (int l = 0; l < P.parts(); ++l) {
-    const int n = P.size(l), g0 = P.first(l);
-    // (no branch around the loads, so that several constraints' are in flight)
-#pragma unroll 4
-    for (int j = lane; j < n; j += 64) {
-      T q[4];
-      P.load(l, j, q);
-      const float s = (float)plane_eval(q[0], q[1], q[2], q[3], p);
-      const float nn = (float)plane_nn(q[0], q[1], q[2]);
-      float u = fmaxf(-(s * fabsf(s)) * __builtin_amdgcn_rcpf(nn), 0.f);
-      const bool fine = nn > 1e-30f && nn < 1e30f && fabsf(s) < 1e15f;
-      if (sizeof(T) == 4) qm = fmaxf(qm, (float)P.err(g0 + j) * __builtin_amdgcn_rsqf(nn));
-      // a plane without a normal holds or fails everywhere; others that are
-      // out of range are left to the walks over all constraints
-      const bool holds = sizeof(T) == 8 && q[0] == T(0) && q[1] == T(0) && q[2] == T(0) &&
-                         (SCAN ? q[3] <= T(0) : q[3] < T(0));
-      bad = bad || !(fine || holds);
-      inf = inf || !fine;
-      u = fine ? u : __builtin_inff();
-      key[g0 + j] = u;
-      best = fminf(best, u);
-    }
+  // constraint g with (signed) plane q and estimate e
+  __device__ __forceinline__ void add(const T* q, T e, const T* p, uint16_t* key, int g) {
+    const float s = (float)plane_eval(q[0], q[1], q[2], q[3], p);
+    const float nn = (float)plane_nn(q[0], q[1], q[2]);
+    const float u = fmaxf(-(s * fabsf(s)) * __builtin_amdgcn_rcpf(nn), 0.f);
+    const bool fine = nn > 1e-30f && nn < 1e30f && fabsf(s) < 1e15f;
+    if (sizeof(T) == 4) qm = fmaxf(qm, (float)e * __builtin_amdgcn_rsqf(nn));
+    // a plane without a normal holds or fails everywhere; others that are out
+    // of range are left to the walks over all constraints
+    const bool holds = sizeof(T) == 8 && q[0] == T(0) && q[1] == T(0) && q[2] == T(0) &&
+                       (SCAN ? q[3] <= T(0) : q[3] < T(0));
+    bad = bad || !(fine || holds);
+    inf = inf || !fine;
+    const uint32_t k = fine ? __float_as_uint(u) >> 16 : 0x7f80u;
+    key[g] = (uint16_t)k;
+    best = min(best, k);
   }
-  if (__any(bad)) return 0;
+};
+
+// Constraints j0, j0 + 64, ... (U of them) of part l.
+template <typename T, bool SCAN, int U, typename Src>
+__device__ __forceinline__ void near_batch(const Src& P, int l, int j0, int n, int g0, const T* p, uint16_t* key,
+                                           NearScan<T, SCAN>& sc) {
+  T q[U][4], e[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int j = min(j0 + 64 * u, n - 1);
+    P.load(l, j, q[u]);
+    e[u] = sizeof(T) == 4 ? T(P.err(g0 + j)) : T(0);
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (j0 + 64 * u < n) sc.add(q[u], e[u], p, key, g0 + j0 + 64 * u);
+}
+
+// sc, skip: the pass so far, and the part of the constraints it has done (-1: none).
+template <typename T, bool SCAN, typename Src>
+__device__ __forceinline__ int near_constraints(const Src& P, int C, const T* p, uint16_t* key, uint16_t* cand, T& r,
+                                                T& qmax, NearScan<T, SCAN> sc, int skip) {
+  const int lane = threadIdx.x;
+  for (int l = 0; l < P.parts(); ++l) {
+    if (l == skip) continue;
+    const int n = P.size(l), g0 = P.first(l);
+    // several constraints' loads in flight: up to four per lane, then their distances
+    int j0 = lane;
+    for (; j0 - lane + 128 < n; j0 += 256) near_batch<T, SCAN, 4>(P, l, j0, n, g0, p, key, sc);
+    for (; j0 - lane < n; j0 += 128) near_batch<T, SCAN, 2>(P, l, j0, n, g0, p, key, sc);
+  }
+  if (__any(sc.bad)) return 0;
   __syncthreads();
   int nfin = C;
-  if (__any(inf))
+  if (__any(sc.inf))
     for (int g0 = 0; g0 < C; g0 += 64)
-      nfin -= __popcll(__ballot(g0 + lane < C && key[g0 + lane] == __builtin_inff()));
-  if (sizeof(T) == 4) qmax = T(-wave_min(-qm));
-  const uint32_t ub = __float_as_uint(best);   // non-negative: the bits order as the values
+      nfin -= __popcll(__ballot(g0 + lane < C && key[g0 + lane] == 0x7f80u));
+  const uint32_t best = sc.best;
+  if (sizeof(T) == 4) qmax = T(-wave_min(-sc.qm));
   for (int KT = 34; KT >= 10; KT -= 12) {
-    uint32_t lim = 0x7f7fffffu;                // every finite one
+    uint32_t lim = 0x7f7fu;                    // every finite one
     if (nfin > AM_NEAR_MAX) {
       uint32_t t = 0u;
 #pragma unroll
-      for (int b = 30; b >= 19; --b) {
+      for (int b = 14; b >= 2; --b) {
         const uint32_t c = t | (1u << b);
-        if (__popcll(__ballot(ub < c)) < KT) t = c;
+        if (__popcll(__ballot(best < c)) < KT) t = c;
       }
-      lim = min(t + (1u << 19) - 1u, 0x7f7fffffu);
+      lim = min(t + 3u, 0x7f7fu);
     }
     int n = 0;
     for (int g0 = 0; g0 < C; g0 += 64) {
       const int g = g0 + lane;
-      const bool keep = g < C && __float_as_uint(key[g]) <= lim;
+      const bool keep = g < C && key[g] <= lim;
       const unsigned long long bal = __ballot(keep);
       const int pos = n + __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0u));
       if (keep && pos < AM_NEAR_MAX) cand[pos] = (uint16_t)g;
@@ -170,7 +198,7 @@ __device__ __forceinline__ int near_constraints(const Src& P, int C, const T* p,
     __syncthreads();
     if (n <= AM_NEAR_MAX) {
       // 1e-5: the FP32 rounding of the squared distances
-      r = n == nfin ? T(1e18) : T(__builtin_sqrtf(__uint_as_float(lim)) * (1.f - 1e-5f));
+      r = n == nfin ? T(1e18) : T(__builtin_sqrtf(__uint_as_float((lim + 1u) << 16)) * (1.f - 1e-5f));
       return n;
     }
   }
@@ -212,7 +240,8 @@ __device__ __forceinline__ bool near_covers(const T* v, const T* p, T r, T E, T 
 template <typename T, bool SCAN, bool FULL, typename Src>
 __device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, const WalkParams& wp, int rid,
                                           int slot_region, const Src& P, const NearLds<T>& S, const T* eq, const T* p,
-                                          int start, T eqe = T(0)) {
+                                          int start, T eqe = T(0), NearScan<T, SCAN> sc = NearScan<T, SCAN>{},
+                                          int skip = -1) {
   constexpr bool per_plane = sizeof(T) == 4;
   const int lane = threadIdx.x;
   const int C = net.C, vm = net.vm;
@@ -231,7 +260,7 @@ __device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, 
     return k;
   };
   if (!FULL) {
-    const int n = near_constraints<T, SCAN>(P, C, p, S.key, S.cand, r, qmax);
+    const int n = near_constraints<T, SCAN>(P, C, p, S.key, S.cand, r, qmax, sc, skip);
     if (n < 3) return NEAR_RETRY;
     have = lane < n;
     g = have ? (int)S.cand[lane] : -1;
@@ -240,7 +269,12 @@ __device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, 
       if (per_plane) sig = P.err(g);
       if (SCAN) key = order_key(a);
     }
-    for (int q = 0; q < 4; ++q) S.pl[lane * 4 + q] = a[q];
+    if constexpr (sizeof(T) == 8) {
+      reinterpret_cast<double2*>(S.pl)[2 * lane] = double2{a[0], a[1]};
+      reinterpret_cast<double2*>(S.pl)[2 * lane + 1] = double2{a[2], a[3]};
+    } else {
+      reinterpret_cast<float4*>(S.pl)[lane] = float4{a[0], a[1], a[2], a[3]};
+    }
     const unsigned long long sb = __ballot(g == start && have);
     if (!sb) return NEAR_RETRY;
     sl = __builtin_ctzll(sb);

@@ -10,7 +10,28 @@
 
 namespace am {
 
-enum TimerSlot { T_CHAIN64 = 0, T_RAY64, T_SCAN64, T_REGION64, T_GEMM, T_WALK, T_INSERT, T_VERT64, T_NEWTON, T_SLOTS };
+enum TimerSlot { T_CHAIN64 = 0, T_RAY64, T_SCAN64, T_GEMM, T_WALK, T_INSERT, T_VERT64, T_NEWTON, T_SLOTS };
+
+// Stage times of a march taken on the device: the first thread of a stage's
+// first kernel charges the time since the last mark to the stage that was
+// running (kernels of a stream run one after another).  No events between the
+// launches (each cost about 4 us of the stream's time), and the same inside a
+// captured graph.  Ticks of wall_clock64(): 100 MHz.
+struct StageClock {
+  unsigned long long acc[T_SLOTS + 1];   // the last entry: between levels
+  unsigned long long last;
+  unsigned long long slot;
+};
+constexpr double kStageTickMs = 1e-5;
+__device__ __forceinline__ void stage_mark_now(StageClock* c, int slot) {
+  const unsigned long long t = wall_clock64();
+  c->acc[c->slot] += t - c->last;
+  c->last = t;
+  c->slot = (unsigned long long)slot;
+}
+__device__ __forceinline__ void stage_mark(StageClock* c, int slot) {
+  if (c && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) stage_mark_now(c, slot);
+}
 
 struct StageTimer {
   std::vector<hipEvent_t> pool;
@@ -21,7 +42,7 @@ struct StageTimer {
   };
   std::vector<Span> spans;
   double acc[T_SLOTS] = {0};
-  bool enabled = true;   // off while launches are captured into a graph (no event nodes)
+  bool enabled = true;   // off: mark() and span() do nothing
 
   static void check(hipError_t e, const char* what) {
     if (e != hipSuccess) throw std::runtime_error(std::string("HIP error: ") + hipGetErrorString(e) + " in " + what);
