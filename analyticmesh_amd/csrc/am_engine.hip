@@ -150,6 +150,7 @@ struct am_ctx {
   std::string err;
   hipStream_t stream = nullptr;
   hipStream_t own_stream = nullptr;   // used when the caller passes no stream
+  hipEvent_t null_ev = nullptr;
   int dev = 0;
   size_t max_lds = 65536;
   long long max_regions = -1;
@@ -216,6 +217,8 @@ struct am_ctx {
   // pinned, coherent host word the device writes scan totals into (arm_host_total)
   int* host_total = nullptr;
   int* host_total_dev = nullptr;
+  int host_seq = 0;
+  DevBuf<int2> levels;                    // [kHostRing] first region and count of the levels in flight
   // pinned staging for am_get_mesh into pageable host arrays (grown, kept)
   unsigned char* mesh_pin = nullptr;
   size_t mesh_pin_bytes = 0;
@@ -280,16 +283,26 @@ void grow_cands(am_ctx* c, size_t n) {
 // networks) keep their cores, and a stream sync after 100 ms, which also
 // reports a failed kernel.  Kernels enqueued after the scan may still run when
 // the word is read; later work on the stream stays ordered behind them.
-void arm_host_total(am_ctx* c) {
+// Scans in flight take the slots of a ring in turn (kHostWords words each: the
+// total, then the counts published with it), so that a level can be launched
+// before the one ahead of it has reported.
+constexpr int kHostRing = 8, kHostWords = 32;
+
+int arm_host_total(am_ctx* c) {
   if (!c->host_total) {
-    HIPCHK(hipHostMalloc((void**)&c->host_total, 256, hipHostMallocMapped | hipHostMallocCoherent));
+    HIPCHK(hipHostMalloc((void**)&c->host_total, kHostRing * kHostWords * sizeof(int),
+                         hipHostMallocMapped | hipHostMallocCoherent));
     HIPCHK(hipHostGetDevicePointer((void**)&c->host_total_dev, c->host_total, 0));
+    c->host_seq = 0;
   }
-  *reinterpret_cast<volatile int*>(c->host_total) = -1;
+  const int slot = c->host_seq;
+  c->host_seq = (slot + 1) % kHostRing;
+  *reinterpret_cast<volatile int*>(c->host_total + slot * kHostWords) = -1;
+  return slot;
 }
 
-int wait_total(am_ctx* c) {
-  volatile int* h = reinterpret_cast<volatile int*>(c->host_total);
+int wait_total(am_ctx* c, int slot) {
+  volatile int* h = reinterpret_cast<volatile int*>(c->host_total + slot * kHostWords);
   const auto t0 = std::chrono::steady_clock::now();
   for (unsigned spins = 0; *h < 0; ++spins) {
     if (spins < 4096) continue;
@@ -308,7 +321,6 @@ void ensure_table(am_ctx* c, size_t entries) {
   if (need > (size_t(1) << 31)) throw CapErr{"visited set would exceed 2^31 slots"};
   if (need == c->table_cap) return;
   const hipStream_t st = c->stream;
-  c->table.release();
   ensure(c->table, need, false, st);
   c->table_cap = need;
   hipLaunchKernelGGL(k_fill_u32, dim3(blocks(need, 256)), dim3(256), 0, st, c->table.p, need, 0xFFFFFFFFu);
@@ -327,6 +339,9 @@ struct InsertPlan {
   size_t n = 0;
   bool early = false;
   int R0 = 0;
+  int slot = 0;                 // ring slot of its total and of the level it finds
+  const int2* lvl = nullptr;    // the level's size on the device (launched ahead: n is a bound)
+  int lvl_bound = 0;
 };
 
 InsertPlan insert_prepare(am_ctx* c, size_t n) {
@@ -343,7 +358,8 @@ InsertPlan insert_prepare(am_ctx* c, size_t n) {
   p.early = (size_t)c->R + n <= c->reg_cap || n <= ((size_t)1 << 22);
   if (p.early) grow_regions(c, (size_t)c->R + n);
   ensure(c->scan_state, scan_commit_tiles(n) + 1, false, c->stream);
-  arm_host_total(c);
+  ensure(c->levels, kHostRing, false, c->stream);
+  p.slot = arm_host_total(c);
   return p;
 }
 
@@ -381,6 +397,9 @@ void insert_launch(am_ctx* c, const InsertPlan& p) {
   io.scan_words = (int)tiles + 1;
   io.zero = c->tcnt.p;
   io.clk = c->clock;
+  io.lvl = p.lvl;
+  io.lvl_bound = p.lvl_bound;
+  io.vm = c->vm;
   hipLaunchKernelGGL(k_insert, dim3(blocks(n, 256)), dim3(256), 0, st, io);
   HIPCHK(hipGetLastError());
   // the new-region flags' scan in one pass; with the store already large
@@ -391,21 +410,27 @@ void insert_launch(am_ctx* c, const InsertPlan& p) {
   sio.n = (int)n;
   sio.tiles = (int)tiles;
   sio.rank = p.early ? nullptr : c->rank.p;
-  sio.total = c->host_total_dev;
+  sio.total = c->host_total_dev + p.slot * kHostWords;
+  sio.lvl = p.lvl;
+  sio.lvl_bound = p.lvl_bound;
+  sio.vm = c->vm;
+  sio.lvl_next = c->levels.p + p.slot;
   sio.clk = c->clock;
   sio.pub = c->pfx.dev.total;
   sio.npub = c->pfx.dev.total ? c->pfx.dev.nd + 1 : 0;
   sio.pub_stride = AM_PFX_TS;
-  sio.pub_out = c->host_total_dev + 1;
+  sio.pub_out = c->host_total_dev + p.slot * kHostWords + 1;
   hipLaunchKernelGGL(k_scan_commit, dim3((unsigned)tiles), dim3(kScanCommitThreads), 0, st, sio);
   HIPCHK(hipGetLastError());
 }
 
-int insert_finish(am_ctx* c, const InsertPlan& p) {
+int insert_finish(am_ctx* c, const InsertPlan& p, int ahead = 0) {
   if (p.n == 0) return 0;
-  const int total = wait_total(c);
-  // (every launch of the level has run: its prefixes are counted)
-  for (int d = 1; d <= c->pfx.dev.nd; ++d) c->pfx.ub[d] = reinterpret_cast<volatile int*>(c->host_total)[1 + d];
+  const int total = wait_total(c, p.slot);
+  // (every launch of the level has run: its prefixes are counted; `ahead`: a
+  // level launched ahead may add more)
+  for (int d = 1; d <= c->pfx.dev.nd; ++d)
+    c->pfx.ub[d] = reinterpret_cast<volatile int*>(c->host_total + p.slot * kHostWords)[1 + d] + ahead;
   if (total == 0) return 0;
   // am_combine indexes (region, vertex slot) items with 32-bit ints: R * vm must stay below 2^31
   long long limit = std::min<long long>((long long)INT_MAX / 2, (long long)INT_MAX / c->vm);
@@ -472,8 +497,9 @@ void launch_as_graph(am_ctx* c, int parity, F&& enqueue) {
 }
 
 // Insert n candidates (already in cand_*) and append the new ones as regions.
-int insert_level(am_ctx* c, size_t n) {
+int insert_level(am_ctx* c, size_t n, int* slot = nullptr) {
   const InsertPlan p = insert_prepare(c, n);
+  if (slot) *slot = p.slot;
   insert_launch(c, p);
   return insert_finish(c, p);
 }
@@ -750,7 +776,8 @@ void prefix_plan(am_ctx* c, int count, size_t chunk) {
 }
 
 // The planes of the regions of one launch (chunk k of the plan).
-void prefix_launch(am_ctx* c, size_t k, const int* ids, int first, int n, const int* dcount, int dbase) {
+void prefix_launch(am_ctx* c, size_t k, const int* ids, int first, int n, const int* dcount, int dbase,
+                   const int2* lvl, int lvl_bound) {
   PrefixStore& s = c->pfx;
   if (s.reset[k]) prefix_clear(c);
   s.dev.clk = c->clock;
@@ -762,6 +789,8 @@ void prefix_launch(am_ctx* c, size_t k, const int* ids, int first, int n, const 
   rg.count = n;
   rg.dcount = dcount;
   rg.dbase = dbase;
+  rg.lvl = lvl;
+  rg.lvl_bound = lvl_bound;
   hipLaunchKernelGGL(k_prefix, dim3(blocks(n, AM_PFX_REGIONS), s.dev.nd), dim3(4 * AM_PFX_REGIONS), 0, c->stream, c->net,
                      s.dev, rg);
   HIPCHK(hipGetLastError());
@@ -795,9 +824,12 @@ void fp64_prepare(am_ctx* c, int count) {
 // -1 when the count is not known on the host): the regions it decided get FP64
 // vertices (k_vertex_fp64, their other records stay as written), the others go
 // through mode 1.
+// With lvl, first and count are those found on the device (a level launched
+// ahead of its size; `count` is its bound).
 // Nothing here waits for the device.
 void run_fp64_regions(am_ctx* c, int lvl_first, int first, int count, const int* ids, int mode, Fp64Counts& t,
-                      long long undecided = -1, const int* dcount = nullptr) {
+                      long long undecided = -1, const int* dcount = nullptr, const int2* lvl = nullptr,
+                      int lvl_bound = 0) {
   const bool after_walk = mode == 2;
   if (after_walk) mode = 1;
   // nets with skips or layers over 256 wide keep the candidate scan's records in every form
@@ -841,10 +873,12 @@ void run_fp64_regions(am_ctx* c, int lvl_first, int first, int count, const int*
     io.dcount = dcount;
     io.dbase = off;
     const int rid0 = first + off;
+    io.lvl = lvl;
+    io.lvl_bound = lvl_bound;
     io.clk = c->clock;
     if (k > 0)   // (the level's first launch finds them cleared)
       hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, c->stream, c->tcnt.p, (size_t)2, 0);
-    prefix_launch(c, k, io.ids, rid0, n, dcount, off);
+    prefix_launch(c, k, io.ids, rid0, n, dcount, off, lvl, lvl_bound);
     t.chain_launches += 1;
     if (after_walk && undecided != count && vert64) {
       hipLaunchKernelGGL(k_vertex_fp64, dim3(n), dim3(64), 0, c->stream, c->net, c->pfx.dev, io, rid0);
@@ -871,6 +905,113 @@ void run_fp64_regions(am_ctx* c, int lvl_first, int first, int count, const int*
                        io, rid0, (const int*)left.cnt, (const int*)left.slots, (const double*)c->teq.p, 0);
     HIPCHK(hipGetLastError());
   }
+}
+
+// Whether a level of up to B regions can be launched behind the one in flight
+// with the buffers as they are (nothing may be allocated or moved under it):
+// the level in flight adds up to B regions to c->R, this one B vm candidates.
+bool ahead_fits(const am_ctx* c, int B) {
+  const size_t n = (size_t)B * c->vm, R = (size_t)c->R + B;
+  const PrefixStore& s = c->pfx;
+  if (R + n > c->reg_cap || 2 * (R + n) > c->table_cap) return false;
+  if (c->cand_mask.n < n * c->Wd || c->cand_start.n < n || c->cand_point.n < 3 * n || c->cand_hash.n < n ||
+      c->slot.n < n || c->rank.n < n || c->rflags.n < (size_t)B || c->scan_state.n < scan_commit_tiles(n) + 1 ||
+      c->teq.n < (size_t)4 * B || c->tslots.n < (size_t)2 * B)
+    return false;
+  const int nd = s.dev.nd;
+  if ((size_t)B > prefix_chunk(c) || s.rslot.n < (size_t)B * std::max(nd, 1) || s.fresh.n < (size_t)(nd + 1) * B)
+    return false;
+  size_t sum = 0;
+  for (int d = 1; d <= nd; ++d) {
+    const size_t ids = (size_t)s.ub[d] + B;
+    if (ids > s.blocks[d].size() * AM_PFX_IDS) return false;
+    sum += ids;
+  }
+  return 2 * sum <= s.cap;
+}
+
+// Buffers so that ahead_fits(B) holds from the level after next on.
+void ahead_grow(am_ctx* c, int B) {
+  const size_t n = (size_t)B * c->vm;
+  grow_cands(c, n);
+  ensure(c->rflags, (size_t)B, false, c->stream);
+  ensure(c->scan_state, scan_commit_tiles(n) + 1, false, c->stream);
+  ensure(c->teq, (size_t)4 * B, false, c->stream);
+  ensure(c->tslots, (size_t)2 * B, false, c->stream);
+  const int nd = c->pfx.dev.nd;
+  ensure(c->pfx.rslot, (size_t)B * std::max(nd, 1), false, c->stream);
+  ensure(c->pfx.fresh, (size_t)(nd + 1) * B, false, c->stream);
+  ensure_table(c, (size_t)c->R + B + n);
+  grow_regions(c, (size_t)c->R + B + n);
+  long long ids[AM_MAX_LINEAR + 1] = {0};
+  for (int d = 1; d <= nd; ++d) ids[d] = c->pfx.ub[d] + 2LL * B;
+  (void)prefix_blocks(c, ids, false);
+}
+
+// The levels of an FP64 march.  While a small level runs, the next one is
+// already in the stream: launched for at most twice the regions (and 256 more),
+// its size read on the device, so the host's round trip (about 20 us: the total's way
+// to the host and the next launches) is off the GPU's path.  When the level
+// turns out larger the launches made ahead find nothing to do and it is launched
+// again; levels over kAheadMax regions take longer than the round trip and are
+// launched when their size is known.
+struct LevelsDone {
+  long long levels = 0, cands = 0;
+};
+constexpr int kAheadMax = 8192;
+
+LevelsDone march_fp64(am_ctx* c, long long first, long long count, int slot, int mode, Fp64Counts& t) {
+  LevelsDone done;
+  auto bound_after = [](long long n) { return (int)(2 * n + 256); };
+  InsertPlan cur;            // the level in flight
+  bool launched = false;     // ... already there, launched ahead
+  while (count > 0) {
+    const size_t ncand = (size_t)count * c->vm;
+    const int B = bound_after(count);
+    if (!launched) {
+      if (count <= kAheadMax) ahead_grow(c, B);
+      grow_cands(c, ncand);
+      ensure(c->rflags, (size_t)count, false, c->stream);
+      fp64_prepare(c, (int)count);
+      cur = insert_prepare(c, ncand);
+      run_fp64_regions(c, (int)first, (int)first, (int)count, nullptr, mode, t);
+      insert_launch(c, cur);
+    }
+    InsertPlan next;
+    const bool ahead = count <= kAheadMax && ahead_fits(c, B);
+    if (ahead) {
+      PrefixStore& s = c->pfx;
+      s.reset.assign(1, 0);
+      s.dev.fresh_stride = B;
+      s.dev.rslot = s.rslot.p;
+      s.dev.fresh = s.fresh.p;
+      for (int d = 1; d <= s.dev.nd; ++d) s.ub[d] += B;
+      next.n = (size_t)B * c->vm;
+      next.early = true;
+      next.slot = arm_host_total(c);
+      next.lvl = c->levels.p + cur.slot;
+      next.lvl_bound = B;
+      run_fp64_regions(c, 0, 0, B, nullptr, mode, t, -1, nullptr, next.lvl, B);
+      insert_launch(c, next);
+    }
+    const long long before = c->R;
+    const int added = insert_finish(c, cur, ahead ? B : 0);
+    done.cands += (long long)ncand;
+    done.levels += 1;
+    first = before;
+    count = added;
+    launched = ahead && added <= B;
+    if (ahead && !launched)
+      for (int d = 1; d <= c->pfx.dev.nd; ++d) c->pfx.ub[d] -= B;
+    if (launched) {
+      cur = next;
+      cur.n = (size_t)added * c->vm;
+      cur.R0 = (int)before;
+      cur.lvl = nullptr;
+    }
+  }
+  (void)slot;
+  return done;
 }
 
 // A device-readable view of a caller's array: the pointer itself when it is
@@ -1376,6 +1517,10 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
     // device-readable views of the weights (host arrays are staged once)
     c->stage_used = 0;
     const size_t esz = dtype == AM_DTYPE_F64 ? 8 : 4;
+    // the caller's device arrays may still be in the making on the null stream
+    if (!c->null_ev) HIPCHK(hipEventCreateWithFlags(&c->null_ev, hipEventDisableTiming));
+    HIPCHK(hipEventRecord(c->null_ev, nullptr));
+    HIPCHK(hipStreamWaitEvent(st, c->null_ev, 0));
     std::vector<const void*> wv(nl), bv(nl);
     wv[0] = dev_view(c, weights[0], (size_t)c->nodes[1] * 3 * esz, st);
     for (int li = 1; li < nl; ++li)
@@ -1495,30 +1640,12 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
     // ---- seeds -> first level (backend/inc/states.h:147-176)
     c->R = 0;
     c->table_cap = 0;
-    c->table.release();
     grow_cands(c, (size_t)n_seeds);
-    {
-      std::vector<uint32_t> m((size_t)n_seeds * c->Wd, 0u);
-      std::vector<uint8_t> hs((size_t)n_seeds * c->L);
-      HIPCHK(hipMemcpy(hs.data(), states, hs.size(), hipMemcpyDefault));
-      for (int s = 0; s < n_seeds; ++s)
-        for (int g = 0; g < c->L; ++g)
-          if (hs[(size_t)s * c->L + g]) m[(size_t)s * c->Wd + (g >> 5)] |= 1u << (g & 31);
-      std::vector<double> pts((size_t)n_seeds * 3);
-      if (dtype == AM_DTYPE_F64) {
-        HIPCHK(hipMemcpy(pts.data(), points, pts.size() * sizeof(double), hipMemcpyDefault));
-      } else {
-        std::vector<float> f(pts.size());
-        HIPCHK(hipMemcpy(f.data(), points, f.size() * sizeof(float), hipMemcpyDefault));
-        for (size_t i = 0; i < f.size(); ++i) pts[i] = f[i];
-      }
-      std::vector<int> startv(n_seeds, -1);
-      HIPCHK(hipMemcpy(c->cand_mask.p, m.data(), m.size() * 4, hipMemcpyHostToDevice));
-      HIPCHK(hipMemcpy(c->cand_point.p, pts.data(), pts.size() * 8, hipMemcpyHostToDevice));
-      HIPCHK(hipMemcpy(c->cand_start.p, startv.data(), startv.size() * 4, hipMemcpyHostToDevice));
-    }
-    hipLaunchKernelGGL(k_hash_keys, dim3(blocks(n_seeds, 256)), dim3(256), 0, st, (const uint32_t*)c->cand_mask.p,
-                       n_seeds, c->Wd, c->cand_hash.p);
+    hipLaunchKernelGGL(k_seeds, dim3(n_seeds), dim3(64), 0, st,
+                       (const uint8_t*)dev_view(c, states, (size_t)n_seeds * c->L, st),
+                       dev_view(c, points, (size_t)n_seeds * 3 * esz, st), dtype == AM_DTYPE_F64 ? 1 : 0, n_seeds,
+                       c->L, c->Wd, c->cand_mask.p, c->cand_hash.p, c->cand_point.p, c->cand_start.p);
+    HIPCHK(hipGetLastError());
     // run counters on the device: [0, 1 + W) the FP64 ray walk's undecided
     // regions and reasons, [1 + W, 2 + 2W) the reduced-precision walk's, then
     // the regions it decided with a vertex left to FP64; then the stage clock
@@ -1537,11 +1664,19 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
                        c->tcnt.p);
     HIPCHK(hipGetLastError());
     long long lvl_first = 0;
-    long long lvl_count = insert_level(c, (size_t)n_seeds);
+    int seed_slot = 0;
+    long long lvl_count = insert_level(c, (size_t)n_seeds, &seed_slot);
     long long levels = 0, cands = 0, launches = 0;
     long long why[AM_WHY_COUNT] = {0};
     Fp64Counts f64;
     c->timer.reset();
+    if (fp64_form && !c->graph_levels && c->max_regions < 0) {
+      const LevelsDone ld = march_fp64(c, lvl_first, lvl_count, seed_slot, c->precision == AM_PREC_FP64 ? 0 : 1, f64);
+      levels = ld.levels;
+      cands = ld.cands;
+      launches = ld.levels;
+      lvl_count = 0;
+    }
     while (lvl_count > 0) {
       if (c->max_regions >= 0 && lvl_first >= c->max_regions) break;
       const size_t ncand = (size_t)lvl_count * c->vm;
@@ -2385,6 +2520,7 @@ am_status am_destroy(am_ctx* c) {
   if (c->host_total) (void)hipHostFree(c->host_total);   // every level waited for its total
   if (c->mesh_pin) (void)hipHostFree(c->mesh_pin);
   for (hipEvent_t e : c->mesh_ev) (void)hipEventDestroy(e);
+  if (c->null_ev) (void)hipEventDestroy(c->null_ev);
   hipStream_t own = c->own_stream;
   delete c;
   if (own) (void)hipStreamDestroy(own);

@@ -71,6 +71,10 @@ struct ScanCommitIO {
   int* rank;
   int* total;
   StageClock* clk = nullptr;
+  // a level launched ahead of its size: n = vm slots per region of lvl, R0 = its end
+  const int2* lvl = nullptr;
+  int lvl_bound = 0, vm = 0;
+  int2* lvl_next = nullptr;     // receives the new regions' first and count
   // further counts handed to the host before the total
   const int* pub = nullptr;
   int npub = 0, pub_stride = 1;
@@ -82,6 +86,9 @@ constexpr int kScanCommitTile = kScanCommitThreads * kScanCommitItems;   // cand
 inline size_t scan_commit_tiles(size_t n) { return (n + kScanCommitTile - 1) / kScanCommitTile; }
 __global__ void k_scan_commit(ScanCommitIO io);
 __global__ void k_hash_keys(const uint32_t* masks, int n, int Wd, uint64_t* out);
+// Seeds as the first candidates: packed masks, key hashes, points, no start plane.
+__global__ void k_seeds(const uint8_t* states, const void* points, int f64, int n, int L, int Wd, uint32_t* mask,
+                        uint64_t* hash, double* point, int* start);
 __global__ void k_rehash(const uint32_t* reg_mask, int R, int Wd, uint32_t* table, uint32_t cap_mask);
 __global__ void k_fingerprint(const uint32_t* reg_mask, const int* info, const int* vpair, int R, int Wd, int Wh,
                               int vm, int L, int net, unsigned long long* out);

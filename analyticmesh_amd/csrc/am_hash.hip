@@ -79,8 +79,9 @@ __global__ __launch_bounds__(256) void k_insert(InsertIO io) {
   if (gtid < io.scan_words) io.scan_state[gtid] = 0ull;
   if (io.zero && gtid < 2) io.zero[gtid] = 0;
   const int c = gtid;
+  const int n = io.lvl ? level_count(io.lvl, io.lvl_bound) * io.vm : io.n;
   bool live = false;
-  if (c < io.n) {
+  if (c < n) {
     live = io.cand_start[c] != -2;
     if (!live) io.slot[c] = -1;
   }
@@ -152,15 +153,22 @@ __global__ __launch_bounds__(kScanCommitThreads) void k_scan_commit(ScanCommitIO
   __shared__ int s_wave[kScanCommitThreads / 64];
   __shared__ int s_list[kScanCommitTile];
   const int tid = threadIdx.x, lane = tid & 63;
+  int n = io.n, R0 = io.cio.R0;
+  if (io.lvl) {
+    n = level_count(io.lvl, io.lvl_bound) * io.vm;
+    R0 = io.lvl->x + io.lvl->y;
+  }
+  const int tiles = max(1, (n + kScanCommitTile - 1) / kScanCommitTile);
   if (tid == 0) s_tile = (int)atomicAdd(&io.state[io.tiles], 1ull);
   __syncthreads();
   const int t = s_tile;
+  if (t >= tiles) return;
   const size_t base = (size_t)t * kScanCommitTile + (size_t)tid * kScanCommitItems;
   int v[kScanCommitItems];
   int sum = 0;
 #pragma unroll
   for (int it = 0; it < kScanCommitItems; ++it) {
-    v[it] = base + it < (size_t)io.n ? first_flag(io.cio, base + it) : 0;
+    v[it] = base + it < (size_t)n ? first_flag(io.cio, base + it) : 0;
     sum += v[it];
   }
   int tot;
@@ -194,7 +202,8 @@ __global__ __launch_bounds__(kScanCommitThreads) void k_scan_commit(ScanCommitIO
     }
     if (lane == 0) {
       s_excl = excl;
-      if (t == io.tiles - 1 && io.total) {
+      if (t == tiles - 1 && io.lvl_next) *io.lvl_next = make_int2(R0, excl + tot);
+      if (t == tiles - 1 && io.total) {
         for (int i = 0; i < io.npub; ++i) io.pub_out[i] = io.pub[i * io.pub_stride];
         if (io.clk) stage_mark_now(io.clk, T_SLOTS);
         if (io.npub) __threadfence_system();
@@ -254,7 +263,7 @@ __global__ __launch_bounds__(kScanCommitThreads) void k_scan_commit(ScanCommitIO
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         if (cc[u] >= 0) {
-          const int rid = ci.R0 + excl + k0 + u * NG;
+          const int rid = R0 + excl + k0 + u * NG;
 #pragma unroll
           for (int t = 0; t < NQ; ++t) {
             const int q = j + t * AM_KG;
@@ -272,7 +281,7 @@ __global__ __launch_bounds__(kScanCommitThreads) void k_scan_commit(ScanCommitIO
   } else {
     for (int k = gid; k < tot; k += NG) {
       const int cc = s_list[k];
-      const int rid = ci.R0 + excl + k;
+      const int rid = R0 + excl + k;
       group_copy(ci.reg_mask + (size_t)rid * ci.Wd, ci.cand_mask + (size_t)cc * ci.Wd, ci.Wd, j);
       if (j == 0) {
         ci.reg_start[rid] = ci.cand_start[cc];
@@ -294,6 +303,31 @@ __global__ void k_commit(CommitIO io, const int* rank, int n) {
 __global__ void k_hash_keys(const uint32_t* masks, int n, int Wd, uint64_t* out) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c < n) out[c] = key_hash_sum(masks + (size_t)c * Wd, Wd);
+}
+
+__global__ __launch_bounds__(64) void k_seeds(const uint8_t* states, const void* points, int f64, int n, int L, int Wd,
+                                              uint32_t* mask, uint64_t* hash, double* point, int* start) {
+  const int s = blockIdx.x, lane = threadIdx.x;
+  if (s >= n) return;
+  uint64_t h = 0;
+  for (int w = 0; w < Wd; w += 2) {
+    const int g = 32 * w + lane;
+    const unsigned long long bal = __ballot(g < L && states[(size_t)s * L + g] != 0);
+    const uint32_t lo = (uint32_t)bal, hi = (uint32_t)(bal >> 32);
+    if (lane == 0) {
+      mask[(size_t)s * Wd + w] = lo;
+      if (w + 1 < Wd) mask[(size_t)s * Wd + w + 1] = hi;
+    }
+    h += word_hash(lo, w);
+    if (w + 1 < Wd) h += word_hash(hi, w + 1);
+  }
+  if (lane == 0) {
+    hash[s] = h;
+    start[s] = -1;
+  }
+  if (lane < 3)
+    point[(size_t)s * 3 + lane] = f64 ? static_cast<const double*>(points)[(size_t)s * 3 + lane]
+                                      : (double)static_cast<const float*>(points)[(size_t)s * 3 + lane];
 }
 
 // Re-insert every region id into an empty (larger) table.

@@ -29,17 +29,34 @@ struct RegionIO {
   const int* ids;             // optional: region ids to process (FP64 re-decision); else first + blockIdx.x
   const int* dcount = nullptr;  // optional: ids past *dcount - dbase are not valid (a launch sized on
   int dbase = 0;                // the host for the worst case; blocks past the device count exit)
+  const int2* lvl = nullptr;    // the level's first region and count on the device (first is not valid then)
+  int lvl_bound = 0;            // largest count the launch is sized for
   StageClock* clk = nullptr;    // the march's stage times, if taken
   uint16_t* reg_jinv = nullptr; // optional [R][vm][9] bf16: per vertex the inverse of its 3x3 system
                                 // from the reduced planes (columns for the new, walked and face plane),
                                 // for the FP64 Newton step (a record with it has info[7] = 1)
 };
 
-// Regions of a launch whose count may be known on the device only.
+// Regions of a launch whose count may be known on the device only: a level
+// launched ahead of its size (lvl: first region and count, none when the count
+// passes the bound it was launched for), or a list (dcount).
 template <typename IO>
 __device__ __forceinline__ int launch_count(const IO& io) {
+  if (io.lvl) {
+    const int n = io.lvl->y;
+    return n <= io.lvl_bound ? min(io.count, n - io.dbase) : 0;
+  }
   return io.dcount ? min(io.count, *io.dcount - io.dbase) : io.count;
 }
+// First region of the launch (host: the value known there), and of its level.
+template <typename IO>
+__device__ __forceinline__ int launch_first(const IO& io, int host) {
+  return io.lvl ? io.lvl->x + io.dbase : host;
+}
+__device__ __forceinline__ int level_first(const RegionIO& io) { return io.lvl ? io.lvl->x : io.first; }
+
+// Regions of a level known on the device (as launch_count).
+__device__ __forceinline__ int level_count(const int2* lvl, int bound) { return lvl->y <= bound ? lvl->y : 0; }
 
 // Visited-set insertion of one level's candidates.
 struct InsertIO {
@@ -54,6 +71,8 @@ struct InsertIO {
   uint32_t cap_mask;
   unsigned long long* scan_state;  // [scan_words] tile states of the level's one-pass scan, cleared here
   int scan_words;
+  const int2* lvl = nullptr;       // as in RegionIO: n is then vm slots per region of the level
+  int lvl_bound = 0, vm = 0;
   int* zero = nullptr;             // two counters of the walks, cleared for the next level
   StageClock* clk = nullptr;
 };
@@ -82,6 +101,8 @@ struct ChainIO {
   int noutp[AM_MAX_LINEAR];         // n_out rounded up to AM_CR
   const int* dcount = nullptr;      // as in RegionIO: regions past *dcount - dbase are not valid
   int dbase = 0;
+  const int2* lvl = nullptr;
+  int lvl_bound = 0;
 };
 
 // A list of chunk-local slots filled by atomics (cnt zeroed before), with

@@ -64,11 +64,10 @@ struct PrefixRegions {
   int first, count;
   const int* dcount = nullptr;  // as in RegionIO
   int dbase = 0;
+  const int2* lvl = nullptr;
+  int lvl_bound = 0;
 };
 
-__device__ __forceinline__ int prefix_count(const PrefixRegions& r) {
-  return r.dcount ? min(r.count, *r.dcount - r.dbase) : r.count;
-}
 __device__ __forceinline__ double2* prefix_planes(const PrefixDev& pf, const NetDev& net, int d, int id) {
   char* b = pf.blk[(size_t)d * AM_PFX_BLOCKS + (id >> AM_PFX_SHIFT)];
   return reinterpret_cast<double2*>(b) + (size_t)(id & (AM_PFX_IDS - 1)) * 2 * net.nodes[d + 1];

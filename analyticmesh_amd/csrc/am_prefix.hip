@@ -27,7 +27,7 @@ __global__ __launch_bounds__(4 * AM_PFX_REGIONS) void k_prefix(NetDev net, Prefi
   __shared__ int s_cnt, s_base;
   const int tid = threadIdx.x, lane = tid & 63;
   const int d = blockIdx.y + 1;
-  const int cnt = prefix_count(rg);
+  const int cnt = launch_count(rg);
   stage_mark(pf.clk, T_CHAIN64);
   if ((int)blockIdx.x * AM_PFX_REGIONS >= cnt) return;
   if (tid == 0) s_cnt = 0;
@@ -36,7 +36,7 @@ __global__ __launch_bounds__(4 * AM_PFX_REGIONS) void k_prefix(NetDev net, Prefi
   const int nw = prefix_words(net, d);
   const int i = blockIdx.x * AM_PFX_REGIONS + (tid >> 2);
   const bool act = i < cnt;
-  const int rid = act ? (rg.ids ? rg.ids[i] : rg.first + i) : 0;
+  const int rid = act ? (rg.ids ? rg.ids[i] : launch_first(rg, rg.first) + i) : 0;
   const uint32_t* m = rg.reg_mask + (size_t)rid * net.Wd;
   uint64_t h = 0;
   if (act)
@@ -470,9 +470,9 @@ __global__ __launch_bounds__(64, SCAN ? 5 : 4) void k_near64(NetDev net, PrefixD
   const int n = launch_count(io);
   if ((int)blockIdx.x >= n) return;
   const int b = xcd_run(blockIdx.x, n);
-  const int rid = io.ids ? io.ids[b] : rid0 + b;
+  const int rid = io.ids ? io.ids[b] : launch_first(io, rid0) + b;
   // a region an earlier walk decided keeps its records (its flag is 0 and stays 0)
-  if (only_undecided && !(io.flags[rid - io.first] & AM_UNDECIDED)) return;
+  if (only_undecided && !(io.flags[rid - level_first(io)] & AM_UNDECIDED)) return;
   const NearLds<double> S = carve_near<double>(smem_raw, net.C, net.Wd, net.vm, false);
   const int start = io.reg_start[rid];
   prefix_bases(net, pf, b, s_bases, threadIdx.x, 64);
@@ -485,10 +485,10 @@ __global__ __launch_bounds__(64, SCAN ? 5 : 4) void k_near64(NetDev net, PrefixD
   face_plane(net, pf, P, S.pl, eq, [&](const double* x, int g) { sc.add(x, 0.0, p, S.key, g); });
   bool done = false;
   if (start >= 0 && start < net.C)
-    done = near_walk<double, SCAN, false>(net, io, wp, rid, rid - io.first, P, S, eq, p, start, 0.0, sc, net.D - 1) ==
+    done = near_walk<double, SCAN, false>(net, io, wp, rid, rid - level_first(io), P, S, eq, p, start, 0.0, sc, net.D - 1) ==
            NEAR_DONE;
   // (thread 0 wrote the flag in finish_region: the orientation may be undecided)
-  if (threadIdx.x == 0 && (!done || (!SCAN && (io.flags[rid - io.first] & AM_UNDECIDED)))) {
+  if (threadIdx.x == 0 && (!done || (!SCAN && (io.flags[rid - level_first(io)] & AM_UNDECIDED)))) {
     for (int q = 0; q < 4; ++q) eqb[(size_t)b * 4 + q] = eq[q];
     near_left(left, b);
   }
@@ -516,7 +516,7 @@ __global__ __launch_bounds__(64, 4) void k_walk_fp64(NetDev net, PrefixDev pf, R
   const int total = min(*count, io.count);
   for (int i = blockIdx.x; i < total; i += gridDim.x) {
     const int b = slots[i];
-    const int rid = io.ids ? io.ids[b] : rid0 + b;
+    const int rid = io.ids ? io.ids[b] : launch_first(io, rid0) + b;
     const int start = io.reg_start[rid];
     prefix_bases(net, pf, b, s_bases, lane, 64);
     double p[3], eq[4];
@@ -528,7 +528,7 @@ __global__ __launch_bounds__(64, 4) void k_walk_fp64(NetDev net, PrefixDev pf, R
       for (int w = lane; w < net.Wd; w += 64) S.mask[w] = io.reg_mask[(size_t)rid * net.Wd + w];
       __syncthreads();
       const PrefixPlanes P{net, s_bases, S.mask};
-      const int done = near_walk<double, true, true>(net, io, wp, rid, rid - io.first, P, S, eq, p, start);
+      const int done = near_walk<double, true, true>(net, io, wp, rid, rid - level_first(io), P, S, eq, p, start);
       __syncthreads();
       if (done == NEAR_DONE) continue;
     }
@@ -547,7 +547,7 @@ __global__ __launch_bounds__(64, 4) void k_walk_fp64(NetDev net, PrefixDev pf, R
         Pc[g] = x[3];
       }
     __syncthreads();
-    walk_region<double, false>(net, io, wp, rid, rid - io.first, Px, Py, Pz, Pc, keys, order, used, smask, eq, p);
+    walk_region<double, false>(net, io, wp, rid, rid - level_first(io), Px, Py, Pz, Pc, keys, order, used, smask, eq, p);
     __syncthreads();   // this region's LDS is free for the next
   }
 }
@@ -573,7 +573,7 @@ __global__ __launch_bounds__(64 * NW, 24 / NW) void k_walk_ray64(NetDev net, Pre
   const int total = min(*list.cnt, io.count);
   for (int i = blockIdx.x; i < total; i += gridDim.x) {
     const int b = list.slots[i];
-    const int rid = io.ids ? io.ids[b] : rid0 + b;
+    const int rid = io.ids ? io.ids[b] : launch_first(io, rid0) + b;
     const int start_in = io.reg_start[rid];
     prefix_bases(net, pf, b, s_bases, tid, 64 * NW);
     for (int w = tid; w < net.Wd; w += 64 * NW) smask[w] = io.reg_mask[(size_t)rid * net.Wd + w];
@@ -591,10 +591,10 @@ __global__ __launch_bounds__(64 * NW, 24 / NW) void k_walk_ray64(NetDev net, Pre
     for (int q = 0; q < 4; ++q) eq[q] = eqb[(size_t)b * 4 + q];
     __syncthreads();
     const PlaneView<double> P{reinterpret_cast<const double*>(Q), Cl, n1, net.W0, net.b[0], smask};
-    walk_ray<double, NW>(net, io, wp, rid, rid - io.first, P, smask, eq, p, rec, start_in);
+    walk_ray<double, NW>(net, io, wp, rid, rid - level_first(io), P, smask, eq, p, rec, start_in);
     // thread 0 wrote the region's flag (finish_region)
     if (tid == 0) {
-      const unsigned f = io.flags[rid - io.first];
+      const unsigned f = io.flags[rid - level_first(io)];
       if (f & AM_UNDECIDED) {
         left.slots[atomicAdd(left.cnt, 1)] = b;
         atomicAdd(left.run, 1);
@@ -621,8 +621,8 @@ __global__ __launch_bounds__(64) void k_vertex_fp64(NetDev net, PrefixDev pf, Re
   const int b = blockIdx.x;
   stage_mark(io.clk, T_VERT64);
   if (b >= launch_count(io)) return;
-  const int rid = io.ids ? io.ids[b] : rid0 + b;
-  if (io.flags && (io.flags[rid - io.first] & AM_UNDECIDED)) return;   // left to the FP64 walk
+  const int rid = io.ids ? io.ids[b] : launch_first(io, rid0) + b;
+  if (io.flags && (io.flags[rid - level_first(io)] & AM_UNDECIDED)) return;   // left to the FP64 walk
   const int vm = net.vm;
   const int nv = io.reg_info[(size_t)rid * AM_INFO_STRIDE + 2];
   prefix_bases(net, pf, b, s_bases, threadIdx.x, 64);
