@@ -845,7 +845,8 @@ void run_fp64_regions(am_ctx* c, int lvl_first, int first, int count, const int*
   const WalkParams& kr = c->chain_mfma ? kRay64Mf : kRay64;
   // the near walk lists the regions it leaves to the walk over all constraints,
   // the ray walk those it leaves to the candidate scan
-  const size_t nlds = near_lds_bytes(c->C, c->Wd, c->vm, 8, false);
+  const bool all = c->C <= AM_ALL_MAX;
+  const size_t nlds = near_lds_bytes(c->C, c->Wd, c->vm, 8, false, all);
   const size_t qlds = std::max(wlds, nlds);
   const NearList near{c->tcnt.p, c->tslots.p};
   const size_t lcap = std::min<size_t>(chunk, (size_t)count);
@@ -885,17 +886,17 @@ void run_fp64_regions(am_ctx* c, int lvl_first, int first, int count, const int*
       HIPCHK(hipGetLastError());
     }
     if (mode == 0) {
-      hipLaunchKernelGGL(k_near64<true>, dim3(n), dim3(64), nlds, c->stream, c->net, c->pfx.dev, io, rid0, kr,
+      hipLaunchKernelGGL((all ? k_near64<true, true> : k_near64<true, false>), dim3(n), dim3(64), nlds, c->stream, c->net, c->pfx.dev, io, rid0, kr,
                          c->teq.p, after_walk ? 1 : 0, near);
       io.flags = nullptr;
       hipLaunchKernelGGL(k_walk_fp64, dim3(std::min(n, c->scan_blocks)), dim3(64), qlds, c->stream, c->net,
-                         c->pfx.dev, io, rid0, (const int*)near.cnt, (const int*)near.slots, (const double*)c->teq.p, 1);
+                         c->pfx.dev, io, rid0, (const int*)near.cnt, (const int*)near.slots, (const double*)c->teq.p, all ? 0 : 1);
       HIPCHK(hipGetLastError());
       t.scanned_host += n;
       continue;
     }
     const SlotList left{c->tcnt.p + 1, c->tslots.p + lcap, c->acc};
-    hipLaunchKernelGGL(k_near64<false>, dim3(n), dim3(64), nlds, c->stream, c->net, c->pfx.dev, io, rid0, kr, c->teq.p,
+    hipLaunchKernelGGL((all ? k_near64<false, true> : k_near64<false, false>), dim3(n), dim3(64), nlds, c->stream, c->net, c->pfx.dev, io, rid0, kr, c->teq.p,
                        after_walk ? 1 : 0, near);
     HIPCHK(hipGetLastError());
     launch_ray64(c, n, rlds, io, rid0, kr, near, left);

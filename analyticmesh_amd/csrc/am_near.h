@@ -33,25 +33,37 @@ namespace am {
 // Scratch of the near walk in dynamic LDS, ahead of the walk records.
 template <typename T>
 struct NearLds {
-  T* pl;            // [64][4] the near constraints' planes, for broadcast reads
+  T* stage;         // [4][66] the face plane's inputs
+  T* pl;            // [64][4] the near constraints' planes, for broadcast reads (over stage); SET_LDS: [C][4] all
   uint16_t* key;    // [C] squared distance of p inside each constraint (0 where outside, +inf: never a
                     // bound), as the upper half of its FP32 bits, i.e. rounded down
   uint16_t* cand;   // [64] near constraints
   uint32_t* mask;   // [Wd]
-  uint32_t* used;   // [C bits] (over key: the walk on all constraints does not need the distances)
+  float* okey;      // [C] order keys (SET_LDS)
+  uint32_t* used;   // [C bits] (over key where that is not used)
   WalkRecs rec;
 };
-__host__ __device__ inline size_t near_lds_bytes(int C, int Wd, int vm, int tsize, bool jinv) {
+#define AM_ALL_MAX 256        // constraints up to which SET_LDS is taken
+__host__ __device__ inline size_t near_lds_bytes(int C, int Wd, int vm, int tsize, bool jinv, bool all = false) {
   auto a16 = [](size_t x) { return (x + 15) & ~(size_t)15; };
-  return (size_t)AM_NEAR_PL * tsize + a16((size_t)C * 2) + AM_NEAR_MAX * 2 + a16((size_t)Wd * 4) +
-         walk_rec_bytes(vm, jinv);
+  // (all: planes behind the face plane's inputs, order keys)
+  return (size_t)AM_NEAR_PL * tsize + (all ? (size_t)C * 4 * tsize + a16((size_t)C * 4) : 0) + a16((size_t)C * 2) +
+         AM_NEAR_MAX * 2 + a16((size_t)Wd * 4) + walk_rec_bytes(vm, jinv);
 }
 template <typename T>
-__device__ inline NearLds<T> carve_near(unsigned char* p, int C, int Wd, int vm, bool jinv) {
+__device__ inline NearLds<T> carve_near(unsigned char* p, int C, int Wd, int vm, bool jinv, bool all = false) {
   auto a16 = [](size_t x) { return (x + 15) & ~(size_t)15; };
   NearLds<T> s;
-  s.pl = reinterpret_cast<T*>(p);
+  s.stage = reinterpret_cast<T*>(p);
+  s.pl = s.stage;
+  s.okey = nullptr;
   p += (size_t)AM_NEAR_PL * sizeof(T);
+  if (all) {
+    s.pl = reinterpret_cast<T*>(p);
+    p += (size_t)C * 4 * sizeof(T);
+    s.okey = reinterpret_cast<float*>(p);
+    p += a16((size_t)C * 4);
+  }
   s.key = reinterpret_cast<uint16_t*>(p);
   s.used = reinterpret_cast<uint32_t*>(p);
   p += a16((size_t)C * 2);
@@ -220,6 +232,22 @@ __device__ __forceinline__ bool near_covers(const T* v, const T* p, T r, T E, T 
   return dx * dx + dy * dy + dz * dz <= T(0.81) * r * r && E <= T(0.01) && T(20) * (E * p1 + F) <= r && u * p1 <= r;
 }
 
+// The scan's order (distance_key).
+template <typename T>
+__device__ __forceinline__ T near_order_key(const T* x, const T* p) {
+  const T s = plane_eval(x[0], x[1], x[2], x[3], p);
+  const T nn = plane_nn(x[0], x[1], x[2]);
+  T k = nn > T(0) ? s * absT(s) / nn : (s > T(0) ? T(__builtin_inf()) : T(-__builtin_inf()));
+  if (k != k) k = -__builtin_inf();
+  return k;
+}
+// Constraint g's plane (and its order key, rounded) into LDS for SET_LDS.
+template <typename T, bool SCAN>
+__device__ __forceinline__ void near_stage(const NearLds<T>& S, int g, const T* x, const T* p) {
+  for (int q = 0; q < 4; ++q) S.pl[g * 4 + q] = x[q];
+  if (SCAN) S.okey[g] = (float)near_order_key<T>(x, p);
+}
+
 // SCAN: the candidate scan's decisions (walk_region<double, false>), bit for
 // bit: the next edge plane is the first unused constraint in distance order
 // whose vertex no constraint violates.  On the line of the current edge that is
@@ -229,20 +257,28 @@ __device__ __forceinline__ bool near_covers(const T* v, const T* p, T r, T E, T 
 // edge's two bounding planes -- so the scan would have passed it over too.
 // Else: the checked ray walk's decisions (walk_ray), same proposals, vertices
 // and bounds.
-// FULL: every constraint takes part (each pass reads all planes again), for a
-// region whose polygon the near constraints do not cover: about one in a hundred
-// on the geometric networks, a third on the trained chair (long thin faces).
+// SET_ALL: every constraint takes part and each pass reads all planes again, for
+// a region whose polygon the near constraints do not cover: about one in a
+// hundred on the geometric networks.
+// SET_LDS: every constraint takes part, planes in LDS (up to AM_ALL_MAX
+// constraints): no distances to sort out and nothing left over; on the trained
+// network a third of the polygons (long thin faces) are not covered by 64 of its
+// 240 constraints.
 // Returns NEAR_DONE (settled, record written), NEAR_RETRY (the constraints at
 // hand do not suffice), or the reason bits (AM_WHY_BIT) for which the checked ray
 // walk would leave the region undecided.
 #define NEAR_DONE 0
 #define NEAR_RETRY (-1)
-template <typename T, bool SCAN, bool FULL, typename Src>
+#define SET_NEAR 0
+#define SET_ALL 1
+#define SET_LDS 2
+template <typename T, bool SCAN, int SET, typename Src>
 __device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, const WalkParams& wp, int rid,
                                           int slot_region, const Src& P, const NearLds<T>& S, const T* eq, const T* p,
                                           int start, T eqe = T(0), NearScan<T, SCAN> sc = NearScan<T, SCAN>{},
                                           int skip = -1) {
   constexpr bool per_plane = sizeof(T) == 4;
+  constexpr bool FULL = SET != SET_NEAR;
   const int lane = threadIdx.x;
   const int C = net.C, vm = net.vm;
   T r = T(1e18), qmax = T(0);
@@ -252,13 +288,7 @@ __device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, 
   T sig = T(0), key = T(0);
   bool have = false;
   int sl = start;
-  auto order_key = [&](const T* x) {   // distance_key
-    const T s = plane_eval(x[0], x[1], x[2], x[3], p);
-    const T nn = plane_nn(x[0], x[1], x[2]);
-    T k = nn > T(0) ? s * absT(s) / nn : (s > T(0) ? T(__builtin_inf()) : T(-__builtin_inf()));
-    if (k != k) k = -__builtin_inf();
-    return k;
-  };
+  auto order_key = [&](const T* x) { return near_order_key<T>(x, p); };
   if (!FULL) {
     const int n = near_constraints<T, SCAN>(P, C, p, S.key, S.cand, r, qmax, sc, skip);
     if (n < 3) return NEAR_RETRY;
@@ -280,6 +310,15 @@ __device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, 
     sl = __builtin_ctzll(sb);
   } else {
     for (int w = lane; w < (C + 31) >> 5; w += 64) S.used[w] = 0u;
+    if (SET == SET_LDS)
+      for (int l = 0; l < P.parts(); ++l) {
+        if (l == skip) continue;   // staged by the caller
+        for (int j = lane; j < P.size(l); j += 64) {
+          T x[4];
+          P.load(l, j, x);
+          near_stage<T, SCAN>(S, P.first(l) + j, x, p);
+        }
+      }
   }
   __syncthreads();
   unsigned long long used = 0ull;      // near: lanes of the polygon's planes (FULL: S.used)
@@ -289,7 +328,7 @@ __device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, 
     else if (lane == 0) S.used[h >> 5] |= 1u << (h & 31);
   };
   auto plane = [&](int h, T* o) {
-    if (FULL) P.get(h, o);
+    if (SET == SET_ALL) P.get(h, o);
     else
       for (int q = 0; q < 4; ++q) o[q] = S.pl[h * 4 + q];
   };
@@ -299,6 +338,12 @@ __device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, 
   auto each = [&](auto&& f) {
     if (!FULL) {
       if (have) f(a, lane, g, sig);
+    } else if (SET == SET_LDS) {
+      for (int h = lane; h < C; h += 64) {
+        T x[4];
+        plane(h, x);
+        f(x, h, h, T(0));
+      }
     } else {
       for (int l = 0; l < P.parts(); ++l) {
         const int n = P.size(l), g0 = P.first(l);
@@ -385,6 +430,7 @@ __device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, 
       if (FULL) kw = order_key(pr);
       else kw = lane_value(key, rl);
       const int gw = index_of(rl);
+      const float kwf = (float)kw;
       bool fail = false;
       each([&](const T* x, int h, int gi, T) {
         if (h == cl || h == rl) return;
@@ -394,7 +440,8 @@ __device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, 
         const T al = fmaT(x[0], dn[0], fmaT(x[1], dn[1], x[2] * dn[2]));
         next.add(-sv, al, al > T(0), h);
         // an unused constraint before the winner in the order
-        if (key_before(FULL ? order_key(x) : key, gi, kw, gw) && (!is_used(h) || (h == sl && ntab >= 3))) {
+        const bool maybe = SET != SET_LDS || S.okey[h] >= kwf;   // (rounding keeps the order)
+        if (maybe && key_before(FULL ? order_key(x) : key, gi, kw, gw) && (!is_used(h) || (h == sl && ntab >= 3))) {
           T vt[3];
           solve3(x, pc, eq, vt);
           fail = fail || !(violates(pr[0], pr[1], pr[2], pr[3], vt) ||
@@ -504,10 +551,10 @@ __device__ __forceinline__ int near_or_full_walk(const NetDev& net, const Region
                                                  int slot_region, const Src& P, const NearLds<T>& S, const T* eq,
                                                  const T* p, int start, T eqe = T(0)) {
   if (start < 0 || start >= net.C) return NEAR_RETRY;
-  const int w = near_walk<T, SCAN, false>(net, io, wp, rid, slot_region, P, S, eq, p, start, eqe);
+  const int w = near_walk<T, SCAN, SET_NEAR>(net, io, wp, rid, slot_region, P, S, eq, p, start, eqe);
   if (w == NEAR_DONE || (sizeof(T) == 4 && w != NEAR_RETRY)) return w;
   __syncthreads();
-  return near_walk<T, SCAN, true>(net, io, wp, rid, slot_region, P, S, eq, p, start, eqe);
+  return near_walk<T, SCAN, SET_ALL>(net, io, wp, rid, slot_region, P, S, eq, p, start, eqe);
 }
 
 // Puts a region the near walk left (slot b of its launch) on the list.

@@ -99,10 +99,11 @@ __global__ void k_prefix_ptrs(char** blk, PrefixPtrs ptrs);
 __global__ void k_pack_pairs(const double* xyz, const double* c, int n, double2* out);
 
 // The near walk, and the walks over all constraints of what it leaves, on
-// prefix planes.  The near walk computes each region's face plane from layer
+// prefix planes.  ALL: the near walk takes every constraint (C <= AM_ALL_MAX).
+// The near walk computes each region's face plane from layer
 // D's planes (the output row's fma chain) and stores those of the regions it
 // leaves in eq.
-template <bool SCAN>
+template <bool SCAN, bool ALL>
 __global__ void k_near64(NetDev net, PrefixDev pf, RegionIO io, int rid0, WalkParams wp, double* eq,
                          int only_undecided, NearList left);
 template <int NW>

@@ -459,8 +459,8 @@ __device__ __forceinline__ int xcd_run(int b, int n) {
   return x * q + min(x, rem) + k;
 }
 
-template <bool SCAN>
-__global__ __launch_bounds__(64, SCAN ? 5 : 4) void k_near64(NetDev net, PrefixDev pf, RegionIO io, int rid0, WalkParams wp,
+template <bool SCAN, bool ALL>
+__global__ __launch_bounds__(64, SCAN && !ALL ? 5 : 4) void k_near64(NetDev net, PrefixDev pf, RegionIO io, int rid0, WalkParams wp,
                                                   double* eqb, int only_undecided, NearList left) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ gplanes s_bases[AM_MAX_LINEAR + 1];
@@ -473,7 +473,7 @@ __global__ __launch_bounds__(64, SCAN ? 5 : 4) void k_near64(NetDev net, PrefixD
   const int rid = io.ids ? io.ids[b] : launch_first(io, rid0) + b;
   // a region an earlier walk decided keeps its records (its flag is 0 and stays 0)
   if (only_undecided && !(io.flags[rid - level_first(io)] & AM_UNDECIDED)) return;
-  const NearLds<double> S = carve_near<double>(smem_raw, net.C, net.Wd, net.vm, false);
+  const NearLds<double> S = carve_near<double>(smem_raw, net.C, net.Wd, net.vm, false, ALL);
   const int start = io.reg_start[rid];
   prefix_bases(net, pf, b, s_bases, threadIdx.x, 64);
   for (int w = threadIdx.x; w < net.Wd; w += 64) S.mask[w] = io.reg_mask[(size_t)rid * net.Wd + w];
@@ -482,19 +482,24 @@ __global__ __launch_bounds__(64, SCAN ? 5 : 4) void k_near64(NetDev net, PrefixD
   __syncthreads();
   const PrefixPlanes P{net, s_bases, S.mask};
   NearScan<double, SCAN> sc;
-  face_plane(net, pf, P, S.pl, eq, [&](const double* x, int g) { sc.add(x, 0.0, p, S.key, g); });
+  face_plane(net, pf, P, S.stage, eq, [&](const double* x, int g) {
+    if (ALL) near_stage<double, SCAN>(S, g, x, p);
+    else sc.add(x, 0.0, p, S.key, g);
+  });
   bool done = false;
   if (start >= 0 && start < net.C)
-    done = near_walk<double, SCAN, false>(net, io, wp, rid, rid - level_first(io), P, S, eq, p, start, 0.0, sc, net.D - 1) ==
-           NEAR_DONE;
+    done = near_walk<double, SCAN, ALL ? SET_LDS : SET_NEAR>(net, io, wp, rid, rid - level_first(io), P, S, eq, p, start,
+                                                             0.0, sc, net.D - 1) == NEAR_DONE;
   // (thread 0 wrote the flag in finish_region: the orientation may be undecided)
   if (threadIdx.x == 0 && (!done || (!SCAN && (io.flags[rid - level_first(io)] & AM_UNDECIDED)))) {
     for (int q = 0; q < 4; ++q) eqb[(size_t)b * 4 + q] = eq[q];
     near_left(left, b);
   }
 }
-template __global__ void k_near64<true>(NetDev, PrefixDev, RegionIO, int, WalkParams, double*, int, NearList);
-template __global__ void k_near64<false>(NetDev, PrefixDev, RegionIO, int, WalkParams, double*, int, NearList);
+template __global__ void k_near64<true, false>(NetDev, PrefixDev, RegionIO, int, WalkParams, double*, int, NearList);
+template __global__ void k_near64<false, false>(NetDev, PrefixDev, RegionIO, int, WalkParams, double*, int, NearList);
+template __global__ void k_near64<true, true>(NetDev, PrefixDev, RegionIO, int, WalkParams, double*, int, NearList);
+template __global__ void k_near64<false, true>(NetDev, PrefixDev, RegionIO, int, WalkParams, double*, int, NearList);
 
 // The listed regions (blocks stride over the list) on all constraints: with
 // `quick` the walk that reads the planes once per vertex, then, for seeds and
@@ -528,7 +533,7 @@ __global__ __launch_bounds__(64, 4) void k_walk_fp64(NetDev net, PrefixDev pf, R
       for (int w = lane; w < net.Wd; w += 64) S.mask[w] = io.reg_mask[(size_t)rid * net.Wd + w];
       __syncthreads();
       const PrefixPlanes P{net, s_bases, S.mask};
-      const int done = near_walk<double, true, true>(net, io, wp, rid, rid - level_first(io), P, S, eq, p, start);
+      const int done = near_walk<double, true, SET_ALL>(net, io, wp, rid, rid - level_first(io), P, S, eq, p, start);
       __syncthreads();
       if (done == NEAR_DONE) continue;
     }
