@@ -28,6 +28,7 @@
 #include "am_adjoint.h"
 #include "am_newton.h"
 #include "am_combine.h"
+#include "am_mem.h"
 #include "am_near.h"
 #include "am_prefix.h"
 #include "am_scan.h"
@@ -44,26 +45,29 @@ template <typename T>
 struct DevBuf {
   T* p = nullptr;
   size_t n = 0;
+  Mem mem;
   DevBuf() = default;
-  DevBuf(const DevBuf&) = delete;
-  DevBuf& operator=(const DevBuf&) = delete;
-  DevBuf(DevBuf&& o) noexcept : p(o.p), n(o.n) {
-    o.p = nullptr;
-    o.n = 0;
-  }
+  DevBuf(DevBuf&& o) noexcept { swap(o); }
   DevBuf& operator=(DevBuf&& o) noexcept {
     if (this != &o) {
       release();
-      p = o.p;
-      n = o.n;
-      o.p = nullptr;
-      o.n = 0;
+      swap(o);
     }
     return *this;
   }
-  ~DevBuf() { release(); }
+  void swap(DevBuf& o) noexcept {
+    std::swap(p, o.p);
+    std::swap(n, o.n);
+    mem.swap(o.mem);
+  }
+  hipError_t take(size_t count) {
+    const hipError_t e = mem.take(MEM_DEVICE, count * sizeof(T));
+    p = static_cast<T*>(mem.p);
+    n = mem.bytes / sizeof(T);
+    return e;
+  }
   void release() {
-    if (p) (void)hipFree(p);
+    mem.release();
     p = nullptr;
     n = 0;
   }
@@ -91,15 +95,10 @@ template <typename T>
 void ensure(DevBuf<T>& b, size_t n, bool keep, hipStream_t st) {
   if (b.n >= n) return;
   size_t cap = std::max<size_t>(n, b.n ? b.n * 2 : 1024);
-  T* q = nullptr;
-  HIPCHK(hipMalloc(&q, cap * sizeof(T)));
-  if (keep && b.p && b.n) HIPCHK(hipMemcpyAsync(q, b.p, b.n * sizeof(T), hipMemcpyDeviceToDevice, st));
-  if (b.p) {
-    HIPCHK(hipStreamSynchronize(st));
-    HIPCHK(hipFree(b.p));
-  }
-  b.p = q;
-  b.n = cap;
+  DevBuf<T> q;
+  HIPCHK(q.take(cap));
+  if (keep && b.p && b.n) HIPCHK(hipMemcpyAsync(q.p, b.p, b.n * sizeof(T), hipMemcpyDeviceToDevice, st));
+  b = std::move(q);   // (the old block goes once the device is done with it)
 }
 
 inline unsigned blocks(size_t n, unsigned t) { return (unsigned)((n + t - 1) / t); }
@@ -141,6 +140,12 @@ struct PrefixStore {
 };
 
 }  // namespace
+
+// Results into pageable host arrays: 16 pinned slots of one chunk, their events.
+struct HostCopy {
+  Mem pin;
+  std::vector<hipEvent_t> ev;
+};
 
 struct am_ctx {
   // architecture
@@ -215,14 +220,12 @@ struct am_ctx {
   size_t stage_used = 0;
 
   // pinned, coherent host word the device writes scan totals into (arm_host_total)
+  Mem host_mem;
   int* host_total = nullptr;
   int* host_total_dev = nullptr;
   int host_seq = 0;
   DevBuf<int2> levels;                    // [kHostRing] first region and count of the levels in flight
-  // pinned staging for am_get_mesh into pageable host arrays (grown, kept)
-  unsigned char* mesh_pin = nullptr;
-  size_t mesh_pin_bytes = 0;
-  std::vector<hipEvent_t> mesh_ev;   // one per 2 MB chunk of the staged copy (created once, kept)
+  HostCopy copy;                     // staging for results going into pageable host arrays (kept)
 
   // tiled FP64 chain (nets without skips, layers up to AM_CHAIN_MAXW wide)
   bool tile_ok = false;
@@ -290,8 +293,8 @@ constexpr int kHostRing = 8, kHostWords = 32;
 
 int arm_host_total(am_ctx* c) {
   if (!c->host_total) {
-    HIPCHK(hipHostMalloc((void**)&c->host_total, kHostRing * kHostWords * sizeof(int),
-                         hipHostMallocMapped | hipHostMallocCoherent));
+    HIPCHK(c->host_mem.take(MEM_COHERENT, kHostRing * kHostWords * sizeof(int)));
+    c->host_total = static_cast<int*>(c->host_mem.p);
     HIPCHK(hipHostGetDevicePointer((void**)&c->host_total_dev, c->host_total, 0));
     c->host_seq = 0;
   }
@@ -692,14 +695,12 @@ bool prefix_blocks(am_ctx* c, const long long* ids, bool must) {
     if (!fits && !must) return false;
     if (!fits) bytes = want;
     DevBuf<char> b;
-    const hipError_t er = hipMalloc(&b.p, bytes);
+    const hipError_t er = b.take(bytes);
     if (er != hipSuccess) {
       (void)hipGetLastError();
-      b.p = nullptr;
-      if (must) throw HipErr{er, "hipMalloc of the activation prefixes' planes"};
+      if (must) throw HipErr{er, "allocation of the activation prefixes' planes"};
       return false;
     }
-    b.n = bytes;
     s.bytes += bytes;
     s.arena_left = bytes;
     s.arena = b.p;
@@ -1119,9 +1120,11 @@ struct am_batch {
   DevBuf<NetDev> nets_d;
   DevBuf<ChainIO> cios_d;
   DevBuf<int4> tiles_d;
+  Mem tiles_mem, hist_mem;
   int4* tiles_h = nullptr;       // pinned staging of a level's tile list
   size_t tiles_cap = 0;
   DevBuf<int> hist_d, sel_flags, sel_rank, sel_ids;
+  DevBuf<uint32_t> sel_words;   // a network's records, gathered for the copy out
   int* hist_h = nullptr;         // pinned: regions per network of the level
 };
 
@@ -1181,10 +1184,9 @@ BatchLevelPlan batch_level_prepare(am_batch* b, long long first, long long count
   if (seg[nn] != count) throw std::runtime_error("batch level: network counts do not add up");
   const size_t max_tiles = (size_t)(count + AM_CT - 1) / AM_CT + (size_t)nn * ((count + chunk - 1) / chunk + 1);
   if (max_tiles > b->tiles_cap) {
-    if (b->tiles_h) HIPCHK(hipHostFree(b->tiles_h));
-    b->tiles_h = nullptr;
     b->tiles_cap = std::max(max_tiles, b->tiles_cap * 2);
-    HIPCHK(hipHostMalloc((void**)&b->tiles_h, b->tiles_cap * sizeof(int4), hipHostMallocDefault));
+    HIPCHK(b->tiles_mem.take(MEM_PINNED, b->tiles_cap * sizeof(int4)));
+    b->tiles_h = static_cast<int4*>(b->tiles_mem.p);
     ensure(b->tiles_d, b->tiles_cap, false, st);
   }
   std::vector<size_t> chunk_tile0;
@@ -2105,6 +2107,92 @@ static void mesh_to_host(am_ctx* c) {
   c->mesh_on_host = true;
 }
 
+namespace {
+
+struct Part {
+  void* dst;   // the caller's array, or null
+  const void* src;
+  size_t bytes;
+};
+
+// Device arrays into the caller's.  Device, pinned or managed ones get them
+// straight from device memory.  Pageable ones: in chunks, each by one DMA into a
+// pinned slot and then by one of eight host threads into the array, while the
+// next chunks are on their way (a plain copy into pageable memory stages through
+// small chunks and one host thread: about 10 GB/s, less into fresh pages; marching
+// eight networks and copying out their 188 MB of records takes 41 ms with it, 28 so).  A thread
+// owns two slots and refills one as soon as it has emptied it.
+void copy_out(am_ctx* c, const std::vector<Part>& all, hipStream_t st) {
+  std::vector<Part> parts;
+  size_t staged = 0;
+  for (const Part& p : all) {
+    if (!p.dst || !p.bytes) continue;
+    if (pageable_host(p.dst)) {
+      parts.push_back(p);
+      staged += p.bytes;
+    } else {
+      HIPCHK(hipMemcpy(p.dst, p.src, p.bytes, hipMemcpyDefault));
+    }
+  }
+  if (!staged) return;
+  const size_t chunk = std::min<size_t>((size_t)2 << 20, std::max<size_t>((size_t)256 << 10, (staged / 16 + 4095) / 4096 * 4096));
+  std::vector<Part> chunks;
+  for (const Part& p : parts)
+    for (size_t a = 0; a < p.bytes; a += chunk)
+      chunks.push_back(Part{(unsigned char*)p.dst + a, (const unsigned char*)p.src + a, std::min(chunk, p.bytes - a)});
+  const size_t nt = std::min<size_t>(8, (chunks.size() + 1) / 2), slots = std::min(2 * nt, chunks.size());
+  if (c->copy.pin.bytes < slots * chunk) HIPCHK(c->copy.pin.take(MEM_PINNED, slots * chunk));
+  while (c->copy.ev.size() < slots) {
+    hipEvent_t e;
+    HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    c->copy.ev.push_back(e);
+  }
+  // chunk k goes through slot k % (2 nt) and is lane k % nt's
+  unsigned char* const pin = static_cast<unsigned char*>(c->copy.pin.p);
+  auto fetch = [&](size_t k) -> hipError_t {
+    const size_t s = k % (2 * nt);
+    const hipError_t e = hipMemcpyAsync(pin + s * chunk, chunks[k].src, chunks[k].bytes, hipMemcpyDeviceToHost, st);
+    return e != hipSuccess ? e : hipEventRecord(c->copy.ev[s], st);
+  };
+  std::atomic<size_t> next{0};
+  std::atomic<int> bad{hipSuccess};
+  for (size_t k = 0; k < slots && bad == hipSuccess; ++k) bad = fetch(k);
+  auto work = [&]() {
+    for (size_t lane; (lane = next++) < nt;)
+      for (size_t k = lane; k < chunks.size(); k += nt) {
+        const size_t s = k % (2 * nt);
+        hipError_t e = bad != hipSuccess ? hipErrorUnknown : hipEventSynchronize(c->copy.ev[s]);
+        if (e == hipSuccess) {
+          std::memcpy(chunks[k].dst, pin + s * chunk, chunks[k].bytes);
+          if (k + 2 * nt < chunks.size()) e = fetch(k + 2 * nt);
+        }
+        if (e != hipSuccess) {
+          int ok = hipSuccess;
+          bad.compare_exchange_strong(ok, e);
+          return;
+        }
+      }
+  };
+  std::vector<std::thread> th;
+  try {
+    th.reserve(nt);
+    while (th.size() + 1 < nt)
+      th.emplace_back([&]() {
+        if (hipSetDevice(c->dev) == hipSuccess) work();
+      });
+  } catch (const std::exception&) {
+    // fewer threads: the others take their lanes
+  }
+  work();
+  for (auto& t : th) t.join();
+  if (bad != hipSuccess) {
+    (void)hipStreamSynchronize(st);   // the slots are written no more
+    throw HipErr{(hipError_t)bad.load(), "copy of the results to host memory"};
+  }
+}
+
+}  // namespace
+
 am_status am_get_mesh(am_ctx* c, double* vertices, int* face_offsets, int* face_indices) {
   if (!c) return AM_ERR_ARG;
   if (!c->has_mesh) return fail(c, AM_ERR_STATE, "am_get_mesh called before am_combine");
@@ -2115,79 +2203,10 @@ am_status am_get_mesh(am_ctx* c, double* vertices, int* face_offsets, int* face_
       if (face_indices) std::memcpy(face_indices, c->mesh_idx.data(), c->mesh_idx.size() * 4);
       return AM_OK;
     }
-    // Device, pinned or managed caller arrays get the arrays straight from
-    // device memory.  Pageable ones: each array goes by one DMA into a pinned
-    // staging buffer the context keeps, then by a host copy over several
-    // threads (a plain copy into pageable memory stages through small chunks
-    // and one host thread: about 10 GB/s).
-    struct Part {
-      void* dst;
-      const void* src;
-      size_t bytes;
-    };
-    Part parts[3] = {{vertices, c->m_xyz.p, vertices ? (size_t)c->mesh_V * 3 * 8 : 0},
-                     {face_offsets, c->m_face_off.p, face_offsets ? (size_t)c->mesh_F * 4 : 0},
-                     {face_indices, c->m_face_idx.p, face_indices ? (size_t)c->mesh_NI * 4 : 0}};
-    size_t staged = 0;
-    bool stage[3] = {false, false, false};
-    for (int i = 0; i < 3; ++i) {
-      if (!parts[i].bytes) continue;
-      stage[i] = pageable_host(parts[i].dst);
-      if (stage[i]) staged += (parts[i].bytes + 255) & ~(size_t)255;
-      else HIPCHK(hipMemcpy(parts[i].dst, parts[i].src, parts[i].bytes, hipMemcpyDefault));
-    }
-    if (staged) {
-      if (staged > c->mesh_pin_bytes) {
-        if (c->mesh_pin) HIPCHK(hipHostFree(c->mesh_pin));
-        c->mesh_pin = nullptr;
-        c->mesh_pin_bytes = 0;
-        HIPCHK(hipHostMalloc((void**)&c->mesh_pin, staged, hipHostMallocDefault));
-        c->mesh_pin_bytes = staged;
-      }
-      // chunks of 2 MB, each DMA followed by an event; host threads copy a
-      // chunk out as soon as its event has passed, so the copies overlap the
-      // later DMAs
-      struct Chunk {
-        void* dst;
-        const unsigned char* src;
-        size_t len;
-      };
-      std::vector<Chunk> chunks;
-      const size_t kChunk = (size_t)2 << 20;
-      size_t o = 0;
-      for (int i = 0; i < 3; ++i)
-        if (stage[i]) {
-          for (size_t a = 0; a < parts[i].bytes; a += kChunk) {
-            const size_t len = std::min(kChunk, parts[i].bytes - a);
-            if (chunks.size() == c->mesh_ev.size()) {
-              hipEvent_t e;
-              HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-              c->mesh_ev.push_back(e);
-            }
-            HIPCHK(hipMemcpyAsync(c->mesh_pin + o + a, (const unsigned char*)parts[i].src + a, len,
-                                  hipMemcpyDeviceToHost, c->stream));
-            HIPCHK(hipEventRecord(c->mesh_ev[chunks.size()], c->stream));
-            chunks.push_back(Chunk{(unsigned char*)parts[i].dst + a, c->mesh_pin + o + a, len});
-          }
-          o += (parts[i].bytes + 255) & ~(size_t)255;
-        }
-      const int nt = (int)std::min<size_t>(8, chunks.size());
-      std::atomic<int> bad{0};
-      auto work = [&](int id) {
-        for (size_t k = id; k < chunks.size(); k += nt) {
-          if (hipEventSynchronize(c->mesh_ev[k]) != hipSuccess) {
-            bad = 1;
-            return;
-          }
-          std::memcpy(chunks[k].dst, chunks[k].src, chunks[k].len);
-        }
-      };
-      std::vector<std::thread> th;
-      for (int id = 1; id < nt; ++id) th.emplace_back(work, id);
-      work(0);
-      for (auto& t : th) t.join();
-      if (bad) HIPCHK(hipStreamSynchronize(c->stream));   // reports the failed copy
-    }
+    copy_out(c, {{vertices, c->m_xyz.p, (size_t)c->mesh_V * 3 * 8},
+                 {face_offsets, c->m_face_off.p, (size_t)c->mesh_F * 4},
+                 {face_indices, c->m_face_idx.p, (size_t)c->mesh_NI * 4}},
+             c->stream);
     if (face_offsets) {
       const int ni = (int)c->mesh_NI;
       HIPCHK(hipMemcpy(face_offsets + c->mesh_F, &ni, 4, hipMemcpyDefault));
@@ -2203,12 +2222,13 @@ am_status am_get_regions(am_ctx* c, uint32_t* masks, int* info, int* tabs, doubl
   return guarded(c, [&]() -> am_status {
     const size_t R = (size_t)c->R;
     if (R == 0) return AM_OK;
-    if (masks) HIPCHK(hipMemcpy(masks, c->reg_mask.p, R * c->Wd * 4, hipMemcpyDeviceToHost));
-    if (info) HIPCHK(hipMemcpy(info, c->reg_info.p, R * AM_INFO_STRIDE * 4, hipMemcpyDeviceToHost));
-    if (tabs) HIPCHK(hipMemcpy(tabs, c->reg_tab.p, R * (c->vm + 1) * 4, hipMemcpyDeviceToHost));
-    if (verts) HIPCHK(hipMemcpy(verts, c->reg_verts.p, R * c->vm * 3 * 8, hipMemcpyDeviceToHost));
-    if (vpairs) HIPCHK(hipMemcpy(vpairs, c->reg_vpair.p, R * c->vm * 2 * 4, hipMemcpyDeviceToHost));
-    if (points) HIPCHK(hipMemcpy(points, c->reg_point.p, R * 3 * 8, hipMemcpyDeviceToHost));
+    copy_out(c, {{masks, c->reg_mask.p, R * c->Wd * 4},
+                 {info, c->reg_info.p, R * AM_INFO_STRIDE * 4},
+                 {tabs, c->reg_tab.p, R * (c->vm + 1) * 4},
+                 {verts, c->reg_verts.p, R * c->vm * 3 * 8},
+                 {vpairs, c->reg_vpair.p, R * c->vm * 2 * 4},
+                 {points, c->reg_point.p, R * 3 * 8}},
+             c->own_stream);   // (a march has ended when am_run returns)
     return AM_OK;
   });
 }
@@ -2515,16 +2535,15 @@ am_status am_destroy(am_ctx* c) {
   if (c->own_stream) (void)hipStreamSynchronize(c->own_stream);
   for (hipGraphExec_t& e : c->gexec)
     if (e) (void)hipGraphExecDestroy(e);
+  const MemQuiet quiet;
   c->timer.release();
-  fast_release(c->fbuf);
   if (c->own_stream) (void)hipStreamSynchronize(c->own_stream);
-  if (c->host_total) (void)hipHostFree(c->host_total);   // every level waited for its total
-  if (c->mesh_pin) (void)hipHostFree(c->mesh_pin);
-  for (hipEvent_t e : c->mesh_ev) (void)hipEventDestroy(e);
+  for (hipEvent_t e : c->copy.ev) (void)hipEventDestroy(e);
   if (c->null_ev) (void)hipEventDestroy(c->null_ev);
   hipStream_t own = c->own_stream;
   delete c;
   if (own) (void)hipStreamDestroy(own);
+  MemPool::get().age();
   return AM_OK;
 }
 
@@ -2690,7 +2709,10 @@ am_status am_batch_run(am_batch* b, const void* const* weights, const void* cons
     HIPCHK(hipMemcpyAsync(b->nets_d.p, b->nets_h.data(), nn * sizeof(NetDev), hipMemcpyHostToDevice, st));
     ensure(b->cios_d, (size_t)nn, false, st);
     ensure(b->hist_d, (size_t)nn, false, st);
-    if (!b->hist_h) HIPCHK(hipHostMalloc((void**)&b->hist_h, (size_t)1 << 22, hipHostMallocDefault));
+    if (!b->hist_h) {
+      HIPCHK(b->hist_mem.take(MEM_PINNED, (size_t)1 << 22));
+      b->hist_h = static_cast<int*>(b->hist_mem.p);
+    }
     if ((size_t)nn * sizeof(int) > ((size_t)1 << 22)) throw CapErr{"too many networks"};
     const size_t clds = batch_chain_lds(b), slds = batch_scan_lds(b), rlds = batch_ray_lds(b);
     if (clds > c->max_lds || slds > c->max_lds) throw CapErr{"networks too wide for the batch kernels' LDS"};
@@ -2871,23 +2893,34 @@ am_status am_batch_get_regions(am_batch* b, int net, long long* n_regions, uint3
     *n_regions = n;
     if (n == 0 || (!masks && !info && !tabs && !verts && !vpairs && !points)) return AM_OK;
     const int vm = c->vm, Wn = b->nets[net].Wn;
-    DevBuf<uint32_t> tmp;
-    auto gather = [&](const void* src, int stride_words, int copy_words, void* dst) {
-      if (!dst) return;
-      ensure(tmp, (size_t)n * copy_words, false, st);
-      const size_t tot = (size_t)n * copy_words;
-      hipLaunchKernelGGL(k_gather_words, dim3(blocks(tot, 256)), dim3(256), 0, st, (const uint32_t*)src,
-                         stride_words, copy_words, (const int*)b->sel_ids.p, n, tmp.p, copy_words);
-      HIPCHK(hipGetLastError());
-      HIPCHK(hipMemcpyAsync(dst, tmp.p, tot * 4, hipMemcpyDeviceToHost, st));
-      HIPCHK(hipStreamSynchronize(st));
+    std::vector<Part> parts;
+    size_t words = 0;
+    struct Field {
+      const void* src;
+      int stride, copy;
+      void* dst;
     };
-    gather(c->reg_mask.p, c->Wd, Wn, masks);
-    gather(c->reg_info.p, AM_INFO_STRIDE, AM_INFO_STRIDE, info);
-    gather(c->reg_tab.p, vm + 1, vm + 1, tabs);
-    gather(c->reg_verts.p, vm * 6, vm * 6, verts);
-    gather(c->reg_vpair.p, vm * 2, vm * 2, vpairs);
-    gather(c->reg_point.p, 6, 6, points);
+    const Field fields[6] = {{c->reg_mask.p, c->Wd, Wn, masks},
+                             {c->reg_info.p, AM_INFO_STRIDE, AM_INFO_STRIDE, info},
+                             {c->reg_tab.p, vm + 1, vm + 1, tabs},
+                             {c->reg_verts.p, vm * 6, vm * 6, verts},
+                             {c->reg_vpair.p, vm * 2, vm * 2, vpairs},
+                             {c->reg_point.p, 6, 6, points}};
+    for (const Field& f : fields)
+      if (f.dst) words += (size_t)n * f.copy;
+    DevBuf<uint32_t>& tmp = b->sel_words;
+    ensure(tmp, words, false, st);
+    size_t at = 0;
+    for (const Field& f : fields) {
+      if (!f.dst) continue;
+      const size_t tot = (size_t)n * f.copy;
+      hipLaunchKernelGGL(k_gather_words, dim3(blocks(tot, 256)), dim3(256), 0, st, (const uint32_t*)f.src, f.stride,
+                         f.copy, (const int*)b->sel_ids.p, n, tmp.p + at, f.copy);
+      parts.push_back(Part{f.dst, tmp.p + at, tot * 4});
+      at += tot;
+    }
+    HIPCHK(hipGetLastError());
+    copy_out(c, parts, st);
     return AM_OK;
   });
 }
@@ -2913,17 +2946,8 @@ const char* am_batch_last_error(const am_batch* b) { return b ? am_last_error(b-
 am_status am_batch_destroy(am_batch* b) {
   if (!b) return AM_ERR_ARG;
   if (b->c) (void)hipStreamSynchronize(b->c->stream);
-  if (b->tiles_h) (void)hipHostFree(b->tiles_h);
-  if (b->hist_h) (void)hipHostFree(b->hist_h);
+  const MemQuiet quiet;
   am_ctx* c = b->c;
-  b->nets.clear();
-  b->nets_d.release();
-  b->cios_d.release();
-  b->tiles_d.release();
-  b->hist_d.release();
-  b->sel_flags.release();
-  b->sel_rank.release();
-  b->sel_ids.release();
   delete b;
   if (c) am_destroy(c);
   return AM_OK;

@@ -7,6 +7,7 @@
 #include <stdint.h>
 
 #include "am_kernels.h"
+#include "am_mem.h"
 #include "am_timer.h"
 #include "am_walk.h"
 
@@ -57,8 +58,7 @@ struct FastNet {
 };
 
 struct FastBuffers {
-  void* mem[64] = {nullptr};
-  size_t bytes[64] = {0};
+  Mem mem[64];
 };
 
 struct FastLevel {
@@ -114,6 +114,5 @@ void fast_level_prepare(FastNet& f, FastBuffers& b, const NetDev& net, int count
 // reduced-precision form: planes [n][AM_PCOMP][Cs] f32 (x, y, z, c signed, then
 // each plane's error estimate sigma), eq [n][AM_EQS] f32 (x, y, z, c, sigma).
 void fast_planes(FastNet& f, const uint32_t* reg_mask, int n, float* planes, float* eq, hipStream_t st);
-void fast_release(FastBuffers& b);
 
 }  // namespace am

@@ -633,15 +633,8 @@ enum Slot {
 
 // Buffer s with at least `bytes`; grows geometrically (levels grow run by run).
 void* slot(FastBuffers& b, int s, size_t bytes) {
-  if (b.bytes[s] < bytes) {
-    const size_t cap = std::max<size_t>({bytes, 2 * b.bytes[s], 256});
-    if (b.mem[s]) (void)hipFree(b.mem[s]);
-    b.mem[s] = nullptr;
-    b.bytes[s] = 0;
-    FCHK(hipMalloc(&b.mem[s], cap));
-    b.bytes[s] = cap;
-  }
-  return b.mem[s];
+  if (b.mem[s].bytes < bytes) FCHK(b.mem[s].take(MEM_DEVICE, std::max<size_t>({bytes, 2 * b.mem[s].bytes, 256})));
+  return b.mem[s].p;
 }
 
 // host copy as float of a device-readable array (ordered after earlier work on st)
@@ -925,14 +918,6 @@ void fast_planes(FastNet& f, const uint32_t* reg_mask, int n, float* planes, flo
     hipLaunchKernelGGL(k_gemm<1>, dim3((n + AM_GT - 1) / AM_GT), dim3(256), glds, st, f.dev, g);
   FCHK(hipGetLastError());
   FCHK(hipStreamSynchronize(st));
-}
-
-void fast_release(FastBuffers& b) {
-  for (int i = 0; i < 64; ++i) {
-    if (b.mem[i]) (void)hipFree(b.mem[i]);
-    b.mem[i] = nullptr;
-    b.bytes[i] = 0;
-  }
 }
 
 }  // namespace am
