@@ -1621,7 +1621,16 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
     // re-decisions; nets it does not take (skips, layers over 256 wide) run
     // those forms on the FP64 region kernel, with the same topology.
     const bool reduced_asked = c->precision == AM_PREC_FP32 || c->precision == AM_PREC_SPLIT_BF16X3;
-    const bool fp64_form = !reduced_asked || !c->tile_ok;
+    // A reduced form whose vertices are all re-solved from FP64 planes (split
+    // BF16; FP32 with reduced_vertices 0) marches on those planes: every region
+    // needs them, and one wave decides a region on them for less than the
+    // reduced product and walk cost before it (a 4x128 network in split BF16, whose
+    // bound decides no region: 20 to 22 ms with them, 12 to 14 without).  Same topology, same
+    // vertices.
+    const bool resolved = reduced_asked && c->fast.walk_mode == 0 &&
+                          (c->precision == AM_PREC_SPLIT_BF16X3 || c->fast.vertex_mode == 0);
+    const bool fp64_form = !reduced_asked || !c->tile_ok || resolved;
+    c->fast.ready = false;
     // FP32 form, Newton vertices: the walk keeps each vertex's inverse system
     // (the Newton kernel takes layers up to AM_CHAIN_MAXW wide, which the
     // reduced forms require anyway, and the ray walk)
@@ -1792,7 +1801,7 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
     HIPCHK(hipMemcpyAsync(&ra, ra_dev, sizeof(ra), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
     const int* acc = ra.acc;
-    const long long redo = fp64_form ? 0 : acc[1 + AM_WHY_COUNT];
+    const long long redo = fp64_form ? (resolved && c->tile_ok ? c->R : 0) : acc[1 + AM_WHY_COUNT];
     const long long vert64 = fp64_form ? 0 : acc[2 + 2 * AM_WHY_COUNT];
     c->timer.resolve();
     const auto t1 = std::chrono::steady_clock::now();
@@ -2240,6 +2249,15 @@ am_status am_planes(am_ctx* c, const uint32_t* masks, int n, float* planes, floa
                                  "reduced forms take: no skips, layers up to 256 wide)");
   return guarded(c, [&]() -> am_status {
     const hipStream_t st = c->stream;
+    if (!c->fast.ready) {
+      // (the march ran on FP64 planes alone: the reduced operands from the FP64 copies)
+      std::vector<const void*> wv, bv;
+      for (int li = 0; li <= c->D; ++li) {
+        wv.push_back(li == 0 ? c->W0.p : c->Wrow[li].p);
+        bv.push_back(c->b[li].p);
+      }
+      fast_prepare(c->fast, c->fbuf, c->net, c->precision, wv.data(), bv.data(), AM_DTYPE_F64, st);
+    }
     const int Cs = c->fast.dev.Cs;
     DevBuf<uint32_t> m;
     DevBuf<float> p, e;

@@ -30,7 +30,7 @@ typedef int am_status;
 
 /* Arithmetic of the constraint planes and of the walk. */
 #define AM_PREC_FP32 0            /* FP32 MFMA planes, FP64 re-decision of undecided regions */
-#define AM_PREC_SPLIT_BF16X3 1    /* split-BF16 (3 products) MFMA planes, FP64 re-decision */
+#define AM_PREC_SPLIT_BF16X3 1    /* split-BF16 (3 products) MFMA planes (am_planes); every region decided in FP64 */
 #define AM_PREC_FP64 2            /* FP64 everywhere (the reference's default dtype) */
 #define AM_PREC_FP64_RAY 3        /* FP64 planes, checked FP64 ray walk, FP64 candidate scan where undecided */
 
@@ -156,7 +156,8 @@ am_status am_topology_fingerprint(am_ctx* ctx, unsigned long long* out5);
  * vertex of a region the reduced walk decides is re-solved from FP64 planes;
  * 1 a region's reduced-plane vertices are kept where the estimate puts all of
  * them within 1e-5 of |v|, the other regions' are re-solved; the split-BF16
- * form always re-solves),
+ * form always re-solves.  Where every vertex is re-solved and the walk is the ray
+ * walk, the march runs on the FP64 planes alone),
  * "adjoint_tiled" (1 default: the
  * adjoint on the tiled FP64 chain and GEMMs; 0 one kernel per region),
  * "adjoint_mfma" (1 default: those GEMMs on the FP64 matrix cores; 0 VALU),
@@ -196,7 +197,7 @@ am_status am_set_option(am_ctx* ctx, const char* key, long long value);
 #define AM_STAT_CHAIN64_LAUNCHES 31 /* launches of the FP64 tiled chain */
 #define AM_STAT_VERT64_MS 32    /* FP64 vertex re-solve of regions the reduced-precision walk decided (HIP events) */
 #define AM_STAT_VERT64_REGIONS 33 /* regions whose vertices were re-solved from FP64 planes */
-#define AM_STAT_FP64_ONLY 34    /* 1: a reduced form ran on the FP64 region kernel (skips or layers over 256 wide) */
+#define AM_STAT_FP64_ONLY 34    /* 1: a reduced form marched on FP64 planes alone (skips, layers over 256 wide, every vertex re-solved) */
 #define AM_STAT_HOST_WAITS 35   /* host waits on the device during the run */
 #define AM_STAT_GRAPH_LAUNCHES 36 /* levels launched as one captured graph ("graph_levels") */
 #define AM_STAT_NEWTON_MS 37    /* FP32 form: FP64 Newton step of the vertices (HIP events, with its vertex dedup) */
