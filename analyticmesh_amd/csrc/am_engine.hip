@@ -515,10 +515,12 @@ size_t region_lds_bytes(const am_ctx* c, int& Cs, int& Csort) {
          (size_t)((c->C + 31) / 32) * 4 + (size_t)c->Wd * 4 + 64;
 }
 
-size_t chain_lds_bytes(const am_ctx* c) {
-  return ((size_t)AM_CXR * AM_CXS + 1) * sizeof(double) + (size_t)c->D * AM_KLS * sizeof(uint16_t) +
-         (size_t)AM_CT * c->Wd * 4 + 16;
+int chain_maxw(const am_ctx* c) {
+  int m = 1;
+  for (int i = 1; i <= c->D + 1; ++i) m = std::max(m, c->nodes[i]);
+  return m;
 }
+size_t chain_lds_bytes(const am_ctx* c) { return chain_tile_lds(chain_maxw(c), c->Wd); }
 
 // Per-run counters of the FP64 stages (kernel times go to the context's timer;
 // the ray walk's undecided count and reasons accumulate on the device).
@@ -1114,18 +1116,16 @@ struct am_batch {
   am_ctx* c = nullptr;
   int precision = AM_PREC_FP64_RAY;
   std::vector<BatchNet> nets;
-  int Wmax = 0, Dmax = 0, Cmax = 0, Lmax = 0;
+  int Wmax = 0, Cmax = 0, Lmax = 0;
   std::vector<NetDev> nets_h;
   std::vector<ChainIO> cios_h;
   DevBuf<NetDev> nets_d;
   DevBuf<ChainIO> cios_d;
   DevBuf<int4> tiles_d;
-  Mem tiles_mem, hist_mem;
-  int4* tiles_h = nullptr;       // pinned staging of a level's tile list
-  size_t tiles_cap = 0;
-  DevBuf<int> hist_d, sel_flags, sel_rank, sel_ids;
+  int maxw = 1;                 // widest layer
+  DevBuf<int> seg_d;            // the networks' first regions of a chunk
+  DevBuf<int> sel_flags, sel_rank, sel_ids;
   DevBuf<uint32_t> sel_words;   // a network's records, gathered for the copy out
-  int* hist_h = nullptr;         // pinned: regions per network of the level
 };
 
 namespace {
@@ -1147,22 +1147,24 @@ size_t batch_ray_lds(const am_batch* b) {
                         walk_rec_bytes(b->c->vm, false));
   return m;
 }
-size_t batch_chain_lds(const am_batch* b) {
-  return ((size_t)AM_CXR * AM_CXS + 1) * sizeof(double) + (size_t)b->Dmax * AM_KLS * sizeof(uint16_t) +
-         (size_t)AM_CT * b->c->Wd * 4 + 16;
+size_t batch_near_lds(const am_batch* b) {
+  return near_lds_bytes(b->Cmax, b->c->Wd, b->c->vm, 8, false, b->Cmax <= AM_ALL_MAX);
 }
+size_t batch_chain_lds(const am_batch* b) { return chain_tile_lds(b->maxw, b->c->Wd); }
 
 // Planes and walks of the level's regions (first .. first + count - 1, grouped
-// by network in ascending order; hist_h has the per-network counts).
+// by network in ascending order).
 struct BatchLevelPlan {
   long long first = 0, count = 0;
-  size_t chunk = 0, nt = 0;
-  std::vector<size_t> chunk_tile0;
+  size_t chunk = 0;
 };
 
-void batch_level_launch(am_batch* b, const BatchLevelPlan& pl, Fp64Counts& t);
+// Tiles of n regions: full ones, and a partial one per network at most.
+int batch_tiles(const am_batch* b, long long n) {
+  return (int)((n + AM_CT - 1) / AM_CT + std::min<long long>((long long)b->nets.size(), n));
+}
 
-// Host part of a level: buffers and the tile list (in pinned memory).
+// Host part of a level: its buffers.
 BatchLevelPlan batch_level_prepare(am_batch* b, long long first, long long count) {
   am_ctx* c = b->c;
   const hipStream_t st = c->stream;
@@ -1175,37 +1177,9 @@ BatchLevelPlan batch_level_prepare(am_batch* b, long long first, long long count
   const size_t cap = std::min<size_t>(chunk, (size_t)count);
   ensure(c->tplanes, cap * 4 * Ch, false, st);
   ensure(c->teq, cap * 4, false, st);
-  ensure(c->tslots, cap, false, st);
-  ensure(c->tcnt, 1, false, st);
-  // tiles: per chunk, per network segment, AM_CT regions (chunk-relative r0)
-  const int nn = (int)b->nets.size();
-  std::vector<long long> seg(nn + 1, 0);
-  for (int i = 0; i < nn; ++i) seg[i + 1] = seg[i] + b->hist_h[i];
-  if (seg[nn] != count) throw std::runtime_error("batch level: network counts do not add up");
-  const size_t max_tiles = (size_t)(count + AM_CT - 1) / AM_CT + (size_t)nn * ((count + chunk - 1) / chunk + 1);
-  if (max_tiles > b->tiles_cap) {
-    b->tiles_cap = std::max(max_tiles, b->tiles_cap * 2);
-    HIPCHK(b->tiles_mem.take(MEM_PINNED, b->tiles_cap * sizeof(int4)));
-    b->tiles_h = static_cast<int4*>(b->tiles_mem.p);
-    ensure(b->tiles_d, b->tiles_cap, false, st);
-  }
-  std::vector<size_t> chunk_tile0;
-  size_t nt = 0;
-  for (long long cs = 0; cs < count; cs += (long long)chunk) {
-    const long long ce = std::min<long long>(cs + (long long)chunk, count);
-    chunk_tile0.push_back(nt);
-    for (int i = 0; i < nn; ++i) {
-      const long long a = std::max(seg[i], cs), e = std::min(seg[i + 1], ce);
-      for (long long r = a; r < e; r += AM_CT) b->tiles_h[nt++] = make_int4(i, (int)(r - cs), (int)std::min<long long>(AM_CT, e - r), 0);
-    }
-  }
-  chunk_tile0.push_back(nt);
+  ensure(c->tslots, 2 * cap, false, st);   // the near walk's leavings, then the ray walk's
+  ensure(b->tiles_d, (size_t)batch_tiles(b, (long long)cap), false, st);
   pl.chunk = chunk;
-  pl.nt = nt;
-  pl.chunk_tile0 = std::move(chunk_tile0);
-  // stream-ordered after the previous level's kernels (which read the old
-  // list) and kept out of graph captures (no memcpy nodes)
-  HIPCHK(hipMemcpyAsync(b->tiles_d.p, b->tiles_h, nt * sizeof(int4), hipMemcpyHostToDevice, st));
   return pl;
 }
 
@@ -1214,29 +1188,35 @@ void batch_level_launch(am_batch* b, const BatchLevelPlan& pl, Fp64Counts& t) {
   am_ctx* c = b->c;
   const hipStream_t st = c->stream;
   const long long first = pl.first, count = pl.count;
-  const size_t chunk = pl.chunk;
-  const std::vector<size_t>& chunk_tile0 = pl.chunk_tile0;
-  const int Ch = (b->Cmax + 63) & ~63;
+  const size_t chunk = pl.chunk, cap = std::min<size_t>(chunk, (size_t)count);
+  const int Ch = (b->Cmax + 63) & ~63, nn = (int)b->nets.size();
   const size_t clds = batch_chain_lds(b), slds = batch_scan_lds(b), rlds = batch_ray_lds(b);
   const bool ray = b->precision == AM_PREC_FP64_RAY && rlds <= c->max_lds;
-  // the ray walk certifies its decisions: its planes may come from the matrix cores
-  const bool mf = ray && c->chain_mfma;
-  const WalkParams& kr = mf ? kRay64Mf : kRay64;
-  StageTimer& tm = c->timer;
-  size_t k = 0;
-  for (long long cs = 0; cs < count; cs += (long long)chunk, ++k) {
+  const WalkParams& kr = c->chain_mfma ? kRay64Mf : kRay64;
+  const bool all = b->Cmax <= AM_ALL_MAX;
+  const size_t nlds = batch_near_lds(b);
+  const NetDev* nd = (const NetDev*)b->nets_d.p;
+  const double* P = c->tplanes.p;
+  const double* E = c->teq.p;
+  const NearList near{c->tcnt.p, c->tslots.p};
+  const SlotList left{c->tcnt.p + 1, c->tslots.p + cap, c->acc};
+  for (long long cs = 0; cs < count; cs += (long long)chunk) {
     const int n = (int)std::min<long long>((long long)chunk, count - cs);
-    const int rid0 = (int)(first + cs);
-    const ChainLevel lv{rid0, n, nullptr, c->tplanes.p, c->teq.p};
-    const int ntile = (int)(chunk_tile0[k + 1] - chunk_tile0[k]);
-    const size_t m0 = tm.mark(st);
-    hipLaunchKernelGGL((mf ? k_chain_tile_fp64_multi<true> : k_chain_tile_fp64_multi<false>), dim3(ntile),
-                       dim3(AM_CHAIN_THREADS), clds, st, (const NetDev*)b->nets_d.p, (const ChainIO*)b->cios_d.p, lv,
-                       (const int4*)(b->tiles_d.p + chunk_tile0[k]));
+    const int rid0 = (int)(first + cs), ntile = batch_tiles(b, n);
+    const ChainLevel lv{rid0, n, nullptr, c->tplanes.p, c->teq.p, c->reg_mask.p, c->clock};
+    if (cs > 0)   // (the level's first launch finds them cleared)
+      hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, c->tcnt.p, (size_t)2, 0);
+    // up to 64 networks one block finds their regions too
+    if (nn > 64)
+      hipLaunchKernelGGL(k_net_seg, dim3(blocks(nn, 4)), dim3(256), 0, st, (const uint32_t*)c->reg_mask.p, c->Wd, rid0, n,
+                         nn, b->seg_d.p);
+    hipLaunchKernelGGL(k_net_tiles, dim3(1), dim3(1024), 0, st, (const uint32_t*)c->reg_mask.p, c->Wd, rid0, n, nn,
+                       nn > 64 ? 0 : 1, b->seg_d.p, AM_CT, b->tiles_d.p, ntile);
+    hipLaunchKernelGGL((b->maxw > 128 ? k_chain_tile_fp64_multi<8> : k_chain_tile_fp64_multi<4>), dim3(ntile),
+                       dim3(b->maxw > 128 ? 512 : 256), clds, st, nd, (const ChainIO*)b->cios_d.p, lv,
+                       (const int4*)b->tiles_d.p, b->maxw);
     HIPCHK(hipGetLastError());
     t.chain_launches += 1;
-    const size_t m1 = tm.mark(st);
-    tm.span(m0, m1, T_CHAIN64);
     RegionIO io;
     io.reg_mask = c->reg_mask.p;
     io.reg_start = c->reg_start.p;
@@ -1255,58 +1235,38 @@ void batch_level_launch(am_batch* b, const BatchLevelPlan& pl, Fp64Counts& t) {
     io.Csort = 0;
     io.flags = ray ? c->rflags.p : nullptr;
     io.ids = nullptr;
+    io.clk = c->clock;
+    const dim3 list(std::min(n, c->scan_blocks));
     if (!ray) {
-      hipLaunchKernelGGL(k_walk_fp64_multi, dim3(n), dim3(64), slds, st, (const NetDev*)b->nets_d.p, io, c->Wd,
-                         rid0, (const int*)nullptr, (const int*)nullptr, (const double*)c->tplanes.p,
-                         (const double*)c->teq.p, Ch);
+      hipLaunchKernelGGL((all ? k_near64_multi<true, true> : k_near64_multi<true, false>), dim3(n), dim3(64), nlds, st, nd,
+                         io, c->Wd, rid0, kr, P, E, Ch, near);
+      hipLaunchKernelGGL(k_walk_fp64_multi, list, dim3(64), slds, st, nd, io, c->Wd, rid0, (const int*)near.cnt,
+                         (const int*)near.slots, P, E, Ch);
       HIPCHK(hipGetLastError());
-      tm.span(m1, tm.mark(st), T_SCAN64);
       t.scanned_host += n;
       continue;
     }
-    {
-      const NetDev* nd = (const NetDev*)b->nets_d.p;
-      const double* P = c->tplanes.p;
-      const double* E = c->teq.p;
-      switch (c->ray_waves) {
-        case 2:
-          hipLaunchKernelGGL(k_walk_ray64_multi<2>, dim3(n), dim3(128), rlds, st, nd, io, c->Wd, rid0, kr, P, E, Ch);
-          break;
-        case 8:
-          hipLaunchKernelGGL(k_walk_ray64_multi<8>, dim3(n), dim3(512), rlds, st, nd, io, c->Wd, rid0, kr, P, E, Ch);
-          break;
-        default:
-          hipLaunchKernelGGL(k_walk_ray64_multi<4>, dim3(n), dim3(256), rlds, st, nd, io, c->Wd, rid0, kr, P, E, Ch);
-      }
+    hipLaunchKernelGGL((all ? k_near64_multi<false, true> : k_near64_multi<false, false>), dim3(n), dim3(64), nlds, st, nd,
+                       io, c->Wd, rid0, kr, P, E, Ch, near);
+    switch (c->ray_waves) {
+      case 2:
+        hipLaunchKernelGGL(k_walk_ray64_multi<2>, list, dim3(128), rlds, st, nd, io, c->Wd, rid0, kr, P, E, Ch, near,
+                           left);
+        break;
+      case 8:
+        hipLaunchKernelGGL(k_walk_ray64_multi<8>, list, dim3(512), rlds, st, nd, io, c->Wd, rid0, kr, P, E, Ch, near,
+                           left);
+        break;
+      default:
+        hipLaunchKernelGGL(k_walk_ray64_multi<4>, list, dim3(256), rlds, st, nd, io, c->Wd, rid0, kr, P, E, Ch, near,
+                           left);
     }
     HIPCHK(hipGetLastError());
-    const size_t m2 = tm.mark(st);
-    tm.span(m1, m2, T_RAY64);
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, c->tcnt.p, (size_t)1, 0);
-    hipLaunchKernelGGL(k_collect_slots, dim3((n + 255) / 256), dim3(256), 0, st, (const unsigned*)c->rflags.p, n,
-                       (const int*)nullptr, 0, (const int*)nullptr, rid0, (int)first, c->tcnt.p, c->tslots.p,
-                       c->runacc.p);
     io.flags = nullptr;
-    hipLaunchKernelGGL(k_walk_fp64_multi, dim3(std::min(n, c->scan_blocks)), dim3(64), slds, st, (const NetDev*)b->nets_d.p,
-                       io, c->Wd, rid0, (const int*)c->tcnt.p, (const int*)c->tslots.p,
-                       (const double*)c->tplanes.p, (const double*)c->teq.p, Ch);
+    hipLaunchKernelGGL(k_walk_fp64_multi, list, dim3(64), slds, st, nd, io, c->Wd, rid0, (const int*)left.cnt,
+                       (const int*)left.slots, P, E, Ch);
     HIPCHK(hipGetLastError());
-    tm.span(m2, tm.mark(st), T_SCAN64);
   }
-}
-
-// Regions per network of level first .. first + count - 1 into b->hist_h (waits for the stream).
-void batch_hist(am_batch* b, long long first, long long count) {
-  am_ctx* c = b->c;
-  const hipStream_t st = c->stream;
-  const int nn = (int)b->nets.size();
-  hipLaunchKernelGGL(k_fill_i32, dim3(blocks(nn, 256)), dim3(256), 0, st, b->hist_d.p, (size_t)nn, 0);
-  if (count > 0)
-    hipLaunchKernelGGL(k_net_hist, dim3(blocks((size_t)count, 256)), dim3(256), 0, st, c->reg_mask.p, c->Wd,
-                       (int)first, (int)count, b->hist_d.p);
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(b->hist_h, b->hist_d.p, nn * sizeof(int), hipMemcpyDeviceToHost, st));
-  HIPCHK(hipStreamSynchronize(st));
 }
 
 }  // namespace
@@ -1315,6 +1275,14 @@ void batch_hist(am_batch* b, long long first, long long count) {
 // C-ABI
 // ---------------------------------------------------------------------------
 namespace {
+
+// A run's counters on the device: [0, 1 + W) the FP64 ray walk's undecided
+// regions and reasons, [1 + W, 2 + 2W) the reduced-precision walk's, then the
+// regions it decided with a vertex left to FP64; and the stage clock.
+struct RunAcc {
+  StageClock clock;
+  int acc[2 * (1 + AM_WHY_COUNT) + 1];
+};
 
 // A run's counters, stage clock and walk counters, cleared.
 __global__ void k_run_begin(int* p, int n, StageClock* clk, int* zero) {
@@ -1612,7 +1580,7 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
       const size_t clds = chain_lds_bytes(c);
       if (clds > c->max_lds) c->tile_ok = false;
       else if (clds > 65536) {
-        HIPCHK(hipFuncSetAttribute((const void*)k_chain_tile_fp64, hipFuncAttributeMaxDynamicSharedMemorySize,
+        HIPCHK(hipFuncSetAttribute((const void*)k_chain_tile_fp64<8>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)clds));
       }
     }
@@ -1658,14 +1626,6 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
                        dev_view(c, points, (size_t)n_seeds * 3 * esz, st), dtype == AM_DTYPE_F64 ? 1 : 0, n_seeds,
                        c->L, c->Wd, c->cand_mask.p, c->cand_hash.p, c->cand_point.p, c->cand_start.p);
     HIPCHK(hipGetLastError());
-    // run counters on the device: [0, 1 + W) the FP64 ray walk's undecided
-    // regions and reasons, [1 + W, 2 + 2W) the reduced-precision walk's, then
-    // the regions it decided with a vertex left to FP64; then the stage clock
-    constexpr int NACC = 2 * (1 + AM_WHY_COUNT) + 1;
-    struct RunAcc {
-      StageClock clock;
-      int acc[NACC];
-    };
     ensure(c->runacc, (sizeof(RunAcc) + 3) / 4, false, st);
     RunAcc* const ra_dev = reinterpret_cast<RunAcc*>(c->runacc.p);
     int* const acc_dev = ra_dev->acc;
@@ -2421,8 +2381,10 @@ am_status am_adjoint(am_ctx* c, const void* grad_vertices, int dtype, void* cons
       io.dcap = dcap;
       const uint32_t* mask0 = c->reg_mask.p + (size_t)r0 * c->Wd;
       if (tiled) {
-        hipLaunchKernelGGL(k_chain_tile_fp64, dim3((cnt + AM_CT - 1) / AM_CT), dim3(AM_CHAIN_THREADS),
-                           chain_lds_bytes(c), st, c->net, chain_io(c, nullptr, r0, cnt, Ch));
+        const int maxw = chain_maxw(c);
+        hipLaunchKernelGGL((maxw > 128 ? k_chain_tile_fp64<8> : k_chain_tile_fp64<4>), dim3((cnt + AM_CT - 1) / AM_CT),
+                           dim3(maxw > 128 ? 512 : 256), chain_lds_bytes(c), st, c->net,
+                           chain_io(c, nullptr, r0, cnt, Ch), maxw);
         hipLaunchKernelGGL(k_adjoint_direct, dim3(cnt), dim3(64), lds, st, c->net, io, (const double*)c->tplanes.p,
                            (const double*)c->teq.p, Ch);
         HIPCHK(hipGetLastError());
@@ -2591,7 +2553,7 @@ am_status am_batch_create(am_batch** out, int n_nets, const int* n_nodes, const 
   }
   am_batch* b = new am_batch();
   b->precision = precision;
-  int Lmax = 0, Dmax = 0, Wmax = 0;
+  int Lmax = 0, Wmax = 0;
   for (int i = 0; i < n_nets; ++i) {
     const int nn = n_nodes[i];
     const int* nd = nodes[i];
@@ -2614,7 +2576,7 @@ am_status am_batch_create(am_batch** out, int n_nets, const int* n_nodes, const 
         return AM_ERR_ARG;
       }
     Lmax = std::max(Lmax, bn.L);
-    Dmax = std::max(Dmax, bn.D);
+    for (size_t k = 1; k < bn.nodes.size(); ++k) b->maxw = std::max(b->maxw, bn.nodes[k]);
     Wmax = std::max(Wmax, bn.Wn);
     b->nets.push_back(std::move(bn));
   }
@@ -2637,7 +2599,6 @@ am_status am_batch_create(am_batch** out, int n_nets, const int* n_nodes, const 
   c->C = Lmax;
   b->c = c;
   b->Wmax = Wmax;
-  b->Dmax = Dmax;
   b->Lmax = Lmax;
   b->Cmax = Lmax;
   *out = b;
@@ -2726,20 +2687,15 @@ am_status am_batch_run(am_batch* b, const void* const* weights, const void* cons
     ensure(b->nets_d, (size_t)nn, false, st);
     HIPCHK(hipMemcpyAsync(b->nets_d.p, b->nets_h.data(), nn * sizeof(NetDev), hipMemcpyHostToDevice, st));
     ensure(b->cios_d, (size_t)nn, false, st);
-    ensure(b->hist_d, (size_t)nn, false, st);
-    if (!b->hist_h) {
-      HIPCHK(b->hist_mem.take(MEM_PINNED, (size_t)1 << 22));
-      b->hist_h = static_cast<int*>(b->hist_mem.p);
-    }
+    HIPCHK(hipMemcpyAsync(b->cios_d.p, b->cios_h.data(), nn * sizeof(ChainIO), hipMemcpyHostToDevice, st));
     if ((size_t)nn * sizeof(int) > ((size_t)1 << 22)) throw CapErr{"too many networks"};
+    ensure(b->seg_d, (size_t)nn, false, st);
     const size_t clds = batch_chain_lds(b), slds = batch_scan_lds(b), rlds = batch_ray_lds(b);
     if (clds > c->max_lds || slds > c->max_lds) throw CapErr{"networks too wide for the batch kernels' LDS"};
-    if (clds > 65536) {
-      HIPCHK(hipFuncSetAttribute((const void*)k_chain_tile_fp64_multi<false>,
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)clds));
-      HIPCHK(hipFuncSetAttribute((const void*)k_chain_tile_fp64_multi<true>,
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)clds));
-    }
+    if (batch_near_lds(b) > c->max_lds) throw CapErr{"networks too wide for the batch kernels' LDS"};
+    if (clds > 65536)
+      HIPCHK(hipFuncSetAttribute((const void*)k_chain_tile_fp64_multi<8>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 (int)clds));
     if (slds > 65536)
       HIPCHK(hipFuncSetAttribute((const void*)k_walk_fp64_multi, hipFuncAttributeMaxDynamicSharedMemorySize,
                                  (int)slds));
@@ -2752,7 +2708,6 @@ am_status am_batch_run(am_batch* b, const void* const* weights, const void* cons
     // seeds of every network -> the first level (network word appended)
     c->R = 0;
     c->table_cap = 0;
-    c->table.release();
     grow_cands(c, (size_t)total_seeds);
     {
       std::vector<uint32_t> m((size_t)total_seeds * c->Wd, 0u);
@@ -2783,33 +2738,25 @@ am_status am_batch_run(am_batch* b, const void* const* weights, const void* cons
       HIPCHK(hipMemcpy(c->cand_point.p, pts.data(), pts.size() * 8, hipMemcpyHostToDevice));
       HIPCHK(hipMemcpy(c->cand_start.p, startv.data(), startv.size() * 4, hipMemcpyHostToDevice));
     }
-    c->timer.reset();
-    constexpr int NACC = 2 * (1 + AM_WHY_COUNT);
-    ensure(c->runacc, NACC, false, st);
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, c->runacc.p, (size_t)NACC, 0);
+    ensure(c->runacc, (sizeof(RunAcc) + 3) / 4, false, st);
+    RunAcc* const ra_dev = reinterpret_cast<RunAcc*>(c->runacc.p);
+    c->acc = ra_dev->acc;
+    c->clock = &ra_dev->clock;
+    ensure(c->tcnt, 2, false, st);
+    hipLaunchKernelGGL(k_run_begin, dim3(1), dim3(256), 0, st, c->runacc.p, (int)(sizeof(RunAcc) / 4), c->clock,
+                       c->tcnt.p);
     hipLaunchKernelGGL(k_hash_keys, dim3(blocks((size_t)total_seeds, 256)), dim3(256), 0, st,
                        (const uint32_t*)c->cand_mask.p, (int)total_seeds, c->Wd, c->cand_hash.p);
     long long lvl_first = 0;
     long long lvl_count = insert_level(c, (size_t)total_seeds);
-    batch_hist(b, lvl_first, lvl_count);
     long long levels = 0, cands = 0, launches = 0, waits = 1;
-    const uint32_t* mask_at_upload = nullptr;
     Fp64Counts f64;
     while (lvl_count > 0) {
       const size_t ncand = (size_t)lvl_count * c->vm;
       grow_cands(c, ncand);
       ensure(c->rflags, (size_t)lvl_count, false, st);
-      // with graph-captured levels the store grows before the level's kernels
-      // are captured, so the chain must see the grown store's masks
       InsertPlan ip;
-      if (c->graph_levels) ip = insert_prepare(c, ncand);
-      if (c->reg_mask.p != mask_at_upload) {
-        // the chain reads region masks through each network's ChainIO
-        for (ChainIO& cio : b->cios_h) cio.reg_mask = c->reg_mask.p;
-        HIPCHK(hipMemcpyAsync(b->cios_d.p, b->cios_h.data(), nn * sizeof(ChainIO), hipMemcpyHostToDevice, st));
-        HIPCHK(hipStreamSynchronize(st));
-        mask_at_upload = c->reg_mask.p;
-      }
+      if (c->graph_levels) ip = insert_prepare(c, ncand);   // (its allocations stay out of the capture)
       const BatchLevelPlan pl = batch_level_prepare(b, lvl_first, lvl_count);
       launches += 1;
       const long long before = c->R;
@@ -2822,23 +2769,21 @@ am_status am_batch_run(am_batch* b, const void* const* weights, const void* cons
         added = insert_finish(c, ip);
       } else {
         batch_level_launch(b, pl, f64);
-        const size_t mi = c->timer.mark(st);
         added = insert_level(c, ncand);
-        c->timer.span(mi, c->timer.mark(st), T_INSERT);
       }
       cands += (long long)ncand;
       levels += 1;
       lvl_first = before;
       lvl_count = added;
-      batch_hist(b, lvl_first, lvl_count);
-      waits += 2;
+      waits += 1;
     }
-    int acc[NACC] = {0};
-    HIPCHK(hipMemcpyAsync(acc, c->runacc.p, sizeof(acc), hipMemcpyDeviceToHost, st));
+    RunAcc ra{};
+    HIPCHK(hipMemcpyAsync(&ra, ra_dev, sizeof(ra), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
-    c->timer.resolve();
+    const int* acc = ra.acc;
     const auto t1 = std::chrono::steady_clock::now();
-    const double* T = c->timer.acc;
+    double T[T_SLOTS];
+    for (int i = 0; i < T_SLOTS; ++i) T[i] = (double)ra.clock.acc[i] * kStageTickMs;
     c->stats[AM_STAT_RUN_MS] = std::chrono::duration<double, std::milli>(t1 - t0).count();
     c->stats[AM_STAT_INSERT_MS] = T[T_INSERT];
     c->stats[AM_STAT_REGION_MS] = T[T_CHAIN64] + T[T_RAY64] + T[T_SCAN64];

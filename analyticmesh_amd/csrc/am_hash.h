@@ -92,7 +92,9 @@ __global__ void k_seeds(const uint8_t* states, const void* points, int f64, int 
 __global__ void k_rehash(const uint32_t* reg_mask, int R, int Wd, uint32_t* table, uint32_t cap_mask);
 __global__ void k_fingerprint(const uint32_t* reg_mask, const int* info, const int* vpair, int R, int Wd, int Wh,
                               int vm, int L, int net, unsigned long long* out);
-__global__ void k_net_hist(const uint32_t* reg_mask, int Wd, int first, int count, int* hist);
+__global__ void k_net_seg(const uint32_t* reg_mask, int Wd, int first, int n, int nn, int* seg);
+__global__ void k_net_tiles(const uint32_t* reg_mask, int Wd, int first, int n, int nn, int find, int* seg, int ct,
+                            int4* tiles, int ntile);
 __global__ void k_net_flags(const uint32_t* reg_mask, int Wd, int R, int net, int* flags);
 __global__ void k_net_scatter(const int* flags, const int* rank, int R, int* ids);
 

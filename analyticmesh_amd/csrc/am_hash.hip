@@ -431,11 +431,70 @@ __global__ __launch_bounds__(256) void k_fingerprint(const uint32_t* reg_mask, c
   if (threadIdx.x < 6) atomicAdd(&out[threadIdx.x], red[threadIdx.x][0]);
 }
 
-// Regions per network of level regions first .. first + count - 1 (network =
-// last mask word).
-__global__ void k_net_hist(const uint32_t* reg_mask, int Wd, int first, int count, int* hist) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < count) atomicAdd(&hist[reg_mask[(size_t)(first + i) * Wd + Wd - 1]], 1);
+// How many of regions first .. first + n - 1 belong to networks before `net`
+// (network = last mask word, ascending): one wave, 64 probes a step.
+__device__ __forceinline__ int net_start(const uint32_t* reg_mask, int Wd, int first, int n, int net) {
+  const int lane = threadIdx.x & 63;
+  int lo = 0, hi = n;
+  while (lo < hi) {
+    const int step = (hi - lo + 63) >> 6, i = lo + lane * step;
+    const bool before = i < hi && (int)reg_mask[(size_t)(first + i) * Wd + Wd - 1] < net;
+    const int k = __popcll(__ballot(before));   // (a prefix of the lanes)
+    if (k == 0) break;
+    hi = min(hi, lo + k * step);
+    lo += (k - 1) * step + 1;
+  }
+  return lo;
+}
+__global__ void k_net_seg(const uint32_t* reg_mask, int Wd, int first, int n, int nn, int* seg) {
+  const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (i >= nn) return;
+  const int s = net_start(reg_mask, Wd, first, n, i);
+  if ((threadIdx.x & 63) == 0) seg[i] = s;
+}
+// The tile list of regions first .. first + n - 1: ct regions of one network per
+// entry (network, first region, regions, -), `ntile` entries, the last ones empty.
+// seg: the networks' first regions, found here (find) or by k_net_seg.  One block.
+__global__ __launch_bounds__(1024) void k_net_tiles(const uint32_t* reg_mask, int Wd, int first, int n, int nn, int find,
+                                                    int* seg, int ct, int4* tiles, int ntile) {
+  __shared__ int s_off[1025], s_seg[1025], s_part[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (find)
+    for (int i = wave; i < nn; i += 16) {
+      const int s = net_start(reg_mask, Wd, first, n, i);
+      if (lane == 0) seg[i] = s;
+    }
+  __syncthreads();
+  int base = 0;
+  for (int b0 = 0; b0 < nn; b0 += 1024) {
+    const int i = b0 + tid;
+    const int s = i < nn ? seg[i] : n, e = i + 1 < nn ? seg[i + 1] : n;
+    s_seg[tid] = s;
+    if (tid == 1023) s_seg[1024] = e;
+    const int t = (e - s + ct - 1) / ct;
+    int x = t;
+    for (int d = 1; d < 64; d <<= 1) {
+      const int y = __shfl_up(x, d);
+      if (lane >= d) x += y;
+    }
+    if (lane == 63) s_part[wave] = x;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) x += s_part[w];
+    s_off[tid + 1] = x;
+    if (tid == 0) s_off[0] = 0;
+    __syncthreads();
+    const int total = s_off[1024];
+    for (int j = tid; j < total; j += 1024) {
+      int k = 0;   // the last network whose tiles start at or before j
+      for (int d = 512; d > 0; d >>= 1)
+        if (s_off[k + d] <= j) k += d;
+      const int r = s_seg[k] + (j - s_off[k]) * ct;
+      if (base + j < ntile) tiles[base + j] = make_int4(b0 + k, r, min(ct, s_seg[k + 1] - r), 0);
+    }
+    base += total;
+    __syncthreads();
+  }
+  for (int j = base + tid; j < ntile; j += 1024) tiles[j] = make_int4(0, 0, 0, 0);
 }
 
 // Ids of the regions of network `net` (last mask word), in region order:

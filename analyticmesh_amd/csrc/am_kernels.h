@@ -78,16 +78,15 @@ struct InsertIO {
 };
 
 // Tiled FP64 chain: the planes of a tile of regions in HBM, for the walk kernel.
-#define AM_CT 16                // regions per chain workgroup
-#define AM_CN (4 * AM_CT)       // chain columns (one per lane): x, y, z, c of each region
+#define AM_CT 8                 // regions per chain workgroup
+#define AM_CN (4 * AM_CT)       // chain columns: x, y, z, c of each region
 #define AM_CXS (AM_CN + 1)      // LDS row stride (doubles) of the chain's layer buffer
-#define AM_CR 16                // output rows per wave
+#define AM_CR 16                // rows the operands are padded to
 #define AM_CHAIN_MAXW 256       // widest layer the tiled chain takes
 #define AM_RAY_WAVES 4          // waves per region in the ray-shooting walks
-#define AM_CPF 16               // k steps of chain operands in flight (k lists are padded to a multiple)
-#define AM_KLS (AM_CHAIN_MAXW + 2 * AM_CPF)   // entries of one layer's active-input list
-#define AM_CXR (AM_CHAIN_MAXW + AM_CPF)       // rows of the chain's layer buffer (list positions + prefetch)
-#define AM_CHAIN_THREADS (64 * AM_CHAIN_MAXW / AM_CR)
+inline size_t chain_tile_lds(int maxw, int Wd) {
+  return (size_t)(maxw + 1) * AM_CXS * 8 + (size_t)(maxw + 32) * 4 + (size_t)AM_CT * Wd * 4;
+}
 struct ChainIO {
   const uint32_t* reg_mask;   // [R][Wd]
   const int* ids;             // optional region ids; else first + tile-local index
@@ -126,28 +125,30 @@ struct ChainLevel {
   const int* ids;
   double* planes;             // [count][4][Cs]
   double* eq;                 // [count][4]
+  const uint32_t* reg_mask;   // [R][Wd]
+  StageClock* clk;
 };
 
-__global__ void k_chain_tile_fp64(NetDev net, ChainIO io);
+// NW waves: 4 for layers up to 128 wide (maxw), 8 up to 256.
+template <int NW>
+__global__ void k_chain_tile_fp64(NetDev net, ChainIO io, int maxw);
 // A batch of networks (each region's network is the last word of its mask):
 // tiles[b] = (network, first slot, regions, -) of one network.
-// MF: the products on the matrix cores (k_chain_tile_mfma).
-template <bool MF>
-__global__ void k_chain_tile_fp64_multi(const NetDev* nets, const ChainIO* cios, ChainLevel lv, const int4* tiles);
+template <int NW>
+__global__ void k_chain_tile_fp64_multi(const NetDev* nets, const ChainIO* cios, ChainLevel lv, const int4* tiles,
+                                        int maxw);
 struct WalkParams;
 // Batch-of-networks forms (region rid0 + b; its network is mask word Wd - 1;
 // the scan's LDS layout follows each network's C, the launch is sized for the
 // widest network).
 __global__ void k_walk_fp64_multi(const NetDev* nets, RegionIO io, int Wd, int rid0, const int* count,
                                   const int* slots, const double* planes, const double* eq, int Cs_hbm);
+template <bool SCAN, bool ALL>
+__global__ void k_near64_multi(const NetDev* nets, RegionIO io, int Wd, int rid0, WalkParams wp, const double* planes,
+                               const double* eq, int Cs_hbm, NearList left);
 template <int NW>
 __global__ void k_walk_ray64_multi(const NetDev* nets, RegionIO io, int Wd, int rid0, WalkParams wp,
-                                   const double* planes, const double* eq, int Cs_hbm);
-// Chunk-local slots of the regions k_walk_ray64 left undecided (cnt[0] counts
-// them); run[0] accumulates the count and run[1 + w] the reasons, per run.
-// With dn, entries past *dn - dbase are not valid.
-__global__ void k_collect_slots(const unsigned* flags, int n, const int* dn, int dbase, const int* ids, int rid0,
-                                int lvl_first, int* cnt, int* slots, int* run);
+                                   const double* planes, const double* eq, int Cs_hbm, NearList list, SlotList left);
 __global__ void k_fill_i32(int* p, size_t n, int v);
 
 // Weight layouts on the device (am_layout.hip): dst[j * ni + i] = src[i * cols + j]
