@@ -245,7 +245,9 @@ __device__ __forceinline__ void walk_fp64_body(const NetDev& net, const RegionIO
                         eqb[(size_t)sl * 4 + 3]};
   __syncthreads();
   const WalkParams wp{0.f, 0.f, 0.f};
-  walk_region<double, false>(net, io, wp, rid, rid - io.first, Px, Py, Pz, Pc, keys, order, used, smask, eq, p);
+  const WalkRecs rec = carve_walk_recs(smem_raw + scan_lds_head(C, N2, net.Wd), net.vm, false);
+  walk_region<double, false>(net, io, wp, rid, rid - io.first, Px, Py, Pz, Pc, keys, order, used, smask, eq, p, rec.tab,
+                             rec.verts, rec.vpair);
   __syncthreads();   // this region's LDS is free for the next
 }
 
@@ -279,43 +281,6 @@ struct TilePlanes {
   __device__ __forceinline__ void get(int g, double* p) const { plane64(net, mask, src, Cs, g, p); }
   __device__ __forceinline__ void load(int l, int j, double* p) const { get(first(l) + j, p); }
 };
-
-// The near walk of a batch's regions (am_near.h), one wave per region; the ones
-// it leaves go on the list of the walks below.  ALL: every network of the batch
-// has up to AM_ALL_MAX constraints.  Eight networks of 48 to 256 constraints
-// (85 levels of up to 5,800 regions): 47 us a level with two-wave ray walks over all
-// constraints, 36 so.
-template <bool SCAN, bool ALL>
-__global__ __launch_bounds__(64, 4) void k_near64_multi(const NetDev* nets, RegionIO io, int Wd, int rid0, WalkParams wp,
-                                                     const double* planes, const double* eqb, int Cs_hbm,
-                                                     NearList left) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  stage_mark(io.clk, SCAN ? T_SCAN64 : T_RAY64);
-  const int b = blockIdx.x;
-  if (b >= io.count) return;
-  const int rid = rid0 + b;
-  const NetDev& net = nets[region_net(io, Wd, rid)];
-  const NearLds<double> S = carve_near<double>(smem_raw, net.C, Wd, net.vm, false, ALL);
-  const int start = io.reg_start[rid];
-  for (int w = threadIdx.x; w < Wd; w += 64) S.mask[w] = io.reg_mask[(size_t)rid * Wd + w];
-  double p[3], eq[4];
-  for (int q = 0; q < 3; ++q) p[q] = io.reg_point[(size_t)rid * 3 + q];
-  for (int q = 0; q < 4; ++q) eq[q] = eqb[(size_t)b * 4 + q];
-  __syncthreads();
-  const TilePlanes P{net, planes + (size_t)b * 4 * Cs_hbm, Cs_hbm, S.mask};
-  bool done = false;
-  if (start >= 0 && start < net.C) {
-    if (ALL) done = near_walk<double, SCAN, SET_LDS>(net, io, wp, rid, rid - io.first, P, S, eq, p, start) == NEAR_DONE;
-    else if (SCAN) done = near_or_full_walk<double, true>(net, io, wp, rid, rid - io.first, P, S, eq, p, start) == NEAR_DONE;
-    else done = near_walk<double, false, SET_NEAR>(net, io, wp, rid, rid - io.first, P, S, eq, p, start) == NEAR_DONE;
-  }
-  // (thread 0 wrote the flag in finish_region: the orientation may be undecided)
-  if (threadIdx.x == 0 && (!done || (!SCAN && (io.flags[rid - io.first] & AM_UNDECIDED)))) near_left(left, b);
-}
-template __global__ void k_near64_multi<true, false>(const NetDev*, RegionIO, int, int, WalkParams, const double*, const double*, int, NearList);
-template __global__ void k_near64_multi<false, false>(const NetDev*, RegionIO, int, int, WalkParams, const double*, const double*, int, NearList);
-template __global__ void k_near64_multi<true, true>(const NetDev*, RegionIO, int, int, WalkParams, const double*, const double*, int, NearList);
-template __global__ void k_near64_multi<false, true>(const NetDev*, RegionIO, int, int, WalkParams, const double*, const double*, int, NearList);
 
 // The candidate scan of the listed slots (blocks stride over the list).
 __global__ __launch_bounds__(64) void k_walk_fp64_multi(const NetDev* nets, RegionIO io, int Wd, int rid0,
@@ -366,6 +331,61 @@ __device__ __forceinline__ void walk_ray64_body(const NetDev& net, const RegionI
   const PlaneView<double> P{reinterpret_cast<const double*>(Q), Cl, n1, net.W0, net.b[0], smask};
   walk_ray<double, NW>(net, io, wp, rid, rid - io.first, P, smask, eq, p, rec, start_in);
 }
+
+// The near walk of a batch's regions (am_near.h), one wave per region; ALL
+// (every network of the batch has up to AM_ALL_MAX constraints): on all of them, and
+// the few regions it leaves, and seeds, take the walks over all constraints in the
+// same wave (two launches for them took 9.6 us a level).  Else they go on a list.  Eight networks of 48 to 256 constraints
+// (85 levels of up to 5,800 regions): 47 us a level with two-wave ray walks over all
+// constraints, 36 so.
+template <bool SCAN, bool ALL>
+__global__ __launch_bounds__(64, 4) void k_near64_multi(const NetDev* nets, RegionIO io, int Wd, int rid0, WalkParams wp,
+                                                     const double* planes, const double* eqb, int Cs_hbm,
+                                                     NearList left, int* run) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  stage_mark(io.clk, SCAN ? T_SCAN64 : T_RAY64);
+  const int b = blockIdx.x;
+  if (b >= io.count) return;
+  const int rid = rid0 + b;
+  const NetDev& net = nets[region_net(io, Wd, rid)];
+  const NearLds<double> S = carve_near<double>(smem_raw, net.C, Wd, net.vm, false, ALL);
+  const int start = io.reg_start[rid];
+  for (int w = threadIdx.x; w < Wd; w += 64) S.mask[w] = io.reg_mask[(size_t)rid * Wd + w];
+  double p[3], eq[4];
+  for (int q = 0; q < 3; ++q) p[q] = io.reg_point[(size_t)rid * 3 + q];
+  for (int q = 0; q < 4; ++q) eq[q] = eqb[(size_t)b * 4 + q];
+  __syncthreads();
+  const TilePlanes P{net, planes + (size_t)b * 4 * Cs_hbm, Cs_hbm, S.mask};
+  bool done = false;
+  if (start >= 0 && start < net.C) {
+    if (ALL) done = near_walk<double, SCAN, SET_LDS>(net, io, wp, rid, rid - io.first, P, S, eq, p, start) == NEAR_DONE;
+    else if (SCAN) done = near_or_full_walk<double, true>(net, io, wp, rid, rid - io.first, P, S, eq, p, start) == NEAR_DONE;
+    else done = near_walk<double, false, SET_NEAR>(net, io, wp, rid, rid - io.first, P, S, eq, p, start) == NEAR_DONE;
+  }
+  if (ALL) {
+    if (done && (SCAN || !(__builtin_amdgcn_readfirstlane(io.flags[rid - io.first]) & AM_UNDECIDED))) return;
+    __syncthreads();
+    if (!SCAN) {
+      walk_ray64_body<1>(net, io, rid, b, wp, planes, eqb, Cs_hbm);
+      const unsigned f = __builtin_amdgcn_readfirstlane(io.flags[rid - io.first]);
+      if (!(f & AM_UNDECIDED)) return;
+      if (threadIdx.x == 0) {
+        atomicAdd(run, 1);
+        for (int w = 0; w < AM_WHY_COUNT; ++w)
+          if (f & AM_WHY_BIT(w)) atomicAdd(run + 1 + w, 1);
+      }
+      __syncthreads();
+    }
+    walk_fp64_body(net, scan_layout(io, net.C), rid, b, planes, eqb, Cs_hbm);
+    return;
+  }
+  // (thread 0 wrote the flag in finish_region: the orientation may be undecided)
+  if (threadIdx.x == 0 && (!done || (!SCAN && (io.flags[rid - io.first] & AM_UNDECIDED)))) near_left(left, b);
+}
+template __global__ void k_near64_multi<true, false>(const NetDev*, RegionIO, int, int, WalkParams, const double*, const double*, int, NearList, int*);
+template __global__ void k_near64_multi<false, false>(const NetDev*, RegionIO, int, int, WalkParams, const double*, const double*, int, NearList, int*);
+template __global__ void k_near64_multi<true, true>(const NetDev*, RegionIO, int, int, WalkParams, const double*, const double*, int, NearList, int*);
+template __global__ void k_near64_multi<false, true>(const NetDev*, RegionIO, int, int, WalkParams, const double*, const double*, int, NearList, int*);
 
 // ... of the listed slots (blocks stride over the list); a region it leaves
 // undecided goes on the candidate scan's list and counts itself and its reasons.

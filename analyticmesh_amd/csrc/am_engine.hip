@@ -838,7 +838,8 @@ void run_fp64_regions(am_ctx* c, int lvl_first, int first, int count, const int*
   // nets with skips or layers over 256 wide keep the candidate scan's records in every form
   if (mode == 1 && (ray64_lds_bytes(c) > c->max_lds || !c->tile_ok)) mode = 0;
   int Cs, Csort;
-  const size_t wlds = region_lds_bytes(c, Cs, Csort);
+  (void)region_lds_bytes(c, Cs, Csort);
+  const size_t wlds = scan_lds_bytes(Cs, Csort, c->Wd, c->vm);
   const size_t rlds = ray64_lds_bytes(c);
   const size_t chunk = prefix_chunk(c);
   // regions the reduced walk may have decided with a vertex left to FP64 (the
@@ -889,11 +890,14 @@ void run_fp64_regions(am_ctx* c, int lvl_first, int first, int count, const int*
       HIPCHK(hipGetLastError());
     }
     if (mode == 0) {
-      hipLaunchKernelGGL((all ? k_near64<true, true> : k_near64<true, false>), dim3(n), dim3(64), nlds, c->stream, c->net, c->pfx.dev, io, rid0, kr,
-                         c->teq.p, after_walk ? 1 : 0, near);
+      // (up to AM_ALL_MAX constraints nothing is left over)
+      hipLaunchKernelGGL((all ? k_near64<true, true> : k_near64<true, false>), dim3(n), dim3(64), all ? qlds : nlds,
+                         c->stream, c->net, c->pfx.dev, io, rid0, kr, c->teq.p, after_walk ? 1 : 0, near);
       io.flags = nullptr;
-      hipLaunchKernelGGL(k_walk_fp64, dim3(std::min(n, c->scan_blocks)), dim3(64), qlds, c->stream, c->net,
-                         c->pfx.dev, io, rid0, (const int*)near.cnt, (const int*)near.slots, (const double*)c->teq.p, all ? 0 : 1);
+      if (!all)
+        hipLaunchKernelGGL(k_walk_fp64, dim3(std::min(n, c->scan_blocks)), dim3(64), qlds, c->stream, c->net,
+                           c->pfx.dev, io, rid0, (const int*)near.cnt, (const int*)near.slots,
+                           (const double*)c->teq.p, 1);
       HIPCHK(hipGetLastError());
       t.scanned_host += n;
       continue;
@@ -1136,7 +1140,7 @@ size_t batch_scan_lds(const am_batch* b) {
   for (const BatchNet& n : b->nets) {
     int Csort = AM_TOPK;
     while (Csort < n.L) Csort <<= 1;
-    m = std::max(m, (size_t)4 * n.L * 8 + (size_t)Csort * 12 + (size_t)((n.L + 31) / 32) * 4 + (size_t)b->c->Wd * 4 + 64);
+    m = std::max(m, scan_lds_bytes(n.L, Csort, b->c->Wd, b->c->vm));
   }
   return m;
 }
@@ -1148,7 +1152,9 @@ size_t batch_ray_lds(const am_batch* b) {
   return m;
 }
 size_t batch_near_lds(const am_batch* b) {
-  return near_lds_bytes(b->Cmax, b->c->Wd, b->c->vm, 8, false, b->Cmax <= AM_ALL_MAX);
+  const bool all = b->Cmax <= AM_ALL_MAX;
+  const size_t m = near_lds_bytes(b->Cmax, b->c->Wd, b->c->vm, 8, false, all);
+  return all ? std::max({m, batch_scan_lds(b), batch_ray_lds(b)}) : m;
 }
 size_t batch_chain_lds(const am_batch* b) { return chain_tile_lds(b->maxw, b->c->Wd); }
 
@@ -1237,17 +1243,19 @@ void batch_level_launch(am_batch* b, const BatchLevelPlan& pl, Fp64Counts& t) {
     io.ids = nullptr;
     io.clk = c->clock;
     const dim3 list(std::min(n, c->scan_blocks));
+    // (up to AM_ALL_MAX constraints the near walk leaves nothing)
+    hipLaunchKernelGGL((all ? (ray ? k_near64_multi<false, true> : k_near64_multi<true, true>)
+                            : (ray ? k_near64_multi<false, false> : k_near64_multi<true, false>)),
+                       dim3(n), dim3(64), nlds, st, nd, io, c->Wd, rid0, kr, P, E, Ch, near, c->acc);
+    HIPCHK(hipGetLastError());
+    if (!ray) t.scanned_host += n;
+    if (all) continue;
     if (!ray) {
-      hipLaunchKernelGGL((all ? k_near64_multi<true, true> : k_near64_multi<true, false>), dim3(n), dim3(64), nlds, st, nd,
-                         io, c->Wd, rid0, kr, P, E, Ch, near);
       hipLaunchKernelGGL(k_walk_fp64_multi, list, dim3(64), slds, st, nd, io, c->Wd, rid0, (const int*)near.cnt,
                          (const int*)near.slots, P, E, Ch);
       HIPCHK(hipGetLastError());
-      t.scanned_host += n;
       continue;
     }
-    hipLaunchKernelGGL((all ? k_near64_multi<false, true> : k_near64_multi<false, false>), dim3(n), dim3(64), nlds, st, nd,
-                       io, c->Wd, rid0, kr, P, E, Ch, near);
     switch (c->ray_waves) {
       case 2:
         hipLaunchKernelGGL(k_walk_ray64_multi<2>, list, dim3(128), rlds, st, nd, io, c->Wd, rid0, kr, P, E, Ch, near,
@@ -1568,9 +1576,9 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
     const size_t lds = region_lds_bytes(c, Cs, Csort);
     if (lds > c->max_lds)
       throw CapErr{"network too wide for the FP64 region kernel's LDS (" + std::to_string(lds) + " bytes)"};
-    if (lds > 65536) {
-      HIPCHK(hipFuncSetAttribute((const void*)k_walk_fp64, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    }
+    const size_t slds = scan_lds_bytes(Cs, Csort, c->Wd, c->vm);
+    if (slds > 65536)
+      HIPCHK(hipFuncSetAttribute((const void*)k_walk_fp64, hipFuncAttributeMaxDynamicSharedMemorySize, (int)slds));
     c->tile_ok = true;
     for (int li = 0; li <= c->D; ++li)
       if (!c->skips[li].empty()) c->tile_ok = false;

@@ -462,9 +462,12 @@ __global__ __launch_bounds__(64) void k_walk_f32(NetDev net, RegionIO io, WalkPa
   const float eq[4] = {eb[0], eb[1], eb[2], eb[3]};
   const float p[3] = {(float)io.reg_point[(size_t)rid * 3 + 0], (float)io.reg_point[(size_t)rid * 3 + 1],
                       (float)io.reg_point[(size_t)rid * 3 + 2]};
+  __shared__ int s_tab[AM_VM_MAX + 2];
+  __shared__ float s_verts[AM_VM_MAX * 3];
+  __shared__ int s_vpair[AM_VM_MAX * 2];
   __syncthreads();
-  walk_region<float, true>(net, io, wp, rid, rid - io.first, Px, Py, Pz, Pc, keys, order, used, smask, eq, p,
-                           with_sigma ? Pe : nullptr, with_sigma ? eb[4] : 0.f);
+  walk_region<float, true>(net, io, wp, rid, rid - io.first, Px, Py, Pz, Pc, keys, order, used, smask, eq, p, s_tab,
+                           s_verts, s_vpair, with_sigma ? Pe : nullptr, with_sigma ? eb[4] : 0.f);
 }
 
 // Ray-shooting FP32 walk: LDS holds only the planes and the mask; NW waves

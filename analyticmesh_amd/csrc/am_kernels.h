@@ -145,7 +145,7 @@ __global__ void k_walk_fp64_multi(const NetDev* nets, RegionIO io, int Wd, int r
                                   const int* slots, const double* planes, const double* eq, int Cs_hbm);
 template <bool SCAN, bool ALL>
 __global__ void k_near64_multi(const NetDev* nets, RegionIO io, int Wd, int rid0, WalkParams wp, const double* planes,
-                               const double* eq, int Cs_hbm, NearList left);
+                               const double* eq, int Cs_hbm, NearList left, int* run);
 template <int NW>
 __global__ void k_walk_ray64_multi(const NetDev* nets, RegionIO io, int Wd, int rid0, WalkParams wp,
                                    const double* planes, const double* eq, int Cs_hbm, NearList list, SlotList left);

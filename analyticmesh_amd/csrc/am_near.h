@@ -39,15 +39,14 @@ struct NearLds {
                     // bound), as the upper half of its FP32 bits, i.e. rounded down
   uint16_t* cand;   // [64] near constraints
   uint32_t* mask;   // [Wd]
-  float* okey;      // [C] order keys (SET_LDS)
   uint32_t* used;   // [C bits] (over key where that is not used)
   WalkRecs rec;
 };
 #define AM_ALL_MAX 256        // constraints up to which SET_LDS is taken
 __host__ __device__ inline size_t near_lds_bytes(int C, int Wd, int vm, int tsize, bool jinv, bool all = false) {
   auto a16 = [](size_t x) { return (x + 15) & ~(size_t)15; };
-  // (all: planes behind the face plane's inputs, order keys)
-  return (size_t)AM_NEAR_PL * tsize + (all ? (size_t)C * 4 * tsize + a16((size_t)C * 4) : 0) + a16((size_t)C * 2) +
+  // (all: planes behind the face plane's inputs)
+  return (size_t)AM_NEAR_PL * tsize + (all ? (size_t)C * 4 * tsize : 0) + a16((size_t)C * 2) +
          AM_NEAR_MAX * 2 + a16((size_t)Wd * 4) + walk_rec_bytes(vm, jinv);
 }
 template <typename T>
@@ -56,13 +55,10 @@ __device__ inline NearLds<T> carve_near(unsigned char* p, int C, int Wd, int vm,
   NearLds<T> s;
   s.stage = reinterpret_cast<T*>(p);
   s.pl = s.stage;
-  s.okey = nullptr;
   p += (size_t)AM_NEAR_PL * sizeof(T);
   if (all) {
     s.pl = reinterpret_cast<T*>(p);
     p += (size_t)C * 4 * sizeof(T);
-    s.okey = reinterpret_cast<float*>(p);
-    p += a16((size_t)C * 4);
   }
   s.key = reinterpret_cast<uint16_t*>(p);
   s.used = reinterpret_cast<uint32_t*>(p);
@@ -241,11 +237,10 @@ __device__ __forceinline__ T near_order_key(const T* x, const T* p) {
   if (k != k) k = -__builtin_inf();
   return k;
 }
-// Constraint g's plane (and its order key, rounded) into LDS for SET_LDS.
-template <typename T, bool SCAN>
-__device__ __forceinline__ void near_stage(const NearLds<T>& S, int g, const T* x, const T* p) {
+// Constraint g's plane into LDS for SET_LDS.
+template <typename T>
+__device__ __forceinline__ void near_stage(const NearLds<T>& S, int g, const T* x) {
   for (int q = 0; q < 4; ++q) S.pl[g * 4 + q] = x[q];
-  if (SCAN) S.okey[g] = (float)near_order_key<T>(x, p);
 }
 
 // SCAN: the candidate scan's decisions (walk_region<double, false>), bit for
@@ -316,7 +311,7 @@ __device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, 
         for (int j = lane; j < P.size(l); j += 64) {
           T x[4];
           P.load(l, j, x);
-          near_stage<T, SCAN>(S, P.first(l) + j, x, p);
+          near_stage<T>(S, P.first(l) + j, x);
         }
       }
   }
@@ -359,10 +354,12 @@ __device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, 
 
   // the start plane's edge: nearest planes both ways along its line
   int cl = sl, ql, rl;   // the plane walked along, the plane come from, the next plane
+  T pc[4], pq[4];        // planes of cl and ql
+  T d[3];                // along cl, towards rl
+  plane(sl, pc);
   {
-    T ps[4];
-    plane(sl, ps);
-    const T d[3] = {ps[1] * eq[2] - ps[2] * eq[1], ps[2] * eq[0] - ps[0] * eq[2], ps[0] * eq[1] - ps[1] * eq[0]};
+    const T(&ps)[4] = pc;
+    for (int q = 0; q < 3; ++q) d[q] = ps[(q + 1) % 3] * eq[(q + 2) % 3] - ps[(q + 2) % 3] * eq[(q + 1) % 3];
     const T pd[4] = {d[0], d[1], d[2], -(d[0] * p[0] + d[1] * p[1] + d[2] * p[2])};
     T x0[3];
     solve3(ps, eq, pd, x0);
@@ -392,9 +389,11 @@ __device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, 
         const int t = rl;
         rl = ql;
         ql = t;
+        for (int q = 0; q < 3; ++q) d[q] = -d[q];
       }
     }
   }
+  plane(ql, pq);
   int ntab = 1, nv = 0;
   use(sl);
   int tab1 = sl, tab2 = -1;           // the last two tab entries
@@ -405,32 +404,39 @@ __device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, 
     // next edge plane rl: its vertex with the plane walked along and f = iso
     if (FULL) __syncthreads();        // S.used
     const bool in_tab = is_used(rl) && !(rl == sl && ntab >= 3);
-    T pr[4], pc[4], v[3];
+    T pr[4], v[3];
     plane(rl, pr);
-    plane(cl, pc);
     double vd[3];
     VertexBound<T> vb{};
     // along the next edge plane, away from the one walked along
     T dn[3] = {pr[1] * eq[2] - pr[2] * eq[1], pr[2] * eq[0] - pr[0] * eq[2], pr[0] * eq[1] - pr[1] * eq[0]};
     if (pc[0] * dn[0] + pc[1] * dn[1] + pc[2] * dn[2] > T(0)) { dn[0] = -dn[0]; dn[1] = -dn[1]; dn[2] = -dn[2]; }
     Nearest<T> next;
-    T n1[4], n2[4];                   // the last two planes of the polygon, for the turn
-    if (ntab >= 2) {
-      plane(tab2, n1);
-      plane(tab1, n2);
-    }
+    const T(&n1)[4] = pq;             // with two planes or more, the last two of the polygon (for the turn)
+    const T(&n2)[4] = pc;
     if (SCAN) {
       solve3(pr, pc, eq, v);
       for (int q = 0; q < 3; ++q) vd[q] = (double)v[q];
       if (in_tab || !near_covers<T>(v, p, r, T(0), T(0)) || (nv > 0 && same_vertex(lastv, vd)) ||
           (ntab >= 2 && !pivot_valid(eq, n1, n2, pr)))
         return NEAR_RETRY;
-      T pq[4], kw;
-      plane(ql, pq);
-      if (FULL) kw = order_key(pr);
-      else kw = lane_value(key, rl);
+      // An unused constraint before rl in the scan's order must have been passed
+      // over: its vertex on this edge's line is outside rl or ql.  Along the line
+      // from v, x crosses at t = -x(v) / (x . d); a crossing that lies outside rl
+      // or ql by far more than v, the scan's vertex and their evaluation can be off
+      // settles it without the order or the vertex: with the condition numbers Kx =
+      // |x| |pc| |eq| / |x . d| and Kv = |pr| |pc| |eq| / |pr . d| that is below 200 u Kx Kv (1 +
+      // |v| + |t d|) per unit normal (1e-11 here is 90,000 u), and 1e-5 covers the
+      // FP32 arithmetic.  The others, few, take the scan's own expressions.
+      const T apr = pr[0] * d[0] + pr[1] * d[1] + pr[2] * d[2], apq = pq[0] * d[0] + pq[1] * d[1] + pq[2] * d[2];
+      const float npr = __builtin_sqrtf((float)plane_nn(pr[0], pr[1], pr[2]));
+      const float npq = __builtin_sqrtf((float)plane_nn(pq[0], pq[1], pq[2]));
+      const float nce = __builtin_sqrtf((float)plane_nn(pc[0], pc[1], pc[2]) * (float)plane_nn(eq[0], eq[1], eq[2]));
+      const float fr = (float)apr, fq = (float)apq, vq = (float)plane_eval(pq[0], pq[1], pq[2], pq[3], v);
+      const float dl = __builtin_sqrtf((float)plane_nn(d[0], d[1], d[2]));
+      const float v1 = 1.f + (float)(absT(v[0]) + absT(v[1]) + absT(v[2]));
+      const float kv = 1e-11f * nce * nce * npr * __builtin_amdgcn_rcpf(fabsf(fr));
       const int gw = index_of(rl);
-      const float kwf = (float)kw;
       bool fail = false;
       each([&](const T* x, int h, int gi, T) {
         if (h == cl || h == rl) return;
@@ -439,9 +445,13 @@ __device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, 
         fail = fail || (sv > T(0) && sv * sv > (Tol<T>::EPS * Tol<T>::EPS) * nn);
         const T al = fmaT(x[0], dn[0], fmaT(x[1], dn[1], x[2] * dn[2]));
         next.add(-sv, al, al > T(0), h);
-        // an unused constraint before the winner in the order
-        const bool maybe = SET != SET_LDS || S.okey[h] >= kwf;   // (rounding keeps the order)
-        if (maybe && key_before(FULL ? order_key(x) : key, gi, kw, gw) && (!is_used(h) || (h == sl && ntab >= 3))) {
+        const T ax = fmaT(x[0], d[0], fmaT(x[1], d[1], x[2] * d[2]));
+        const float ra = __builtin_amdgcn_rcpf((float)ax), t = -(float)sv * ra;
+        const float far = 1e-17f + kv * __builtin_sqrtf((float)nn) * fabsf(ra) * (v1 + fabsf(t) * dl);
+        const float tr = fr * t, tq = fq * t;
+        const bool passed = tr > npr * far || vq + tq > npq * far + 1e-5f * (fabsf(vq) + fabsf(tq));
+        if (!passed && (!is_used(h) || (h == sl && ntab >= 3)) &&
+            key_before(FULL ? order_key(x) : key, gi, order_key(pr), gw)) {
           T vt[3];
           solve3(x, pc, eq, vt);
           fail = fail || !(violates(pr[0], pr[1], pr[2], pr[3], vt) ||
@@ -531,6 +541,11 @@ __device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, 
     ql = cl;
     cl = rl;
     rl = nx;
+    for (int q = 0; q < 4; ++q) {
+      pq[q] = pc[q];
+      pc[q] = pr[q];
+    }
+    for (int q = 0; q < 3; ++q) d[q] = dn[q];
   }
   __syncthreads();
   if constexpr (SCAN)

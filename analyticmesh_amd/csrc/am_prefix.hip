@@ -391,7 +391,7 @@ __device__ __forceinline__ double fma_chain16(double acc, double w, const double
       "v_fmac_f64_dpp %0, %1, %15 row_newbcast:13 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %0, %1, %16 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
       "v_fmac_f64_dpp %0, %1, %17 row_newbcast:15 row_mask:0xf bank_mask:0xf\n"
-      : "+v"(acc)
+      : "+&v"(acc)
       : "v"(w), "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(x[4]), "v"(x[5]), "v"(x[6]), "v"(x[7]), "v"(x[8]),
         "v"(x[9]), "v"(x[10]), "v"(x[11]), "v"(x[12]), "v"(x[13]), "v"(x[14]), "v"(x[15]));
   return acc;
@@ -451,6 +451,40 @@ __device__ __forceinline__ void face_plane(const NetDev& net, const PrefixDev& p
   eq[3] = eq[3] - net.iso;
 }
 
+// The candidate scan of one region, all its planes into LDS.
+__device__ __forceinline__ void scan_prefix_region(const NetDev& net, const RegionIO& io, int rid, const gplanes* bases,
+                                                   unsigned char* smem, const double* eq, const double* p) {
+  const int C = net.C, Cs = io.Cs, N2 = io.Csort, lane = threadIdx.x;
+  double* Px = reinterpret_cast<double*>(smem);
+  double* Py = Px + Cs;
+  double* Pz = Py + Cs;
+  double* Pc = Pz + Cs;
+  double* keys = Pc + Cs;
+  int* order = reinterpret_cast<int*>(keys + N2);
+  uint32_t* used = reinterpret_cast<uint32_t*>(order + N2);
+  uint32_t* smask = used + ((C + 31) >> 5);
+  for (int w = lane; w < net.Wd; w += 64) smask[w] = io.reg_mask[(size_t)rid * net.Wd + w];
+  for (int w = lane; w < ((C + 31) >> 5); w += 64) used[w] = 0u;
+  __syncthreads();
+  const PrefixPlanes P{net, bases, smask};
+  for (int l = 0; l < P.parts(); ++l)
+    for (int j = lane; j < P.size(l); j += 64) {
+      double x[4];
+      P.load(l, j, x);
+      const int g = P.first(l) + j;
+      Px[g] = x[0];
+      Py[g] = x[1];
+      Pz[g] = x[2];
+      Pc[g] = x[3];
+    }
+  __syncthreads();
+  const WalkParams wp{0.f, 0.f, 0.f};
+  const WalkRecs rec = carve_walk_recs(smem + scan_lds_head(C, N2, net.Wd), net.vm, false);
+  walk_region<double, false>(net, io, wp, rid, rid - level_first(io), Px, Py, Pz, Pc, keys, order, used, smask, eq, p, rec.tab,
+                             rec.verts, rec.vpair);
+  __syncthreads();   // this region's LDS is free for the next
+}
+
 // Consecutive blocks go to the eight XCDs in turn; this gives each XCD a run of
 // consecutive regions instead: neighbours share prefixes, and with them the
 // planes in the XCD's L2.
@@ -460,7 +494,7 @@ __device__ __forceinline__ int xcd_run(int b, int n) {
 }
 
 template <bool SCAN, bool ALL>
-__global__ __launch_bounds__(64, SCAN && !ALL ? 5 : 4) void k_near64(NetDev net, PrefixDev pf, RegionIO io, int rid0, WalkParams wp,
+__global__ __launch_bounds__(64, 4) void k_near64(NetDev net, PrefixDev pf, RegionIO io, int rid0, WalkParams wp,
                                                   double* eqb, int only_undecided, NearList left) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ gplanes s_bases[AM_MAX_LINEAR + 1];
@@ -483,13 +517,21 @@ __global__ __launch_bounds__(64, SCAN && !ALL ? 5 : 4) void k_near64(NetDev net,
   const PrefixPlanes P{net, s_bases, S.mask};
   NearScan<double, SCAN> sc;
   face_plane(net, pf, P, S.stage, eq, [&](const double* x, int g) {
-    if (ALL) near_stage<double, SCAN>(S, g, x, p);
+    if (ALL) near_stage<double>(S, g, x);
     else sc.add(x, 0.0, p, S.key, g);
   });
   bool done = false;
   if (start >= 0 && start < net.C)
     done = near_walk<double, SCAN, ALL ? SET_LDS : SET_NEAR>(net, io, wp, rid, rid - level_first(io), P, S, eq, p, start,
                                                              0.0, sc, net.D - 1) == NEAR_DONE;
+  if (SCAN && ALL) {
+    // (a launch of its own for the seeds and the few others took 4.6 us a level)
+    if (!done) {
+      __syncthreads();
+      scan_prefix_region(net, io, rid, s_bases, smem_raw, eq, p);
+    }
+    return;
+  }
   // (thread 0 wrote the flag in finish_region: the orientation may be undecided)
   if (threadIdx.x == 0 && (!done || (!SCAN && (io.flags[rid - level_first(io)] & AM_UNDECIDED)))) {
     for (int q = 0; q < 4; ++q) eqb[(size_t)b * 4 + q] = eq[q];
@@ -509,15 +551,7 @@ __global__ __launch_bounds__(64, 4) void k_walk_fp64(NetDev net, PrefixDev pf, R
   extern __shared__ __align__(16) unsigned char smem_raw[];
   __shared__ gplanes s_bases[AM_MAX_LINEAR + 1];
   if (!quick) stage_mark(io.clk, T_SCAN64);
-  const int C = net.C, Cs = io.Cs, N2 = io.Csort, lane = threadIdx.x;
-  double* Px = reinterpret_cast<double*>(smem_raw);
-  double* Py = Px + Cs;
-  double* Pz = Py + Cs;
-  double* Pc = Pz + Cs;
-  double* keys = Pc + Cs;
-  int* order = reinterpret_cast<int*>(keys + N2);
-  uint32_t* used = reinterpret_cast<uint32_t*>(order + N2);
-  uint32_t* smask = used + ((C + 31) >> 5);
+  const int lane = threadIdx.x;
   const int total = min(*count, io.count);
   for (int i = blockIdx.x; i < total; i += gridDim.x) {
     const int b = slots[i];
@@ -527,9 +561,9 @@ __global__ __launch_bounds__(64, 4) void k_walk_fp64(NetDev net, PrefixDev pf, R
     double p[3], eq[4];
     for (int q = 0; q < 3; ++q) p[q] = io.reg_point[(size_t)rid * 3 + q];
     for (int q = 0; q < 4; ++q) eq[q] = eqb[(size_t)b * 4 + q];
-    const WalkParams wp{0.f, 0.f, 0.f};
-    if (quick && start >= 0 && start < C) {
-      const NearLds<double> S = carve_near<double>(smem_raw, C, net.Wd, net.vm, false);
+    if (quick && start >= 0 && start < net.C) {
+      const WalkParams wp{0.f, 0.f, 0.f};
+      const NearLds<double> S = carve_near<double>(smem_raw, net.C, net.Wd, net.vm, false);
       for (int w = lane; w < net.Wd; w += 64) S.mask[w] = io.reg_mask[(size_t)rid * net.Wd + w];
       __syncthreads();
       const PrefixPlanes P{net, s_bases, S.mask};
@@ -537,23 +571,7 @@ __global__ __launch_bounds__(64, 4) void k_walk_fp64(NetDev net, PrefixDev pf, R
       __syncthreads();
       if (done == NEAR_DONE) continue;
     }
-    for (int w = lane; w < net.Wd; w += 64) smask[w] = io.reg_mask[(size_t)rid * net.Wd + w];
-    for (int w = lane; w < ((C + 31) >> 5); w += 64) used[w] = 0u;
-    __syncthreads();
-    const PrefixPlanes P{net, s_bases, smask};
-    for (int l = 0; l < P.parts(); ++l)
-      for (int j = lane; j < P.size(l); j += 64) {
-        double x[4];
-        P.load(l, j, x);
-        const int g = P.first(l) + j;
-        Px[g] = x[0];
-        Py[g] = x[1];
-        Pz[g] = x[2];
-        Pc[g] = x[3];
-      }
-    __syncthreads();
-    walk_region<double, false>(net, io, wp, rid, rid - level_first(io), Px, Py, Pz, Pc, keys, order, used, smask, eq, p);
-    __syncthreads();   // this region's LDS is free for the next
+    scan_prefix_region(net, io, rid, s_bases, smem_raw, eq, p);
   }
 }
 

@@ -263,6 +263,24 @@ __device__ __forceinline__ int lane_check(const T* Px, const T* Py, const T* Pz,
   return verdict;
 }
 
+// Sum over the wave, in every lane (DPP moves, as wave_argmin).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint64_t dpp_add_step(uint64_t x) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)x, CTRL, ROWS, 0xf, false);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(x >> 32), CTRL, ROWS, 0xf, false);
+  return x + (((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ uint64_t wave_sum_u64(uint64_t x) {
+  x = dpp_add_step<0x111, 0xf>(x);
+  x = dpp_add_step<0x112, 0xf>(x);
+  x = dpp_add_step<0x114, 0xf>(x);
+  x = dpp_add_step<0x118, 0xf>(x);
+  x = dpp_add_step<0x142, 0xa>(x);
+  x = dpp_add_step<0x143, 0xc>(x);
+  return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(x >> 32), 63) << 32) |
+         (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, 63);
+}
+
 // Orientation, region record and neighbour candidates of a finished walk
 // (backend/inc/kernel.h:1325-1474).  In CHECKED mode an undecided region only
 // raises its flag: the FP64 redo writes its record and candidate slots.
@@ -323,13 +341,14 @@ __device__ void finish_region(const NetDev& net, const RegionIO& io, const WalkP
 
   // ---- neighbour candidates (backend/inc/kernel.h:1390-1474)
   const size_t slot0 = (size_t)slot_region * vm;
+  // lane m of every wave: entry m of the polygon, where it makes a candidate
+  int tm = -1;
+  if ((lane & 63) < vm && (lane & 63) + 1 < ntab) tm = s_tab[lane & 63];
+  if (tm >= L) tm = -1;
   if (lane < vm) {
     const int m = lane;
-    int t = -1;
-    if (m + 1 < ntab) t = s_tab[m];
-    const bool valid = t >= 0 && t < L;
     V mid[3] = {V(0), V(0), V(0)};
-    if (valid) {
+    if (tm >= 0) {
       const int m_ = (m == 0) ? ntab - 1 : m;
       int cnt = -1, v1 = -1;
       for (int i = 1; i < ntab; ++i) {
@@ -337,47 +356,34 @@ __device__ void finish_region(const NetDev& net, const RegionIO& io, const WalkP
         if (i == m_) v1 = cnt;
       }
       if (nv > 0 && v1 >= 0) {
-        int v2 = (v1 + 1) % nv;
+        if (v1 >= nv) v1 %= nv;   // (one vertex per entry: not taken)
+        const int v2 = v1 + 1 < nv ? v1 + 1 : 0;
         const int w1 = rev ? nv - 1 - v1 : v1, w2 = rev ? nv - 1 - v2 : v2;
         for (int c = 0; c < 3; ++c) mid[c] = (s_verts[w1 * 3 + c] + s_verts[w2 * 3 + c]) / V(2);
       }
     }
-    io.cand_start[slot0 + m] = valid ? t : -2;
+    io.cand_start[slot0 + m] = tm >= 0 ? tm : -2;
     io.cand_point[(slot0 + m) * 3 + 0] = (double)mid[0];
     io.cand_point[(slot0 + m) * 3 + 1] = (double)mid[1];
     io.cand_point[(slot0 + m) * 3 + 2] = (double)mid[2];
   }
+  // candidate m's mask: waves take candidates, lanes hold the region's words
   const int Wd = net.Wd;
-  // candidate m's mask: waves take candidates, lanes take words (no division)
-  for (int m = lane >> 6; m < vm; m += (nth + 63) >> 6) {
-    int t = -1;
-    if (m + 1 < ntab) t = s_tab[m];
-    if (t >= 0 && t < L)
-      for (int w = lane & 63; w < Wd; w += 64) {
-        uint32_t word = smask[w];
-        if ((t >> 5) == w) word ^= 1u << (t & 31);
-        io.cand_mask[(slot0 + m) * Wd + w] = word;
-      }
+  const uint32_t word = (lane & 63) < Wd ? smask[lane & 63] : 0u;   // (Wd <= 64)
+  const int nm = min(vm, ntab - 1);
+  for (int m = __builtin_amdgcn_readfirstlane(lane >> 6); m < nm; m += (nth + 63) >> 6) {
+    const int t = __builtin_amdgcn_readlane(tm, m);
+    if (t >= 0 && (lane & 63) < Wd)
+      io.cand_mask[(slot0 + m) * Wd + (lane & 63)] = (t >> 5) == (lane & 63) ? word ^ (1u << (t & 31)) : word;
   }
   // each candidate's key hash: the region's sum of word hashes with the
   // flipped word's term swapped (wave 0; Wd <= 64 and vm <= 64)
   if (lane < 64) {
-    uint64_t g = 0;
-    if (lane < Wd) g = word_hash(smask[lane], lane);
-#pragma unroll
-    for (int d = 32; d > 0; d >>= 1) {
-      const uint32_t lo = (uint32_t)__shfl_xor((int)(uint32_t)g, d, 64);
-      const uint32_t hi = (uint32_t)__shfl_xor((int)(uint32_t)(g >> 32), d, 64);
-      g += ((uint64_t)hi << 32) | lo;
-    }
-    if (lane < vm) {
-      int t = -1;
-      if (lane + 1 < ntab) t = s_tab[lane];
-      if (t >= 0 && t < L) {
-        const int wt = t >> 5;
-        const uint32_t x = smask[wt];
-        io.cand_hash[slot0 + lane] = g - word_hash(x, wt) + word_hash(x ^ (1u << (t & 31)), wt);
-      }
+    const uint64_t g = wave_sum_u64(lane < Wd ? word_hash(word, lane) : 0ull);
+    if (tm >= 0) {
+      const int wt = tm >> 5;
+      const uint32_t x = smask[wt];
+      io.cand_hash[slot0 + lane] = g - word_hash(x, wt) + word_hash(x ^ (1u << (tm & 31)), wt);
     }
   }
 }
@@ -501,20 +507,17 @@ __device__ void wave_top64(const T* Px, const T* Py, const T* Pz, const T* Pc, i
 }
 
 // Pe, eqe: per-plane error estimates of the constraints and the face plane
-// (coarse planes, per-plane mode with wp.lam > 0), as in walk_ray.
+// (coarse planes, per-plane mode with wp.lam > 0), as in walk_ray.  s_tab [vm + 2],
+// s_verts [vm][3], s_vpair [vm][2]: LDS for the records.
 template <typename T, bool CHECKED>
 __device__ void walk_region(const NetDev& net, const RegionIO& io, const WalkParams& wp, int rid, int slot_region,
                             T* Px, T* Py, T* Pz, T* Pc, T* keys, int* order, uint32_t* used,
-                            const uint32_t* smask, const T* eq_in, const T* p, const T* Pe = nullptr,
-                            T eqe = T(0)) {
+                            const uint32_t* smask, const T* eq_in, const T* p, int* s_tab, T* s_verts, int* s_vpair,
+                            const T* Pe = nullptr, T eqe = T(0)) {
   const bool per_plane = CHECKED && sizeof(T) == 4 && wp.lam > 0.f && Pe != nullptr;
   const T lam = per_plane ? T(wp.lam) : T(0);
   const T* Pg = per_plane ? Pe : nullptr;
   bool vinacc = false;
-  __shared__ int s_tab[AM_VM_MAX + 2];
-  __shared__ T s_verts[AM_VM_MAX * 3];
-  __shared__ int s_vpair[AM_VM_MAX * 2];
-
   const int C = net.C, vm = net.vm, N2 = io.Csort;
   const int lane = threadIdx.x;
   const T eq[4] = {eq_in[0], eq_in[1], eq_in[2], eq_in[3]};
@@ -1032,6 +1035,14 @@ __device__ inline WalkRecs carve_walk_recs(unsigned char* p, int vm, bool jinv) 
   p += a16((size_t)(vm + 2) * 4);
   r.jinv = jinv ? reinterpret_cast<float*>(p) : nullptr;
   return r;
+}
+
+// LDS of the FP64 candidate scan over C constraints, its records behind the rest.
+__host__ __device__ inline size_t scan_lds_head(int C, int Csort, int Wd) {
+  return ((size_t)4 * C * 8 + (size_t)Csort * 12 + (size_t)((C + 31) / 32) * 4 + (size_t)Wd * 4 + 15) & ~(size_t)15;
+}
+__host__ __device__ inline size_t scan_lds_bytes(int C, int Csort, int Wd, int vm) {
+  return scan_lds_head(C, Csort, Wd) + walk_rec_bytes(vm, false);
 }
 
 // Reduced-precision walk by ray shooting.  From the start plane's edge each
