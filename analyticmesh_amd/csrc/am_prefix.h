@@ -39,7 +39,7 @@ namespace am {
 struct PrefixDev {
   int nd;
   uint32_t cap_mask;
-  unsigned long long* tab;      // [cap] depth << 32 | a region with that prefix, or empty
+  unsigned long long* tab;      // [cap] prefix_key << 32 | a region with that prefix, or empty
   int* tab_id;                  // [cap] its id
   int* total;                   // [nd + 1] ids given per depth, AM_PFX_TS apart
   int* done;                    // [nd + 1] ids whose planes are there
