@@ -915,16 +915,54 @@ void run_fp64_regions(am_ctx* c, int lvl_first, int first, int count, const int*
   }
 }
 
+// Buffers of a reduced form's level of `count` regions, beside fp64_prepare's.
+void reduced_prepare(am_ctx* c, int count) {
+  fast_level_prepare(c->fast, c->fbuf, c->net, count);
+  ensure(c->redo_ids, (size_t)count, false, c->stream);
+  ensure(c->redo_cnt, 1, false, c->stream);
+  ensure_zeroed(c->redo_state, redo_state_words(count), c->stream);
+}
+
+// A reduced form's level: face kernel and checked walk, then FP64 planes of the
+// regions the walk left to FP64 only (their list, made by fast_level's last
+// launch, and its count stay on the device; the launches are sized for the whole
+// level and their blocks past the count exit): the ones it decided with a vertex
+// it could not vouch for get their vertices re-solved from them; the undecided
+// ones are re-decided in place (records and candidate slots rewritten) by the
+// checked FP64 ray walk, and by the candidate scan where that is undecided too.
+// lvl: as in run_fp64_regions.  Returns the launches of the face kernel.
+int run_reduced_level(am_ctx* c, int first, int count, Fp64Counts& t, const int2* lvl = nullptr, int lvl_bound = 0) {
+  FastLevel fl;
+  fl.first = first;
+  fl.count = count;
+  fl.reg_mask = c->reg_mask.p; fl.reg_start = c->reg_start.p; fl.reg_point = c->reg_point.p;
+  fl.reg_info = c->reg_info.p; fl.reg_tab = c->reg_tab.p; fl.reg_verts = c->reg_verts.p;
+  fl.reg_vpair = c->reg_vpair.p; fl.cand_mask = c->cand_mask.p; fl.cand_start = c->cand_start.p;
+  fl.cand_point = c->cand_point.p;
+  fl.cand_hash = c->cand_hash.p;
+  fl.reg_jinv = c->jinv_on ? c->reg_jinv.p : nullptr;
+  fl.lvl = lvl;
+  fl.lvl_bound = lvl_bound;
+  const RedoList redo{c->redo_ids.p, c->redo_cnt.p, c->redo_state.p};
+  FastTimes ft{};
+  fast_level(c->fast, c->fbuf, c->net, fl, c->stream, c->clock, ft, c->rflags.p, c->acc + 1 + AM_WHY_COUNT, redo, true);
+  run_fp64_regions(c, first, first, count, c->redo_ids.p, 2, t, -1, c->redo_cnt.p, lvl, lvl_bound);
+  return ft.launches;
+}
+
 // Whether a level of up to B regions can be launched behind the one in flight
 // with the buffers as they are (nothing may be allocated or moved under it):
 // the level in flight adds up to B regions to c->R, this one B vm candidates.
-bool ahead_fits(const am_ctx* c, int B) {
+bool ahead_fits(const am_ctx* c, int B, bool reduced) {
   const size_t n = (size_t)B * c->vm, R = (size_t)c->R + B;
   const PrefixStore& s = c->pfx;
   if (R + n > c->reg_cap || 2 * (R + n) > c->table_cap) return false;
   if (c->cand_mask.n < n * c->Wd || c->cand_start.n < n || c->cand_point.n < 3 * n || c->cand_hash.n < n ||
       c->slot.n < n || c->rank.n < n || c->rflags.n < (size_t)B || c->scan_state.n < scan_commit_tiles(n) + 1 ||
       c->teq.n < (size_t)4 * B || c->tslots.n < (size_t)2 * B)
+    return false;
+  if (reduced && (!fast_level_fits(c->fast, c->fbuf, B) || c->redo_ids.n < (size_t)B ||
+                  c->redo_state.n < redo_state_words(B)))
     return false;
   const int nd = s.dev.nd;
   if ((size_t)B > prefix_chunk(c) || s.rslot.n < (size_t)B * std::max(nd, 1) || s.fresh.n < (size_t)(nd + 1) * B)
@@ -939,13 +977,14 @@ bool ahead_fits(const am_ctx* c, int B) {
 }
 
 // Buffers so that ahead_fits(B) holds from the level after next on.
-void ahead_grow(am_ctx* c, int B) {
+void ahead_grow(am_ctx* c, int B, bool reduced) {
   const size_t n = (size_t)B * c->vm;
   grow_cands(c, n);
   ensure(c->rflags, (size_t)B, false, c->stream);
   ensure(c->scan_state, scan_commit_tiles(n) + 1, false, c->stream);
   ensure(c->teq, (size_t)4 * B, false, c->stream);
   ensure(c->tslots, (size_t)2 * B, false, c->stream);
+  if (reduced) reduced_prepare(c, B);
   const int nd = c->pfx.dev.nd;
   ensure(c->pfx.rslot, (size_t)B * std::max(nd, 1), false, c->stream);
   ensure(c->pfx.fresh, (size_t)(nd + 1) * B, false, c->stream);
@@ -956,7 +995,7 @@ void ahead_grow(am_ctx* c, int B) {
   (void)prefix_blocks(c, ids, false);
 }
 
-// The levels of an FP64 march.  While a small level runs, the next one is
+// The levels of a march.  While a small level runs, the next one is
 // already in the stream: launched for at most twice the regions (and 256 more),
 // its size read on the device, so the host's round trip (about 20 us: the total's way
 // to the host and the next launches) is off the GPU's path.  When the level
@@ -964,12 +1003,19 @@ void ahead_grow(am_ctx* c, int B) {
 // again; levels over kAheadMax regions take longer than the round trip and are
 // launched when their size is known.
 struct LevelsDone {
-  long long levels = 0, cands = 0;
+  long long levels = 0, cands = 0, launches = 0;
 };
 constexpr int kAheadMax = 8192;
 
-LevelsDone march_fp64(am_ctx* c, long long first, long long count, int slot, int mode, Fp64Counts& t) {
+// mode: as in run_fp64_regions; 2: a reduced form.
+LevelsDone march_levels(am_ctx* c, long long first, long long count, int mode, Fp64Counts& t) {
   LevelsDone done;
+  const bool reduced = mode == 2;
+  auto launch = [&](int f, int n, const int2* lvl, int bound) -> int {
+    if (reduced) return run_reduced_level(c, f, n, t, lvl, bound);
+    run_fp64_regions(c, f, f, n, nullptr, mode, t, -1, nullptr, lvl, bound);
+    return 1;
+  };
   auto bound_after = [](long long n) { return (int)(2 * n + 256); };
   InsertPlan cur;            // the level in flight
   bool launched = false;     // ... already there, launched ahead
@@ -977,16 +1023,17 @@ LevelsDone march_fp64(am_ctx* c, long long first, long long count, int slot, int
     const size_t ncand = (size_t)count * c->vm;
     const int B = bound_after(count);
     if (!launched) {
-      if (count <= kAheadMax) ahead_grow(c, B);
+      if (count <= kAheadMax) ahead_grow(c, B, reduced);
       grow_cands(c, ncand);
       ensure(c->rflags, (size_t)count, false, c->stream);
       fp64_prepare(c, (int)count);
+      if (reduced) reduced_prepare(c, (int)count);
       cur = insert_prepare(c, ncand);
-      run_fp64_regions(c, (int)first, (int)first, (int)count, nullptr, mode, t);
+      done.launches += launch((int)first, (int)count, nullptr, 0);
       insert_launch(c, cur);
     }
     InsertPlan next;
-    const bool ahead = count <= kAheadMax && ahead_fits(c, B);
+    const bool ahead = count <= kAheadMax && ahead_fits(c, B, reduced);
     if (ahead) {
       PrefixStore& s = c->pfx;
       s.reset.assign(1, 0);
@@ -999,7 +1046,7 @@ LevelsDone march_fp64(am_ctx* c, long long first, long long count, int slot, int
       next.slot = arm_host_total(c);
       next.lvl = c->levels.p + cur.slot;
       next.lvl_bound = B;
-      run_fp64_regions(c, 0, 0, B, nullptr, mode, t, -1, nullptr, next.lvl, B);
+      done.launches += launch(0, B, next.lvl, B);
       insert_launch(c, next);
     }
     const long long before = c->R;
@@ -1018,7 +1065,6 @@ LevelsDone march_fp64(am_ctx* c, long long first, long long count, int slot, int
       cur.lvl = nullptr;
     }
   }
-  (void)slot;
   return done;
 }
 
@@ -1644,17 +1690,17 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
                        c->tcnt.p);
     HIPCHK(hipGetLastError());
     long long lvl_first = 0;
-    int seed_slot = 0;
-    long long lvl_count = insert_level(c, (size_t)n_seeds, &seed_slot);
+    long long lvl_count = insert_level(c, (size_t)n_seeds);
     long long levels = 0, cands = 0, launches = 0;
     long long why[AM_WHY_COUNT] = {0};
     Fp64Counts f64;
     c->timer.reset();
-    if (fp64_form && !c->graph_levels && c->max_regions < 0) {
-      const LevelsDone ld = march_fp64(c, lvl_first, lvl_count, seed_slot, c->precision == AM_PREC_FP64 ? 0 : 1, f64);
+    if ((fp64_form || fast_ahead(c->fast)) && !c->graph_levels && c->max_regions < 0) {
+      const LevelsDone ld =
+          march_levels(c, lvl_first, lvl_count, !fp64_form ? 2 : c->precision == AM_PREC_FP64 ? 0 : 1, f64);
       levels = ld.levels;
       cands = ld.cands;
-      launches = ld.levels;
+      launches = fp64_form ? ld.levels : ld.launches;
       lvl_count = 0;
     }
     while (lvl_count > 0) {
@@ -1681,42 +1727,20 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
         lvl_count = added;
         continue;
       }
-      // the reduced forms' level: face kernel and checked walk, then the FP64
-      // redo of the regions the walk left to FP64
-      auto fast_level_of = [&]() {
-        FastLevel fl;
-        fl.first = (int)lvl_first;
-        fl.count = (int)lvl_count;
-        fl.reg_mask = c->reg_mask.p; fl.reg_start = c->reg_start.p; fl.reg_point = c->reg_point.p;
-        fl.reg_info = c->reg_info.p; fl.reg_tab = c->reg_tab.p; fl.reg_verts = c->reg_verts.p;
-        fl.reg_vpair = c->reg_vpair.p; fl.cand_mask = c->cand_mask.p; fl.cand_start = c->cand_start.p;
-        fl.cand_point = c->cand_point.p;
-        fl.cand_hash = c->cand_hash.p;
-        fl.reg_jinv = c->jinv_on ? c->reg_jinv.p : nullptr;
-        return fl;
-      };
       if (!fp64_form && c->graph_levels) {
         // as the FP64 forms' graph above: the host work first (buffers, the
         // region store's growth), then every launch of the level in one graph
         fp64_prepare(c, (int)lvl_count);
-        fast_level_prepare(c->fast, c->fbuf, n, (int)lvl_count);
-        ensure(c->redo_ids, (size_t)lvl_count, false, st);
-        ensure(c->redo_cnt, 1, false, st);
-        ensure_zeroed(c->redo_state, redo_state_words((int)lvl_count), st);
+        reduced_prepare(c, (int)lvl_count);
         const InsertPlan plan = insert_prepare(c, ncand);
-        const FastLevel fl = fast_level_of();
-        const RedoList redo{c->redo_ids.p, c->redo_cnt.p, c->redo_state.p};
-        FastTimes ft{};
+        int face = 0;
         launch_as_graph(c, (int)levels, [&]() {
-          fast_level(c->fast, c->fbuf, n, fl, st, c->clock, ft, c->rflags.p, acc_dev + 1 + AM_WHY_COUNT, redo,
-                     true);
-          run_fp64_regions(c, (int)lvl_first, (int)lvl_first, (int)lvl_count, c->redo_ids.p, 2, f64, -1,
-                           c->redo_cnt.p);
+          face = run_reduced_level(c, (int)lvl_first, (int)lvl_count, f64);
           insert_launch(c, plan);
         });
         const long long before = c->R;
         const int added = insert_finish(c, plan);
-        launches += ft.launches;
+        launches += face;
         cands += (long long)ncand;
         levels += 1;
         lvl_first = before;
@@ -1729,24 +1753,8 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
                          c->precision == AM_PREC_FP64 ? 0 : 1, f64);
         launches += 1;
       } else {
-        const FastLevel fl = fast_level_of();
-        ensure(c->redo_ids, (size_t)lvl_count, false, st);
-        ensure(c->redo_cnt, 1, false, st);
-        ensure_zeroed(c->redo_state, redo_state_words((int)lvl_count), st);
-        const RedoList redo{c->redo_ids.p, c->redo_cnt.p, c->redo_state.p};
-        FastTimes ft{};
-        fast_level(c->fast, c->fbuf, n, fl, st, c->clock, ft, c->rflags.p, acc_dev + 1 + AM_WHY_COUNT, redo);
-        // FP64 planes of the regions the walk left to FP64 only (their list,
-        // made by fast_level's last launch, and count stay on the device;
-        // the launches are sized for the whole
-        // level and their blocks past the count exit): the ones it decided
-        // with a vertex it could not vouch for get their vertices re-solved
-        // from them; the undecided ones are re-decided in place (records and
-        // candidate slots rewritten) by the checked FP64 ray walk, and by the
-        // candidate scan where that is undecided too.
-        run_fp64_regions(c, (int)lvl_first, (int)lvl_first, (int)lvl_count, c->redo_ids.p, 2, f64, -1,
-                         c->redo_cnt.p);
-        launches += ft.launches;
+        reduced_prepare(c, (int)lvl_count);
+        launches += run_reduced_level(c, (int)lvl_first, (int)lvl_count, f64);
       }
       const long long before = c->R;
       const int added = insert_level(c, ncand);   // waits once: the next level's size

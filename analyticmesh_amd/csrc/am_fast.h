@@ -75,6 +75,8 @@ struct FastLevel {
   double* cand_point;
   uint64_t* cand_hash;
   uint16_t* reg_jinv = nullptr;   // optional: the walk's inverse vertex systems (Newton vertices)
+  const int2* lvl = nullptr;      // as in RegionIO: a level launched ahead (near walk only; up to one chunk)
+  int lvl_bound = 0;
 };
 
 struct FastTimes {
@@ -109,6 +111,9 @@ void fast_level(FastNet& f, FastBuffers& b, const NetDev& net, const FastLevel& 
                 StageClock* clk, FastTimes& t, unsigned* flags, int* acc, const RedoList& redo,
                 bool prepared = false);
 // Buffers and launch attributes of fast_level for a level of `count` regions.
+// Whether levels past the seeds can be launched ahead, and whether one of `count` regions fits the buffers.
+bool fast_ahead(const FastNet& f);
+bool fast_level_fits(const FastNet& f, const FastBuffers& b, int count);
 void fast_level_prepare(FastNet& f, FastBuffers& b, const NetDev& net, int count);
 // Planes of n given regions (their masks in `reg_mask`) with the prepared
 // reduced-precision form: planes [n][AM_PCOMP][Cs] f32 (x, y, z, c signed, then

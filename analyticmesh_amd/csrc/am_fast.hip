@@ -46,6 +46,10 @@ struct GemmIO {
   float* planes;    // [count][4][Cs]
   float* eq;        // [count][4]
   StageClock* clk = nullptr;
+  const int* dcount = nullptr;   // as in RegionIO
+  int dbase = 0;
+  const int2* lvl = nullptr;
+  int lvl_bound = 0;
 };
 
 __device__ __forceinline__ uint16_t bf16_rn(float x) {
@@ -157,11 +161,12 @@ __global__ __launch_bounds__(256, PREC == 0 ? 4 : 1) void k_gemm(FastNetDev f, G
   auto xq_at = [&](int k, int t) -> uint16_t& { return Ypad[k * 2 * AM_XS + t]; };
   __shared__ int s_nk[AM_MAX_LINEAR];
   const int r0 = blockIdx.x * AM_GT;
-  const int nreg = min(AM_GT, io.count - r0);
+  const int nreg = min(AM_GT, launch_count(io) - r0), first = launch_first(io, io.first);
+  if (nreg <= 0) return;
 
   for (int idx = tid; idx < AM_GT * f.Wd; idx += 256) {
     const int t = idx / f.Wd, w = idx - t * f.Wd;
-    mk[idx] = t < nreg ? io.reg_mask[(size_t)(io.first + r0 + t) * f.Wd + w] : 0u;
+    mk[idx] = t < nreg ? io.reg_mask[(size_t)(first + r0 + t) * f.Wd + w] : 0u;
   }
   // (FP32: every LDS element a step reads is written first -- list positions
   // by the staging and the compaction, parked rows below n_out -- so no clear)
@@ -528,8 +533,8 @@ __global__ __launch_bounds__(64, 5) void k_near_f32(NetDev net, RegionIO io, Wal
   stage_mark(io.clk, T_WALK);
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int b = blockIdx.x;
-  if (b >= io.count) return;
-  const int rid = chunk_first + b;
+  if (b >= launch_count(io)) return;
+  const int rid = launch_first(io, chunk_first) + b, slot = rid - level_first(io);
   const NearLds<float> S = carve_near<float>(smem_raw, net.C, net.Wd, net.vm, true);
   const int start = io.reg_start[rid];
   for (int w = threadIdx.x; w < net.Wd; w += 64) S.mask[w] = io.reg_mask[(size_t)rid * net.Wd + w];
@@ -539,9 +544,9 @@ __global__ __launch_bounds__(64, 5) void k_near_f32(NetDev net, RegionIO io, Wal
                       (float)io.reg_point[(size_t)rid * 3 + 2]};
   __syncthreads();
   const FacePlanes P{planes + (size_t)b * AM_PCOMP * Cs_hbm, Cs_hbm, net.C};
-  const int w = near_or_full_walk<float, false>(net, io, wp, rid, rid - io.first, P, S, eq, p, start, eb[4]);
+  const int w = near_or_full_walk<float, false>(net, io, wp, rid, slot, P, S, eq, p, start, eb[4]);
   if (w != NEAR_DONE && threadIdx.x == 0)
-    io.flags[rid - io.first] = AM_UNDECIDED | (w > 0 ? (unsigned)w : AM_WHY_BIT(AM_WHY_SEED));
+    io.flags[slot] = AM_UNDECIDED | (w > 0 ? (unsigned)w : AM_WHY_BIT(AM_WHY_SEED));
 }
 
 // The level's regions the walk left to FP64 in one launch: their ids (first +
@@ -551,7 +556,11 @@ __global__ __launch_bounds__(64, 5) void k_near_f32(NetDev net, RegionIO io, Wal
 // acc[1 + AM_WHY_COUNT] (one atomic per wave and counter).
 constexpr int kRedoThreads = 256, kRedoItems = 8, kRedoTile = kRedoThreads * kRedoItems;
 __global__ __launch_bounds__(kRedoThreads) void k_redo_list(const unsigned* flags, int n, int first, int* acc,
-                                                           RedoList out, int tiles) {
+                                                           RedoList out, int tiles, const int2* lvl, int lvl_bound) {
+  if (lvl) {
+    n = level_count(lvl, lvl_bound);
+    first = lvl->x;
+  }
   __shared__ int s_tile, s_excl;
   __shared__ int s_wave[kRedoThreads / 64];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -814,6 +823,12 @@ size_t walk_ray_lds(const NetDev& net) {
 }
 }  // namespace
 
+bool fast_ahead(const FastNet& f) { return f.walk_mode == 0 && f.precision != 1; }
+bool fast_level_fits(const FastNet& f, const FastBuffers& b, int count) {
+  return count <= kLevelChunk && b.mem[S_PLANES].bytes >= (size_t)count * AM_PCOMP * f.dev.Cs * 4 &&
+         b.mem[S_EQ].bytes >= (size_t)count * AM_EQS * 4;
+}
+
 void fast_level_prepare(FastNet& f, FastBuffers& b, const NetDev& net, int count) {
   const FastNetDev& d = f.dev;
   const int chunk = std::min(count, kLevelChunk);
@@ -856,6 +871,8 @@ void fast_level(FastNet& f, FastBuffers& b, const NetDev& net, const FastLevel& 
     g.planes = planes;
     g.eq = eqb;
     g.clk = clk;
+    g.lvl = lvl.lvl;
+    g.lvl_bound = lvl.lvl_bound;
     if (prec == 0)
       hipLaunchKernelGGL(k_gemm<0>, dim3((n + AM_GT - 1) / AM_GT), dim3(256), glds, st, d, g);
     else
@@ -882,8 +899,10 @@ void fast_level(FastNet& f, FastBuffers& b, const NetDev& net, const FastLevel& 
     io.flags = flags;
     io.clk = clk;
     io.ids = nullptr;
+    io.lvl = lvl.lvl;
+    io.lvl_bound = lvl.lvl_bound;
     // a level past the seeds, planes with estimates: the near walk
-    if (f.walk_mode == 0 && prec == 0 && lvl.first > 0)
+    if (fast_ahead(f) && (lvl.first > 0 || lvl.lvl))
       hipLaunchKernelGGL(k_near_f32, dim3(n), dim3(64), nlds, st, net, io, f.wp, planes, eqb, d.Cs, lvl.first + c0);
     else if (f.walk_mode == 0 && f.ray_waves == 2)
       hipLaunchKernelGGL(k_walk_ray_f32<2>, dim3(n), dim3(128), rlds, st, net, io, f.wp, planes, eqb, d.Cs,
@@ -902,7 +921,7 @@ void fast_level(FastNet& f, FastBuffers& b, const NetDev& net, const FastLevel& 
   }
   const int tiles = (int)redo_state_words(lvl.count) - 2;
   hipLaunchKernelGGL(k_redo_list, dim3(tiles), dim3(kRedoThreads), 0, st, (const unsigned*)flags, lvl.count,
-                     lvl.first, acc, redo, tiles);
+                     lvl.first, acc, redo, tiles, lvl.lvl, lvl.lvl_bound);
   FCHK(hipGetLastError());
 }
 

@@ -42,11 +42,12 @@ struct RegionIO {
 // passes the bound it was launched for), or a list (dcount).
 template <typename IO>
 __device__ __forceinline__ int launch_count(const IO& io) {
+  if (io.dcount) return min(io.count, *io.dcount - io.dbase);
   if (io.lvl) {
     const int n = io.lvl->y;
     return n <= io.lvl_bound ? min(io.count, n - io.dbase) : 0;
   }
-  return io.dcount ? min(io.count, *io.dcount - io.dbase) : io.count;
+  return io.count;
 }
 // First region of the launch (host: the value known there), and of its level.
 template <typename IO>
