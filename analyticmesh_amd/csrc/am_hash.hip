@@ -203,16 +203,21 @@ __global__ __launch_bounds__(kScanCommitThreads) void k_scan_commit(ScanCommitIO
     if (lane == 0) {
       s_excl = excl;
       if (t == tiles - 1 && io.lvl_next) *io.lvl_next = make_int2(R0, excl + tot);
-      if (t == tiles - 1 && io.total) {
-        for (int i = 0; i < io.npub; ++i) io.pub_out[i] = io.pub[i * io.pub_stride];
-        if (io.clk) stage_mark_now(io.clk, T_SLOTS);
-        if (io.npub) __threadfence_system();
-        *io.total = excl + tot;
-      }
     }
   }
   __syncthreads();
   const int excl = s_excl;
+  // The host's words, by the last tile's first wave behind its share of the
+  // commit (the system-scope fence takes about 2 us).
+  auto publish = [&]() {
+    if (t != tiles - 1 || !io.total || tid >= 64) return;
+    if (lane < io.npub) io.pub_out[lane] = io.pub[lane * io.pub_stride];
+    if (io.npub) __threadfence_system();
+    if (lane == 0) {
+      *io.total = excl + tot;
+      if (io.clk) stage_mark_now(io.clk, T_SLOTS);
+    }
+  };
   int run = off;
 #pragma unroll
   for (int it = 0; it < kScanCommitItems; ++it) {
@@ -222,7 +227,10 @@ __global__ __launch_bounds__(kScanCommitThreads) void k_scan_commit(ScanCommitIO
     }
     run += v[it];
   }
-  if (io.rank) return;
+  if (io.rank) {
+    publish();
+    return;
+  }
   __syncthreads();
   const CommitIO& ci = io.cio;
   const int j = tid & (AM_KG - 1), gid = tid / AM_KG;
@@ -291,6 +299,7 @@ __global__ __launch_bounds__(kScanCommitThreads) void k_scan_commit(ScanCommitIO
       }
     }
   }
+  publish();
 }
 
 // New regions get ids R0 + rank in candidate order (rank from a stored scan).

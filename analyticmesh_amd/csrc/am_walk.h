@@ -345,15 +345,20 @@ __device__ void finish_region(const NetDev& net, const RegionIO& io, const WalkP
   int tm = -1;
   if ((lane & 63) < vm && (lane & 63) + 1 < ntab) tm = s_tab[lane & 63];
   if (tm >= L) tm = -1;
+  const bool holes = ntab > 64 || __any((lane & 63) < ntab && s_tab[min(lane & 63, ntab - 1)] < 0);
   if (lane < vm) {
     const int m = lane;
     V mid[3] = {V(0), V(0), V(0)};
     if (tm >= 0) {
       const int m_ = (m == 0) ? ntab - 1 : m;
-      int cnt = -1, v1 = -1;
-      for (int i = 1; i < ntab; ++i) {
-        if (s_tab[i] >= 0) ++cnt;
-        if (i == m_) v1 = cnt;
+      int v1 = m_ - 1;   // (every entry of the polygon is a vertex, unless one is negative)
+      if (holes) {
+        int cnt = -1;
+        v1 = -1;
+        for (int i = 1; i < ntab; ++i) {
+          if (s_tab[i] >= 0) ++cnt;
+          if (i == m_) v1 = cnt;
+        }
       }
       if (nv > 0 && v1 >= 0) {
         if (v1 >= nv) v1 %= nv;   // (one vertex per entry: not taken)
