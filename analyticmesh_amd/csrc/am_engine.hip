@@ -800,7 +800,7 @@ void prefix_launch(am_ctx* c, size_t k, const int* ids, int first, int n, const 
   const size_t lds = prefix_layer_lds(c);
   for (int d = 1; d <= s.dev.nd; ++d) {
     const int nout = c->nodes[d + 1];
-    hipLaunchKernelGGL((c->skips[d].empty() ? k_layer<false> : k_layer<true>), dim3(blocks(n, AM_PT), (nout + 127) / 128),
+    hipLaunchKernelGGL((c->skips[d].empty() ? k_layer<false> : k_layer<true>), dim3(blocks(n, AM_PT), n <= 4096 ? (nout + 63) / 64 : (nout + 127) / 128),
                        dim3(256), lds, c->stream, c->net, s.dev, rg, d);
     HIPCHK(hipGetLastError());
   }

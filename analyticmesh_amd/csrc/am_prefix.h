@@ -83,7 +83,7 @@ inline size_t prefix_block_bytes(int n) { return (size_t)AM_PFX_IDS * (32 * (siz
 #define AM_PFX_REGIONS 256              // regions per block of k_prefix
 // Finds or adds the prefixes of the launch's regions (grid: ceil(count / AM_PFX_REGIONS) x nd).
 __global__ void k_prefix(NetDev net, PrefixDev pf, PrefixRegions rg);
-// Planes of layer d + 1 for the new ids of depth d (grid: ceil(count / AM_PT) x ceil(n_out / 128),
+// Planes of layer d + 1 for the new ids of depth d (grid: ceil(count / AM_PT) x ceil(n_out / 128) or ceil(n_out / 64),
 // 256 threads, layer_lds bytes).  SKIPS: additive skips lead into the layer.
 template <bool SKIPS>
 __global__ void k_layer(NetDev net, PrefixDev pf, PrefixRegions rg, int d);

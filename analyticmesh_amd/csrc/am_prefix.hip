@@ -189,8 +189,14 @@ __global__ __launch_bounds__(256, SKIPS ? 4 : 5) void k_layer(NetDev net, Prefix
   // the tile's regions: every lane t % AM_PT knows prefix t's
   const int2 reg = pf.fresh[(size_t)d * pf.fresh_stride + blockIdx.x * AM_PT + min(lane & (AM_PT - 1), np - 1)];
   const int l16 = lane & 15, l4 = lane >> 4, q_l = l16 & 3;
-  const int row0 = (int)blockIdx.y * 128 + wave * 32;
-  const int nrb = row0 >= nout ? 0 : (row0 + 16 >= nout ? 1 : 2);   // the wave's row blocks with rows
+  // rows per wave: 32, or 16 where that leaves no wave idle (layers up to 64 wide) or
+  // where the tiles do not fill half the chip (a grid of 64-row blocks then; the
+  // second half of it exits when they do)
+  const int tiles = (pf.total[d * AM_PFX_TS] - pf.done[d] + AM_PT - 1) / AM_PT, rows128 = (nout + 127) >> 7;
+  const int rpw = nout <= 64 || ((int)gridDim.y > rows128 && tiles * rows128 <= 128) ? 16 : 32;
+  if ((int)blockIdx.y * 4 * rpw >= nout) return;
+  const int row0 = (int)blockIdx.y * 4 * rpw + wave * rpw;
+  const int nrb = row0 >= nout ? 0 : (rpw == 16 || row0 + 16 >= nout ? 1 : 2);   // the wave's row blocks with rows
   am_f64x4 acc[2][2];
 #pragma unroll
   for (int rb = 0; rb < 2; ++rb)
@@ -308,7 +314,7 @@ __global__ __launch_bounds__(256, SKIPS ? 4 : 5) void k_layer(NetDev net, Prefix
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int row = row0 + 16 * rb + l4 + 4 * v;
-        if (row < nout) {
+        if (rb < nrb && row < nout) {
           acc[rb][0][v] = f(acc[rb][0][v], row, l16 >> 2);
           acc[rb][1][v] = f(acc[rb][1][v], row, 4 + (l16 >> 2));
         }
