@@ -817,6 +817,8 @@ void fp64_prepare(am_ctx* c, int count) {
   prefix_plan(c, count, chunk);
 }
 
+bool ray64_form(const am_ctx* c) { return ray64_lds_bytes(c) <= c->max_lds && c->tile_ok; }
+
 // FP64 planes + walk of `count` regions (region ids first.., or ids[0..count)),
 // in chunks; candidate slots and flags are numbered from `lvl_first`.  Planes
 // come from the activation prefixes, the walk is the near walk and, for what it
@@ -836,7 +838,7 @@ void run_fp64_regions(am_ctx* c, int lvl_first, int first, int count, const int*
   const bool after_walk = mode == 2;
   if (after_walk) mode = 1;
   // nets with skips or layers over 256 wide keep the candidate scan's records in every form
-  if (mode == 1 && (ray64_lds_bytes(c) > c->max_lds || !c->tile_ok)) mode = 0;
+  if (mode == 1 && !ray64_form(c)) mode = 0;
   int Cs, Csort;
   (void)region_lds_bytes(c, Cs, Csort);
   const size_t wlds = scan_lds_bytes(Cs, Csort, c->Wd, c->vm);
@@ -899,7 +901,7 @@ void run_fp64_regions(am_ctx* c, int lvl_first, int first, int count, const int*
                            c->pfx.dev, io, rid0, (const int*)near.cnt, (const int*)near.slots,
                            (const double*)c->teq.p, 1);
       HIPCHK(hipGetLastError());
-      t.scanned_host += n;
+      if (!lvl) t.scanned_host += n;   // (launched ahead: n is a bound, march_levels counts)
       continue;
     }
     const SlotList left{c->tcnt.p + 1, c->tslots.p + lcap, c->acc};
@@ -1059,6 +1061,7 @@ LevelsDone march_levels(am_ctx* c, long long first, long long count, int mode, F
     if (ahead && !launched)
       for (int d = 1; d <= c->pfx.dev.nd; ++d) c->pfx.ub[d] -= B;
     if (launched) {
+      if (mode == 0 || (mode == 1 && !ray64_form(c))) t.scanned_host += added;
       cur = next;
       cur.n = (size_t)added * c->vm;
       cur.R0 = (int)before;
