@@ -9,7 +9,7 @@ Two shapes are chosen per network shape (widest hidden layer, depth):
   walk leaves undecided (a block-stride loop over a count the device holds).
 
 ``tune()`` marches the given workload once per candidate, reads the kernel time
-of the stage each shape affects from the engine's HIP-event counters, checks
+of the stage each shape affects from the engine's stage counters, checks
 that every candidate gives the same topology fingerprint (the shapes must not
 change the result), and stores the fastest in ``tuning.json`` beside this file.
 ``Engine`` and ``BatchEngine`` apply the stored shape of the nearest network

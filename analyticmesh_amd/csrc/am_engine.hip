@@ -229,7 +229,7 @@ struct am_ctx {
 
   // tiled FP64 chain (nets without skips, layers up to AM_CHAIN_MAXW wide)
   bool tile_ok = false;
-  bool chain_mfma = true;     // the certified forms' FP64 chain on the matrix cores ("chain_mfma")
+  bool chain_mfma = true;     // the FP64 ray walk's wider plane bound ("chain_mfma")
   DevBuf<double> tplanes, teq;
   // planes shared by activation prefix (am_prefix.h)
   PrefixStore pfx;
@@ -531,9 +531,10 @@ struct Fp64Counts {
 // Checked FP64 ray walk: planes are exact FP64, so eps only covers the walk's
 // own rounding (the vertex solve's share is added per system).
 const WalkParams kRay64{1e-13f, 1e-12f, 1e6f};
-// The same walk on planes from the matrix-core chain (another summation
-// order: up to a few 1e-14 of a plane's largest coefficient from the
-// sequential-fma planes on the 4x256 net); the bound keeps a margin of 10x.
+// The default ("chain_mfma" 1): ten times that bound.  It was set for planes
+// summed in another order (a few 1e-14 of their largest coefficient away); the
+// planes are the canonical ones now, and the bound stays so that the same regions
+// go on to the scan.
 const WalkParams kRay64Mf{1e-12f, 1e-11f, 1e6f};
 
 // planes past hidden layer 1 (the walk rebuilds layer 1's) and the mask

@@ -26,10 +26,9 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
 PEAK_TFLOPS = {"fp32": 157.3, "bf16x3": 2516.6 / 3.0, "fp64": 78.6, "fp64ray": 78.6}
-GEMM_KERNEL = {"fp32": "k_gemm<0>", "bf16x3": "k_gemm<1>", "fp64ray": "k_chain_tile_mfma", "fp64": "k_chain_tile_fp64"}
-# the FP64 chain of the certified forms runs on the matrix cores; the bit-exact FP64 form's on VALU
-CHAIN_KERNEL = {"fp32": "k_chain_tile_mfma", "bf16x3": "k_chain_tile_mfma", "fp64ray": "k_chain_tile_mfma",
-                "fp64": "k_chain_tile_fp64"}
+# the reduced FP32 planes; every other form's come from the FP64 layer products shared by activation prefix
+GEMM_KERNEL = "k_gemm<0>"
+CHAIN_KERNEL = "k_layer"
 
 
 def log(*a):
@@ -171,6 +170,22 @@ def traffic_per_launch(kernel, regions, launches):
     regions per launch."""
     b = profile_value("hbm_traffic.txt", kernel)
     return None if b is None else round(b * regions / max(1.0, launches), 1)
+
+
+def prefix_flops(spec, masks):
+    """FLOPs of the hidden planes and the face plane when regions with the same activations up to
+    layer l share the planes of layer l + 1: 8 n_out n_in per activation prefix, 8 n_D per region."""
+    n = list(spec.nodes)
+    m = np.ascontiguousarray(masks).view(np.uint32).reshape(len(masks), -1)
+    total, off = 8.0 * n[-2] * len(m), 0
+    for li in range(1, len(n) - 2):
+        off += n[li]
+        words = m[:, :(off + 31) // 32].copy()
+        if off % 32:
+            words[:, -1] &= np.uint32((1 << (off % 32)) - 1)
+        rows = np.ascontiguousarray(words).view(np.dtype((np.void, words.shape[1] * 4))).ravel()
+        total += 8.0 * n[li + 1] * n[li] * len(np.unique(rows))
+    return total
 
 
 VALU_PEAK_G = 256 * 4 * 2.4 / 4   # G wave64 VALU instructions/s: one per SIMD every 4 cycles at 2.4 GHz
@@ -316,43 +331,43 @@ def main():
     head = "fp32" if out.get("fp32") else next(f for f in forms if out.get(f))
     h = out[head]
     st = h["stats"]
-    # plane kernels of the head form: its own GEMM (reduced forms) and the FP64
-    # chain (every region in every form: the reduced forms re-solve the
-    # vertices of the regions they decide from FP64 planes and re-decide the
-    # others on them); the roofline line is the one that took longer
+    # plane kernels of the head form: the FP32 GEMM (every region), and the FP64 layer products, whose
+    # planes the regions with the same activations up to a layer share (in the FP32 form for the
+    # regions its walk left to FP64: no FLOP count there); the roofline line is the one that took longer
     kernels = []
-    if head in ("fp32", "bf16x3"):
-        kernels.append(dict(kernel=GEMM_KERNEL[head], ms=float(st[3]), regions=h["regions"], peak=PEAK_TFLOPS[head],
-                            launches=max(1.0, float(st[11]))))
+    if head == "fp32":
+        kernels.append(dict(kernel=GEMM_KERNEL, ms=float(st[3]), regions=h["regions"], peak=PEAK_TFLOPS[head],
+                            launches=max(1.0, float(st[11])), flops=flops_region * h["regions"]))
         if float(st[13]) > 0:
-            # the FP64 chain runs on the regions the reduced walk left to FP64 (undecided, or
-            # decided with vertices re-solved from FP64 planes)
-            kernels.append(dict(kernel=CHAIN_KERNEL[head], ms=float(st[13]), regions=int(st[9]) + int(st[33]),
-                                peak=PEAK_TFLOPS["fp64"], launches=max(1.0, float(st[31]))))
+            kernels.append(dict(kernel=CHAIN_KERNEL, ms=float(st[13]), regions=int(st[9]) + int(st[33]),
+                                peak=PEAK_TFLOPS["fp64"], launches=max(1.0, float(st[31])), flops=None))
     else:
-        kernels.append(dict(kernel=CHAIN_KERNEL[head.split("+")[0]], ms=float(st[13]), regions=h["regions"],
-                            peak=PEAK_TFLOPS["fp64"], launches=max(1.0, float(st[31]))))
+        kernels.append(dict(kernel=CHAIN_KERNEL, ms=float(st[13]), regions=h["regions"], peak=PEAK_TFLOPS["fp64"],
+                            launches=max(1.0, float(st[31])), flops=prefix_flops(spec, h["res"].masks)))
     lines = []
     for k in kernels:
-        ach = flops_region * k["regions"] / (k["ms"] / 1e3) / 1e12 if k["ms"] > 0 else 0.0
-        lines.append({"bound": "fp64 valu" if k["kernel"] == "k_chain_tile_fp64" else "mfma", "kernel": k["kernel"],
-                      "achieved": round(ach, 3), "peak": k["peak"], "unit": "TFLOP/s",
-                      "frac": round(ach / k["peak"], 5),
+        ach = k["flops"] / (k["ms"] / 1e3) / 1e12 if k["flops"] and k["ms"] > 0 else None
+        lines.append({"bound": "mfma", "kernel": k["kernel"],
+                      "achieved": None if ach is None else round(ach, 3), "peak": k["peak"], "unit": "TFLOP/s",
+                      "frac": None if ach is None else round(ach / k["peak"], 5),
                       "traffic": traffic_per_launch(k["kernel"], k["regions"], k["launches"]),
                       "kernel_ms": round(k["ms"], 3), "launches": int(k["launches"]),
                       "avg_launch_ms": round(k["ms"] / k["launches"], 4),
-                      "regions": k["regions"], "flops_per_region": flops_region})
+                      "regions": k["regions"],
+                      "flops_per_region": None if k["flops"] is None else round(k["flops"] / k["regions"], 1)})
     lines.sort(key=lambda r: -r["kernel_ms"])
     roofline = lines[0]
-    # walk kernels of the head form: the reduced-precision walk over every region, the FP64 ray
-    # walk over the regions it left undecided (every region in the fp64ray form)
+    # walk kernels of the head form: the FP32 near walk over every region and the FP64 one over the
+    # regions it left undecided; the FP64 near walk over every region in the other forms
     walks = []
     nlev = max(1.0, float(st[6]))
-    if head in ("fp32", "bf16x3"):
-        walks.append(walk_roofline("k_walk_ray_f32", float(st[4]), h["regions"], nlev))
-        walks.append(walk_roofline("k_walk_ray64<4>", float(st[28]), int(st[9]), float(st[31])))
-    elif head == "fp64ray":
-        walks.append(walk_roofline("k_walk_ray64<4>", float(st[28]), h["regions"], float(st[31])))
+    if head == "fp32":
+        walks.append(walk_roofline("k_near_f32", float(st[4]), h["regions"], nlev))
+        walks.append(walk_roofline("k_near64<false,false>", float(st[28]), int(st[9]), float(st[31])))
+    elif head == "fp64":
+        walks.append(walk_roofline("k_near64<true,false>", float(st[14]), h["regions"], nlev))
+    else:
+        walks.append(walk_roofline("k_near64<false,false>", float(st[28]), h["regions"], float(st[31])))
     walks = [w for w in walks if w]
 
     topo = {}

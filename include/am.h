@@ -161,21 +161,19 @@ am_status am_topology_fingerprint(am_ctx* ctx, unsigned long long* out5);
  * "adjoint_tiled" (1 default: the
  * adjoint on the tiled FP64 chain and GEMMs; 0 one kernel per region),
  * "adjoint_mfma" (1 default: those GEMMs on the FP64 matrix cores; 0 VALU),
- * "chain_mfma" (1 default: the FP64 plane chain of the forms that certify
- * their decisions -- the FP64 ray walk, the reduced forms' FP64 redo, the
- * batch engine's ray walk -- runs on the FP64 matrix cores, planes equal to
- * the sequential-fma chain's up to the rounding of another summation order,
- * same topology; 0: the sequential-fma chain everywhere.  The bit-exact FP64
- * form always uses the sequential-fma chain). */
+ * "chain_mfma" (1 default: the FP64 ray walk bounds its planes' error at 1e-12 of
+ * their largest coefficient, 0: at 1e-13; the FP64 planes themselves are the
+ * canonical sequential-fma ones, on the matrix cores, in every form). */
 am_status am_set_option(am_ctx* ctx, const char* key, long long value);
 
-/* Timings and counters of the last am_run/am_combine; see AM_STAT_* indices. */
+/* Timings and counters of the last am_run/am_combine; see AM_STAT_* indices.  Stage times are
+ * taken on the device (the Newton step's by events). */
 #define AM_STAT_RUN_MS 0        /* am_run wall time, seeds in -> records in device memory */
-#define AM_STAT_REGION_MS 1     /* region kernels (HIP events) */
-#define AM_STAT_INSERT_MS 2     /* visited-set insertion + compaction (HIP events) */
-#define AM_STAT_GEMM_MS 3       /* plane GEMM kernels (HIP events; reduced precisions) */
-#define AM_STAT_WALK_MS 4       /* walk kernels after the GEMM (HIP events; reduced precisions) */
-#define AM_STAT_REDO_MS 5       /* FP64 re-decision kernels (HIP events) */
+#define AM_STAT_REGION_MS 1     /* region kernels */
+#define AM_STAT_INSERT_MS 2     /* visited-set insertion + compaction */
+#define AM_STAT_GEMM_MS 3       /* plane GEMM kernels (the FP32 form; the plane stage of the others) */
+#define AM_STAT_WALK_MS 4       /* walk kernels after the GEMM (the FP32 form's; the FP64 ones of the others) */
+#define AM_STAT_REDO_MS 5       /* FP64 re-decision kernels */
 #define AM_STAT_LEVELS 6
 #define AM_STAT_REGIONS 7
 #define AM_STAT_CANDIDATES 8
@@ -183,24 +181,24 @@ am_status am_set_option(am_ctx* ctx, const char* key, long long value);
 #define AM_STAT_COMBINE_MS 10
 #define AM_STAT_REGION_LAUNCHES 11
 #define AM_STAT_ADJOINT_MS 12   /* am_adjoint kernels (wall time) */
-#define AM_STAT_CHAIN64_MS 13   /* FP64 tiled plane chain, all launches (HIP events) */
-#define AM_STAT_WALK64_MS 14    /* FP64 walk after the tiled chain, all launches (HIP events) */
+#define AM_STAT_CHAIN64_MS 13   /* FP64 tiled plane chain, all launches */
+#define AM_STAT_WALK64_MS 14    /* FP64 walk after the tiled chain, all launches */
 #define AM_STAT_SETUP_MS 15     /* am_run set-up: weight uploads and operand layouts (wall time) */
 #define AM_STAT_WHY0 16         /* 16..27: regions the reduced-precision walk left to FP64, per reason:
                                    seed shot, start edge, plane already in polygon, sign within bound,
                                    proposed vertex infeasible, ill-conditioned system, turn within bound,
                                    vertex cap, open edge, orientation within bound, candidate scan,
                                    same vertex */
-#define AM_STAT_RAY64_MS 28     /* FP64 checked ray walk (HIP events) */
+#define AM_STAT_RAY64_MS 28     /* FP64 checked ray walk */
 #define AM_STAT_SCAN64_REGIONS 29 /* regions decided by the FP64 candidate scan */
 #define AM_STAT_RAY64_UNDECIDED 30 /* regions the FP64 ray walk left to the scan */
 #define AM_STAT_CHAIN64_LAUNCHES 31 /* launches of the FP64 tiled chain */
-#define AM_STAT_VERT64_MS 32    /* FP64 vertex re-solve of regions the reduced-precision walk decided (HIP events) */
+#define AM_STAT_VERT64_MS 32    /* FP64 vertex re-solve of regions the reduced-precision walk decided */
 #define AM_STAT_VERT64_REGIONS 33 /* regions whose vertices were re-solved from FP64 planes */
 #define AM_STAT_FP64_ONLY 34    /* 1: a reduced form marched on FP64 planes alone (skips, layers over 256 wide, every vertex re-solved) */
 #define AM_STAT_HOST_WAITS 35   /* host waits on the device during the run */
 #define AM_STAT_GRAPH_LAUNCHES 36 /* levels launched as one captured graph ("graph_levels") */
-#define AM_STAT_NEWTON_MS 37    /* FP32 form: FP64 Newton step of the vertices (HIP events, with its vertex dedup) */
+#define AM_STAT_NEWTON_MS 37    /* FP32 form: FP64 Newton step of the vertices (with its vertex dedup) */
 #define AM_STAT_NEWTON_VERTICES 38 /* vertices it refined */
 #define AM_STAT_COUNT 39
 am_status am_get_stats(am_ctx* ctx, double* out, int n);
