@@ -2264,8 +2264,7 @@ am_status am_planes(am_ctx* c, const uint32_t* masks, int n, float* planes, floa
     HIPCHK(hipMemcpy(he.data(), e.p, he.size() * 4, hipMemcpyDeviceToHost));
     for (int r = 0; r < n; ++r) {
       for (int q = 0; q < 4; ++q) {
-        std::memcpy(planes + ((size_t)r * 4 + q) * c->C, hp.data() + ((size_t)r * AM_PCOMP + q) * Cs,
-                    (size_t)c->C * 4);
+        for (int g = 0; g < c->C; ++g) planes[((size_t)r * 4 + q) * c->C + g] = hp[(size_t)r * AM_PCOMP * Cs + 4 * (size_t)g + q];
         eq[(size_t)r * 4 + q] = he[(size_t)r * AM_EQS + q];
       }
       if (sigma && c->fast.dev.sig) {

@@ -8,17 +8,18 @@
 // middle of an edge of the neighbour it was found from); the up to 64 nearest
 // become one constraint per lane, and the walk runs on those alone.  Every
 // excluded plane has p inside it by at least the radius r, so it holds at any
-// vertex within r/2 of p by a margin above the rounding of its evaluation
+// vertex within 0.9 r of p by a margin above the rounding of its evaluation
 // (near_covers): the walk takes a vertex only there.  A region it cannot settle
-// (a seed, a vertex beyond r/2, a turn or sign that is not certain) goes on the
+// (a seed, a vertex beyond that, a turn or sign that is not certain) goes on the
 // list of the walks over all constraints, so the near walk never decides
 // otherwise than they do.
 //
 // What bounds it: VALU issue and the planes' read (32 bytes per constraint).
 // The walks over all constraints read every plane once per vertex, from LDS
 // that leaves 4 to 6 regions per CU.  4x256 network, 1,022,340 regions, one
-// MI355X: candidate scan 75.3 -> 9.2 ms, FP64 ray walk 21.4 -> 9.9 ms, FP32 ray
-// walk 17.5 -> 10.8 ms; the trained 4x60 network (248,231 regions) 11.6 -> 3.8 ms.
+// MI355X: candidate scan 75.3 -> 9.8 ms, FP64 ray walk 21.4 -> 9.3 ms, FP32 ray
+// walk 17.5 -> 10.9 ms; the trained 4x60 network (248,231 regions) 11.6 -> 3.6 ms.
+// In small levels it is one region's serial chain: 21 us a level of 140 regions.
 #pragma once
 #include "am_device.h"
 #include "am_kernels.h"
