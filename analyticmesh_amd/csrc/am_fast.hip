@@ -511,7 +511,7 @@ __global__ __launch_bounds__(64 * NW, 24 / NW) void k_walk_ray_f32(NetDev net, R
 // One region's FP32 planes and error estimates as the face kernel stores them: 16
 // bytes a plane, so that the near constraints, picked after the pass over all, touch
 // one sector each instead of four (they made it read the record twice from memory:
-// 48 KB a region; 4x256 march, walk 11.6 -> 10.9 ms, whole call 48.2 -> 46.9).
+// 48 KB a region, now 40; 4x256 march, walk 11.6 -> 10.9 ms, whole call 48.2 -> 46.9).
 struct FacePlanes {
   const float* src;
   int Cs, C;
