@@ -166,12 +166,15 @@ __device__ __forceinline__ void raw_plane64(const NetDev& net, const uint32_t* m
 // out: G of the output plane, the sums as a list per distinct tight hidden
 // neuron, and the masked inputs P.  The pull-back through the weights is left
 // to the GEMMs over all regions, and k_adj_scatter adds the lists to it.
+// Bound by memory (the planes in, P out) as far as enough waves are in flight: the
+// sums take LDS per list entry, not per neuron (18 KB at 512 neurons, so 6 regions a
+// CU; now 3 KB, 10): 241,000 regions of a 4x128 network 2.67 -> 1.53 ms.
 __global__ __launch_bounds__(64) void k_adjoint_direct(NetDev net, AdjointIO io, const double* planes,
                                                        const double* eqb, int Cs) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   const int L = net.L;
-  double* G = reinterpret_cast<double*>(smem_raw);   // [4][L]
-  int* mark = reinterpret_cast<int*>(G + 4 * L);      // [L]: neuron already in the list
+  double* G = reinterpret_cast<double*>(smem_raw);               // [2 vm][4] sums, one entry per neuron of the list
+  int* mark = reinterpret_cast<int*>(G + (size_t)8 * io.vm);      // [L]: its entry + 1, 0: not in the list
   __shared__ int s_list[2 * AM_VM_MAX];
   __shared__ int s_nd;
   __shared__ double s_c[AM_VM_MAX][12];
@@ -186,7 +189,7 @@ __global__ __launch_bounds__(64) void k_adjoint_direct(NetDev net, AdjointIO io,
   const int nv = io.info[(size_t)r * AM_INFO_STRIDE + 2];
   const uint32_t* mask = io.reg_mask + (size_t)r * net.Wd;
   const double* src = planes + (size_t)b * 4 * Cs;
-  for (int g = lane; g < 4 * L; g += 64) G[g] = 0.0;
+  for (int g = lane; g < 8 * vm; g += 64) G[g] = 0.0;
   for (int g = lane; g < L; g += 64) mark[g] = 0;
   const int item0 = (int)(io.item_off[r] & 0xffffffffu);
   const bool mine = lane < vm && lane < nv && nv >= 3 && io.vfirst[item0 + lane];
@@ -225,13 +228,16 @@ __global__ __launch_bounds__(64) void k_adjoint_direct(NetDev net, AdjointIO io,
     for (int k = 0; k < nv && k < vm; ++k) {
       if (!s_own[k]) continue;
       const int lo = s_lohi[k][0], hi = s_lohi[k][1];
-      if (lo < L) {
-        for (int c = 0; c < 4; ++c) G[c * L + lo] -= s_c[k][c];
-        if (!mark[lo]) { mark[lo] = 1; s_list[nd++] = lo; }
-      }
-      if (hi < L) {
-        for (int c = 0; c < 4; ++c) G[c * L + hi] -= s_c[k][4 + c];
-        if (!mark[hi]) { mark[hi] = 1; s_list[nd++] = hi; }
+      for (int side = 0; side < 2; ++side) {
+        const int g = side ? hi : lo;
+        if (g >= L) continue;
+        int e = mark[g] - 1;
+        if (e < 0) {
+          e = nd++;
+          mark[g] = nd;
+          s_list[e] = g;
+        }
+        for (int c = 0; c < 4; ++c) G[e * 4 + c] -= s_c[k][4 * side + c];
       }
       for (int c = 0; c < 4; ++c) ge[c] -= s_c[k][8 + c];
     }
@@ -247,7 +253,7 @@ __global__ __launch_bounds__(64) void k_adjoint_direct(NetDev net, AdjointIO io,
   for (int j = lane; j < nd; j += 64) {
     const int g = s_list[j];
     io.dg[(size_t)b * io.dcap + j] = g;
-    for (int c = 0; c < 4; ++c) io.dv[((size_t)b * io.dcap + j) * 4 + c] = G[c * L + g];
+    for (int c = 0; c < 4; ++c) io.dv[((size_t)b * io.dcap + j) * 4 + c] = G[j * 4 + c];
   }
   // masked inputs of linear layers 1..D (zero for a region owning no vertex:
   // its G rows are zero)
@@ -451,15 +457,18 @@ __global__ void k_adj_scatter(const int* dn, const int* dg, const double* dv, in
 
 // part[y][j] = sum over the 256 regions b of block y of G[b][qsel][j]: 64
 // columns per block, four partial sums per column added in LDS in a fixed
-// order.  k_slice_sum adds the blocks' partials.
+// order, 16 loads in flight (21.5 -> 9 us a layer of 128).  k_slice_sum adds the
+// blocks' partials.
 __global__ __launch_bounds__(256) void k_col_sum(const double* G, int count, int M, int qsel, double* part) {
   __shared__ double ps[4][64];
   const int jx = threadIdx.x & 63, by = threadIdx.x >> 6;
   const int j = blockIdx.x * 64 + jx;
   const int b0 = blockIdx.y * 256, b1 = min(count, b0 + 256);
   double acc = 0.0;
-  if (j < M)
+  if (j < M) {
+#pragma unroll 16
     for (int b = b0 + by; b < b1; b += 4) acc += G[((size_t)b * 4 + qsel) * M + j];
+  }
   ps[by][jx] = acc;
   __syncthreads();
   if (by == 0 && j < M) part[(size_t)blockIdx.y * M + j] = ((ps[0][jx] + ps[1][jx]) + ps[2][jx]) + ps[3][jx];
@@ -484,22 +493,26 @@ __global__ __launch_bounds__(256) void k_col_sum4(const double* G, int count, in
 }
 
 // out[i * ostride] += the sum over slices z < nslice of part[z][i] (slice z at
-// part + z * sstride), i < n: eight running sums over z = u mod 8, u = 0..7,
-// then added pairwise in a fixed order (the loads of eight slices are in
-// flight at once; the result does not depend on timing).
+// part + z * sstride), i < n: eight running sums over z = u mod 8, u = 0..7, one
+// thread each, then added pairwise in a fixed order (the result does not depend on
+// timing).  32 outputs a block: with all eight sums in one thread the 16,384
+// outputs of a 128 x 128 layer filled 64 blocks, 8.4 us a launch.
 __global__ __launch_bounds__(256) void k_slice_sum(const double* part, int nslice, size_t sstride, int n, double* out,
                                                    int ostride) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  double a[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-  int z = 0;
-  for (; z + 8 <= nslice; z += 8) {
-#pragma unroll
-    for (int u = 0; u < 8; ++u) a[u] += part[(size_t)(z + u) * sstride + i];
+  __shared__ double a[8][32];
+  const int x = threadIdx.x & 31, u = threadIdx.x >> 5;
+  const int i = blockIdx.x * 32 + x;
+  double s = 0.0;
+  if (i < n) {
+#pragma unroll 8
+    for (int z = u; z < nslice; z += 8) s += part[(size_t)z * sstride + i];
   }
-  for (int u = 0; z + u < nslice; ++u) a[u] += part[(size_t)(z + u) * sstride + i];
-  const double s = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
-  out[(size_t)i * ostride] = out[(size_t)i * ostride] + s;
+  a[u][x] = s;
+  __syncthreads();
+  if (u == 0 && i < n) {
+    const double t = ((a[0][x] + a[1][x]) + (a[2][x] + a[3][x])) + ((a[4][x] + a[5][x]) + (a[6][x] + a[7][x]));
+    out[(size_t)i * ostride] = out[(size_t)i * ostride] + t;
+  }
 }
 
 }  // namespace am

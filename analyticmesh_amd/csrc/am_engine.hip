@@ -2355,7 +2355,7 @@ am_status am_adjoint(am_ctx* c, const void* grad_vertices, int dtype, void* cons
       ensure(c->adj_dn, (size_t)chunk, false, st);
       ensure(c->adj_dg, (size_t)chunk * dcap, false, st);
       ensure(c->adj_dv, (size_t)chunk * dcap * 4, false, st);
-      lds = (size_t)4 * c->L * 8 + (size_t)c->L * 4;
+      lds = (size_t)8 * c->vm * 8 + (size_t)c->L * 4;
       if (lds > c->max_lds) throw CapErr{"network too wide for the adjoint kernel's LDS"};
       if (lds > 65536)
         HIPCHK(hipFuncSetAttribute((const void*)k_adjoint_direct, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -2442,7 +2442,7 @@ am_status am_adjoint(am_ctx* c, const void* grad_vertices, int dtype, void* cons
       const int K = cnt * 4, ny = (cnt + 255) / 256;
       double* part = c->adj_part.p;
       auto slice_sum = [&](const double* src, int nslice, size_t sstride, int n, double* out, int ostride) {
-        hipLaunchKernelGGL(k_slice_sum, dim3((n + 255) / 256), dim3(256), 0, st, src, nslice, sstride, n, out,
+        hipLaunchKernelGGL(k_slice_sum, dim3((n + 31) / 32), dim3(256), 0, st, src, nslice, sstride, n, out,
                            ostride);
       };
       for (int li = 1; li < nl; ++li) {

@@ -3,8 +3,8 @@
 // A context (one call of a training loop makes and drops one) needs some 60
 // buffers, grown as its march grows: hipMalloc takes 0.1 to 0.4 ms whatever the
 // size, hipFree as much and a wait for the device, pinned memory more: the
-// 4x128 training step, which makes a context a step, took 51 ms and takes 32 so.  Freed blocks therefore wait
-// here for the next context: bounded (4 GiB of device memory, 256 MiB pinned),
+// 4x128 training step, which makes a context a step, took 51 ms and takes 32
+// so.  Freed blocks therefore wait here for the next context: bounded (4 GiB of device memory, 256 MiB pinned),
 // given back to the device when eight contexts have ended without using them,
 // when the bound is passed (oldest first), or when an allocation fails.
 // A block is given only when no work on it is pending (its stream has been
