@@ -948,7 +948,7 @@ int run_reduced_level(am_ctx* c, int first, int count, Fp64Counts& t, const int2
   fl.lvl_bound = lvl_bound;
   const RedoList redo{c->redo_ids.p, c->redo_cnt.p, c->redo_state.p};
   FastTimes ft{};
-  fast_level(c->fast, c->fbuf, c->net, fl, c->stream, c->clock, ft, c->rflags.p, c->acc + 1 + AM_WHY_COUNT, redo, true);
+  fast_level(c->fast, c->fbuf, c->net, fl, c->stream, c->clock, ft, c->rflags.p, c->acc + 1 + AM_WHY_COUNT, redo);
   run_fp64_regions(c, first, first, count, c->redo_ids.p, 2, t, -1, c->redo_cnt.p, lvl, lvl_bound);
   return ft.launches;
 }

@@ -105,19 +105,18 @@ size_t redo_state_words(int count);
 // ones to acc[0], their reasons to acc[1 + w] and the AM_VERT64 ones to
 // acc[1 + AM_WHY_COUNT] on the device; nothing here waits.
 // Kernel times go to `clk` (T_GEMM, T_WALK).
-// With `prepared`, fast_level_prepare(f, b, net, lvl.count) has run before
-// (then fast_level only enqueues launches: it can be captured into a graph).
+// fast_level_prepare(f, b, net, lvl.count) has run before; here launches are only
+// enqueued (they can be captured into a graph).
 void fast_level(FastNet& f, FastBuffers& b, const NetDev& net, const FastLevel& lvl, hipStream_t st,
-                StageClock* clk, FastTimes& t, unsigned* flags, int* acc, const RedoList& redo,
-                bool prepared = false);
-// Buffers and launch attributes of fast_level for a level of `count` regions.
+                StageClock* clk, FastTimes& t, unsigned* flags, int* acc, const RedoList& redo);
 // Whether levels past the seeds can be launched ahead, and whether one of `count` regions fits the buffers.
 bool fast_ahead(const FastNet& f);
 bool fast_level_fits(const FastNet& f, const FastBuffers& b, int count);
+// Buffers and launch attributes of fast_level for a level of `count` regions.
 void fast_level_prepare(FastNet& f, FastBuffers& b, const NetDev& net, int count);
 // Planes of n given regions (their masks in `reg_mask`) with the prepared
-// reduced-precision form: planes [n][AM_PCOMP][Cs] f32 (x, y, z, c signed, then
-// each plane's error estimate sigma), eq [n][AM_EQS] f32 (x, y, z, c, sigma).
+// reduced-precision form: planes [n][AM_PCOMP * Cs] f32 ([Cs] x, y, z, c signed,
+// then [Cs] error estimates sigma), eq [n][AM_EQS] f32 (x, y, z, c, sigma).
 void fast_planes(FastNet& f, const uint32_t* reg_mask, int n, float* planes, float* eq, hipStream_t st);
 
 }  // namespace am

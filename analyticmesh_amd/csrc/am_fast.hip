@@ -850,11 +850,10 @@ void fast_level_prepare(FastNet& f, FastBuffers& b, const NetDev& net, int count
 }
 
 void fast_level(FastNet& f, FastBuffers& b, const NetDev& net, const FastLevel& lvl, hipStream_t st,
-                StageClock* clk, FastTimes& t, unsigned* flags, int* acc, const RedoList& redo, bool prepared) {
+                StageClock* clk, FastTimes& t, unsigned* flags, int* acc, const RedoList& redo) {
   const FastNetDev& d = f.dev;
   const int prec = f.precision == 1 ? 1 : 0;
   t.launches = 0;
-  if (!prepared) fast_level_prepare(f, b, net, lvl.count);
   const int CH = kLevelChunk;
   const int chunk = std::min(lvl.count, CH);
   float* planes = (float*)slot(b, S_PLANES, (size_t)chunk * AM_PCOMP * d.Cs * 4);
