@@ -2115,15 +2115,15 @@ struct Part {
   size_t bytes;
 };
 
-// Device arrays into the caller's.  Device, pinned or managed ones get them
-// straight from device memory.  Pageable ones: in chunks, each by one DMA into a
+// Device arrays into the caller's, once the work on st is done.  Device, pinned or
+// managed ones get them straight from device memory.  Pageable ones: in chunks, each by one DMA into a
 // pinned slot and then by one of eight host threads into the array, while the
 // next chunks are on their way (a plain copy into pageable memory stages through
 // small chunks and one host thread: about 10 GB/s, less into fresh pages; marching
 // eight networks and copying out their 188 MB of records takes 41 ms with it, 28 so).  A thread
 // owns two slots and refills one as soon as it has emptied it.
 void copy_out(am_ctx* c, const std::vector<Part>& all, hipStream_t st) {
-  std::vector<Part> parts;
+  std::vector<Part> parts, direct;
   size_t staged = 0;
   for (const Part& p : all) {
     if (!p.dst || !p.bytes) continue;
@@ -2131,8 +2131,20 @@ void copy_out(am_ctx* c, const std::vector<Part>& all, hipStream_t st) {
       parts.push_back(p);
       staged += p.bytes;
     } else {
-      HIPCHK(hipMemcpy(p.dst, p.src, p.bytes, hipMemcpyDefault));
+      direct.push_back(p);
     }
+  }
+  if (!direct.empty()) {
+    // behind the kernels on st that still write the sources (st need not wait for the
+    // null stream, nor that for st), and on the null stream, behind what the caller
+    // has queued there for its arrays
+    HIPCHK(hipStreamSynchronize(st));
+    hipError_t e = hipSuccess;
+    for (const Part& p : direct)
+      if (e == hipSuccess) e = hipMemcpyAsync(p.dst, p.src, p.bytes, hipMemcpyDefault, nullptr);
+    const hipError_t w = hipStreamSynchronize(nullptr);
+    if (e == hipSuccess) e = w;
+    if (e != hipSuccess) throw HipErr{e, "copy of the results into the caller's arrays"};
   }
   if (!staged) return;
   const size_t chunk = std::min<size_t>((size_t)2 << 20, std::max<size_t>((size_t)256 << 10, (staged / 16 + 4095) / 4096 * 4096));
