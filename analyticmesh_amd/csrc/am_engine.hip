@@ -15,7 +15,7 @@
 #include <thread>
 #include <climits>
 #include <cstdio>
-#include <cstring>
+#include <exception>
 #include <fstream>
 #include <string>
 #include <deque>
@@ -1127,6 +1127,18 @@ void upload_pad(am_ctx* c, DevBuf<double>& wdst, DevBuf<double>& bdst, const voi
   HIPCHK(hipGetLastError());
 }
 
+// When an exception leaves its scope, waits for the stream: a level launched ahead,
+// or a copy out of a caller's array, may still be under way, and the caller may give
+// the arrays back or run the context on another stream.
+struct DrainOnThrow {
+  hipStream_t st;
+  int n = std::uncaught_exceptions();
+  explicit DrainOnThrow(hipStream_t s) : st(s) {}
+  ~DrainOnThrow() {
+    if (std::uncaught_exceptions() > n) (void)hipStreamSynchronize(st);
+  }
+};
+
 am_status fail(am_ctx* c, am_status s, const std::string& m) {
   if (c) c->err = m;
   return s;
@@ -1532,6 +1544,7 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
       }
     c->stream = stream ? (hipStream_t)stream : c->own_stream;
     const hipStream_t st = c->stream;
+    const DrainOnThrow drain(st);
     const auto t0 = std::chrono::steady_clock::now();
     for (int i = 0; i < AM_STAT_COUNT; ++i) c->stats[i] = 0;
     c->has_run = false;
@@ -2675,6 +2688,7 @@ am_status am_batch_run(am_batch* b, const void* const* weights, const void* cons
     if (total_seeds > INT_MAX / 2) throw CapErr{"too many seeds"};
     c->stream = stream ? (hipStream_t)stream : c->own_stream;
     const hipStream_t st = c->stream;
+    const DrainOnThrow drain(st);
     const auto t0 = std::chrono::steady_clock::now();
     for (double& x : c->stats) x = 0;
     c->has_run = false;
