@@ -1692,7 +1692,7 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
     c->R = 0;
     c->table_cap = 0;
     grow_cands(c, (size_t)n_seeds);
-    hipLaunchKernelGGL(k_seeds, dim3(n_seeds), dim3(64), 0, st,
+    hipLaunchKernelGGL(k_seeds, dim3(std::min(n_seeds, 1 << 20)), dim3(64), 0, st,
                        (const uint8_t*)dev_view(c, states, (size_t)n_seeds * c->L, st),
                        dev_view(c, points, (size_t)n_seeds * 3 * esz, st), dtype == AM_DTYPE_F64 ? 1 : 0, n_seeds,
                        c->L, c->Wd, c->cand_mask.p, c->cand_hash.p, c->cand_point.p, c->cand_start.p);

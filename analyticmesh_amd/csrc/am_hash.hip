@@ -314,29 +314,32 @@ __global__ void k_hash_keys(const uint32_t* masks, int n, int Wd, uint64_t* out)
   if (c < n) out[c] = key_hash_sum(masks + (size_t)c * Wd, Wd);
 }
 
+// Blocks stride over the seeds: one each would pass 2^32 threads at 2^26 of them, and
+// the launch then covers what is left of the count modulo that.
 __global__ __launch_bounds__(64) void k_seeds(const uint8_t* states, const void* points, int f64, int n, int L, int Wd,
                                               uint32_t* mask, uint64_t* hash, double* point, int* start) {
-  const int s = blockIdx.x, lane = threadIdx.x;
-  if (s >= n) return;
-  uint64_t h = 0;
-  for (int w = 0; w < Wd; w += 2) {
-    const int g = 32 * w + lane;
-    const unsigned long long bal = __ballot(g < L && states[(size_t)s * L + g] != 0);
-    const uint32_t lo = (uint32_t)bal, hi = (uint32_t)(bal >> 32);
-    if (lane == 0) {
-      mask[(size_t)s * Wd + w] = lo;
-      if (w + 1 < Wd) mask[(size_t)s * Wd + w + 1] = hi;
+  const int lane = threadIdx.x;
+  for (long long s = blockIdx.x; s < n; s += gridDim.x) {
+    uint64_t h = 0;
+    for (int w = 0; w < Wd; w += 2) {
+      const int g = 32 * w + lane;
+      const unsigned long long bal = __ballot(g < L && states[(size_t)s * L + g] != 0);
+      const uint32_t lo = (uint32_t)bal, hi = (uint32_t)(bal >> 32);
+      if (lane == 0) {
+        mask[(size_t)s * Wd + w] = lo;
+        if (w + 1 < Wd) mask[(size_t)s * Wd + w + 1] = hi;
+      }
+      h += word_hash(lo, w);
+      if (w + 1 < Wd) h += word_hash(hi, w + 1);
     }
-    h += word_hash(lo, w);
-    if (w + 1 < Wd) h += word_hash(hi, w + 1);
+    if (lane == 0) {
+      hash[s] = h;
+      start[s] = -1;
+    }
+    if (lane < 3)
+      point[(size_t)s * 3 + lane] = f64 ? static_cast<const double*>(points)[(size_t)s * 3 + lane]
+                                        : (double)static_cast<const float*>(points)[(size_t)s * 3 + lane];
   }
-  if (lane == 0) {
-    hash[s] = h;
-    start[s] = -1;
-  }
-  if (lane < 3)
-    point[(size_t)s * 3 + lane] = f64 ? static_cast<const double*>(points)[(size_t)s * 3 + lane]
-                                      : (double)static_cast<const float*>(points)[(size_t)s * 3 + lane];
 }
 
 // Re-insert every region id into an empty (larger) table.
