@@ -428,15 +428,24 @@ __device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, 
       // settles it without the order or the vertex: with the condition numbers Kx =
       // |x| |pc| |eq| / |x . d| and Kv = |pr| |pc| |eq| / |pr . d| that is below 200 u Kx Kv (1 +
       // |v| + |t d|) per unit normal (1e-11 here is 90,000 u), and 1e-5 covers the
-      // FP32 arithmetic.  The others, few, take the scan's own expressions.
+      // FP32 arithmetic.  The others, few, take the scan's own expressions.  The planes
+      // of a network scaled by 2^k are all scaled by it, so a product of norms is taken
+      // in FP32 together with the quotient that undoes its scale (1e-11 |pc|^2 |eq|^2 |pr| on its
+      // own is 0 from 2^-23 on), and normals of 1e-15 or less settle nothing here.  (The
+      // instruction's square root, within an ulp: a rounded one takes 15 in its place.)
       const T apr = pr[0] * d[0] + pr[1] * d[1] + pr[2] * d[2], apq = pq[0] * d[0] + pq[1] * d[1] + pq[2] * d[2];
-      const float npr = __builtin_sqrtf((float)plane_nn(pr[0], pr[1], pr[2]));
-      const float npq = __builtin_sqrtf((float)plane_nn(pq[0], pq[1], pq[2]));
-      const float nce = __builtin_sqrtf((float)plane_nn(pc[0], pc[1], pc[2]) * (float)plane_nn(eq[0], eq[1], eq[2]));
+      const float nnr = (float)plane_nn(pr[0], pr[1], pr[2]), nnq = (float)plane_nn(pq[0], pq[1], pq[2]);
+      const float nnc = (float)plane_nn(pc[0], pc[1], pc[2]), nne = (float)plane_nn(eq[0], eq[1], eq[2]);
+      const float npr = __builtin_amdgcn_sqrtf(nnr), npq = __builtin_amdgcn_sqrtf(nnq);
+      const float nce = __builtin_amdgcn_sqrtf(nnc) * __builtin_amdgcn_sqrtf(nne);
       const float fr = (float)apr, fq = (float)apq, vq = (float)plane_eval(pq[0], pq[1], pq[2], pq[3], v);
-      const float dl = __builtin_sqrtf((float)plane_nn(d[0], d[1], d[2]));
+      const float ince = __builtin_amdgcn_rcpf(nce);
+      const float dx = (float)d[0] * ince, dy = (float)d[1] * ince, dz = (float)d[2] * ince;
+      const float dl = nce * __builtin_amdgcn_sqrtf(dx * dx + dy * dy + dz * dz);
       const float v1 = 1.f + (float)(absT(v[0]) + absT(v[1]) + absT(v[2]));
-      const float kv = 1e-11f * nce * nce * npr * __builtin_amdgcn_rcpf(fabsf(fr));
+      const float kv = fminf(fminf(nnr, nnq), fminf(nnc, nne)) > 1e-30f
+                           ? (1e-11f * nce) * ((nce * npr) * __builtin_amdgcn_rcpf(fabsf(fr)))
+                           : __builtin_inff();
       const int gw = index_of(rl);
       bool fail = false;
       each([&](const T* x, int h, int gi, T) {
@@ -448,9 +457,11 @@ __device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, 
         next.add(-sv, al, al > T(0), h);
         const T ax = fmaT(x[0], d[0], fmaT(x[1], d[1], x[2] * d[2]));
         const float ra = __builtin_amdgcn_rcpf((float)ax), t = -(float)sv * ra;
-        const float far = 1e-17f + kv * __builtin_sqrtf((float)nn) * fabsf(ra) * (v1 + fabsf(t) * dl);
+        const float fn = (float)nn;
+        const float far = 1e-17f + kv * (__builtin_amdgcn_sqrtf(fn) * fabsf(ra)) * (v1 + fabsf(t) * dl);
         const float tr = fr * t, tq = fq * t;
-        const bool passed = tr > npr * far || vq + tq > npq * far + 1e-5f * (fabsf(vq) + fabsf(tq));
+        const bool passed =
+            fn > 1e-30f && (tr > npr * far || vq + tq > npq * far + 1e-5f * (fabsf(vq) + fabsf(tq)));
         if (!passed && (!is_used(h) || (h == sl && ntab >= 3)) &&
             key_before(FULL ? order_key(x) : key, gi, order_key(pr), gw)) {
           T vt[3];
