@@ -507,12 +507,11 @@ int insert_level(am_ctx* c, size_t n, int* slot = nullptr) {
   return insert_finish(c, p);
 }
 
-size_t region_lds_bytes(const am_ctx* c, int& Cs, int& Csort) {
+// The candidate scan's plane stride and sort width.
+void scan_sizes(const am_ctx* c, int& Cs, int& Csort) {
   Cs = c->C;
   Csort = AM_TOPK;   // the walk's top-64 order lives in keys/order[0, 64)
   while (Csort < c->C) Csort <<= 1;
-  return (size_t)4 * Cs * sizeof(double) + (size_t)Csort * (sizeof(double) + sizeof(int)) +
-         (size_t)((c->C + 31) / 32) * 4 + (size_t)c->Wd * 4 + 64;
 }
 
 int chain_maxw(const am_ctx* c) {
@@ -841,7 +840,7 @@ void run_fp64_regions(am_ctx* c, int lvl_first, int first, int count, const int*
   // nets with skips or layers over 256 wide keep the candidate scan's records in every form
   if (mode == 1 && !ray64_form(c)) mode = 0;
   int Cs, Csort;
-  (void)region_lds_bytes(c, Cs, Csort);
+  scan_sizes(c, Cs, Csort);
   const size_t wlds = scan_lds_bytes(Cs, Csort, c->Wd, c->vm);
   const size_t rlds = ray64_lds_bytes(c);
   const size_t chunk = prefix_chunk(c);
@@ -1636,10 +1635,10 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
     n.flip = flip_insideout ? 1 : 0;
 
     int Cs, Csort;
-    const size_t lds = region_lds_bytes(c, Cs, Csort);
-    if (lds > c->max_lds)
-      throw CapErr{"network too wide for the FP64 region kernel's LDS (" + std::to_string(lds) + " bytes)"};
+    scan_sizes(c, Cs, Csort);
     const size_t slds = scan_lds_bytes(Cs, Csort, c->Wd, c->vm);
+    if (slds > c->max_lds)
+      throw CapErr{"network too wide for the FP64 candidate scan's LDS (" + std::to_string(slds) + " bytes)"};
     if (slds > 65536)
       HIPCHK(hipFuncSetAttribute((const void*)k_walk_fp64, hipFuncAttributeMaxDynamicSharedMemorySize, (int)slds));
     c->tile_ok = true;

@@ -568,11 +568,14 @@ template __global__ void k_near64<false, true>(NetDev, PrefixDev, RegionIO, int,
 
 // The listed regions (blocks stride over the list) on all constraints: with
 // `quick` the walk that reads the planes once per vertex, then, for seeds and
-// what that does not settle, the candidate scan.
+// what that does not settle, the candidate scan.  The planes' pointers lie where
+// the scan keeps its records, which it writes once the planes are in LDS (past
+// all of the other walk's scratch): 136 bytes more would leave no room for them at
+// the largest constraint counts.
 __global__ __launch_bounds__(64, 4) void k_walk_fp64(NetDev net, PrefixDev pf, RegionIO io, int rid0, const int* count,
                                                   const int* slots, const double* eqb, int quick) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  __shared__ gplanes s_bases[AM_MAX_LINEAR + 1];
+  gplanes* const bases = reinterpret_cast<gplanes*>(smem_raw + scan_lds_head(net.C, io.Csort, net.Wd));
   if (!quick) stage_mark(io.clk, T_SCAN64);
   const int lane = threadIdx.x;
   const int total = min(*count, io.count);
@@ -580,7 +583,7 @@ __global__ __launch_bounds__(64, 4) void k_walk_fp64(NetDev net, PrefixDev pf, R
     const int b = slots[i];
     const int rid = io.ids ? io.ids[b] : launch_first(io, rid0) + b;
     const int start = io.reg_start[rid];
-    prefix_bases(net, pf, b, s_bases, lane, 64);
+    prefix_bases(net, pf, b, bases, lane, 64);
     double p[3], eq[4];
     for (int q = 0; q < 3; ++q) p[q] = io.reg_point[(size_t)rid * 3 + q];
     for (int q = 0; q < 4; ++q) eq[q] = eqb[(size_t)b * 4 + q];
@@ -589,12 +592,12 @@ __global__ __launch_bounds__(64, 4) void k_walk_fp64(NetDev net, PrefixDev pf, R
       const NearLds<double> S = carve_near<double>(smem_raw, net.C, net.Wd, net.vm, false);
       for (int w = lane; w < net.Wd; w += 64) S.mask[w] = io.reg_mask[(size_t)rid * net.Wd + w];
       __syncthreads();
-      const PrefixPlanes P{net, s_bases, S.mask};
+      const PrefixPlanes P{net, bases, S.mask};
       const int done = near_walk<double, true, SET_ALL>(net, io, wp, rid, rid - level_first(io), P, S, eq, p, start);
       __syncthreads();
       if (done == NEAR_DONE) continue;
     }
-    scan_prefix_region(net, io, rid, s_bases, smem_raw, eq, p);
+    scan_prefix_region(net, io, rid, bases, smem_raw, eq, p);
   }
 }
 
