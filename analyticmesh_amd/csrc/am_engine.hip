@@ -1035,6 +1035,7 @@ LevelsDone march_levels(am_ctx* c, long long first, long long count, int mode, F
       insert_launch(c, cur);
     }
     InsertPlan next;
+    const long long faces = done.launches, chains = t.chain_launches;
     const bool ahead = count <= kAheadMax && ahead_fits(c, B, reduced);
     if (ahead) {
       PrefixStore& s = c->pfx;
@@ -1060,6 +1061,11 @@ LevelsDone march_levels(am_ctx* c, long long first, long long count, int mode, F
     launched = ahead && added <= B;
     if (ahead && !launched)
       for (int d = 1; d <= c->pfx.dev.nd; ++d) c->pfx.ub[d] -= B;
+    if (ahead && !(launched && added > 0)) {
+      // (nothing was there for those launches, or too much: they are not counted)
+      done.launches = faces;
+      t.chain_launches = chains;
+    }
     if (launched) {
       if (mode == 0 || (mode == 1 && !ray64_form(c))) t.scanned_host += added;
       cur = next;
