@@ -2589,6 +2589,11 @@ am_status am_destroy(am_ctx* c) {
   return AM_OK;
 }
 
+am_status am_trim_memory(void) {
+  MemPool::get().clear();
+  return AM_OK;
+}
+
 const char* am_last_error(const am_ctx* c) {
   if (!c) return g_create_error.c_str();
   return c->err.c_str();

@@ -6,7 +6,9 @@
 // 4x128 training step, which makes a context a step, took 51 ms and takes 32
 // so.  Freed blocks therefore wait here for the next context: bounded (4 GiB of device memory, 256 MiB pinned),
 // given back to the device when eight contexts have ended without using them,
-// when the bound is passed (oldest first), or when an allocation fails.
+// when the bound is passed (oldest first), when an allocation fails, or by
+// am_trim_memory().  Contexts that end are what ages them: the
+// blocks of a process's last ones stay until that call or the process's end.
 // A block is given only when no work on it is pending (its stream has been
 // waited for), so any stream may take it next.  Safe from several threads.
 #pragma once
@@ -14,6 +16,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <new>
 #include <utility>
 #include <vector>
 
@@ -87,27 +90,33 @@ struct MemPool {
   }
   // Nothing that uses the block may be pending.
   void give(int kind, void* p, size_t bytes, int dev) {
+    bool in = true;
     {
       std::lock_guard<std::mutex> lock(m);
-      kept[kind].push_back(Block{p, bytes, dev, epoch});
-      total[kind] += bytes;
+      try {
+        kept[kind].push_back(Block{p, bytes, dev, epoch});
+        total[kind] += bytes;
+      } catch (const std::bad_alloc&) {
+        in = false;
+      }
     }
+    if (!in) drop(kind, Block{p, bytes, dev, 0});
     trim(kind, bound(kind), -1);
   }
   // Frees kept blocks, oldest first, down to `most` bytes, and those given before epoch `since`.
   void trim(int kind, size_t most, long long since) {
-    std::vector<Block> out;
-    {
-      std::lock_guard<std::mutex> lock(m);
-      std::vector<Block>& k = kept[kind];
-      size_t i = 0;
-      while (i < k.size() && (total[kind] > most || k[i].epoch < since)) {
-        total[kind] -= k[i].bytes;
-        out.push_back(k[i++]);
+    for (;;) {
+      Block b;
+      {
+        std::lock_guard<std::mutex> lock(m);
+        std::vector<Block>& k = kept[kind];
+        if (k.empty() || !(total[kind] > most || k[0].epoch < since)) return;
+        b = k[0];
+        total[kind] -= b.bytes;
+        k.erase(k.begin());
       }
-      k.erase(k.begin(), k.begin() + i);
+      drop(kind, b);
     }
-    for (const Block& b : out) drop(kind, b);
   }
   // A context has ended.
   void age() {
@@ -117,6 +126,9 @@ struct MemPool {
       now = ++epoch;
     }
     for (int k = 0; k < MEM_KINDS; ++k) trim(k, bound(k), now - 8);
+  }
+  void clear() {
+    for (int k = 0; k < MEM_KINDS; ++k) trim(k, 0, -1);
   }
 };
 

@@ -281,6 +281,7 @@ PYBIND11_MODULE(_am, m) {
   m.attr("PREC_FP64_RAY") = AM_PREC_FP64_RAY;
   m.attr("DTYPE_F32") = AM_DTYPE_F32;
   m.attr("DTYPE_F64") = AM_DTYPE_F64;
+  m.def("trim_memory", []() { am_trim_memory(); }, py::call_guard<py::gil_scoped_release>());
   py::class_<Engine>(m, "Engine")
       .def(py::init<const std::vector<int>&, py::array_t<int, py::array::c_style | py::array::forcecast>, int, int>(),
            py::arg("nodes"), py::arg("arc_table"), py::arg("num_extra_constraints"), py::arg("precision"))

@@ -17,7 +17,7 @@ walk, leaving only undecided regions to the candidate scan (float64 tensors).
 import numpy as np
 import torch
 
-from .engine import Engine, MarchResult
+from .engine import Engine, MarchResult, trim_memory
 
 _S = {"engine": None, "float_type": "", "nodes": None, "arc": None, "E": 0, "result": None}
 
@@ -52,8 +52,7 @@ def Init(float_type, nodesnum, arc_table, num_extra_constraints):
     for row in arc_table.tolist():
         _check(1 + 2 * row[0] <= arc_table.size(1), "arc_table row declares more skips than it holds")
     _check(int(num_extra_constraints) >= 0, "num_extra_constraints >= 0")
-    if _S["engine"] is not None:
-        Destroy()
+    _drop()
     _S["engine"] = Engine(nodesnum, arc_table.tolist(), int(num_extra_constraints), precision=_PRECISION[float_type])
     _S["float_type"] = float_type
     _S["nodes"] = nodesnum
@@ -122,9 +121,17 @@ def ExportMesh(file_path, is_polymesh, is_float32):
     _S["result"].export_ply(file_path, bool(is_polymesh), bool(is_float32))
 
 
-def Destroy():
-    """backend/src/cuam_kernel.cu:153-179."""
+def _drop():
     _S.update(engine=None, float_type="", nodes=None, arc=None, E=0, result=None)
+
+
+def Destroy():
+    """backend/src/cuam_kernel.cu:153-179.  Frees: nothing is kept for a later ``Init`` (one that
+    replaces a live context takes that one's memory over instead)."""
+    had = _S["engine"] is not None
+    _drop()
+    if had:
+        trim_memory()
 
 
 def last_result():

@@ -31,6 +31,13 @@ def native():
     return _mod
 
 
+def trim_memory():
+    """Give the memory that ended engines have left for later ones back to the device and the system (up to
+    4 GiB of device memory and 256 MiB each of two kinds of pinned host memory stay otherwise).  An engine ends
+    when it and its results are gone."""
+    native().trim_memory()
+
+
 def _as_ptr(a):
     """Address of a torch tensor or numpy array (host or device)."""
     if hasattr(a, "data_ptr"):

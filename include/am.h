@@ -85,8 +85,19 @@ am_status am_combine_noalloc(am_ctx* ctx, double scale, const double* center3, d
  * binary little-endian PLY, polygons or fan triangles, float or double xyz. */
 am_status am_export_ply(am_ctx* ctx, const char* path, int is_polymesh, int is_float32);
 
-/* Replaces Destroy() (backend/src/cuam_kernel.cu:153-179). */
+/* Replaces Destroy() (backend/src/cuam_kernel.cu:153-179).  The context's memory
+ * stays in the process for the next context: up to 4 GiB of device memory and
+ * 256 MiB each of pinned and coherent host memory, of all ended contexts together
+ * (allocations of other libraries do not get at it).  Blocks go back when eight
+ * further contexts have ended without using them, when the engine itself runs
+ * short of memory, and with am_trim_memory. */
 am_status am_destroy(am_ctx* ctx);
+
+/* Gives everything that ended contexts have left back to the device and the system
+ * (no counterpart in the reference, whose Destroy frees).  Live contexts keep
+ * theirs, among it up to 4 GiB of constraint planes each that a later march reuses.
+ * Waits for the device; may be called from any thread, at any time. */
+am_status am_trim_memory(void);
 
 /* Message of the last failing call on ctx (or of a failed am_create when ctx is NULL). */
 const char* am_last_error(const am_ctx* ctx);
