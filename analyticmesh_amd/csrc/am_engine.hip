@@ -136,6 +136,7 @@ struct PrefixStore {
   size_t cap = 0;                          // table slots in use
   long long ub[AM_MAX_LINEAR + 1] = {0};   // upper bounds of the ids given per depth
   std::vector<char> reset;                 // per chunk of the planned level: start over first
+  long long restarts = 0;                  // times this run's table has started over
   PrefixDev dev{};
 };
 
@@ -668,6 +669,7 @@ void prefix_setup(am_ctx* c, const void* const* tms, int dtype) {
   prefix_table(c, std::max(cap, s.cap));
   prefix_clear(c);
   std::fill(s.ub, s.ub + AM_MAX_LINEAR + 1, 0);
+  s.restarts = 0;
 }
 
 // Storage for `ids` ids of every depth: more blocks where needed, cut from
@@ -690,9 +692,17 @@ bool prefix_blocks(am_ctx* c, const long long* ids, bool must) {
     size_t bytes = std::max<size_t>(want, std::min<size_t>(s.bytes, kPrefixBytes > s.bytes ? kPrefixBytes - s.bytes : 0));
     bool fits = s.bytes + want <= kPrefixBytes;
     if (fits && s.bytes + bytes > ((size_t)512 << 20)) {
-      // many contexts may share the device: leave a quarter of it free
-      size_t fr = 0, all = 0;
-      fits = hipMemGetInfo(&fr, &all) == hipSuccess && fr > all / 4 + bytes;
+      // many contexts may share the device: leave a quarter of it free (the blocks
+      // that ended contexts have left are given back before it counts as short)
+      auto room = [&]() {
+        size_t fr = 0, all = 0;
+        return hipMemGetInfo(&fr, &all) == hipSuccess && fr > all / 4 + bytes;
+      };
+      fits = room();
+      if (!fits) {
+        MemPool::get().trim(MEM_DEVICE, 0, -1);
+        fits = room();
+      }
     }
     if (!fits && !must) return false;
     if (!fits) bytes = want;
@@ -782,7 +792,10 @@ void prefix_plan(am_ctx* c, int count, size_t chunk) {
 void prefix_launch(am_ctx* c, size_t k, const int* ids, int first, int n, const int* dcount, int dbase,
                    const int2* lvl, int lvl_bound) {
   PrefixStore& s = c->pfx;
-  if (s.reset[k]) prefix_clear(c);
+  if (s.reset[k]) {
+    prefix_clear(c);
+    s.restarts += 1;
+  }
   s.dev.clk = c->clock;
   if (s.dev.nd == 0) return;
   PrefixRegions rg;
@@ -1841,6 +1854,7 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
     c->stats[AM_STAT_GRAPH_LAUNCHES] = c->graph_levels ? (double)levels : 0.0;
     c->stats[AM_STAT_NEWTON_MS] = T[T_NEWTON];
     c->stats[AM_STAT_NEWTON_VERTICES] = (double)newton_n;
+    c->stats[AM_STAT_PREFIX_RESTARTS] = (double)c->pfx.restarts;
     for (int w = 0; w < AM_WHY_COUNT && AM_STAT_WHY0 + w < AM_STAT_COUNT; ++w) c->stats[AM_STAT_WHY0 + w] = (double)why[w];
     c->has_run = true;
     return AM_OK;

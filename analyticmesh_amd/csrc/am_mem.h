@@ -6,8 +6,8 @@
 // 4x128 training step, which makes a context a step, took 51 ms and takes 32
 // so.  Freed blocks therefore wait here for the next context: bounded (4 GiB of device memory, 256 MiB pinned),
 // given back to the device when eight contexts have ended without using them,
-// when the bound is passed (oldest first), when an allocation fails, or by
-// am_trim_memory().  Contexts that end are what ages them: the
+// when the bound is passed (oldest first), when an allocation fails or the device is
+// short of memory, or by am_trim_memory().  Contexts that end are what ages them: the
 // blocks of a process's last ones stay until that call or the process's end.
 // A block is given only when no work on it is pending (its stream has been
 // waited for), so any stream may take it next.  Safe from several threads.

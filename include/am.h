@@ -211,7 +211,8 @@ am_status am_set_option(am_ctx* ctx, const char* key, long long value);
 #define AM_STAT_GRAPH_LAUNCHES 36 /* levels launched as one captured graph ("graph_levels") */
 #define AM_STAT_NEWTON_MS 37    /* FP32 form: FP64 Newton step of the vertices (with its vertex dedup) */
 #define AM_STAT_NEWTON_VERTICES 38 /* vertices it refined */
-#define AM_STAT_COUNT 39
+#define AM_STAT_PREFIX_RESTARTS 39 /* times the shared planes' storage was full and their table started over */
+#define AM_STAT_COUNT 40
 am_status am_get_stats(am_ctx* ctx, double* out, int n);
 
 /* ---- Many networks in one job (no counterpart in the reference, which marches

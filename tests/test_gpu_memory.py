@@ -1,4 +1,6 @@
-"""Memory of ended engines: kept for the next one, given back by trim_memory() and by the drop-in Destroy()."""
+"""Memory of ended engines: kept for the next one, given back by trim_memory() and by the drop-in Destroy(), not
+counted as used when the planes' storage grows on a nearly full device; and marches whose planes' table starts
+over again and again there give the same topology."""
 import gc
 
 import numpy as np
@@ -6,11 +8,12 @@ import pytest
 
 from _common import workload
 from analyticmesh_amd import configs
-from analyticmesh_amd.engine import march, trim_memory
+from analyticmesh_amd.engine import Engine, march, trim_memory
 
 pytestmark = pytest.mark.gpu
 
 MB = 1 << 20
+RESTARTS = 39   # AM_STAT_PREFIX_RESTARTS
 
 
 def _free():
@@ -73,3 +76,40 @@ def test_destroy_of_the_drop_in_frees():
     first, second = use(), use()      # (the first loads kernels)
     assert first[1] - second[0] > 256 * MB
     assert first[1] - second[1] < 16 * MB
+
+
+def test_planes_storage_on_a_nearly_full_device():
+    """The 4x256 network's planes take more than their storage holds.  With 2 GiB over the quarter that stays
+    free, and as much kept of ended engines, it is as large as with nothing kept; the marches agree."""
+    import torch
+    base = _base()
+    spec, pts, st = workload("deep")
+    args = ([np.asarray(w, np.float64) for w in spec.weights], [np.asarray(b, np.float64) for b in spec.biases], pts, st)
+
+    def run():
+        r = Engine(spec.nodes, precision="fp64ray").run(*args)
+        return r.fingerprint(), int(r.stats[RESTARTS])
+
+    print("[memory] free device", flush=True)
+    want, fewest = run()
+    assert fewest > 0
+    total = torch.cuda.mem_get_info()[1]
+    gc.collect()
+    trim_memory()
+    hold = torch.empty(_free() - total // 4 - 2048 * MB, dtype=torch.uint8, device="cuda")
+    try:
+        print("[memory] nothing kept", flush=True)
+        got, alone = run()
+        assert got == want and alone >= fewest
+        print("[memory] blocks kept", flush=True)
+        march(*workload("sphere"), table_log2=29)     # leaves a table of 2 GiB
+        gc.collect()
+        got, kept = run()
+        print(f"[memory] restarts: {fewest} on a free device, {alone} nearly full, {kept} with blocks kept", flush=True)
+        assert got == want and kept <= alone
+    finally:
+        del hold
+        torch.cuda.empty_cache()
+        gc.collect()
+        trim_memory()
+    assert abs(base - _free()) < 64 * MB
