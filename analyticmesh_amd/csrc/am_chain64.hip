@@ -60,8 +60,8 @@ __device__ __forceinline__ void load_planes64(const NetDev& net, const uint32_t*
 
 typedef double am_f64x4 __attribute__((ext_vector_type(4)));
 
-// The planes of one tile: regions r0 .. r0 + nreg - 1 of lv (ids[r0 + t] or
-// first + r0 + t), written at planes slots r0 + t.  io supplies the plane stride
+// The planes of one tile: regions first + r0 .. + nreg - 1 of lv, written at planes
+// slots r0 + t.  io supplies the plane stride
 // and the layer operands; maxw >= the network's layer widths (LDS layout).
 template <int NW>
 __device__ __forceinline__ void chain_tile(const NetDev& net, const ChainIO& io, const ChainLevel& lv, int r0, int nreg,
@@ -77,7 +77,7 @@ __device__ __forceinline__ void chain_tile(const NetDev& net, const ChainIO& io,
   const int Wd = net.Wd, Cs = io.Cs;
   for (int idx = tid; idx < AM_CT * Wd; idx += NT) {
     const int t = idx / Wd, w = idx - t * Wd, r = r0 + min(t, nreg - 1);
-    mk[idx] = lv.reg_mask[(size_t)(lv.ids ? lv.ids[r] : lv.first + r) * Wd + w];
+    mk[idx] = lv.reg_mask[(size_t)(lv.first + r) * Wd + w];
   }
   for (int idx = tid; idx < AM_CN * net.E; idx += NT) {
     const int col = idx / net.E, e = idx - col * net.E, t = col >> 2, q = col & 3;
@@ -197,7 +197,7 @@ template <int NW>
 __global__ __launch_bounds__(64 * NW) void k_chain_tile_fp64(NetDev net, ChainIO io, int maxw) {
   const int r0 = blockIdx.x * AM_CT;
   if (r0 >= io.count) return;
-  const ChainLevel lv{io.first, io.count, io.ids, io.planes, io.eq, io.reg_mask, nullptr};
+  const ChainLevel lv{io.first, io.count, io.planes, io.eq, io.reg_mask, nullptr};
   chain_tile<NW>(net, io, lv, r0, min(AM_CT, io.count - r0), maxw);
 }
 template __global__ void k_chain_tile_fp64<4>(NetDev, ChainIO, int);

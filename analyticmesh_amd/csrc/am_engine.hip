@@ -172,7 +172,7 @@ struct am_ctx {
 
   // network (device)
   DevBuf<double> W0, ew, eb;
-  std::vector<DevBuf<double>> WT, Wrow, b, tm, tmT;
+  std::vector<DevBuf<double>> WT, Wrow, b, tm;
   std::vector<int> tm_h, tm_w;
   NetDev net{};
   FastNet fast{};
@@ -543,12 +543,11 @@ size_t ray64_lds_bytes(const am_ctx* c) {
          walk_rec_bytes(c->vm, false);
 }
 
-// The tiled chain's arguments for regions first .. first + n - 1 (or ids),
-// planes into the context's tile buffers with component stride Ch.
-ChainIO chain_io(const am_ctx* c, const int* ids, int first, int n, int Ch) {
+// The tiled chain's arguments for regions first .. first + n - 1, planes into the
+// context's tile buffers with component stride Ch.
+ChainIO chain_io(const am_ctx* c, int first, int n, int Ch) {
   ChainIO cio;
   cio.reg_mask = c->reg_mask.p;
-  cio.ids = ids;
   cio.first = first;
   cio.count = n;
   cio.Cs = Ch;
@@ -1289,7 +1288,7 @@ void batch_level_launch(am_batch* b, const BatchLevelPlan& pl, Fp64Counts& t) {
   for (long long cs = 0; cs < count; cs += (long long)chunk) {
     const int n = (int)std::min<long long>((long long)chunk, count - cs);
     const int rid0 = (int)(first + cs), ntile = batch_tiles(b, n);
-    const ChainLevel lv{rid0, n, nullptr, c->tplanes.p, c->teq.p, c->reg_mask.p, c->clock};
+    const ChainLevel lv{rid0, n, c->tplanes.p, c->teq.p, c->reg_mask.p, c->clock};
     if (cs > 0)   // (the level's first launch finds them cleared)
       hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, c->tcnt.p, (size_t)2, 0);
     // up to 64 networks one block finds their regions too
@@ -1597,17 +1596,13 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
     for (int li = 1; li < nl; ++li)
       upload_pad(c, c->WTp[li], c->bpad[li], wv[li], bv[li], c->nodes[li + 1], c->nodes[li], dtype, st);
     c->tm.resize(n_tm);
-    c->tmT.resize(n_tm);
     c->tm_h.assign(n_tm, 0);
     c->tm_w.assign(n_tm, 0);
     for (int t = 0; t < n_tm; ++t) {
       const int h = tm_shapes[2 * t], w = tm_shapes[2 * t + 1];
       c->tm_h[t] = h;
       c->tm_w[t] = w;
-      if (h > 0 && w > 0) {
-        upload(c, c->tm[t], tms[t], (size_t)h * w, dtype, st);
-        upload_T(c, c->tmT[t], tms[t], h, w, dtype, st);
-      }
+      if (h > 0 && w > 0) upload(c, c->tm[t], tms[t], (size_t)h * w, dtype, st);
     }
     // skip shape checks (backend/src/cuam.cpp:160-172)
     for (int li = 1; li < c->D; ++li)
@@ -1644,7 +1639,6 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
     }
     for (int t = 0; t < n_tm; ++t) {
       n.tm[t] = c->tm[t].p;
-      n.tmT[t] = c->tmT[t].p;
       n.tm_h[t] = c->tm_h[t];
       n.tm_w[t] = c->tm_w[t];
     }
@@ -1967,7 +1961,7 @@ long long newton_refine(am_ctx* c) {
   if (n > 0) {
     const int Ch = (c->C + 63) & ~63;
     hipLaunchKernelGGL(k_newton_fp64, dim3((unsigned)((n + AM_NT - 1) / AM_NT)), dim3(AM_NEWTON_THREADS),
-                       newton_lds_bytes(c->Wd), st, c->net, chain_io(c, nullptr, 0, 0, Ch), io);
+                       newton_lds_bytes(c->Wd), st, c->net, chain_io(c, 0, 0, Ch), io);
     HIPCHK(hipGetLastError());
   }
   hipLaunchKernelGGL(k_newton_scatter, dim3(blocks((size_t)N, 256)), dim3(256), 0, st, io, (const uint32_t*)w.table,
@@ -2460,7 +2454,7 @@ am_status am_adjoint(am_ctx* c, const void* grad_vertices, int dtype, void* cons
         const int maxw = chain_maxw(c);
         hipLaunchKernelGGL((maxw > 128 ? k_chain_tile_fp64<8> : k_chain_tile_fp64<4>), dim3((cnt + AM_CT - 1) / AM_CT),
                            dim3(maxw > 128 ? 512 : 256), chain_lds_bytes(c), st, c->net,
-                           chain_io(c, nullptr, r0, cnt, Ch), maxw);
+                           chain_io(c, r0, cnt, Ch), maxw);
         hipLaunchKernelGGL(k_adjoint_direct, dim3(cnt), dim3(64), lds, st, c->net, io, (const double*)c->tplanes.p,
                            (const double*)c->teq.p, Ch);
         HIPCHK(hipGetLastError());

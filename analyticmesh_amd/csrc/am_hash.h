@@ -44,18 +44,6 @@ __device__ __forceinline__ void commit_one(const CommitIO& io, size_t c, int ran
   io.table[io.slot[c]] = (uint32_t)rid;
 }
 
-// scan source: 1 for a candidate that becomes a region
-struct FirstSrc {
-  CommitIO io;
-  __device__ int operator()(size_t c) const { return first_flag(io, c); }
-};
-// scan sink that commits each new region as its rank is known
-struct CommitSink {
-  CommitIO io;
-  __device__ void operator()(size_t c, int prefix, int v) const {
-    if (v) commit_one(io, c, prefix);
-  }
-};
 __global__ void k_commit(CommitIO io, const int* rank, int n);
 
 // One-pass scan of the new-region flags of a level and the commit of the new

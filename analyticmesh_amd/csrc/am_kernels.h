@@ -90,7 +90,6 @@ inline size_t chain_tile_lds(int maxw, int Wd) {
 }
 struct ChainIO {
   const uint32_t* reg_mask;   // [R][Wd]
-  const int* ids;             // optional region ids; else first + tile-local index
   int first, count;           // regions of this launch
   int Cs;                     // stride of one component array in `planes` (>= C)
   double* planes;             // [count][4][Cs]: signed constraint planes, extras appended; entries of
@@ -99,10 +98,6 @@ struct ChainIO {
   const double* Wp[AM_MAX_LINEAR];  // li >= 1: W_li^T padded, [n_li][noutp[li]] (zero rows past n_out)
   const double* bp[AM_MAX_LINEAR];  // li >= 1: b_li padded to noutp[li]
   int noutp[AM_MAX_LINEAR];         // n_out rounded up to AM_CR
-  const int* dcount = nullptr;      // as in RegionIO: regions past *dcount - dbase are not valid
-  int dbase = 0;
-  const int2* lvl = nullptr;
-  int lvl_bound = 0;
 };
 
 // A list of chunk-local slots filled by atomics (cnt zeroed before), with
@@ -122,8 +117,7 @@ struct NearList {
 
 // The regions and plane buffers of one tiled-chain launch.
 struct ChainLevel {
-  int first, count;           // regions first .. first + count - 1 (or ids[0 .. count))
-  const int* ids;
+  int first, count;           // regions first .. first + count - 1
   double* planes;             // [count][4][Cs]
   double* eq;                 // [count][4]
   const uint32_t* reg_mask;   // [R][Wd]

@@ -38,7 +38,6 @@ struct NetDev {
   int skip_from[AM_MAX_LINEAR][AM_MAX_SKIPS];
   int skip_tm[AM_MAX_LINEAR][AM_MAX_SKIPS];
   const double* tm[AM_MAX_TMS];     // row-major (h, w) as given
-  const double* tmT[AM_MAX_TMS];    // transposed (w, h)
   int tm_h[AM_MAX_TMS];
   int tm_w[AM_MAX_TMS];
   const double* ew;                 // (E, 3)

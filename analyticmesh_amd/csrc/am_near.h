@@ -397,7 +397,6 @@ __device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, 
   plane(ql, pq);
   int ntab = 1, nv = 0;
   use(sl);
-  int tab1 = sl, tab2 = -1;           // the last two tab entries
   double lastv[3] = {0.0, 0.0, 0.0};
   bool vinacc = false;
   if (lane == 0) S.rec.tab[0] = start;
@@ -544,8 +543,6 @@ __device__ __forceinline__ int near_walk(const NetDev& net, const RegionIO& io, 
     nv += 1;
     ntab += 1;
     use(rl);
-    tab2 = tab1;
-    tab1 = rl;
     if (ntab >= 4 && rl == sl) break;       // closed
     if (ntab >= vm + 1) return SCAN ? NEAR_RETRY : (int)AM_WHY_BIT(AM_WHY_TRUNC);
     const int nx = next.take();
