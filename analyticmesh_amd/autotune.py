@@ -2,11 +2,11 @@
 
 Two shapes are chosen per network shape (widest hidden layer, depth):
 
-* ``ray_waves``: waves per region of the FP64 ray walk (2, 4 or 8).  More waves
-  split each region's constraint sweeps further but add block-wide
-  reductions; the best count depends on the number of constraints.
-* ``scan_blocks``: the grid of the candidate scan over the regions the ray
-  walk leaves undecided (a block-stride loop over a count the device holds).
+* ``ray_waves``: waves per region of the FP64 ray walk over all constraints (2, 4
+  or 8), which takes the regions the near walk leaves.  More waves split each
+  region's constraint sweeps further but add block-wide reductions.
+* ``scan_blocks``: the grid of the walks over the regions that the ones before
+  leave (a block-stride loop over a count the device holds).
 
 ``tune()`` marches the given workload once per candidate, reads the kernel time
 of the stage each shape affects from the engine's stage counters, checks

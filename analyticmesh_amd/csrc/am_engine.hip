@@ -1,10 +1,9 @@
 // Host side of the engine: the C-ABI of include/am.h.
 //
 // The marching loop is breadth first: a level is the set of regions found by
-// the previous level.  Per level the engine launches the region kernel (one
-// wave64 per region), inserts the level's neighbour candidates into the
-// visited set, and compacts the new regions into the region store, which
-// becomes the next level.  The reference instead pops LIFO batches of 1024
+// the previous level.  Per level the engine launches the plane and walk kernels,
+// inserts the level's neighbour candidates into the visited set, and compacts the
+// new regions into the region store, which becomes the next level.  The reference instead pops LIFO batches of 1024
 // (backend/src/cuam_kernel.cu:53-98); both orders reach the same regions.
 #include <cstring>
 #include <hip/hip_runtime.h>
@@ -1668,9 +1667,8 @@ am_status am_run(am_ctx* c, const void* const* weights, const void* const* biase
       }
     }
     prefix_setup(c, tms, dtype);
-    // The reduced forms need the tiled FP64 chain for their vertices and
-    // re-decisions; nets it does not take (skips, layers over 256 wide) run
-    // those forms on the FP64 region kernel, with the same topology.
+    // The reduced kernels take no skips and layers up to 256 wide; other nets run
+    // those forms on the FP64 planes alone, with the same topology.
     const bool reduced_asked = c->precision == AM_PREC_FP32 || c->precision == AM_PREC_SPLIT_BF16X3;
     // A reduced form whose vertices are all re-solved from FP64 planes (split
     // BF16; FP32 with reduced_vertices 0) marches on those planes: every region

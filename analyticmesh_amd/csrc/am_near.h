@@ -17,8 +17,8 @@
 // What bounds it: VALU issue and the planes' read (32 bytes per constraint).
 // The walks over all constraints read every plane once per vertex, from LDS
 // that leaves 4 to 6 regions per CU.  4x256 network, 1,022,340 regions, one
-// MI355X: candidate scan 75.3 -> 9.8 ms, FP64 ray walk 21.4 -> 9.3 ms, FP32 ray
-// walk 17.5 -> 10.9 ms; the trained 4x60 network (248,231 regions) 11.6 -> 3.6 ms.
+// MI355X: candidate scan 75.3 -> 9.3 ms, FP64 ray walk 21.4 -> 9.3 ms, FP32 ray
+// walk 17.5 -> 10.2 ms; the trained 4x60 network (248,231 regions) 11.6 -> 3.5 ms.
 // In small levels it is one region's serial chain: 21 us a level of 140 regions.
 #pragma once
 #include "am_device.h"

@@ -9,7 +9,8 @@
 // computes the planes of the ids that are new, and the walks find a region's
 // planes through the ids of its prefixes.  On the 4x256 network that is 29% of
 // the chain's arithmetic (1/16 + 4/16 + 9/16 of a layer's product per region
-// instead of 3).
+// instead of 3), and a third of it with what is done again: its 7.2 GB of planes
+// fill the storage, and the table starts over once or twice a march.
 //
 // The products run on the FP64 matrix cores in the canonical order:
 // v_mfma_f64_16x16x4f64 rounds like four fused multiply-adds in ascending k

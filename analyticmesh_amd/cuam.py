@@ -10,7 +10,8 @@ One process-wide context, as in the reference; create
 
 ``float_type`` selects the arithmetic: ``"float64"`` runs the FP64 form (the
 reference's default dtype); ``"float32"`` runs the FP32-MFMA form with FP64
-re-decision; ``"bf16x3"`` runs the split-BF16 MFMA form (float32 tensors);
+re-decision; ``"bf16x3"`` (float32 tensors) gives the split-BF16 MFMA planes through
+``Engine.planes`` and decides every region on the FP64 planes, as ``"fp64ray"`` does;
 ``"fp64ray"`` builds the FP64 planes and walks them with the checked FP64 ray
 walk, leaving only undecided regions to the candidate scan (float64 tensors).
 """

@@ -154,7 +154,7 @@ class Engine:
                  reduced_vertices="newton_where_needed"):
         """ray_waves / scan_blocks: launch shapes (see ``autotune``); None takes the tuned
         shape stored for the nearest network shape.  graph_levels: launch each level as one
-        captured hipGraph (every form; the stage times of the stats are then not taken).  reduced_vertices (fp32 form):
+        captured hipGraph (every form; not while other threads use the engine).  reduced_vertices (fp32 form):
         "newton_where_needed" (default) gives one FP64 Newton step after the march to each vertex
         solved from the reduced planes that the face kernel's error estimate does not put within
         1e-5 of |v|; "newton" gives every such vertex the step; "fp64" re-solves every vertex from

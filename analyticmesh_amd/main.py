@@ -218,8 +218,8 @@ def AnalyticMarching(model, save_ply_path="mesh.ply", iso=0.0, scale=1.0, center
     """Mesh the iso level set of ``model`` into ``save_ply_path`` (backend/main.py:335-559).
 
     ``precision`` (optional) overrides the arithmetic chosen by ``dtype``:
-    "fp64", "fp32" (FP32 MFMA + FP64 re-decision), "bf16x3" (split-BF16 MFMA) or
-    "fp64ray" (FP64 planes, checked FP64 ray walk, candidate scan where undecided).
+    "fp64", "fp32" (FP32 MFMA + FP64 re-decision), "fp64ray" (FP64 planes, checked FP64 ray
+    walk, candidate scan where undecided) or "bf16x3" (float32 tensors; decided as "fp64ray").
     Returns {"init_point_time", "init_cuda_time", "am_time", "export_time"} in seconds.
     """
     assert w_extra_constraints_.shape[0] == b_extra_constraints_.shape[0]

@@ -150,12 +150,14 @@ am_status am_topology_fingerprint(am_ctx* ctx, unsigned long long* out5);
  * processed, -1 = unlimited), "region_limit" (am_run fails with
  * AM_ERR_CAPACITY once more regions than this would be stored; -1 = the
  * engine's own limit, min(2^30, (2^31 - 1) / vm)), "ray_waves" (waves per
- * region of the FP64 ray walk: 2, 4 (default) or 8; the records do not depend
- * on it), "scan_blocks" (grid of the candidate scan over the regions the ray
- * walk leaves undecided, default 2048), "graph_levels" (1: each breadth-first
+ * region of the FP64 ray walk over all constraints, which takes the regions that
+ * the near walk leaves: 2, 4 (default) or 8; the records do not depend on it),
+ * "scan_blocks" (grid of the walks over the regions that the ones before leave,
+ * default 2048), "graph_levels" (1: each breadth-first
  * level's launches, every form, are captured into a hipGraph and launched as
- * one; the executable graph is updated in place from level to level; the
- * per-stage kernel times of the stats are not taken then),
+ * one; the executable graph is updated in place from level to level.  Not while
+ * other threads use the engine or the null stream: what they do there ends a
+ * capture under way, and am_run fails with AM_ERR_HIP),
  * "walk" (0 ray walk, 1
  * candidate scan, for the reduced forms), "ray_waves_reduced" (waves per
  * region of the reduced forms' ray walk: 2, 4 (default) or 8; 4 measured
@@ -180,7 +182,7 @@ am_status am_set_option(am_ctx* ctx, const char* key, long long value);
 /* Timings and counters of the last am_run/am_combine; see AM_STAT_* indices.  Stage times are
  * taken on the device (the Newton step's by events). */
 #define AM_STAT_RUN_MS 0        /* am_run wall time, seeds in -> records in device memory */
-#define AM_STAT_REGION_MS 1     /* region kernels */
+#define AM_STAT_REGION_MS 1     /* planes and walks (the reduced FP32 ones, without the FP64 redo) */
 #define AM_STAT_INSERT_MS 2     /* visited-set insertion + compaction */
 #define AM_STAT_GEMM_MS 3       /* plane GEMM kernels (the FP32 form; the plane stage of the others) */
 #define AM_STAT_WALK_MS 4       /* walk kernels after the GEMM (the FP32 form's; the FP64 ones of the others) */
@@ -192,18 +194,18 @@ am_status am_set_option(am_ctx* ctx, const char* key, long long value);
 #define AM_STAT_COMBINE_MS 10
 #define AM_STAT_REGION_LAUNCHES 11
 #define AM_STAT_ADJOINT_MS 12   /* am_adjoint kernels (wall time) */
-#define AM_STAT_CHAIN64_MS 13   /* FP64 tiled plane chain, all launches */
-#define AM_STAT_WALK64_MS 14    /* FP64 walk after the tiled chain, all launches */
+#define AM_STAT_CHAIN64_MS 13   /* FP64 planes (shared by activation prefix; batches: the tiled chain) */
+#define AM_STAT_WALK64_MS 14    /* FP64 candidate scan, with the near walk that takes its decisions */
 #define AM_STAT_SETUP_MS 15     /* am_run set-up: weight uploads and operand layouts (wall time) */
 #define AM_STAT_WHY0 16         /* 16..27: regions the reduced-precision walk left to FP64, per reason:
                                    seed shot, start edge, plane already in polygon, sign within bound,
                                    proposed vertex infeasible, ill-conditioned system, turn within bound,
                                    vertex cap, open edge, orientation within bound, candidate scan,
                                    same vertex */
-#define AM_STAT_RAY64_MS 28     /* FP64 checked ray walk */
+#define AM_STAT_RAY64_MS 28     /* FP64 checked ray walk, with the near walk that takes its decisions */
 #define AM_STAT_SCAN64_REGIONS 29 /* regions decided by the FP64 candidate scan */
 #define AM_STAT_RAY64_UNDECIDED 30 /* regions the FP64 ray walk left to the scan */
-#define AM_STAT_CHAIN64_LAUNCHES 31 /* launches of the FP64 tiled chain */
+#define AM_STAT_CHAIN64_LAUNCHES 31 /* launches of the FP64 plane stage (one or more a level) */
 #define AM_STAT_VERT64_MS 32    /* FP64 vertex re-solve of regions the reduced-precision walk decided */
 #define AM_STAT_VERT64_REGIONS 33 /* regions whose vertices were re-solved from FP64 planes */
 #define AM_STAT_FP64_ONLY 34    /* 1: a reduced form marched on FP64 planes alone (skips, layers over 256 wide, every vertex re-solved) */
